@@ -23,12 +23,8 @@
 using namespace hr;
 
 namespace {
-// element layers per z-chunk: fused tile classes (sweep of 3..8 at 64x64x32: 7 first) and
-// split path (chunks from the regular domain's bottom; sweep of 5..26 at 64x64x32, PML 6:
-// 10 first, 9 and 13 3 % and 14 % slower)
+// element layers per z-chunk of the fused tile classes (sweep of 3..8 at 64x64x32: 7 first)
 constexpr int DEFAULT_TZ = 7;
-constexpr int DEFAULT_TZ_SPLIT = 10;
-int default_tz(int version) { return version == 4 ? DEFAULT_TZ_SPLIT : DEFAULT_TZ; }
 constexpr int DEFAULT_TY = 3;
 constexpr int DEFAULT_VERSION = 4;   // 4 = split stage path, 3 = fused tile classes
 
@@ -73,7 +69,7 @@ struct hr_ctx {
   // state (device, 9*NN each)
   double* x[3] = {nullptr, nullptr, nullptr};
   double* y[3] = {nullptr, nullptr, nullptr};
-  double* gs[3] = {nullptr, nullptr, nullptr};
+  double* gs[3] = {nullptr, nullptr, nullptr};   // a1, a2, a3 of an RK4 step
   double* tmp = nullptr;                    // lattice scratch for hr_apply
   double* tmp2 = nullptr;
   Shell shell[3];
@@ -154,20 +150,18 @@ struct hr_ctx {
   // path: on the second side stream), so that it runs beside the stage kernels
   // instead of between stages.  The next launch_stage consumes it.
   std::vector<std::function<int()>> deferred;
-  // split stage path (version 4): the PML nodes' positions in lattice order (host;
-  // the kernels walk that order without a list), the tile list of its
-  // regular-domain kernel (the mixed and regular-domain tiles), the flux records
-  // and interface sums of split_shots shots, source entries by pull block
-  std::vector<std::pair<long long, int>> pnode_pos;   // (lattice index, position in lattice order), by lattice index
+  // split stage path (version 4): the flux records and interface sums of
+  // split_shots shots, source entries by pull block and at regular-domain-only nodes
   bool split_ok = false;                      // the lattice fits the split path
   int pnblk = 0;                              // SPLIT_NT-node blocks of the PML nodes (nodal pull)
   int pnblk_nodal = 0;                        // SPLIT_OWN-node blocks of the PML nodes (nodal pass)
-  int* d_tl_split = nullptr;
-  int ntl_split = 0;
   double* d_D = nullptr;
-  double* d_E = nullptr;
+  double* d_E = nullptr;                      // two fields: 3 NN doubles per shot each
   int split_shots = 0;
-  int *d_psrc_ptr = nullptr, *d_psrc_idx = nullptr, *d_prec_ptr = nullptr, *d_prec_idx = nullptr;
+  int rd_tz = 0;                              // layers per z-chunk of the element pass (0: rd_chunk's rule)
+  struct PullLists {
+    int *ptr = nullptr, *idx = nullptr, *slot = nullptr, *rd_idx = nullptr, *rd_shot = nullptr;
+  } pl_src, pl_rec;
   // stage-kernel version and tile-class lists
   int version = DEFAULT_VERSION;
   std::vector<int> zb;                      // z-chunk boundaries (element layers)
@@ -316,29 +310,53 @@ int upload(hr_ctx* ctx, T** d, const std::vector<T>& h) {
   return 0;
 }
 
-// Source entries at PML nodes by block of the split path's nodal pull: the
-// (shot, block) lists of entry indices, in entry order (ptr: the (shot, tile)
-// lists of nshot shots over nt tiles)
-int build_pull_blocks(hr_ctx* ctx, const std::vector<int>& ptr, const std::vector<long long>& node, int nshot, int nt,
-                      int** d_ptr, int** d_idx, Src3& h3) {
+// Source entries of the split path: those at PML nodes by (shot, block) of the
+// nodal pull, in node order, the others in (shot, node) order (ptr: the (shot,
+// tile) lists of nshot shots over nt tiles)
+int build_pull_lists(hr_ctx* ctx, const std::vector<int>& ptr, const std::vector<long long>& node, int nshot, int nt,
+                     hr_ctx::PullLists& pl, Src3& h3) {
+  const Geo& g = ctx->g;
   const int nblk = ctx->pnblk;
-  std::vector<std::pair<long long, int>> kv;
+  const int gh[2] = {g.rhi[0], g.rhi[1]};
+  struct Entry {
+    long long key;       // (shot, position in lattice order) of a PML node, (shot, node) of another
+    int jj, shot;
+  };
+  std::vector<Entry> pml, rd;
   for (int q = 0; q < nshot; ++q)
     for (int jj = ptr[(size_t)q * nt]; jj < ptr[(size_t)(q + 1) * nt]; ++jj) {
-      auto it = std::lower_bound(ctx->pnode_pos.begin(), ctx->pnode_pos.end(), std::make_pair(node[jj], -1));
-      if (it == ctx->pnode_pos.end() || it->first != node[jj]) continue;
-      kv.push_back({(long long)q * nblk + it->second / SPLIT_NT, jj});
+      const int i = (int)(node[jj] % g.NX), j = (int)((node[jj] / g.NX) % g.NY), k = (int)(node[jj] / ((long long)g.NX * g.NY));
+      if (h_pml_node(g, i, j, k))
+        pml.push_back({(long long)q * nblk * SPLIT_NT + (long long)sp_pml_pos(i, j, k, g.NX, g.NY, g.rlo, gh), jj, q});
+      else
+        rd.push_back({(long long)q * g.NN + node[jj], jj, q});
     }
-  std::sort(kv.begin(), kv.end());
-  std::vector<int> bp((size_t)nshot * nblk + 1, 0), idx;
-  for (auto& e : kv) { bp[e.first + 1]++; idx.push_back(e.second); }
+  auto less = [](const Entry& a, const Entry& b) { return a.key != b.key ? a.key < b.key : a.jj < b.jj; };
+  std::sort(pml.begin(), pml.end(), less);
+  std::sort(rd.begin(), rd.end(), less);
+  std::vector<int> bp((size_t)nshot * nblk + 1, 0), idx, slot, ri, rs;
+  for (const Entry& e : pml) {
+    bp[e.key / SPLIT_NT + 1]++;
+    idx.push_back(e.jj);
+    slot.push_back((int)(e.key % SPLIT_NT));
+  }
   for (size_t b = 0; b + 1 < bp.size(); ++b) bp[b + 1] += bp[b];
-  if (int rc = upload(ctx, d_ptr, bp)) return rc;
-  if (int rc = upload(ctx, d_idx, idx)) return rc;
-  h3.pblk_ptr = *d_ptr;
-  h3.pblk_idx = *d_idx;
+  for (const Entry& e : rd) {
+    ri.push_back(e.jj);
+    rs.push_back(e.shot);
+  }
+  if (int rc = upload(ctx, &pl.ptr, bp)) return rc;
+  if (int rc = upload(ctx, &pl.idx, idx)) return rc;
+  if (int rc = upload(ctx, &pl.slot, slot)) return rc;
+  if (int rc = upload(ctx, &pl.rd_idx, ri)) return rc;
+  if (int rc = upload(ctx, &pl.rd_shot, rs)) return rc;
+  h3.pblk_ptr = pl.ptr;
+  h3.pblk_idx = pl.idx;
+  h3.pblk_slot = pl.slot;
   h3.pnblk = nblk;
-  h3.ptop = idx.empty() ? 0 : 1;
+  h3.rd_idx = pl.rd_idx;
+  h3.rd_shot = pl.rd_shot;
+  h3.nrd = (int)ri.size();
   return 0;
 }
 
@@ -420,38 +438,68 @@ int drain_events(hr_ctx* ctx) {
   return 0;
 }
 
+Geo3 geo3(const hr_ctx* ctx) {
+  Geo3 o;
+  std::memset(&o, 0, sizeof(o));
+  const Geo& g = ctx->g;
+  o.NX = g.NX; o.NY = g.NY; o.NZ = g.NZ; o.NN = (int)g.NN;
+  o.nex = g.nex; o.ney = g.ney; o.nez = g.nez;
+  for (int a = 0; a < 3; ++a) o.rlo[a] = g.rlo[a];
+  o.rhi[0] = g.rhi[0]; o.rhi[1] = g.rhi[1];
+  o.top_rule = g.top_rule;
+  o.tiles0 = g.tiles[0]; o.tiles1 = g.tiles[1]; o.tz = g.tz;
+  for (size_t c = 0; c < ctx->zb.size() && c <= (size_t)HR_MAX_ZCHUNKS; ++c) o.zb[c] = ctx->zb[c];
+  for (int a = 0; a < 3; ++a) o.dxi[a] = g.dxi[a];
+  o.detj = g.detj;
+  return o;
+}
+
+// source parameters of a launch (Stage3Args, SplitArgs)
+template <class Args>
+void set_source(const hr_ctx* ctx, const Src3Spec* sp, Args& B) {
+  if (!(sp && sp->mode)) return;
+  B.src = *sp->lists; B.src_mode = sp->mode; B.ra = sp->ra; B.rb = sp->rb; B.ca = sp->ca; B.cb = sp->cb;
+  B.rb_on = sp->rb_on ? 1 : 0;
+  B.step = sp->step; B.fcol = sp->fcol;
+  B.step_dev = ctx->dyn ? ctx->d_step : nullptr;
+}
+
 Stage3Args args3(hr_ctx* ctx, const StageArgs& A, const Src3Spec* sp) {
   Stage3Args B;
   std::memset(&B, 0, sizeof(B));
-  const Geo& g = ctx->g;
-  B.g.NX = g.NX; B.g.NY = g.NY; B.g.NZ = g.NZ; B.g.NN = (int)g.NN;
-  B.g.nex = g.nex; B.g.ney = g.ney; B.g.nez = g.nez;
-  for (int a = 0; a < 3; ++a) B.g.rlo[a] = g.rlo[a];
-  B.g.rhi[0] = g.rhi[0]; B.g.rhi[1] = g.rhi[1];
-  B.g.top_rule = g.top_rule;
-  B.g.tiles0 = g.tiles[0]; B.g.tiles1 = g.tiles[1]; B.g.tz = g.tz;
-  for (size_t c = 0; c < ctx->zb.size() && c <= (size_t)HR_MAX_ZCHUNKS; ++c) B.g.zb[c] = ctx->zb[c];
-  for (int a = 0; a < 3; ++a) B.g.dxi[a] = g.dxi[a];
-  B.g.detj = g.detj;
+  B.g = geo3(ctx);
   for (int q = 0; q < 6; ++q) B.in[q] = A.in[q];
   B.out = A.out;
   for (int q = 0; q < 3; ++q) B.xnew[q] = A.xnew[q];
   B.node = ctx->d_node;
   B.tab = ctx->d_tab;
-  B.minvu = ctx->d_minvu;
-  B.rwp = ctx->d_rwp;
   B.set_mask = A.set_mask;
-  B.hh = A.hh; B.h = A.h; B.h6 = A.h6;
-  if (sp && sp->mode) {
-    B.src = *sp->lists; B.src_mode = sp->mode; B.ra = sp->ra; B.rb = sp->rb; B.ca = sp->ca; B.cb = sp->cb;
-    B.rb_on = sp->rb_on ? 1 : 0;
-    B.step = sp->step; B.fcol = sp->fcol;
-    B.step_dev = ctx->dyn ? ctx->d_step : nullptr;
-  }
+  B.hh = A.hh; B.h = A.h; B.h6 = A.h6; B.h4 = A.h4;
+  set_source(ctx, sp, B);
   // stage launches over the state buffers cover every shot; hr_apply works on one field
   B.nshot = A.stage > 0 ? ctx->nshot : 1;
   B.shot_stride = (long long)field_size(ctx);
   return B;
+}
+
+// Element layers per z-chunk of the split path's element pass.  A block marches
+// up its chunk and computes one halo layer below it; 512 blocks (two per CU) run
+// at a time.  The chunk is the one with the fewest layers in sequence, rounds of
+// blocks times layers per block; of equals the longest, which repeats the
+// fewest halo layers.
+int rd_chunk(const hr_ctx* ctx, int nshot) {
+  if (ctx->rd_tz > 0) return ctx->rd_tz;
+  const int layers = ctx->g.nez - ctx->g.rlo[2];
+  long long best = -1;
+  int tz = layers;
+  for (int c = layers; c >= 1; --c) {
+    int t[3];
+    rd_tiles(ctx->g, c, t);
+    const long long rounds = ((long long)t[0] * t[1] * t[2] * nshot + 511) / 512;
+    const long long cost = rounds * (c + (t[2] > 1 ? 1 : 0));
+    if (best < 0 || cost < best) { best = cost; tz = c; }
+  }
+  return tz;
 }
 
 // queue the deferred per-step work on the main stream (in the order it was deferred)
@@ -469,7 +517,12 @@ int launch_stage(hr_ctx* ctx, StageArgs& A, const Src3Spec* sp = nullptr) {
   if (counted) ctx->prof_all[A.stage] += 1;
   const bool prof = counted && (ctx->prof_tick++ % PROF_PERIOD) == 0;
   const bool split = ctx->version == 4 && A.stage >= 1 && A.stage <= 4;
-  hr_ctx::StageEv ev{A.stage, ctx->concurrent ? (split ? 2 : 3) : 1, {nullptr, nullptr, nullptr}, {nullptr, nullptr, nullptr}};
+  // the split path runs its two kernels of stages 1 and 3 side by side where the
+  // nodal pass has more blocks than the GPU's CUs; below that the event waits cost
+  // more than the overlap gives (16x16x8: 17.9 ms against 22.5 ms per 200 steps,
+  // 70 blocks; 37x29x19: equal, 480 blocks)
+  const bool fork = ctx->concurrent && (A.stage & 1) && (long long)ctx->pnblk_nodal * ctx->nshot > 384;
+  hr_ctx::StageEv ev{A.stage, !ctx->concurrent ? 1 : (!split ? 3 : (fork ? 2 : 1)), {nullptr, nullptr, nullptr}, {nullptr, nullptr, nullptr}};
   if (prof) {
     if (ctx->ev_open.size() >= 4096) if (int rc = drain_events(ctx)) return rc;
     for (int q = 0; q < ev.n; ++q) {
@@ -489,26 +542,57 @@ int launch_stage(hr_ctx* ctx, StageArgs& A, const Src3Spec* sp = nullptr) {
       return fail(ctx, 3, "stage sign pattern not supported by the v3 kernel");
     if (A.nsrc_tiles && !(sp && sp->mode)) return fail(ctx, 3, "v3 stage launch without its source lists");
     if (split) {
-      // nodal pass (main stream) beside the regular-domain kernel (side stream),
-      // then the nodal pull, which reads the interface sums of the latter
-      Stage3Args B = args3(ctx, A, sp);
+      SplitArgs B;
+      std::memset(&B, 0, sizeof(B));
+      B.g = geo3(ctx);
+      B.nshot = ctx->nshot;
+      B.shot_stride = (long long)field_size(ctx);
       if (ctx->split_shots < B.nshot || !ctx->d_D || !ctx->split_ok)
         return fail(ctx, 3, "split stage path without its buffers for %d shots", B.nshot);
+      const bool last = A.stage == 4;
+      for (int a = 0; a < 3; ++a) { B.v[a] = A.in[a]; B.x[a] = A.in[3 + a]; }
+      B.xn[0] = A.xnew[0]; B.xn[1] = A.xnew[1];
+      B.out = last ? A.xnew[2] : A.out;
+      B.node = ctx->d_node; B.tab = ctx->d_tab; B.minvu = ctx->d_minvu; B.rwp = ctx->d_rwp;
+      set_source(ctx, sp, B);
+      B.h = A.h; B.h2 = A.hh; B.h3 = A.h6; B.h4 = A.h4;
+      B.sc = last ? A.h4 : 1.0;
+      B.pnb = ctx->pnblk; B.pnbn = ctx->pnblk_nodal;
       B.D = ctx->d_D;
-      B.E = ctx->d_E;
-      // all node blocks
-      Stage3Args Ball = B;
-      Ball.pb0 = 0;
-      Ball.pnb = ctx->pnblk;
-      Ball.pnbn = ctx->pnblk_nodal;
-      if (ctx->concurrent) {
+      // the element pass before stages 1 and 3 forms the interface sums of two stages
+      const size_t ne = 3 * (size_t)ctx->g.NN * ctx->split_shots;
+      double* const E[2] = {ctx->d_E, ctx->d_E + ne};
+      B.E = E[(A.stage - 1) & 1];
+      const bool elements = A.stage == 1 || A.stage == 3;
+      RdArgs R;
+      if (elements) {
+        std::memset(&R, 0, sizeof(R));
+        R.g = B.g;
+        int t[3];
+        R.tz = rd_chunk(ctx, B.nshot);
+        rd_tiles(ctx->g, R.tz, t);
+        R.ntx = t[0]; R.nty = t[1]; R.ntz = t[2];
+        const bool update = A.stage == 3;
+        // K inputs of this stage and the next: x2, x3, then a1, a2
+        R.in[0] = update ? ctx->gs[0] : ctx->x[1];
+        R.in[1] = update ? ctx->gs[1] : ctx->x[2];
+        R.x[0] = ctx->x[1]; R.x[1] = ctx->x[2];
+        R.out[0] = update ? ctx->y[1] : ctx->gs[0];
+        R.out[1] = update ? ctx->y[2] : ctx->gs[1];
+        R.E[0] = E[0]; R.E[1] = E[1];
+        R.node = ctx->d_node; R.minvu = ctx->d_minvu;
+        R.nshot = B.nshot; R.shot_stride = B.shot_stride;
+        R.h = A.h; R.h2 = A.hh; R.h3 = A.h6; R.h4 = A.h4;
+      }
+      const int upd = A.stage == 3 ? 1 : 0;
+      if (fork) {
         // the nodal pass on a side stream, the deferred per-step kernels on the
-        // other, the regular-domain kernel (the longer one) on the main stream,
-        // which then runs the pull once both side streams have joined
+        // other, the element pass on the main stream, which then runs the pull
+        // once the side streams have joined
         HIPC(hipEventRecord(ctx->ev_fork, ctx->stream));
         HIPC(hipStreamWaitEvent(ctx->cstream[0], ctx->ev_fork, 0));
         if (prof) HIPC(hipEventRecord(ev.start[1], ctx->cstream[0]));
-        HIPC(launch_split_nodal(Ball, A.stage, A.transpose, ctx->cstream[0]));
+        HIPC(launch_split_nodal(B, last, A.transpose, ctx->cstream[0]));
         if (prof) HIPC(hipEventRecord(ev.end[1], ctx->cstream[0]));
         HIPC(hipEventRecord(ctx->ev_join[0], ctx->cstream[0]));
         const bool side_work = !ctx->deferred.empty();
@@ -523,19 +607,17 @@ int launch_stage(hr_ctx* ctx, StageArgs& A, const Src3Spec* sp = nullptr) {
           HIPC(hipEventRecord(ctx->ev_join[1], ctx->cstream[1]));
         }
         if (prof) HIPC(hipEventRecord(ev.start[0], ctx->stream));
-        HIPC(launch_split_rd(B, A.stage, A.transpose, ctx->d_tl_split, ctx->ntl_split, ctx->stream));
+        HIPC(launch_rd_pair(R, upd, ctx->stream));
         HIPC(hipStreamWaitEvent(ctx->stream, ctx->ev_join[0], 0));
         if (side_work) HIPC(hipStreamWaitEvent(ctx->stream, ctx->ev_join[1], 0));
-        HIPC(launch_split_pull(Ball, A.stage, A.transpose, ctx->stream));
-        if (prof) HIPC(hipEventRecord(ev.end[0], ctx->stream));
       } else {
         if (int rc = run_deferred(ctx)) return rc;
         if (prof) HIPC(hipEventRecord(ev.start[0], ctx->stream));
-        HIPC(launch_split_nodal(Ball, A.stage, A.transpose, ctx->stream));
-        HIPC(launch_split_rd(B, A.stage, A.transpose, ctx->d_tl_split, ctx->ntl_split, ctx->stream));
-        HIPC(launch_split_pull(Ball, A.stage, A.transpose, ctx->stream));
-        if (prof) HIPC(hipEventRecord(ev.end[0], ctx->stream));
+        if (elements) HIPC(launch_rd_pair(R, upd, ctx->stream));
+        HIPC(launch_split_nodal(B, last, A.transpose, ctx->stream));
       }
+      HIPC(launch_split_pull(B, A.transpose, ctx->stream));
+      if (prof) HIPC(hipEventRecord(ev.end[0], ctx->stream));
       if (prof) ctx->ev_open.push_back(ev);
       return 0;
     }
@@ -581,20 +663,15 @@ int setup_tiles(hr_ctx* ctx) {
   Geo& g = ctx->g;
   g.tiles[0] = (g.nex + g.tx - 1) / g.tx;
   g.tiles[1] = (g.ney + g.ty - 1) / g.ty;
-  // z-chunks of tz element layers (the v3 kernel reads the boundaries, so chunks could differ;
-  // for the fused tile classes, aligning one with the bottom PML interface measured slower:
-  // PML-only slabs cost as much).  The split path's tile kernel covers regular-domain
-  // elements only: its chunks start at the regular domain's bottom layer (the layers
-  // below are one chunk, run by the fused kernels of single-operator applies only)
+  // z-chunks of tz element layers (the kernel reads the boundaries, so chunks could differ;
+  // aligning one with the bottom PML interface measured slower: PML-only slabs cost as much)
   std::vector<int>& zb = ctx->zb;
   zb.assign(1, 0);
-  const int z0 = (ctx->version == 4 && g.rlo[2] > 0 && g.rlo[2] < g.nez) ? g.rlo[2] : 0;
-  if (z0 > 0) zb.push_back(z0);
-  for (int z = z0 + g.tz; z < g.nez; z += g.tz) zb.push_back(z);
+  for (int z = g.tz; z < g.nez; z += g.tz) zb.push_back(z);
   zb.push_back(g.nez);
   if ((int)zb.size() - 1 > HR_MAX_ZCHUNKS) return fail(ctx, 1, "too many z-chunks (%d); raise tz", (int)zb.size() - 1);
   g.tiles[2] = (int)zb.size() - 1;
-  std::vector<int> lists[3], rd_any;
+  std::vector<int> lists[3];
   const int nt = ntiles(g);
   // list order: x fastest, then z, then y, so that the z-neighbour whose top slab is a
   // chunk's halo slab runs on the same XCD soon after (measured 2 % faster than x, y, z)
@@ -609,7 +686,6 @@ int setup_tiles(hr_ctx* ctx) {
           if (rd) has_rd = true; else has_pml = true;
         }
     lists[(has_rd && has_pml) ? 0 : (has_rd ? 1 : 2)].push_back(b);
-    if (has_rd) rd_any.push_back(b);
   }
   // Each XCD (blockIdx mod 8) takes a contiguous run of a class list.  A Morton order of the
   // runs measured more fabric traffic.
@@ -617,11 +693,6 @@ int setup_tiles(hr_ctx* ctx) {
     ctx->ntl[c] = (int)lists[c].size();
     if (int rc = upload(ctx, &ctx->d_tl[c], lists[c])) return rc;
   }
-  // the split path's regular-domain kernel runs every tile with a regular-domain
-  // element, in the same traversal order, so that each XCD's contiguous run mixes
-  // interface and interior tiles as the domain does
-  ctx->ntl_split = (int)rd_any.size();
-  if (int rc = upload(ctx, &ctx->d_tl_split, rd_any)) return rc;
   // per-tile source lists of an earlier forward no longer match the tiles
   ctx->have_src = false;
   ctx->f_nstep = 0;
@@ -642,7 +713,7 @@ int check_ready(hr_ctx* ctx) {
 // stay zero (the pull reads them)
 int ensure_split(hr_ctx* ctx) {
   if (ctx->version != 4 || ctx->split_shots >= ctx->shot_cap) return 0;
-  const size_t nd = 12 * (size_t)ctx->g.NN * ctx->shot_cap, ne = 3 * (size_t)ctx->g.NN * ctx->shot_cap;
+  const size_t nd = 12 * (size_t)ctx->g.NN * ctx->shot_cap, ne = 6 * (size_t)ctx->g.NN * ctx->shot_cap;
   if (int rc = dalloc(ctx, &ctx->d_D, nd)) return rc;
   if (int rc = dalloc(ctx, &ctx->d_E, ne)) return rc;
   HIPC(hipMemsetAsync(ctx->d_D, 0, nd * sizeof(double), ctx->stream));
@@ -674,20 +745,23 @@ int zero_state(hr_ctx* ctx) {
   return 0;
 }
 
-// One RK4 step of every shot on (x) -> (y), then swap.  dir = +1 forward, -1 adjoint.
+// One RK4 step of every shot on (x) -> (y), then swap.  dir = +1 forward, -1
+// adjoint.  Stage s reads the vectors s .. s + 2 of x1, x2, x3, a1, a2, a3
+// (hr_split.hip gives the scheme); the last one writes the new state.
 int rk4_step(hr_ctx* ctx, double dt, int dir, int transpose, const double sgn[3], const Src3Spec* sp4) {
-  const double hh = dir * (0.5 * dt), h = dir * dt, h6 = dir * (dt / 6.0);
+  const double h = dir * dt;
+  double* const z[6] = {ctx->x[0], ctx->x[1], ctx->x[2], ctx->gs[0], ctx->gs[1], ctx->gs[2]};
   for (int s = 1; s <= 4; ++s) {
     StageArgs A = base_args(ctx);
     A.stage = s;
     A.set_mask = 7;
     A.transpose = transpose;
     for (int a = 0; a < 3; ++a) A.sgn[a] = sgn[a];
-    A.hh = hh; A.h = h; A.h6 = h6;
-    A.in[0] = ctx->x[0]; A.in[1] = ctx->x[1]; A.in[2] = ctx->x[2];
-    A.in[3] = ctx->gs[0]; A.in[4] = ctx->gs[1]; A.in[5] = ctx->gs[2];
+    A.h = h; A.hh = 0.5 * h * h; A.h6 = h * h * h / 6.0; A.h4 = h * h * h * h / 24.0;
+    for (int a = 0; a < 3; ++a) A.in[a] = z[s - 1 + a];
     if (s < 4) A.out = ctx->gs[s - 1];
-    else { A.xnew[0] = ctx->y[0]; A.xnew[1] = ctx->y[1]; A.xnew[2] = ctx->y[2]; }
+    else
+      for (int a = 0; a < 3; ++a) { A.in[3 + a] = ctx->x[a]; A.xnew[a] = ctx->y[a]; }
     if (sp4 && sp4[s - 1].mode) A.nsrc_tiles = 1;
     if (int rc = launch_stage(ctx, A, sp4 ? &sp4[s - 1] : nullptr)) return rc;
   }
@@ -716,11 +790,11 @@ int store_slice(hr_ctx* ctx, double* base, size_t rows, size_t row) {
   return 0;
 }
 
-// forward sources of step n: B values times f(T), f(T + dt/2), f(T + dt)
+// forward sources of step n: B values times s1, s2, s4 of the stages (stage 3 has none)
 void forward_sources(hr_ctx* ctx, int n, Src3Spec sp4[4]) {
   for (int s = 0; s < 4; ++s) {
     sp4[s] = Src3Spec();
-    if (!ctx->have_src) continue;
+    if (!ctx->have_src || s == 2) continue;
     sp4[s].lists = &ctx->src3_fwd;
     sp4[s].mode = 1;
     sp4[s].step = n;
@@ -884,7 +958,7 @@ int hr_ctx_create(const hr_mesh_desc* d, hr_ctx** out) {
   g.top_rule = d->top_stress_bc ? 1 : 0;
   g.tx = 4;
   g.ty = DEFAULT_TY;
-  g.tz = default_tz(ctx->version);
+  g.tz = DEFAULT_TZ;
   // affine element: DJ = diag(h/2); DETJ and DJI as in ELEMENT_K_3D
   const double j11 = d->h[0] * 0.5, j22 = d->h[1] * 0.5, j33 = d->h[2] * 0.5;
   const double detj = j11 * j22 * j33 + 0.0 * 0.0 * 0.0 + 0.0 * 0.0 * 0.0 - 0.0 * j22 * 0.0 - 0.0 * 0.0 * j11 - j33 * 0.0 * 0.0;
@@ -920,21 +994,14 @@ int hr_ctx_create(const hr_mesh_desc* d, hr_ctx** out) {
   // byte offsets use the fused tile classes
   if (96.0 * (double)g.NN < 4294967296.0) {
     // the nodal kernels walk the PML nodes in lattice order (sp_pml_node; measured
-    // 20 % faster per gradient than with the interface nodes last); their
-    // positions in that order, for the pull's per-block source lists
-    int pos = 0;
-    for (int k = 0; k < g.NZ; ++k)
-      for (int j = 0; j < g.NY; ++j)
-        for (int i = 0; i < g.NX; ++i)
-          if (h_pml_node(g, i, j, k)) ctx->pnode_pos.push_back({lat(g, i, j, k), pos++});
-    int gl[3] = {g.rlo[0], g.rlo[1], g.rlo[2]}, gh[2] = {g.rhi[0], g.rhi[1]};
-    if ((unsigned)pos != sp_pml_count(g.NX, g.NY, g.NZ, gl, gh)) return fail(ctx, 3, "PML node count mismatch");
+    // 20 % faster per gradient than with the interface nodes last)
+    const int gh[2] = {g.rhi[0], g.rhi[1]};
+    const int pos = (int)sp_pml_count(g.NX, g.NY, g.NZ, g.rlo, gh);
     ctx->pnblk = (pos + SPLIT_NT - 1) / SPLIT_NT;
     ctx->pnblk_nodal = (pos + SPLIT_OWN - 1) / SPLIT_OWN;
     ctx->split_ok = true;
   } else {
     ctx->version = 3;
-    g.tz = default_tz(ctx->version);
   }
   if (int rc = setup_tiles(ctx)) return rc;
   if (int rc = upload(ctx, &ctx->d_eq_slot, ctx->eq_slot)) return rc;
@@ -985,8 +1052,10 @@ int hr_ctx_destroy(hr_ctx* ctx) {
   F(ctx->d_obs_sorted);
   F(ctx->d_img); F(ctx->d_restr); F(ctx->d_reg); F(ctx->d_cost_el); F(ctx->d_red); F(ctx->d_pm); F(ctx->d_pg);
   for (int c = 0; c < 3; ++c) F(ctx->d_tl[c]);
-  F(ctx->d_tl_split); F(ctx->d_D); F(ctx->d_E);
-  F(ctx->d_psrc_ptr); F(ctx->d_psrc_idx); F(ctx->d_prec_ptr); F(ctx->d_prec_idx);
+  F(ctx->d_D); F(ctx->d_E);
+  for (hr_ctx::PullLists* pl : {&ctx->pl_src, &ctx->pl_rec}) {
+    F(pl->ptr); F(pl->idx); F(pl->slot); F(pl->rd_idx); F(pl->rd_shot);
+  }
   if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
   if (ctx->gexec) (void)hipGraphExecDestroy(ctx->gexec);
   if (ctx->graph) (void)hipGraphDestroy(ctx->graph);
@@ -1235,7 +1304,8 @@ int hr_set_tiling(hr_ctx* ctx, int ty, int tz, int version) {
   if (version) ctx->version = version;
   g.tx = 4;
   g.ty = t;
-  g.tz = tz ? tz : default_tz(ctx->version);
+  g.tz = tz ? tz : DEFAULT_TZ;
+  ctx->rd_tz = tz;
   if (int rc = ensure_split(ctx)) return rc;
   return setup_tiles(ctx);
 }
@@ -1243,7 +1313,7 @@ int hr_set_tiling(hr_ctx* ctx, int ty, int tz, int version) {
 int hr_get_tiling(hr_ctx* ctx, int* ty, int* tz, int* version) {
   if (!ctx) return 1;
   if (ty) *ty = ctx->g.ty;
-  if (tz) *tz = ctx->g.tz;
+  if (tz) *tz = ctx->version == 4 ? rd_chunk(ctx, ctx->nshot) : ctx->g.tz;
   if (version) *version = ctx->version;
   return 0;
 }
@@ -1444,6 +1514,16 @@ int forward_impl(hr_ctx* ctx, int nshot, int nstep, double dt, const double* fta
   ctx->ftab.resize(nft);
   if (dev && scheme == 0) HIPC(hipMemcpy(ctx->ftab.data(), ftab, nft * sizeof(double), hipMemcpyDeviceToHost));
   else std::memcpy(ctx->ftab.data(), ftab, nft * sizeof(double));
+  if (scheme == 0) {
+    // f0, fm, f1 of a step -> the sources of stages 1, 2 and 4 (hr_split.hip).  The
+    // differences come first: where they vanish, a small dt cannot make 0 x inf of them
+    for (size_t q = 0; q < (size_t)nstep * nshot; ++q) {
+      double* f = ctx->ftab.data() + 3 * q;
+      const double f0 = f[0], fm = f[1], f1 = f[2];
+      f[1] = 2.0 * (fm - f0) / dt;
+      f[2] = 4.0 * ((f0 - fm) + (f1 - fm)) / dt / dt / dt;
+    }
+  }
   if (ctx->ftab_cap < nft) {
     if (int rc = dalloc(ctx, &ctx->d_ftab, nft)) return rc;
     ctx->ftab_cap = nft;
@@ -1482,7 +1562,7 @@ int forward_impl(hr_ctx* ctx, int nshot, int nstep, double dt, const double* fta
     h3.tile_ptr = ctx->d_src_tile_ptr; h3.node = ctx->d_src_node; h3.comp = ctx->d_src_comp;
     h3.m = ctx->d_src_m; h3.val = ctx->d_src_val; h3.ftab = ctx->d_ftab; h3.nstep = nstep; h3.ntiles = nt;
     if (ctx->split_ok)
-      if (int rc = build_pull_blocks(ctx, ptr, node, nshot, nt, &ctx->d_psrc_ptr, &ctx->d_psrc_idx, h3)) return rc;
+      if (int rc = build_pull_lists(ctx, ptr, node, nshot, nt, ctx->pl_src, h3)) return rc;
     ctx->src3_fwd = h3;
     ctx->have_src = true;
   } else {
@@ -1757,8 +1837,7 @@ int hr_adjoint_gradient(hr_ctx* ctx, int nstep, double dt, int nrec, const long 
     h3.m = ctx->d_rec_m; h3.tr = ctx->d_tr_sorted; h3.obs = ctx->d_obs_sorted; h3.nrec = nrec;
     h3.nstep = nstep; h3.ntiles = ntiles(ctx->g);
     if (ctx->split_ok)
-      if (int rc = build_pull_blocks(ctx, rptr, rnode, nshot, h3.ntiles, &ctx->d_prec_ptr, &ctx->d_prec_idx, h3))
-        return rc;
+      if (int rc = build_pull_lists(ctx, rptr, rnode, nshot, h3.ntiles, ctx->pl_rec, h3)) return rc;
     ctx->src3_adj = h3;
   }
   if (nrec) {
@@ -1812,16 +1891,17 @@ int hr_adjoint_gradient(hr_ctx* ctx, int nstep, double dt, int nrec, const long 
         return 0;
       });
     }
-    // misfit sources at t_n (stage 1), t_{n-1} (stage 4), mean (stages 2, 3)
+    // misfit sources r(t_n), their mean with r(t_{n-1}) and r(t_{n-1}) over the step of
+    // -dt: s1 = r(t_n), s2 = (r(t_n) - r(t_{n-1})) / dt, s4 = 0 (the mean is exact)
     Src3Spec sp4[4];
     for (int st = 0; st < 4; ++st) {
       sp4[st] = Src3Spec();
-      if (!nrec) continue;
+      if (!nrec || st > 1) continue;
       sp4[st].lists = &ctx->src3_adj;
       sp4[st].mode = 2;
-      if (st == 0) { sp4[st].ra = n; sp4[st].ca = 1.0; }
-      else if (st == 3) { sp4[st].ra = n - 1; sp4[st].ca = 1.0; }
-      else { sp4[st].ra = n; sp4[st].ca = 0.5; sp4[st].rb = n - 1; sp4[st].cb = 0.5; sp4[st].rb_on = true; }
+      sp4[st].ra = n;
+      if (st == 0) sp4[st].ca = 1.0;
+      else { sp4[st].ca = 1.0 / dt; sp4[st].rb = n - 1; sp4[st].cb = -1.0 / dt; sp4[st].rb_on = true; }
     }
     use(P, PY);
     const int rc = rk4_step(ctx, dt, -1, 1, sgn, sp4);
@@ -1958,15 +2038,15 @@ int hr_autotune(hr_ctx* ctx, int nshot, int steps, int* tz_best, double* ms_per_
   hipEvent_t e0 = nullptr, e1 = nullptr;
   HIPC(hipEventCreate(&e0));
   HIPC(hipEventCreate(&e1));
-  const int tz0 = ctx->g.tz;
+  const int tz0 = ctx->g.tz, rd0 = ctx->rd_tz;
   const double sgn[3] = {1.0, 1.0, 1.0};
   double best = -1.0;
   int bt = tz0;
   int status = 0;
   // z-chunk candidates: element layers per chunk of the stage-kernel tiles
-  for (int tz : {3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 14}) {
+  for (int tz : {1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 16, 18, 20, 26, 32, 40}) {
     if (tz > ctx->g.nez) continue;
-    ctx->g.tz = tz;
+    ctx->g.tz = ctx->rd_tz = tz;
     if (setup_tiles(ctx) != 0) continue;      // too many chunks for this mesh
     // timed RK4 steps on the zero state without sources: the same launches and traffic
     if ((status = zero_state(ctx))) break;
@@ -1986,6 +2066,7 @@ int hr_autotune(hr_ctx* ctx, int nshot, int steps, int* tz_best, double* ms_per_
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   ctx->g.tz = status ? tz0 : bt;
+  ctx->rd_tz = status ? rd0 : bt;
   if (int rc = setup_tiles(ctx)) return rc;
   if (int rc = zero_state(ctx)) return rc;
   if (status) return status;

@@ -25,13 +25,13 @@ struct Geo {
 
 struct StageArgs {
   Geo g;
-  const double* in[6];             // stage: x1 x2 x3 g1 g2 g3; apply: in[0] = x
+  const double* in[6];             // as Stage3Args
   int stage;                       // 0 = apply (raw operator), 1..4 = RK4 stage, 5 = central difference
   int set_mask;                    // bit0: G on v1, bit1: K on v2, bit2: C on v3
   int transpose;                   // 1: apply the transposed operator
-  double sgn[3];                   // multipliers on v1, v2, v3
-  double hh, h, h6;                // 0.5 dt, dt, dt / 6 (signed); stage 5: dt^2, dt, dt^3
-  double* out;                     // stage 1-3: g_s; apply: raw result
+  double sgn[3];                   // multipliers on v1, v2, v3 (the kernels fix them by the transpose)
+  double h, hh, h6, h4;            // as Stage3Args
+  double* out;                     // stage 1-3: a_s; apply: raw result
   double* xnew[3];                 // stage 4: updated x1, x2, x3; stage 5: u_{n+1}, u_his
   int nsrc_tiles;                  // 0: no source
 };
@@ -126,22 +126,28 @@ struct Src3 {                      // device-resident source entries of one solv
   int nstep;
   int ntiles;
   // the same entries at PML nodes, by block of the nodal PML pull: entries of
-  // (shot, block) are pblk_idx[pblk_ptr[s*pnblk+b] .. pblk_ptr[s*pnblk+b+1])
+  // (shot, block) are pblk_idx[pblk_ptr[s*pnblk+b] .. pblk_ptr[s*pnblk+b+1]), in node
+  // order, pblk_slot their node's place in the block
   const int* pblk_ptr;
   const int* pblk_idx;
+  const int* pblk_slot;
   int pnblk;
-  int ptop;                        // some entry is at a PML node: the pull walks its block runs top-first
+  // and those at regular-domain-only nodes, in (shot, node) order
+  const int* rd_idx;
+  const int* rd_shot;
+  int nrd;
 };
 
 struct Stage3Args {
   Geo3 g;
-  const double* in[6];             // stage: x1 x2 x3 g1 g2 g3; apply: in[0] = x
-  double* out;                     // stage 1-3: g_s; apply: raw result
+  // RK4 stage: the operator inputs v1, v2, v3 (stage 1 x1 x2 x3, 2 x2 x3 a1, 3 x3 a1
+  // a2, 4 a1 a2 a3; hr_split.hip gives the scheme), stage 4 then x1, x2, x3;
+  // apply: in[0] = x; stage 5: u_n, u_{n-1}, u_his
+  const double* in[6];
+  double* out;                     // stage 1-3: a_s; apply: raw result
   double* xnew[3];                 // stage 4: updated x1, x2, x3; stage 5: u_{n+1}, u_his
   const double* node;              // node table
   const double* tab;               // small table
-  const double* minvu;             // split path: M^-1 of the displacement rows per node (NN)
-  const double* rwp;               // split path: sum of rho W over the PML elements per node (NN)
   Src3 src;                        // source entries, used when src_mode != 0
   int set_mask;                    // apply: bit0 G, bit1 K, bit2 C
   int src_mode;                    // 0 none, 1 forward: f * B * m, 2 adjoint misfit
@@ -151,30 +157,56 @@ struct Stage3Args {
   const int* step_dev;             // captured loops: step, ra, rb are offsets from *step_dev
   int nshot;                       // shots in the launch; state vectors are shot-major
   long long shot_stride;           // elements per shot of a state vector (9 NN)
-  double hh, h, h6;                // 0.5 dt, dt, dt / 6 (signed); stage 5: dt^2, dt, dt^3
-  // split stage path (RK4 stages): the nodal pull covers the SPLIT_NT-node
-  // blocks [pb0, pb0 + pnb) of the PML nodes in lattice order, the nodal pass its
-  // pnbn blocks of SPLIT_OWN nodes; the y- and z-line flux records D (12 NN
-  // doubles per shot) and the regular-domain K sums of interface nodes E (3 NN
-  // doubles per shot)
-  int pb0, pnb;
-  int pnbn;                        // blocks of the nodal pass (SPLIT_OWN list entries each)
-  double* D;
-  double* E;
+  double h, hh, h6, h4;            // stage 4: h, h^2/2, h^3/6, h^4/24 (h = +-dt); stage 5: h, hh, h6 = dt, dt^2, dt^3
+};
+
+// Split stage path (hr_split.hip): the nodal kernels of one RK4 stage
+struct SplitArgs {
+  Geo3 g;
+  const double* v[3];              // operator inputs
+  const double* x[3];              // last stage: the state
+  double* xn[2];                   // last stage: updated x1, x2
+  double* out;                     // a_s; last stage: updated x3
+  const double *node, *tab;        // node table (lambda, mu pairs), small table
+  const double *minvu, *rwp;       // M^-1 of the displacement rows, sum of rho W over the PML elements per node (NN each)
+  Src3 src;                        // as in Stage3Args
+  int src_mode, step, fcol, ra, rb, rb_on;
+  double ca, cb;
+  const int* step_dev;
+  int nshot;
+  long long shot_stride;
+  double h, h2, h3, h4;            // h, h^2/2, h^3/6, h^4/24
+  double sc;                       // scale of the stage's a in its output: 1, last stage h^4/24
+  int pnb, pnbn;                   // blocks of the pull (SPLIT_NT PML nodes) and of the nodal pass (SPLIT_OWN)
+  double* D;                       // y- and z-line flux records, 12 NN doubles per shot
+  const double* E;                 // regular-domain K sums of interface nodes, 3 NN doubles per shot
+};
+
+// and its regular-domain element pass over two fields
+struct RdArgs {
+  Geo3 g;
+  int ntx, nty, ntz, tz;           // tiles, element layers per z-chunk
+  const double* in[2];             // x2, x3 (update: a1, a2)
+  const double* x[2];              // update: x2, x3
+  double* out[2];                  // a1, a2 (update: new x2, x3)
+  double* E[2];                    // K sums of interface nodes per field
+  const double *node, *minvu;
+  int nshot;
+  long long shot_stride;
+  double h, h2, h3, h4;
 };
 
 // stage 0 = apply; transposed stages 1..4 carry the adjoint signs (-G, +K, -C)
 hipError_t launch_stage3(const Stage3Args& A, int stage, int transpose, int tile_class, const int* tiles, int ntiles,
                          hipStream_t s);
-// split stage path, RK4 stages 1..4: the nodal pass over the PML nodes (flux
-// records, node-local terms, stage-4 x1 x2), the regular-domain kernel over the
-// tiles with regular-domain elements (finishes regular-domain-only nodes, K
-// contribution of interface nodes into E) and the nodal pull over the PML nodes
+// split stage path: the nodal pass over the PML nodes, the nodal pull, and the
+// regular-domain element pass
 constexpr int SPLIT_NT = 256;
 // list entries a nodal-pass block owns: it also computes two entries on each
 // side, for the x flux records of its own entries' x-lines
 constexpr int SPLIT_OWN = SPLIT_NT - 4;      // nodes (threads) per block of the nodal kernels
-hipError_t launch_split_nodal(const Stage3Args& A, int stage, int transpose, hipStream_t s);
-hipError_t launch_split_rd(const Stage3Args& A, int stage, int transpose, const int* tiles, int ntiles, hipStream_t s);
-hipError_t launch_split_pull(const Stage3Args& A, int stage, int transpose, hipStream_t s);
+hipError_t launch_split_nodal(const SplitArgs& A, int last, int transpose, hipStream_t s);
+hipError_t launch_split_pull(const SplitArgs& A, int transpose, hipStream_t s);
+void rd_tiles(const Geo& g, int tz, int t[3]);   // element pass tiles per axis (x, y, z-chunks)
+hipError_t launch_rd_pair(const RdArgs& A, int update, hipStream_t s);
 }  // namespace hr

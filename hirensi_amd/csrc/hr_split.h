@@ -124,6 +124,19 @@ constexpr bool sp_pml_node(unsigned t, int NX, int NY, int NZ, const int lo[3], 
   return true;
 }
 
+// and back: the entry of PML node (i, j, k)
+constexpr unsigned sp_pml_pos(int i, int j, int k, int NX, int NY, const int lo[3], const int hi[2]) {
+  const unsigned nx = (unsigned)NX, nxy = nx * (unsigned)NY;
+  if (k <= 2 * lo[2]) return (unsigned)k * nxy + (unsigned)j * nx + (unsigned)i;
+  const unsigned ax = (unsigned)(2 * (hi[0] - lo[0]) - 1), ay = (unsigned)(2 * (hi[1] - lo[1]) - 1);
+  const unsigned base = (unsigned)(2 * lo[2] + 1) * nxy + (unsigned)(k - 2 * lo[2] - 1) * (nxy - ax * ay);
+  const unsigned R0 = (unsigned)(2 * lo[1] + 1) * nx, W = nx - ax;
+  if (j <= 2 * lo[1]) return base + (unsigned)j * nx + (unsigned)i;
+  if (j < 2 * hi[1])
+    return base + R0 + (unsigned)(j - 2 * lo[1] - 1) * W + (unsigned)(i <= 2 * lo[0] ? i : i - (int)ax);
+  return base + R0 + ay * W + (unsigned)(j - 2 * hi[1]) * nx + (unsigned)i;
+}
+
 // number of PML nodes
 constexpr unsigned sp_pml_count(int NX, int NY, int NZ, const int lo[3], const int hi[2]) {
   const unsigned nxy = (unsigned)NX * (unsigned)NY;

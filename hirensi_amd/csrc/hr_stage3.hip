@@ -4,9 +4,11 @@
 //
 // The operator is the one the reference assembles into AK, AC, AG
 // (Assemble_PETSc_3D.F90:6-436, element blocks Element_Matrices_3D.F90:7-882)
-// and the stage is the VecWAXPY/MatMultAdd sequence of
-// Solver_PETSc_Explicit.F90:1001-1046 (forward) and :1319-1364 (adjoint,
-// transposed with the signs -G, +K, -C).
+// and the stage is one of the four of Solver_PETSc_Explicit.F90:1001-1046 (forward)
+// and :1319-1364 (adjoint, transposed with the signs -G, +K, -C), taken as
+// successive time derivatives (the scheme is in hr_split.hip, which runs the RK4
+// stages by default; this kernel runs single operators, the central-difference
+// step, lattices too large for the split path and stage-kernel version 3).
 //
 // Work decomposition (same tiles as the v2 kernel): a workgroup owns TX x TY
 // elements in x-y and a chunk of tz element layers, and streams up the chunk
@@ -22,7 +24,7 @@
 //    (F[X][x] depends on y and z only, ...): 9 derivatives per element side
 //    instead of 27;
 //  * each owner thread loads its own node, keeps the diagonal terms (and for
-//    stage 4 x3 and the partial g-sum) in registers, and writes the x1, x2
+//    stage 4 the x3 carry) in registers, and writes the x1, x2
 //    updates of stage 4 at load time; helpers load the low-side halo;
 //  * state vectors keep a node's components contiguous (displacement block
 //    [3 n + c], then stress block [SB + 6 n + m], SB = 3 NN rounded up to
@@ -34,8 +36,7 @@
 
 #include <hip/hip_runtime.h>
 #include <type_traits>
-#include "hr_device.h"
-#include "hr_split.h"
+#include "hr_lattice.h"
 
 // Fused multiply-add is allowed here: the parity bar is a tolerance, and FMA
 // halves the FP64 instruction count of the stencils.
@@ -46,70 +47,6 @@ namespace {
 
 constexpr int NT3 = 256;
 constexpr int SRC_LDS = 64;   // source entries of a tile staged in LDS (more: read from memory)
-
-__device__ __forceinline__ void sto(double* p, unsigned off, double v) {
-  *reinterpret_cast<double*>(reinterpret_cast<char*>(p) + off) = v;
-}
-// two consecutive doubles at a 16-byte aligned offset
-__device__ __forceinline__ void ld2(const double* p, unsigned off, double& a, double& b) {
-  const double2 t = *reinterpret_cast<const double2*>(reinterpret_cast<const char*>(p) + off);
-  a = t.x;
-  b = t.y;
-}
-// three consecutive components of a node (8-byte aligned): one 16-byte and one
-// 8-byte access instead of three 8-byte ones
-struct alignas(8) D3 {
-  double v[3];
-};
-__device__ __forceinline__ void ld3(const double* p, unsigned off, double& a, double& b, double& c) {
-  const D3 t = *reinterpret_cast<const D3*>(reinterpret_cast<const char*>(p) + off);
-  a = t.v[0];
-  b = t.v[1];
-  c = t.v[2];
-}
-__device__ __forceinline__ void st3(double* p, unsigned off, double a, double b, double c) {
-  D3 t;
-  t.v[0] = a;
-  t.v[1] = b;
-  t.v[2] = c;
-  *reinterpret_cast<D3*>(reinterpret_cast<char*>(p) + off) = t;
-}
-// six consecutive components at a 16-byte aligned offset: three 16-byte stores
-__device__ __forceinline__ void st6(double* p, unsigned off, const double* v) {
-  char* q = reinterpret_cast<char*>(p) + off;
-#pragma unroll
-  for (int a = 0; a < 3; ++a) *reinterpret_cast<double2*>(q + 16 * a) = make_double2(v[2 * a], v[2 * a + 1]);
-}
-// stores of three consecutive components, each only where its bit of act is set
-__device__ __forceinline__ void st3m(double* p, unsigned off, int act, double a, double b, double c) {
-  if (act == 7) {
-    st3(p, off, a, b, c);
-  } else {
-    if (act & 1) sto(p, off, a);
-    if (act & 2) sto(p, off + 8u, b);
-    if (act & 4) sto(p, off + 16u, c);
-  }
-}
-
-__device__ __forceinline__ bool in_dom3(const Geo3& g, int i, int j, int k) {
-  return i >= 0 && j >= 0 && k >= 0 && i < g.NX && j < g.NY && k < g.NZ;
-}
-__device__ __forceinline__ bool u_act3(const Geo3& g, int i, int j, int k) {
-  return !(i == 0 || j == 0 || k == 0 || i == g.NX - 1 || j == g.NY - 1);
-}
-// node touched by at least one PML element
-__device__ __forceinline__ bool pml3(const Geo3& g, int i, int j, int k) {
-  return !(i > 2 * g.rlo[0] && i < 2 * g.rhi[0] && j > 2 * g.rlo[1] && j < 2 * g.rhi[1] && k > 2 * g.rlo[2]);
-}
-// active stress components (bit m) of a PML node
-__device__ __forceinline__ int smask3(const Geo3& g, int i, int j, int k) {
-  if (g.top_rule && k == g.NZ - 1 && !((i & 1) && (j & 1))) return 0x3f & ~((1 << 2) | (1 << 4) | (1 << 5));
-  return 0x3f;
-}
-__device__ __forceinline__ bool rd3(const Geo3& g, int ex, int ey, int ez) {
-  return ex >= g.rlo[0] && ex < g.rhi[0] && ey >= g.rlo[1] && ey < g.rhi[1] && ez >= g.rlo[2];
-}
-__device__ __forceinline__ int sym3(int i, int k) { return i == k ? i : i + k + 2; }
 
 // 3-point GLL rule on xi = -1, 0, 1: weights and DM(a, c) = l_c'(xi_a)
 __device__ __forceinline__ constexpr double gll_w(int a) { return a == 1 ? 4.0 / 3.0 : 1.0 / 3.0; }
@@ -145,9 +82,10 @@ __device__ __forceinline__ void axis_stencil(int i, int nel, double c[5], double
   }
 }
 
-// Stage-S inputs (v1, v2, v3) of one field component from its raw inputs X
-// (x1 x2 x3 g1 g2 g3; apply: x) in the reference's nested VecWAXPY order.
-// NEG: adjoint signs on v1, v3.  S = 5 is one step of the central-difference
+// Inputs (v1, v2, v3) of the G, K and C operators for one field component from
+// its raw inputs X.  NEG: adjoint signs on v1, v3.  The RK4 stages read the three
+// operator inputs as they are stored (hr_device.h, Stage3Args).  S = 0 (apply):
+// X[0] = x, the sets in mask.  S = 5 is one step of the central-difference
 // variant (X = u_n, u_{n-1}, u_his; hh = dt^2, h = dt, h6 = dt^3): the G, K
 // and C inputs whose operator sum, scaled by -M^-1, is that step's update.
 template <int S, bool NEG>
@@ -158,39 +96,18 @@ __device__ __forceinline__ void combine(const double* X, double hh, double h, do
     v2 = (mask & 2) ? X[0] : 0.0;
     v3 = (mask & 4) ? X[0] : 0.0;
     return;
-  } else if constexpr (S == 1) {
-    v1 = X[0]; v2 = X[1]; v3 = X[2];
-  } else if constexpr (S == 2) {
-    v1 = X[0] + hh * X[1]; v2 = X[1] + hh * X[2]; v3 = X[2] + hh * X[3];
-  } else if constexpr (S == 3) {
-    v1 = X[0] + hh * (X[1] + hh * X[2]); v2 = X[1] + hh * (X[2] + hh * X[3]); v3 = X[2] + hh * X[4];
   } else if constexpr (S == 5) {
     v1 = h6 * X[0] + hh * X[2]; v2 = hh * X[0]; v3 = h * (X[0] - X[1]);
   } else {
-    v1 = X[0] + h * (X[1] + hh * (X[2] + hh * X[3])); v2 = X[1] + h * (X[2] + hh * X[4]); v3 = X[2] + h * X[5];
+    v1 = X[0]; v2 = X[1]; v3 = X[2];
   }
   if constexpr (NEG) { v1 = -v1; v3 = -v3; }
 }
 
-// raw input q enters the K-set input v2 of stage S
+// raw input q enters the K-set input v2
 template <int S>
 __device__ __forceinline__ constexpr bool v2_input(int q) {
-  return S == 0 ? q == 0 : (S == 1 ? q == 1 : (S == 2 ? (q == 1 || q == 2) : (S == 3 ? (q >= 1 && q <= 3) : (S == 5 ? q == 0 : (q == 1 || q == 2 || q == 4)))));
-}
-
-// Stage-4 update of x1 and x2 (no g4 needed), and the x3 carry
-// c3 = x3 + dt/6 (g1 + 2 g2 + 2 g3), so that x3_new = c3 + dt/6 g4
-// (Solver_PETSc_Explicit.F90:1036-1046)
-__device__ __forceinline__ void rk4_update12(const double* X, double hh, double h, double h6, double& xn0, double& xn1,
-                                             double& c3) {
-  const double x1 = X[0], x2 = X[1], x3v = X[2], g1 = X[3], g2 = X[4], g3 = X[5];
-  const double k2t = x2 + hh * x3v, k3t = x2 + hh * (x3v + hh * g1), k4t = x2 + h * (x3v + hh * g2);
-  const double k2m = x3v + hh * g1, k3m = x3v + hh * g2, k4m = x3v + h * g3;
-  const double ht = 0.0 + (((1.0 * x2 + 2.0 * k2t) + 2.0 * k3t) + 1.0 * k4t);
-  const double hm = 0.0 + (((1.0 * x3v + 2.0 * k2m) + 2.0 * k3m) + 1.0 * k4m);
-  xn0 = x1 + h6 * ht;
-  xn1 = x2 + h6 * hm;
-  c3 = x3v + h6 * ((1.0 * g1 + 2.0 * g2) + 2.0 * g3);
+  return S == 0 || S == 5 ? q == 0 : q == 1;
 }
 
 template <int TX, int TY>
@@ -207,13 +124,10 @@ struct Shape3 {
 // register allocations that measured 6 %, 1.5 % and 2 % faster in the whole
 // gradient (the compiler reports the unmet targets).  At stage 4 the PML-only
 // class would then need more than 256 registers.
-// SPLIT (regular-domain class only): the kernel also runs the tiles that hold
-// PML elements, skips them, and leaves the PML nodes to the nodal kernels: their
-// stage-4 x1, x2 updates are not written here and their regular-domain K sums go
-// to A.E instead of being finished.
-template <int TX, int TY, bool HAS_RD, bool HAS_PML, int S, bool TR, bool SPLIT = false>
-__global__ void __launch_bounds__(NT3, HAS_RD ? (HAS_PML ? 3 : 5) : (S >= 1 && S <= 3 ? 3 : 2)) stage_kernel3(const Stage3Args A, const int* __restrict__ tiles, int ntl) {
-  static_assert(!SPLIT || (HAS_RD && !HAS_PML && S >= 1 && S <= 4), "split form: regular-domain RK4 stages");
+// S: 0 one operator, 1 the RK4 stages 1-3, 4 the last RK4 stage, 5 a
+// central-difference step.
+template <int TX, int TY, bool HAS_RD, bool HAS_PML, int S, bool TR>
+__global__ void __launch_bounds__(NT3, HAS_RD ? (HAS_PML ? 3 : 5) : (S == 1 ? 3 : 2)) stage_kernel3(const Stage3Args A, const int* __restrict__ tiles, int ntl) {
   using SH = Shape3<TX, TY>;
   constexpr int WX = SH::WX, WP = SH::WP, NEW = SH::NEW, OX = SH::OX, OC = SH::OC, HP = SH::HP;
   static_assert(OC <= 64 && NT3 == 256, "one owner plane group per wavefront, plus one helper wavefront");
@@ -274,9 +188,7 @@ __global__ void __launch_bounds__(NT3, HAS_RD ? (HAS_PML ? 3 : 5) : (S >= 1 && S
   const int gi0 = 2 * ex0 - 2, gj0 = 2 * ey0 - 2;
   const int own_i1 = (ex0 + TX >= g.nex) ? g.NX : 2 * (ex0 + TX);
   const int own_j1 = (ey0 + TY >= g.ney) ? g.NY : 2 * (ey0 + TY);
-  // split form: no regular-domain element lies below layer rlo[2], so the slabs
-  // under it hold no work for this kernel (their nodes are PML nodes)
-  const int ez_first = SPLIT ? max(max(ez0 - 1, 0), g.rlo[2]) : max(ez0 - 1, 0);
+  const int ez_first = max(ez0 - 1, 0);
   const int mask = (S == 0) ? A.set_mask : 7;
   const bool useG = mask & 1, useK = mask & 2, useC = mask & 4;
   const unsigned NN8 = (unsigned)g.NN * 8u;   // bytes of one double per lattice node
@@ -352,7 +264,7 @@ __global__ void __launch_bounds__(NT3, HAS_RD ? (HAS_PML ? 3 : 5) : (S >= 1 && S
   }
 
   // owner registers: accumulators, diagonal terms, stage-4 carry
-  // c3o: stage 4 x3 + dt/6 (g1 + 2 g2 + 2 g3); stage 5 2 u_n - u_{n-1}.  chs: stage 5 u_his
+  // c3o: stage 4 the x3 carry of rk4_update; stage 5 2 u_n - u_{n-1}.  chs: stage 5 u_his
   // acc starts at the node's diagonal terms (set when the owner loads its node)
   double acc[9], c3o[NS], chs[S == 5 ? NS : 1];
   double lam_o = 0.0, mu_o = 0.0, minvu_o = 0.0, minvs_o = 0.0;
@@ -367,12 +279,13 @@ __global__ void __launch_bounds__(NT3, HAS_RD ? (HAS_PML ? 3 : 5) : (S >= 1 && S
   // The loads of a node class are issued unconditionally, so that they leave
   // in one batch: inactive lattice entries are zero in every state vector and
   // never written, and contribute nothing.  Activity only gates the stores.
-  constexpr int NIN = (S == 0) ? 1 : (S == 5 ? 3 : 2 + S);   // x1 x2 x3 g1 g2 g3 prefix (apply: x)
   // COL: the node is in the lane's owner column (ii, jj = i, j) and its plane kk is
   // the same for the whole wavefront
   auto load = [&](auto own_tag, auto col_tag, int ii, int jj, int kk, int r, int slot, bool own_plane) {
     constexpr bool OWN = decltype(own_tag)::value;
     constexpr bool COL = decltype(col_tag)::value;
+    // raw inputs: the operator inputs (apply: x); owners of the last stage also the state x1, x2, x3
+    constexpr int NIN = (S == 0) ? 1 : ((S == 4 && OWN) ? 6 : 3);
     constexpr bool ALL_U = HAS_PML || (OWN && UPD);      // v1 and v3 of u, or the state update
     if constexpr (OWN) {
       // a newly loaded owned node starts its sums at its diagonal terms (zero off the PML)
@@ -415,10 +328,10 @@ __global__ void __launch_bounds__(NT3, HAS_RD ? (HAS_PML ? 3 : 5) : (S >= 1 && S
         }
       }
       if constexpr (OWN && S == 4) {
-        if (own_plane && ua && !(SPLIT && pml3(g, ii, jj, kk))) {
+        if (own_plane && ua) {
           double xn0[3], xn1[3];
 #pragma unroll
-          for (int c = 0; c < 3; ++c) rk4_update12(XU[c], A.hh, A.h, A.h6, xn0[c], xn1[c], c3o[c]);
+          for (int c = 0; c < 3; ++c) rk4_update(XU[c], A.h, A.hh, A.h6, A.h4, xn0[c], xn1[c], c3o[c]);
           st3(xnp[0], offu, xn0[0], xn0[1], xn0[2]);
           st3(xnp[1], offu, xn1[0], xn1[1], xn1[2]);
         }
@@ -544,7 +457,7 @@ __global__ void __launch_bounds__(NT3, HAS_RD ? (HAS_PML ? 3 : 5) : (S >= 1 && S
 #pragma unroll
                   for (int t = 0; t < 3; ++t) {
                     double c3v;
-                    rk4_update12(XS[t], A.hh, A.h, A.h6, xn0[t], xn1[t], c3v);
+                    rk4_update(XS[t], A.h, A.hh, A.h6, A.h4, xn0[t], xn1[t], c3v);
                     if constexpr (NS == 9) c3o[3 + 3 * hf + t] = c3v;
                   }
                   const int act = (sm >> (3 * hf)) & 7;
@@ -805,13 +718,6 @@ __global__ void __launch_bounds__(NT3, HAS_RD ? (HAS_PML ? 3 : 5) : (S >= 1 && S
         const unsigned n = (unsigned)i + (unsigned)g.NX * ((unsigned)j + (unsigned)g.NY * (unsigned)k);
         const unsigned offu = n * 24u, offs = SB + n * 48u;
         const bool ua = u_act3(g, i, j, k);
-        if constexpr (SPLIT) {
-          if (pml3(g, i, j, k)) {
-            // interface node: its regular-domain K sums, finished by the nodal pull
-            if (ua) st3(A.E + (long long)shot * 3 * g.NN, offu, acc[0], acc[1], acc[2]);
-            goto next_slab;
-          }
-        }
         const int sm = pn ? smask3(g, i, j, k) : 0;
         double raw[9];
 #pragma unroll
@@ -830,23 +736,7 @@ __global__ void __launch_bounds__(NT3, HAS_RD ? (HAS_PML ? 3 : 5) : (S >= 1 && S
               const long long nd = src_lds ? sSrcNode[jj - src_j0] : sp->node[jj];
               if (nd != (long long)n) continue;
               const int cpt = src_lds ? sSrcComp[jj - src_j0] : sp->comp[jj];
-              const double mm = sp->m[jj];
-              double val;
-              if (A.src_mode == 1) {
-                const double f = sp->ftab[((size_t)shot * sp->nstep + (A.step + sdyn)) * 3 + A.fcol];
-                val = f * (sp->val[jj] * mm);
-              } else {
-                const size_t nr = (size_t)sp->nrec;
-                const size_t base = (size_t)shot * ((size_t)sp->nstep + 1) * nr + ((size_t)jj - (size_t)shot * nr);
-                const size_t ra = (size_t)(A.ra + sdyn);
-                const double va = sp->tr[base + ra * nr] - sp->obs[base + ra * nr];
-                val = A.ca * (va * mm);
-                if (A.rb_on) {
-                  const size_t rb = (size_t)(A.rb + sdyn);
-                  const double vb = sp->tr[base + rb * nr] - sp->obs[base + rb * nr];
-                  val = val + A.cb * (vb * mm);
-                }
-              }
+              const double val = src_value(A, jj, shot, sdyn);
               if (cpt == 0) srcv[0] += val;
               else if (cpt == 1) srcv[1] += val;
               else srcv[2] += val;
@@ -861,7 +751,7 @@ __global__ void __launch_bounds__(NT3, HAS_RD ? (HAS_PML ? 3 : 5) : (S >= 1 && S
               out[m] = gout;
             } else if constexpr (S == 4) {
               const int cm = (NS == 9) ? m : (m < 3 ? m : 0);
-              out[m] = c3o[cm] + A.h6 * gout;
+              out[m] = c3o[cm] + A.h4 * gout;
             } else {
               const int cm = (NS == 9) ? m : (m < 3 ? m : 0);
               out[m] = c3o[cm] + gout;                        // u_{n+1}
@@ -890,456 +780,7 @@ __global__ void __launch_bounds__(NT3, HAS_RD ? (HAS_PML ? 3 : 5) : (S >= 1 && S
         }
       }
     }
-  next_slab:
     if constexpr (RING == 3) __syncthreads();
-  }
-}
-
-// ------------------------------------------------------------ split stage path
-// Blocks of consecutive PML nodes in lattice order (sp_pml_node), one node per
-// thread (nodal pull: SPLIT_NT nodes; nodal pass: SPLIT_OWN nodes and two on each
-// side).  XCD x = blockIdx % 8 takes the
-// logical blocks [x C, (x + 1) C) of the launch, so that each XCD's L2 holds a
-// contiguous run of the list (the neighbouring rows and planes of its nodes); a
-// launch has 8 C blocks and starts at logical block A.pb0.
-__device__ __forceinline__ int split_block(int nblk) {
-  const int C = (nblk + 7) / 8;
-  return (blockIdx.x & 7) * C + (blockIdx.x >> 3);
-}
-// the same runs, each walked from its end: a nodal pull whose sources include
-// PML nodes dispatches the top planes (surface sources and receivers, and with
-// them the blocks that also add source terms) first instead of last
-__device__ __forceinline__ int split_block_rev(int nblk) {
-  const int C = (nblk + 7) / 8;
-  return (blockIdx.x & 7) * C + (C - 1 - (int)(blockIdx.x >> 3));
-}
-
-__device__ __forceinline__ void st2(double* p, unsigned off, double a, double b) {
-  *reinterpret_cast<double2*>(reinterpret_cast<char*>(p) + off) = make_double2(a, b);
-}
-
-// Flux records D of the split path, per shot 12 NN doubles: two arrays (ax =
-// y, z) of six doubles per lattice node, (G_{x,ax}, G_{y,ax}, G_{z,ax},
-// w_{ax,x}, w_{ax,y}, w_{ax,z}) with G_{i,ax} the nodal PML flux and w_{ax,i}
-// the F-weighted inputs: a line along ax reads three 16-byte pairs per node.
-// The x-lines are summed by the nodal pass itself, from LDS.
-__device__ __forceinline__ unsigned d_rec(int ax, unsigned NN, unsigned n) {
-  return 48u * ((unsigned)(ax - 1) * NN + n);
-}
-
-// Node-local part of RK4 stage S at one PML node: its stage inputs from the raw
-// inputs (the fused kernel's PML window load, once per node), the flux records
-// of its y- and z-lines, and into the stage output the node-local terms: stages
-// 1-3 -M^-1 (diagonal terms + x-line sums), stage 4 the carry x3 + dt/6 (g1 +
-// 2 g2 + 2 g3) minus dt/6 M^-1 (diagonal terms + x-line sums), with the x1, x2
-// updates written here.  The x-line sums read the x records of the block's
-// entries from LDS: consecutive list entries are x-neighbours.
-template <int S, bool TR>
-__global__ void __launch_bounds__(SPLIT_NT, S == 4 ? 2 : 3) pml_nodal_kernel(const Stage3Args A) {
-  constexpr bool NEG = TR;
-  constexpr int NIN = 2 + S;
-  __shared__ double sXr[6][SPLIT_NT];     // x flux records of the block's entries
-  __shared__ unsigned sXn[SPLIT_NT];      // their lattice nodes (~0: no entry)
-  const Geo3& g = A.g;
-  const int lb = split_block(A.pnbn);
-  if (lb >= A.pnbn) return;
-  const int tid = threadIdx.x;
-  // list entry of this thread: the block owns [lb SPLIT_OWN, (lb + 1) SPLIT_OWN) and
-  // computes two more on each side for their x records; a thread without an
-  // entry runs node 0 (in bounds) and stores nothing
-  const long long t = (long long)lb * SPLIT_OWN - 2 + tid;
-  int i = 0, j = 0, k = 0;
-  const bool valid = t >= 0 && sp_pml_node((unsigned)t, g.NX, g.NY, g.NZ, g.rlo, g.rhi, i, j, k);
-  if (!valid) i = j = k = 0;
-  const bool own = valid && tid >= 2 && tid < SPLIT_NT - 2;
-  const int shot = blockIdx.y;
-  const unsigned n = (unsigned)i + (unsigned)g.NX * ((unsigned)j + (unsigned)g.NY * (unsigned)k);
-  const long long so = (long long)shot * A.shot_stride;
-  const unsigned NN = (unsigned)g.NN;
-  const unsigned SB = 8u * (3u * NN + (NN & 1u));
-  const unsigned offu = n * 24u, offs = SB + n * 48u;
-  const double* __restrict__ tab = A.tab;
-  const double* __restrict__ nodet = A.node;
-
-  double XU[3][NIN], XS6[6][NIN];
-#pragma unroll
-  for (int q = 0; q < NIN; ++q) {
-    const double* ip = A.in[q] + so;
-    ld3(ip, offu, XU[0][q], XU[1][q], XU[2][q]);
-    ld2(ip, offs, XS6[0][q], XS6[1][q]);
-    ld2(ip, offs + 16u, XS6[2][q], XS6[3][q]);
-    ld2(ip, offs + 32u, XS6[4][q], XS6[5][q]);
-  }
-  double lam, mu, ax, bx, ay, by, az, bz;
-  ld2(nodet, n * 16u, lam, mu);
-  const double minv_u = A.minvu[n], rwp = A.rwp[n];
-  ld2(tab, 8u * (unsigned)(TAB_STRETCH + 2 * i), ax, bx);
-  ld2(tab, 8u * (unsigned)(TAB_STRETCH + 2 * g.NX + 2 * j), ay, by);
-  ld2(tab, 8u * (unsigned)(TAB_STRETCH + 2 * g.NX + 2 * g.NY + 2 * k), az, bz);
-  // the node's sides per axis; its PML weight sum and the stress rows' M^-1
-  const SpAxis AX = sp_axis(i, g.nex, g.rlo[0], g.rhi[0]), AY = sp_axis(j, g.ney, g.rlo[1], g.rhi[1]),
-               AZ = sp_axis(k, g.nez, g.rlo[2], g.nez);
-  const double wps = g.detj * sp_pml_weight(AX, AY, AZ);
-  const double minv_s = 1.0 / (((ax * ay) * az) * wps);
-  const bool ua = u_act3(g, i, j, k);
-  const int sm = smask3(g, i, j, k);
-
-  double v1u[3], vu2[3], v3u[3];
-#pragma unroll
-  for (int c = 0; c < 3; ++c) combine<S, NEG>(XU[c], A.hh, A.h, A.h6, 7, v1u[c], vu2[c], v3u[c]);
-  // F[set][k], set 0 = w (G, v1), 1 = p (K, v2), 2 = e (C, v3)
-  double F[3][3];
-  F[2][0] = ay * az; F[2][1] = ax * az; F[2][2] = ax * ay;
-  F[1][0] = ay * bz + az * by; F[1][1] = ax * bz + az * bx; F[1][2] = ax * by + ay * bx;
-  F[0][0] = by * bz; F[0][1] = bx * bz; F[0][2] = bx * by;
-  double wv[9];
-#pragma unroll
-  for (int d = 0; d < 3; ++d)
-#pragma unroll
-    for (int c = 0; c < 3; ++c) wv[3 * d + c] = ((0.0 + F[0][d] * v1u[c]) + F[1][d] * vu2[c]) + F[2][d] * v3u[c];
-  // diagonal terms rho W (b v3 + c v2 + d v1) of ELEMENT_EM/EN (PML.F90 items 7..10)
-  const double qb = ax * ay * bz + ax * az * by + ay * az * bx;
-  const double qc = ax * by * bz + ay * bx * bz + az * bx * by;
-  const double qd = bx * by * bz;
-  auto diag = [&](double wm, double a1, double a2, double a3) { return wm * (((0.0 + qb * a3) + qc * a2) + qd * a1); };
-  double dg[9], c3[9], Gv[9];
-#pragma unroll
-  for (int m = 0; m < 9; ++m) { c3[m] = 0.0; Gv[m] = 0.0; }
-#pragma unroll
-  for (int c = 0; c < 3; ++c) dg[c] = diag(rwp, v1u[c], vu2[c], v3u[c]);
-  double* const x1n = A.xnew[0] ? A.xnew[0] + so : nullptr;
-  double* const x2n = A.xnew[1] ? A.xnew[1] + so : nullptr;
-  if constexpr (S == 4) {
-    double xn0[3], xn1[3];
-#pragma unroll
-    for (int c = 0; c < 3; ++c) rk4_update12(XU[c], A.hh, A.h, A.h6, xn0[c], xn1[c], c3[c]);
-    if (own && ua) {
-      st3(x1n, offu, xn0[0], xn0[1], xn0[2]);
-      st3(x2n, offu, xn1[0], xn1[1], xn1[2]);
-    }
-  }
-  const double l2m = lam + 2.0 * mu, m2 = 2.0 * mu;
-#pragma unroll
-  for (int hf = 0; hf < 2; ++hf) {
-    const double(*XS)[NIN] = &XS6[3 * hf];
-    double s1[3], s2[3], s3[3];
-#pragma unroll
-    for (int tt = 0; tt < 3; ++tt) combine<S, NEG>(XS[tt], A.hh, A.h, A.h6, 7, s1[tt], s2[tt], s3[tt]);
-#pragma unroll
-    for (int X = 0; X < 3; ++X) {
-      const double* sv = X == 0 ? s1 : (X == 1 ? s2 : s3);
-      if (hf == 0) {
-        if constexpr (!TR) {
-          // T(s): stress of the auxiliary strain (ELEMENT_EA_3D lower block), normal part
-          const double Txx = l2m * sv[0] + lam * sv[1] + lam * sv[2];
-          const double Tyy = lam * sv[0] + l2m * sv[1] + lam * sv[2];
-          const double Tzz = lam * sv[0] + lam * sv[1] + l2m * sv[2];
-          Gv[0] -= F[X][0] * Txx; Gv[4] -= F[X][1] * Tyy; Gv[8] -= F[X][2] * Tzz;
-        } else {
-          Gv[0] += F[X][0] * sv[0]; Gv[4] += F[X][1] * sv[1]; Gv[8] += F[X][2] * sv[2];
-        }
-      } else {
-        if constexpr (!TR) {
-          const double Txy = m2 * sv[0], Txz = m2 * sv[1], Tyz = m2 * sv[2];
-          Gv[1] -= F[X][1] * Txy; Gv[2] -= F[X][2] * Txz; Gv[3] -= F[X][0] * Txy;
-          Gv[5] -= F[X][2] * Tyz; Gv[6] -= F[X][0] * Txz; Gv[7] -= F[X][1] * Tyz;
-        } else {
-          Gv[1] += F[X][1] * sv[0]; Gv[2] += F[X][2] * sv[1]; Gv[3] += F[X][0] * sv[0];
-          Gv[5] += F[X][2] * sv[2]; Gv[6] += F[X][0] * sv[1]; Gv[7] += F[X][1] * sv[2];
-        }
-      }
-    }
-    const double wm = hf == 0 ? wps : 2.0 * wps;
-#pragma unroll
-    for (int tt = 0; tt < 3; ++tt) dg[3 + 3 * hf + tt] = diag(wm, s1[tt], s2[tt], s3[tt]);
-    if constexpr (S == 4) {
-      double xn0[3], xn1[3];
-#pragma unroll
-      for (int tt = 0; tt < 3; ++tt) rk4_update12(XS[tt], A.hh, A.h, A.h6, xn0[tt], xn1[tt], c3[3 + 3 * hf + tt]);
-      const int act = own ? (sm >> (3 * hf)) & 7 : 0;
-      if (act) {
-        st3m(x1n, offs + 24u * hf, act, xn0[0], xn0[1], xn0[2]);
-        st3m(x2n, offs + 24u * hf, act, xn1[0], xn1[1], xn1[2]);
-      }
-    }
-  }
-  // node-local terms of the stage output, without the x-line sums
-  const double sc = S == 4 ? A.h6 : 1.0;
-  double pre[9];
-#pragma unroll
-  for (int m = 0; m < 9; ++m) {
-    const double minv = m < 3 ? minv_u : (m < 6 ? minv_s : 0.5 * minv_s);
-    pre[m] = c3[m] - sc * (minv * dg[m]);
-  }
-  // x records to LDS; y and z records to memory
-  sXn[tid] = valid ? n : ~0u;
-  sXr[0][tid] = Gv[0]; sXr[1][tid] = Gv[3]; sXr[2][tid] = Gv[6];
-  sXr[3][tid] = wv[0]; sXr[4][tid] = wv[1]; sXr[5][tid] = wv[2];
-  // flux records: (G_{x,ax}, G_{y,ax}, G_{z,ax}, w_{ax,x}, w_{ax,y}, w_{ax,z}), Gv[3 i + ax], wv[3 ax + i]
-  double* const Dp = A.D + (long long)shot * 12 * g.NN;
-  if (own) {
-#pragma unroll
-    for (int a = 1; a < 3; ++a) {
-      const unsigned o = d_rec(a, NN, n);
-      st2(Dp, o, Gv[a], Gv[3 + a]);
-      st2(Dp, o + 16u, Gv[6 + a], wv[3 * a]);
-      st2(Dp, o + 32u, wv[3 * a + 1], wv[3 * a + 2]);
-    }
-  }
-  __syncthreads();
-  if (!own) return;
-  // the x-line of the pull: side-scaled stencil over the x-neighbours' records.
-  // The neighbour at lattice offset di (|di| <= 2) is at most |di| entries away
-  // in the list (no PML node between, or one); one that is not a PML node (a
-  // regular-domain node) has no record, and offsets outside the lattice have zero
-  // coefficients.
-  double cs0, cs1, cu[5];
-  sp_side_scales(AX, AY, AZ, cs0, cs1);
-  sp_stencil(AX.odd, cs0, cs1, cu);
-  double sux[3] = {0.0, 0.0, 0.0}, sdx[3] = {0.0, 0.0, 0.0};
-#pragma unroll
-  for (int d = 0; d < 5; ++d) {
-    const int di = d - 2;
-    int slot = -1;
-    if (di == 0) {
-      slot = tid;
-    } else if (i + di >= 0 && i + di < g.NX) {
-      const unsigned ne = (unsigned)((int)n + di);
-      const int near = tid + (di > 0 ? 1 : -1);
-      if (di == 2 || di == -2) slot = sXn[tid + di] == ne ? tid + di : (sXn[near] == ne ? near : -1);
-      else slot = sXn[near] == ne ? near : -1;
-    }
-    // u rows with cu, s rows with every offset but 0 negated
-    const double cw = d == 2 ? cu[d] : -cu[d];
-    if (slot >= 0) {
-      sux[0] += cu[d] * sXr[0][slot]; sux[1] += cu[d] * sXr[1][slot]; sux[2] += cu[d] * sXr[2][slot];
-      sdx[0] += cw * sXr[3][slot]; sdx[1] += cw * sXr[4][slot]; sdx[2] += cw * sXr[5][slot];
-    }
-  }
-  // its terms of the sums, taken into the node-local terms
-  double rx[9];
-#pragma unroll
-  for (int c = 0; c < 3; ++c) rx[c] = g.detj * (g.dxi[0] * sux[c]);
-  const double cx = g.detj * g.dxi[0];
-  const double ddx0 = cx * sdx[0], ddx1 = cx * sdx[1], ddx2 = cx * sdx[2];
-  if constexpr (!TR) {
-    rx[3] = ddx0; rx[4] = 0.0; rx[5] = 0.0; rx[6] = ddx1; rx[7] = ddx2; rx[8] = 0.0;
-  } else {
-    rx[3] = -(l2m * ddx0); rx[4] = -(lam * ddx0); rx[5] = -(lam * ddx0);
-    rx[6] = -(m2 * ddx1); rx[7] = -(m2 * ddx2); rx[8] = 0.0;
-  }
-#pragma unroll
-  for (int m = 0; m < 9; ++m) {
-    const double minv = m < 3 ? minv_u : (m < 6 ? minv_s : 0.5 * minv_s);
-    pre[m] = pre[m] - sc * (minv * rx[m]);
-  }
-  double* const dst = (S == 4 ? A.xnew[2] : A.out) + so;
-  if (ua) st3(dst, offu, pre[0], pre[1], pre[2]);
-  if (sm == 0x3f) st6(dst, offs, &pre[3]);
-  else {
-    if (sm & 7) st3m(dst, offs, sm & 7, pre[3], pre[4], pre[5]);
-    if (sm & 56) st3m(dst, offs + 24u, (sm >> 3) & 7, pre[6], pre[7], pre[8]);
-  }
-}
-
-// Pull of RK4 stage S at one PML node: the PML elements' terms from the flux
-// records along the y- and z-lines through the node (side-scaled 5-point
-// stencils; the x-line terms are in the node-local terms), the regular-domain K
-// sums of an interface node from E, the sources, then out = (node-local terms)
-// + sc (src - M^-1 sums), sc = 1 or dt/6.
-template <int S, bool TR>
-__global__ void __launch_bounds__(SPLIT_NT, 2) pml_pull_kernel(const Stage3Args A) {
-  __shared__ int sPn[SRC_LDS], sPj[SRC_LDS], sPc[SRC_LDS];   // the block's source entries
-  const Geo3& g = A.g;
-  const int lb = (A.src_mode && A.src.ptop) ? split_block_rev(A.pnb) : split_block(A.pnb);
-  if (lb >= A.pnb) return;
-  const int blk = A.pb0 + lb;
-  const int shot = blockIdx.y;
-  // this block's source entries (a uniform range), staged in LDS: lattice node,
-  // entry and component, so that each node scans them without global loads
-  int e0 = 0, e1 = 0;
-  if (A.src_mode) {
-    const int pb = shot * A.src.pnblk + blk;
-    e0 = A.src.pblk_ptr[pb];
-    e1 = A.src.pblk_ptr[pb + 1];
-  }
-  const bool src_lds = e1 - e0 <= SRC_LDS;
-  if (e1 > e0 && src_lds) {
-    for (int t = threadIdx.x; t < e1 - e0; t += SPLIT_NT) {
-      const int jj = A.src.pblk_idx[e0 + t];
-      sPj[t] = jj;
-      sPn[t] = (int)A.src.node[jj];
-      sPc[t] = A.src.comp[jj];
-    }
-    __syncthreads();
-  }
-  int i, j, k;
-  if (!sp_pml_node((unsigned)(blk * SPLIT_NT) + threadIdx.x, g.NX, g.NY, g.NZ, g.rlo, g.rhi, i, j, k)) return;
-  const unsigned n = (unsigned)i + (unsigned)g.NX * ((unsigned)j + (unsigned)g.NY * (unsigned)k);
-  const long long so = (long long)shot * A.shot_stride;
-  const unsigned NN = (unsigned)g.NN;
-  const unsigned SB = 8u * (3u * NN + (NN & 1u));
-  const unsigned offu = n * 24u, offs = SB + n * 48u;
-  const double* __restrict__ nodet = A.node;
-
-  // node-local terms the nodal pass wrote, and M^-1, issued with the records
-  double* const dst = (S == 4 ? A.xnew[2] : A.out) + so;
-  const double minv_u = A.minvu[n];
-  const double* __restrict__ tab = A.tab;
-  const double sax = tab[TAB_STRETCH + 2 * i], say = tab[TAB_STRETCH + 2 * g.NX + 2 * j],
-               saz = tab[TAB_STRETCH + 2 * g.NX + 2 * g.NY + 2 * k];
-  double pre[9];
-  ld3(dst, offu, pre[0], pre[1], pre[2]);
-  ld2(dst, offs, pre[3], pre[4]);
-  ld2(dst, offs + 16u, pre[5], pre[6]);
-  ld2(dst, offs + 32u, pre[7], pre[8]);
-  double lam = 0.0, mu = 0.0;
-  if constexpr (TR) ld2(nodet, n * 16u, lam, mu);
-  // interface sums, read with the first batch where a regular-domain element
-  // holds the node; other lanes read the shot's first entry (one shared line)
-  // and drop it
-  const SpAxis ax3[3] = {sp_axis(i, g.nex, g.rlo[0], g.rhi[0]), sp_axis(j, g.ney, g.rlo[1], g.rhi[1]),
-                         sp_axis(k, g.nez, g.rlo[2], g.nez)};
-  const bool iface = sp_iface(ax3[0], ax3[1], ax3[2]);
-  double e3[3];
-  ld3(A.E + (long long)shot * 3 * g.NN, iface ? offu : 0u, e3[0], e3[1], e3[2]);
-  // M^-1 of the stress rows: 1 / (a W), a the stretch-factor product, W the PML weight sum
-  const double minv_s = 1.0 / (((sax * say) * saz) * (g.detj * sp_pml_weight(ax3[0], ax3[1], ax3[2])));
-  const double* const Dp = A.D + (long long)shot * 12 * g.NN;
-  const int cc[3] = {i, j, k};
-  const int nax[3] = {g.NX, g.NY, g.NZ};
-  const int str[3] = {1, g.NX, g.NX * g.NY};
-  // y- and z-lines (the x-line terms are in the node-local terms): per axis
-  // su = sum_d cu[d] G_{.,ax}(n + (d - 2) str), sd the same with the s-row
-  // stencil (every offset but 0 negated) on w_{ax,.}
-  double su[3][3], sd[3][3];
-#pragma unroll
-  for (int ax = 1; ax < 3; ++ax) {
-    double s0, s1, cu[5];
-    sp_side_scales(ax3[ax], ax3[ax == 0 ? 1 : 0], ax3[ax == 2 ? 1 : 2], s0, s1);
-    sp_stencil(ax3[ax].odd, s0, s1, cu);
-#pragma unroll
-    for (int c = 0; c < 3; ++c) { su[ax][c] = 0.0; sd[ax][c] = 0.0; }
-#pragma unroll
-    for (int d = 0; d < 5; ++d) {
-      // odd coordinates have no +-2 terms: skipped (a row of consecutive list
-      // entries shares the y and z coordinates)
-      if ((d == 0 || d == 4) && ax3[ax].odd) continue;
-      // offsets outside the lattice have zero coefficients: read the node itself
-      const int p = cc[ax] + d - 2;
-      const unsigned m = (p >= 0 && p < nax[ax]) ? (unsigned)((int)n + (d - 2) * str[ax]) : n;
-      const unsigned o = d_rec(ax, NN, m);
-      double G0, G1, G2, W0, W1, W2;
-      ld2(Dp, o, G0, G1);
-      ld2(Dp, o + 16u, G2, W0);
-      ld2(Dp, o + 32u, W1, W2);
-      const double cw = d == 2 ? cu[d] : -cu[d];
-      su[ax][0] += cu[d] * G0; su[ax][1] += cu[d] * G1; su[ax][2] += cu[d] * G2;
-      sd[ax][0] += cw * W0; sd[ax][1] += cw * W1; sd[ax][2] += cw * W2;
-    }
-  }
-  double raw[9];
-#pragma unroll
-  for (int c = 0; c < 3; ++c) raw[c] = g.detj * ((0.0 + g.dxi[1] * su[1][c]) + g.dxi[2] * su[2][c]);
-#pragma unroll
-  for (int c = 0; c < 3; ++c) raw[c] += iface ? e3[c] : 0.0;
-  double dd[3][3];
-#pragma unroll
-  for (int ax = 1; ax < 3; ++ax)
-#pragma unroll
-    for (int c = 0; c < 3; ++c) dd[ax][c] = (g.detj * g.dxi[ax]) * sd[ax][c];
-  const double aE[6] = {0.0, dd[1][1], dd[2][2], dd[1][0], dd[2][0], dd[2][1] + dd[1][2]};
-  if constexpr (!TR) {
-#pragma unroll
-    for (int m = 0; m < 6; ++m) raw[3 + m] = aE[m];
-  } else {
-    const double l2m = lam + 2.0 * mu, m2 = 2.0 * mu;
-    raw[3] = -(l2m * aE[0] + lam * aE[1] + lam * aE[2]);
-    raw[4] = -(lam * aE[0] + l2m * aE[1] + lam * aE[2]);
-    raw[5] = -(lam * aE[0] + lam * aE[1] + l2m * aE[2]);
-    raw[6] = -(m2 * aE[3]);
-    raw[7] = -(m2 * aE[4]);
-    raw[8] = -(m2 * aE[5]);
-  }
-  // sources of this node (the entries of this block, a uniform range)
-  const bool ua = u_act3(g, i, j, k);
-  double src[3] = {0.0, 0.0, 0.0};
-  if (e1 > e0 && ua) {
-    const Src3& sp = A.src;
-    const int sdyn = A.step_dev ? *A.step_dev : 0;
-    for (int e = e0; e < e1; ++e) {
-      const int jj = src_lds ? sPj[e - e0] : sp.pblk_idx[e];
-      if ((src_lds ? (long long)sPn[e - e0] : sp.node[jj]) != (long long)n) continue;
-      const double mm = sp.m[jj];
-      double val;
-      if (A.src_mode == 1) {
-        const double f = sp.ftab[((size_t)shot * sp.nstep + (A.step + sdyn)) * 3 + A.fcol];
-        val = f * (sp.val[jj] * mm);
-      } else {
-        const size_t nr = (size_t)sp.nrec;
-        const size_t base = (size_t)shot * ((size_t)sp.nstep + 1) * nr + ((size_t)jj - (size_t)shot * nr);
-        const size_t ra = (size_t)(A.ra + sdyn);
-        const double va = sp.tr[base + ra * nr] - sp.obs[base + ra * nr];
-        val = A.ca * (va * mm);
-        if (A.rb_on) {
-          const size_t rb = (size_t)(A.rb + sdyn);
-          const double vb = sp.tr[base + rb * nr] - sp.obs[base + rb * nr];
-          val = val + A.cb * (vb * mm);
-        }
-      }
-      const int cpt = src_lds ? sPc[e - e0] : sp.comp[jj];
-      src[0] += cpt == 0 ? val : 0.0;
-      src[1] += cpt == 1 ? val : 0.0;
-      src[2] += cpt == 2 ? val : 0.0;
-    }
-  }
-  // finish on the node-local terms
-  const int sm = smask3(g, i, j, k);
-  const double sc = S == 4 ? A.h6 : 1.0;
-  double out[9];
-#pragma unroll
-  for (int m = 0; m < 9; ++m) {
-    const double minv = m < 3 ? minv_u : (m < 6 ? minv_s : 0.5 * minv_s);
-    const double sv = m < 3 ? src[m] : 0.0;
-    out[m] = pre[m] + sc * (sv - minv * raw[m]);
-  }
-  if (ua) st3(dst, offu, out[0], out[1], out[2]);
-  if (sm == 0x3f) st6(dst, offs, &out[3]);
-  else {
-    if (sm & 7) st3m(dst, offs, sm & 7, out[3], out[4], out[5]);
-    if (sm & 56) st3m(dst, offs + 24u, (sm >> 3) & 7, out[6], out[7], out[8]);
-  }
-}
-
-template <int S, bool TR>
-hipError_t launch_split(const Stage3Args& A, int part, const int* tiles, int ntl, hipStream_t s) {
-  if (A.nshot <= 0) return hipSuccess;
-  if (part == 1) {
-    if (ntl <= 0) return hipSuccess;
-    const int nb = 8 * ((ntl * A.nshot + 7) / 8);
-    stage_kernel3<4, 3, true, false, S, TR, true><<<nb, NT3, 0, s>>>(A, tiles, ntl);
-  } else {
-    const int nb = part == 0 ? A.pnbn : A.pnb;
-    if (nb <= 0) return hipSuccess;
-    const dim3 grid(8 * ((nb + 7) / 8), A.nshot);
-    if (part == 0) pml_nodal_kernel<S, TR><<<grid, SPLIT_NT, 0, s>>>(A);
-    else pml_pull_kernel<S, TR><<<grid, SPLIT_NT, 0, s>>>(A);
-  }
-  return hipGetLastError();
-}
-
-hipError_t launch_split_any(const Stage3Args& A, int stage, int transpose, int part, const int* tiles, int ntl,
-                            hipStream_t s) {
-  switch (stage * 2 + (transpose ? 1 : 0)) {
-    case 2: return launch_split<1, false>(A, part, tiles, ntl, s);
-    case 3: return launch_split<1, true>(A, part, tiles, ntl, s);
-    case 4: return launch_split<2, false>(A, part, tiles, ntl, s);
-    case 5: return launch_split<2, true>(A, part, tiles, ntl, s);
-    case 6: return launch_split<3, false>(A, part, tiles, ntl, s);
-    case 7: return launch_split<3, true>(A, part, tiles, ntl, s);
-    case 8: return launch_split<4, false>(A, part, tiles, ntl, s);
-    case 9: return launch_split<4, true>(A, part, tiles, ntl, s);
-    default: return hipErrorInvalidValue;
   }
 }
 
@@ -1359,30 +800,17 @@ hipError_t launch3(const Stage3Args& A, int cls, const int* tiles, int ntl, hipS
 
 hipError_t launch_stage3(const Stage3Args& A, int stage, int transpose, int cls, const int* tiles, int ntl,
                          hipStream_t s) {
-  switch (stage * 2 + (transpose ? 1 : 0)) {
+  // stages 1-3 are one kernel: they differ in the vectors they read
+  switch ((stage == 2 || stage == 3 ? 1 : stage) * 2 + (transpose ? 1 : 0)) {
     case 0: return launch3<0, false>(A, cls, tiles, ntl, s);
     case 1: return launch3<0, true>(A, cls, tiles, ntl, s);
     case 2: return launch3<1, false>(A, cls, tiles, ntl, s);
     case 3: return launch3<1, true>(A, cls, tiles, ntl, s);
-    case 4: return launch3<2, false>(A, cls, tiles, ntl, s);
-    case 5: return launch3<2, true>(A, cls, tiles, ntl, s);
-    case 6: return launch3<3, false>(A, cls, tiles, ntl, s);
-    case 7: return launch3<3, true>(A, cls, tiles, ntl, s);
     case 8: return launch3<4, false>(A, cls, tiles, ntl, s);
     case 9: return launch3<4, true>(A, cls, tiles, ntl, s);
     case 10: return launch3<5, false>(A, cls, tiles, ntl, s);
     default: return hipErrorInvalidValue;
   }
-}
-
-hipError_t launch_split_nodal(const Stage3Args& A, int stage, int transpose, hipStream_t s) {
-  return launch_split_any(A, stage, transpose, 0, nullptr, 0, s);
-}
-hipError_t launch_split_rd(const Stage3Args& A, int stage, int transpose, const int* tiles, int ntl, hipStream_t s) {
-  return launch_split_any(A, stage, transpose, 1, tiles, ntl, s);
-}
-hipError_t launch_split_pull(const Stage3Args& A, int stage, int transpose, hipStream_t s) {
-  return launch_split_any(A, stage, transpose, 2, nullptr, 0, s);
 }
 
 }  // namespace hr

@@ -1,0 +1,58 @@
+"""The split stage path at the sizes where its kernels' tiles, layers and lists end:
+regular domains that do not fill the element pass's 4 x 4 tiles, chunks of one
+layer, one per column and in between, sources and receivers on regular-domain
+nodes inside and on the interface, in the PML, and more receivers on one block of
+the pull than it has threads.  Against the CPU oracle's textbook RK4 at the
+parity bar of the time loops (1e-10 relative L2 on traces and gradients)."""
+import numpy as np
+import pytest
+
+from hirensi_amd import solver as S
+from hirensi_amd.mesh import BoxMesh, receiver_dofs
+from oracle import oracle as O
+from tests.helpers import random_model, rel_l2
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("shape,npml,tz", [((7, 11, 6), (1, 1, 1, 2, 1), 1), ((7, 11, 6), (1, 1, 1, 2, 1), 0),
+                                           ((8, 6, 7), (2, 1, 1, 1, 2), 2), ((6, 7, 5), (1, 4, 2, 2, 1), 3),
+                                           ((11, 6, 9), (1, 2, 1, 1, 1), 8)])
+def test_split_path_at_tile_and_chunk_edges(shape, npml, tz):
+    mesh = BoxMesh(*shape, npml=npml)
+    model, true = random_model(mesh, seed=4), random_model(mesh, seed=5)
+    lo, hi, top = mesh.rd_lo, mesh.rd_hi, mesh.NZ - 1
+    ci, cj = lo[0] + hi[0], lo[1] + hi[1]                    # a node in the middle of the regular domain
+    nodes = [mesh.node_index(i, j, top) for j in range(2 * lo[1], 2 * hi[1] + 1) for i in range(2 * lo[0], 2 * hi[0] + 1)]
+    nodes += [mesh.node_index(ci, cj, top - 1), mesh.node_index(1, cj, top - 2)]
+    rec_eq = receiver_dofs(mesh, nodes)
+    # the interface corner's DOFs many times over: more entries than a pull block's threads
+    rec_eq = np.concatenate([rec_eq, np.repeat(rec_eq[:3], 100)])
+    src_eq = np.array([mesh.dof(mesh.node_index(ci, cj, top), 2), mesh.dof(mesh.node_index(ci, cj, top), 2),
+                       mesh.dof(mesh.node_index(ci, cj, top - 3), 0), mesh.dof(mesh.node_index(2 * lo[0], cj, top), 1),
+                       mesh.dof(mesh.node_index(1, 1, top), 2)], dtype=np.int64)
+    src_val = np.array([1.0, 0.25, -0.5, 0.75, 0.5])
+    nstep, dt, fr = 90, 1.0e-4, 60.0
+    print(f"split path {shape} npml={npml} tz={tz} neq={mesh.neq} receivers={len(rec_eq)}", flush=True)
+    B = np.zeros(mesh.neq)
+    np.add.at(B, src_eq, src_val)
+    row = {int(e): r for r, e in enumerate(mesh.store_eq)}
+    inside = np.array([int(e) in row for e in rec_eq])
+    rows = np.array([row[int(e)] for e in rec_eq[inside]])
+    rec_eq = rec_eq[inside]                                  # the oracle's traces are regular-domain DOFs
+    dobs = O.System(mesh, true).forward(B, nstep, dt, lcase=2, fr=fr)[:, rows].copy()
+    ctx = S.Context(mesh, model, tz=tz)
+    assert ctx.version() == 4
+    tr = S.explicit_rk4_petsc_pml_3d(ctx, nstep, dt, S.time_table(nstep, dt, 2, fr), src_eq, src_val, rec_eq)
+    gl, gm, _ = S.explicit_rk4_petsc_pml_3d_adjoint_otd(ctx, nstep, dt, rec_eq, dobs)
+    so = O.System(mesh, model)
+    U = so.forward(B, nstep, dt, lcase=2, fr=fr)
+    P = so.adjoint(U, nstep, dt, rec_eq, dobs)
+    glr, gmr = so.control(U, P, nstep, dt)
+    assert np.abs(U[:, rows]).max() > 0 and np.abs(glr).max() > 0
+    assert rel_l2(tr, U[:, rows]) < 1e-10
+    assert rel_l2(gl, glr) < 1e-10 and rel_l2(gm, gmr) < 1e-10
+    # the fused tile classes take the same stages
+    c3 = S.Context(mesh, model, version=3)
+    tr3 = S.explicit_rk4_petsc_pml_3d(c3, nstep, dt, S.time_table(nstep, dt, 2, fr), src_eq, src_val, rec_eq)
+    assert rel_l2(tr3, tr) < 1e-12
