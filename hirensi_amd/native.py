@@ -34,6 +34,11 @@ NN_EXPORTS = (
     "hr_nn_to_bf16",
 )
 
+# hirensi_amd/csrc/hr_nn_fused.h: fused forms the package calls itself
+NN_FUSED_EXPORTS = (
+    "hr_nn_conv3d_fused", "hr_nn_transpose_layers", "hr_nn_avgpool2_grad_act", "hr_nn_upsample2_grad_act",
+)
+
 
 class MeshDesc(C.Structure):
     _fields_ = [

@@ -55,7 +55,7 @@ _P = C.c_void_p
 
 
 def lib():
-    """The HIP library with the hr_nn_* signatures set."""
+    """The HIP library with the hr_nn_* signatures set (hirensi_nn.h, csrc/hr_nn_fused.h)."""
     L = native.load()
     if getattr(L, "_nn_ready", False):
         return L
@@ -71,7 +71,11 @@ def lib():
     L.hr_nn_mse.argtypes = [_P, _P, _LL, _P, _P, _P, _P]
     L.hr_nn_adam.argtypes = [_P, _P, _P, _P, _P, _LL, _F, _F, _F, _F, _I, _P]
     L.hr_nn_to_bf16.argtypes = [_P, _P, _LL, _P]
-    for name in native.NN_EXPORTS:
+    L.hr_nn_conv3d_fused.argtypes = [_P, _P, _P, _P, _P, _F, _P, _I, _I, _I, _I, _I, _I, _P]
+    L.hr_nn_transpose_layers.argtypes = [_P, _P, _I, _P, _P, _P]
+    L.hr_nn_avgpool2_grad_act.argtypes = [_P, _P, _P, _LL, _I, _I, _I, _F, _P]
+    L.hr_nn_upsample2_grad_act.argtypes = [_P, _P, _P, _LL, _I, _I, _I, _F, _P]
+    for name in native.NN_EXPORTS + native.NN_FUSED_EXPORTS:
         getattr(L, name).restype = C.c_int
     L._nn_ready = True
     return L
@@ -129,28 +133,32 @@ class ConvNet:
         self._transpose()
 
     def _transpose(self):
-        for li, (_, ci, co, _) in enumerate(LAYERS):
-            o = 2 * self.woff[li]
-            _check(self.L.hr_nn_transpose_weights(self.wb.data_ptr() + o, self.wt.data_ptr() + o, ci, co, self.stream),
-                   "transpose_weights")
+        n = len(LAYERS)
+        ci, co = (_I * n)(*(l[1] for l in LAYERS)), (_I * n)(*(l[2] for l in LAYERS))
+        _check(self.L.hr_nn_transpose_layers(self.wb.data_ptr(), self.wt.data_ptr(), n, ci, co, self.stream),
+               "transpose_layers")
 
     def _empty(self, nb, c, dims):
         return self.torch.empty((nb, c) + tuple(dims), dtype=self.torch.float32, device=self.dev)
 
-    def _conv(self, li, x, out, dims, accumulate=False):
+    def _conv(self, li, x, out, dims, add=None, slope=SLOPE):
+        """out = leaky ReLU of the convolution (+ add); slope 1: no activation."""
         _, ci, co, _ = LAYERS[li]
         nb = x.shape[0]
-        _check(self.L.hr_nn_conv3d(x.data_ptr(), self.wb.data_ptr() + 2 * self.woff[li],
-                                   self.b.data_ptr() + 4 * self.boff[li], out.data_ptr(), ci, co, nb, *dims,
-                                   int(accumulate), self.stream), f"conv {LAYERS[li][0]}")
+        _check(self.L.hr_nn_conv3d_fused(x.data_ptr(), self.wb.data_ptr() + 2 * self.woff[li],
+                                         self.b.data_ptr() + 4 * self.boff[li],
+                                         None if add is None else add.data_ptr(), None, slope, out.data_ptr(), ci, co,
+                                         nb, *dims, self.stream), f"conv {LAYERS[li][0]}")
 
-    def _conv_dx(self, li, dy, dims):
-        """Input gradient of layer li: the convolution with the mirrored, transposed weights."""
+    def _conv_dx(self, li, dy, dims, y=None):
+        """Input gradient of layer li: the convolution with the mirrored, transposed
+        weights; with the input's activation output y, through the activation too."""
         _, ci, co, _ = LAYERS[li]
         nb = dy.shape[0]
         dx = self._empty(nb, ci, dims)
-        _check(self.L.hr_nn_conv3d(dy.data_ptr(), self.wt.data_ptr() + 2 * self.woff[li], None, dx.data_ptr(), co, ci,
-                                   nb, *dims, 0, self.stream), f"conv_dx {LAYERS[li][0]}")
+        _check(self.L.hr_nn_conv3d_fused(dy.data_ptr(), self.wt.data_ptr() + 2 * self.woff[li], None, None,
+                                         None if y is None else y.data_ptr(), 1.0 if y is None else SLOPE,
+                                         dx.data_ptr(), co, ci, nb, *dims, self.stream), f"conv_dx {LAYERS[li][0]}")
         return dx
 
     def _wgrad(self, li, x, dy, dims):
@@ -164,25 +172,17 @@ class ConvNet:
                                          self.gw.data_ptr() + 4 * self.woff[li], self.gb.data_ptr() + 4 * self.boff[li],
                                          ci, co, nb, *dims, self.stream), f"wgrad {LAYERS[li][0]}")
 
-    def _act(self, x):
-        _check(self.L.hr_nn_leaky_relu(x.data_ptr(), x.numel(), SLOPE, self.stream), "leaky_relu")
-        return x
-
-    def _act_grad(self, y, dy):
-        _check(self.L.hr_nn_leaky_relu_grad(y.data_ptr(), dy.data_ptr(), dy.numel(), SLOPE, self.stream),
-               "leaky_relu_grad")
-        return dy
-
     def _pool(self, x, dims):
         nb, c = x.shape[:2]
         out = self._empty(nb, c, [d // 2 for d in dims])
         _check(self.L.hr_nn_avgpool2(x.data_ptr(), out.data_ptr(), nb * c, *dims, self.stream), "avgpool2")
         return out
 
-    def _pool_grad(self, dy, dx, dims):
+    def _pool_grad(self, dy, y, dx, dims):
+        """dx + pooling backward of dy, through the activation with output y."""
         nb, c = dx.shape[:2]
-        _check(self.L.hr_nn_avgpool2_grad(dy.data_ptr(), dx.data_ptr(), nb * c, *dims, 1, self.stream),
-               "avgpool2_grad")
+        _check(self.L.hr_nn_avgpool2_grad_act(dy.data_ptr(), y.data_ptr(), dx.data_ptr(), nb * c, *dims, SLOPE,
+                                              self.stream), "avgpool2_grad")
 
     def _up(self, x, dims):
         nb, c = x.shape[:2]
@@ -190,11 +190,12 @@ class ConvNet:
         _check(self.L.hr_nn_upsample2(x.data_ptr(), out.data_ptr(), nb * c, *dims, self.stream), "upsample2")
         return out
 
-    def _up_grad(self, dy, dims):
+    def _up_grad(self, dy, y, dims):
+        """Upsampling backward of dy, through the activation with output y."""
         nb, c = dy.shape[:2]
         dx = self._empty(nb, c, [d // 2 for d in dims])
-        _check(self.L.hr_nn_upsample2_grad(dy.data_ptr(), dx.data_ptr(), nb * c, *dims, self.stream),
-               "upsample2_grad")
+        _check(self.L.hr_nn_upsample2_grad_act(dy.data_ptr(), y.data_ptr(), dx.data_ptr(), nb * c, *dims, SLOPE,
+                                               self.stream), "upsample2_grad")
         return dx
 
     # ------------------------------------------------------------ passes
@@ -213,10 +214,8 @@ class ConvNet:
             la, lb = 2 * lev, 2 * lev + 1
             h = self._empty(nb, LAYERS[la][2], dims[lev])
             self._conv(la, enc_in, h, dims[lev])
-            self._act(h)
             e = self._empty(nb, LAYERS[lb][2], dims[lev])
             self._conv(lb, h, e, dims[lev])
-            self._act(e)
             a[f"h{lev}"], a[f"e{lev}"] = h, e
             if lev < LEVELS - 1:
                 enc_in = self._pool(e, dims[lev])
@@ -226,16 +225,14 @@ class ConvNet:
             la = 2 * LEVELS + 2 * (LEVELS - 2 - lev)
             lb = la + 1
             u = self._up(dec, dims[lev])
-            z = a[f"e{lev}"].clone()           # skip: conv(u) + e
-            self._conv(la, u, z, dims[lev], accumulate=True)
-            self._act(z)
+            z = self._empty(nb, LAYERS[la][2], dims[lev])
+            self._conv(la, u, z, dims[lev], add=a[f"e{lev}"])   # skip: conv(u) + e
             d = self._empty(nb, LAYERS[lb][2], dims[lev])
             self._conv(lb, z, d, dims[lev])
-            self._act(d)
             a[f"u{lev}"], a[f"z{lev}"], a[f"d{lev}"] = u, z, d
             dec = d
         y = self._empty(nb, 1, dims[0])
-        self._conv(len(LAYERS) - 1, dec, y, dims[0])
+        self._conv(len(LAYERS) - 1, dec, y, dims[0], slope=1.0)
         if keep:
             self._acts, self._dims = a, dims
         return y
@@ -245,29 +242,26 @@ class ConvNet:
         a, dims = self._acts, self._dims
         lo = len(LAYERS) - 1
         self._wgrad(lo, a["d0"], dy, dims[0])
-        g = self._conv_dx(lo, dy, dims[0])
+        g = self._conv_dx(lo, dy, dims[0], a["d0"])
         ge = {}
         for lev in range(LEVELS - 1):            # decoder, finest level first
             la = 2 * LEVELS + 2 * (LEVELS - 2 - lev)
             lb = la + 1
-            self._act_grad(a[f"d{lev}"], g)
             self._wgrad(lb, a[f"z{lev}"], g, dims[lev])
-            g = self._conv_dx(lb, g, dims[lev])
-            self._act_grad(a[f"z{lev}"], g)
+            g = self._conv_dx(lb, g, dims[lev], a[f"z{lev}"])
             self._wgrad(la, a[f"u{lev}"], g, dims[lev])
             ge[lev] = g                           # the skip's gradient into e_lev
             gu = self._conv_dx(la, g, dims[lev])
-            g = self._up_grad(gu, dims[lev])      # gradient of the coarser decoder output
+            # gradient of the coarser decoder output (the bottleneck's below the last level)
+            g = self._up_grad(gu, a[f"d{lev + 1}" if lev < LEVELS - 2 else f"e{lev + 1}"], dims[lev])
         # bottleneck output e3 receives g; then the encoder, coarsest level first
         for lev in range(LEVELS - 1, -1, -1):
             la, lb = 2 * lev, 2 * lev + 1
             if lev < LEVELS - 1:
                 g = ge[lev]
-                self._pool_grad(gp, g, dims[lev])   # + pooling path
-            self._act_grad(a[f"e{lev}"], g)
+                self._pool_grad(gp, a[f"e{lev}"], g, dims[lev])   # + pooling path
             self._wgrad(lb, a[f"h{lev}"], g, dims[lev])
-            g = self._conv_dx(lb, g, dims[lev])
-            self._act_grad(a[f"h{lev}"], g)
+            g = self._conv_dx(lb, g, dims[lev], a[f"h{lev}"])
             xin = a["x"] if lev == 0 else a[f"p{lev}"]
             self._wgrad(la, xin, g, dims[lev])
             if lev > 0:

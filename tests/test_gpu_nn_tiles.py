@@ -1,0 +1,81 @@
+"""The tiled convolution kernels of the learned preconditioner at the sizes where
+their tiles, channel chunks and staged ranges end: channel counts around 16 and
+32, volumes smaller than a block's columns (several samples a block) and of odd
+size (steps of 16 columns across samples), rows too long for the staging (gather
+kernels), and the fused epilogues.  Against PyTorch in FP32 on the same
+BF16-rounded operands; FP32 summation order is the only difference, so 1e-5 of
+the largest output, as in test_gpu_nn.py."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+F = torch.nn.functional
+
+
+def bf(x):
+    return x.to(torch.bfloat16).to(torch.float32)
+
+
+def bits(x):
+    return x.to(torch.bfloat16).view(torch.int16).to("cuda:0")
+
+
+def rel(a, b):
+    return float((a.cpu() - b).abs().max() / max(float(b.abs().max()), 1e-30))
+
+
+CASES = [
+    # cin, cout, NB, (D, H, W), slices
+    (1, 1, 1, (1, 1, 1), 1), (17, 16, 5, (2, 2, 4), 2), (16, 17, 3, (3, 5, 7), 3), (33, 48, 2, (4, 4, 4), 1),
+    (15, 65, 2, (9, 5, 6), 4), (32, 130, 1, (2, 8, 8), 2), (16, 16, 3, (8, 31, 33), 9), (5, 3, 2, (2, 3, 400), 3),
+    (16, 32, 2, (16, 32, 33), 20), (64, 64, 1, (6, 16, 40), 5),
+]
+
+
+@pytest.mark.parametrize("cin,cout,nb,dims,ns", CASES)
+def test_tiled_convolutions(cin, cout, nb, dims, ns):
+    from hirensi_amd import precond as PC
+    print(f"tiled conv cin={cin} cout={cout} nb={nb} dims={dims} slices={ns}", flush=True)
+    L, s = PC.lib(), torch.cuda.current_stream().cuda_stream
+    g = torch.Generator().manual_seed(cin * 131 + cout)
+    x, dy = torch.randn((nb, cin) + dims, generator=g), torch.randn((nb, cout) + dims, generator=g)
+    w, b = torch.randn(cout, cin * 27, generator=g) / np.sqrt(27.0 * cin), torch.randn(cout, generator=g)
+    add, gate = torch.randn(dy.shape, generator=g), torch.randn(dy.shape, generator=g)
+    ref = F.conv3d(bf(x), bf(w).view(cout, cin, 3, 3, 3), b, padding=1)
+    xd, wd, bd, addd, gated, dyd = (v.to("cuda:0") if v.dtype == torch.float32 else v
+                                    for v in (x, bits(w), b, add, gate, dy))
+    y = torch.empty_like(dyd)
+
+    def conv(a, gt, slope):
+        assert L.hr_nn_conv3d_fused(xd.data_ptr(), wd.data_ptr(), bd.data_ptr(), a, gt, slope, y.data_ptr(), cin, cout,
+                                    nb, *dims, s) == 0
+        return y
+    assert rel(conv(None, None, 1.0), ref) < 1e-5
+    assert rel(conv(addd.data_ptr(), None, 0.1), F.leaky_relu(ref + add, 0.1)) < 1e-5
+    assert rel(conv(None, gated.data_ptr(), 0.1), torch.where(gate > 0, ref, 0.1 * ref)) < 1e-5
+    dw, db = torch.empty(cout * cin * 27, device="cuda:0"), torch.empty(cout, device="cuda:0")
+    part = torch.empty(ns * dw.numel(), device="cuda:0")
+    assert L.hr_nn_conv3d_wgrad(xd.data_ptr(), dyd.data_ptr(), part.data_ptr(), ns, dw.data_ptr(), db.data_ptr(), cin,
+                                cout, nb, *dims, s) == 0
+    ref_dw = torch.nn.grad.conv3d_weight(bf(x), (cout, cin, 3, 3, 3), bf(dy), padding=1).reshape(-1)
+    assert rel(dw, ref_dw) < 1e-5
+    assert rel(db, dy.sum(dim=(0, 2, 3, 4))) < 1e-5
+
+
+def test_infinite_and_nan_inputs_stay_in_their_neighbourhood():
+    """Padding columns and K entries past the last channel multiply nothing: a
+    non-finite voxel reaches its 27 neighbours and no others."""
+    from hirensi_amd import precond as PC
+    print("tiled conv with inf and nan voxels", flush=True)
+    L, s = PC.lib(), torch.cuda.current_stream().cuda_stream
+    cin, cout, nb, dims = 3, 5, 2, (5, 6, 7)
+    g = torch.Generator().manual_seed(2)
+    x, w = torch.randn((nb, cin) + dims, generator=g), torch.randn(cout, cin * 27, generator=g)
+    x[0, 2, 4, 5, 6], x[1, 0, 0, 0, 0] = float("nan"), float("inf")
+    ref = F.conv3d(x, w.view(cout, cin, 3, 3, 3), None, padding=1)
+    xd, wd = x.to("cuda:0"), bits(w)
+    y = torch.empty((nb, cout) + dims, device="cuda:0")
+    assert L.hr_nn_conv3d(xd.data_ptr(), wd.data_ptr(), None, y.data_ptr(), cin, cout, nb, *dims, 0, s) == 0
+    assert torch.equal(torch.isfinite(y.cpu()), torch.isfinite(ref))
