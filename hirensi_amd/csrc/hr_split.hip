@@ -486,10 +486,13 @@ __global__ void __launch_bounds__(SPLIT_NT, 2) pml_pull_kernel(const SplitArgs A
 // stresses at the owners instead took 27 LDS reads per node and element, in
 // branches by the nodes' parities, and 10 us per layer.  A z-line's thread reads its own
 // column once for the three points and keeps the column's lambda, mu in registers.
-// The loads of the next layer are in flight while a layer is computed.  Both
-// fields share the window pass and lambda, mu (50 KB of LDS).  Two blocks per CU: the
-// registers of three (168) spilled 90 of them and took twice the time.  About 4.5 us
-// per layer of a lone block (barriers and LDS latency), 90 us a pass at 64x64x32.
+// The loads of the finish and of the next layer are issued when the stresses have
+// freed their registers.  Both fields share the window pass and lambda, mu.
+// LDS bounds it: at 64x64x32 elements 52 of 78 us alone (counters), a quarter of that
+// bank conflicts that no padding of the window or the forces removed.  Beside the
+// nodal pass it takes 88 us there; the loads ahead of the stresses 100 us, three
+// blocks per CU (register spills) 92-112 us, and a form with one lattice column per
+// thread and half the LDS traffic 180 us (its widest parity class needs 300 registers).
 constexpr int RT = 4, RW = 2 * RT + 3, RWP = RW * RW, RNE = (RT + 1) * (RT + 1), RO = 2 * RT + 1;
 constexpr int REW = 7;                     // elements per wavefront (9 lanes each)
 static_assert(4 * REW >= RNE && 2 * RWP <= 256 && 3 * RO * RO <= 256, "one block of four wavefronts");
@@ -497,7 +500,7 @@ static_assert(4 * REW >= RNE && 2 * RWP <= 256 && 3 * RO * RO <= 256, "one block
 template <bool UPDATE>
 __global__ void __launch_bounds__(256, 2) rd_pair_kernel(const RdArgs A) {
   __shared__ double sV[2][3][3][RWP];      // field, plane (k % 3), component, window position
-  __shared__ double sR[2][3][RNE * 27];    // nodal forces of the elements per field and component
+  __shared__ double sR[2][3][RNE * 27 + 1];   // nodal forces of the elements per field and component, a spare
   const Geo3& g = A.g;
   const int tid = threadIdx.x, lane = tid & 63;
   // XCD-aware order: XCD x = blockIdx % 8 takes a contiguous run of the (shot, y, z, x) tiles
@@ -532,16 +535,16 @@ __global__ void __launch_bounds__(256, 2) rd_pair_kernel(const RdArgs A) {
   const bool elm = lane < 9 * REW && se < RNE && sex >= g.rlo[0] && sex < g.rhi[0] && sey >= g.rlo[1] && sey < g.rhi[1];
   const int spc = elm ? 2 * (se % (RT + 1)) + slx + RW * (2 * (se / (RT + 1)) + sly) : slx + RW * sly;   // column in the window
   const unsigned sn = elm ? (unsigned)((2 * sex + slx) + g.NX * (2 * sey + sly)) : 0u;
-  // derivative coefficients DM(l, .) of the line's points, transposed ones DM(a, l)
-  // for a = l, l + 1, l + 2 (mod 3), both in physical units, and the lanes of those lines
-  double fx[3], fy[3], hx[3], hy[3];
+  // the derivative of a, b, c at local point l is (c - a) / 2 + (l - 1) (a - 2 b + c);
+  // transposed coefficients DM(a, l) for a = l, l + 1, l + 2 (mod 3) in physical units,
+  // and the lanes of those lines
+  const double px = slx - 1, py = sly - 1;
+  double hx[3], hy[3];
   int nx[3], ny[3];
 #pragma unroll
   for (int c = 0; c < 3; ++c) {
     auto dm = [](int a, int b) { return b == 0 ? (a - 1) - 0.5 : (b == 1 ? -2.0 * (a - 1) : (a - 1) + 0.5); };
     const int ax = (slx + c) % 3, ay = (sly + c) % 3;
-    fx[c] = g.dxi[0] * dm(slx, c);
-    fy[c] = g.dxi[1] * dm(sly, c);
     hx[c] = g.dxi[0] * dm(ax, slx);
     hy[c] = g.dxi[1] * dm(ay, sly);
     nx[c] = 9 * le + ax + 3 * sly;
@@ -595,10 +598,9 @@ __global__ void __launch_bounds__(256, 2) rd_pair_kernel(const RdArgs A) {
   }
   load_plane(2 * ez_first + 1 + lp, r0, r1);
   // lambda, mu of the line's three points: index 2 of a layer is index 0 of the next
-  double lm[3][2], lmn[2][2];
-  ld2(A.node, (sn + NXY * (unsigned)(2 * ez_first)) * 16u, lm[2][0], lm[2][1]);
+  double lm[3][2];
 #pragma unroll
-  for (int z = 0; z < 2; ++z) ld2(A.node, (sn + NXY * (unsigned)(2 * ez_first + 1 + z)) * 16u, lmn[z][0], lmn[z][1]);
+  for (int z = 0; z < 3; ++z) ld2(A.node, (sn + NXY * (unsigned)(2 * ez_first + z)) * 16u, lm[z][0], lm[z][1]);
 
   double acc[2][3];
 #pragma unroll
@@ -609,29 +611,11 @@ __global__ void __launch_bounds__(256, 2) rd_pair_kernel(const RdArgs A) {
     const int p = ((P - 2 * ez) % 3 + 3) % 3;       // this group's plane within the layer
     const int k = 2 * ez + p;
     put_plane(2 * ez + 1 + lp, r0, r1);
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      lm[0][c] = lm[2][c];
-      lm[1][c] = lmn[0][c];
-      lm[2][c] = lmn[1][c];
-    }
-    if (ez + 1 < ez_end) {
-      load_plane(2 * ez + 3 + lp, r0, r1);
-#pragma unroll
-      for (int z = 0; z < 2; ++z) ld2(A.node, (sn + NXY * (unsigned)(2 * ez + 3 + z)) * 16u, lmn[z][0], lmn[z][1]);
-    }
     // the nodes finished in this layer: two planes, the top one at the surface
     const bool fin = owned && !halo && (p < 2 || ez == g.nez - 1);
     const bool ifc = fin && pml3(g, i, j, k);       // interface node
     const unsigned n = fin ? (unsigned)i + (unsigned)g.NX * (unsigned)j + NXY * (unsigned)k : 0u;
     double minv = 0.0, x2[3], x3[3], own[2][3];
-    if (fin) {
-      minv = A.minvu[n];
-      if constexpr (UPDATE) {
-        ld3(A.x[0] + so, n * 24u, x2[0], x2[1], x2[2]);
-        ld3(A.x[1] + so, n * 24u, x3[0], x3[1], x3[2]);
-      }
-    }
     __syncthreads();
     const int zs[3] = {(2 * ez) % 3, (2 * ez + 1) % 3, (2 * ez + 2) % 3};
 #pragma unroll
@@ -654,8 +638,10 @@ __global__ void __launch_bounds__(256, 2) rd_pair_kernel(const RdArgs A) {
           for (int c = 0; c < 3; ++c) {
             const double* U = sV[f][zs[z]][c];
             const int rx = spc - slx, ry = spc - RW * sly;
-            gx[c] = fx[0] * U[rx] + fx[1] * U[rx + 1] + fx[2] * U[rx + 2];
-            gy[c] = fy[0] * U[ry] + fy[1] * U[ry + RW] + fy[2] * U[ry + 2 * RW];
+            const double a0 = U[rx], a1 = U[rx + 1], a2 = U[rx + 2];
+            const double b0 = U[ry], b1 = U[ry + RW], b2 = U[ry + 2 * RW];
+            gx[c] = g.dxi[0] * (0.5 * (a2 - a0) + px * ((a0 + a2) - 2.0 * a1));
+            gy[c] = g.dxi[1] * (0.5 * (b2 - b0) + py * ((b0 + b2) - 2.0 * b1));
           }
           const double W = swxy * (z == 1 ? 4.0 / 3.0 : 1.0 / 3.0);
           const double lam = W * lm[z][0], mu = W * lm[z][1];
@@ -678,16 +664,42 @@ __global__ void __launch_bounds__(256, 2) rd_pair_kernel(const RdArgs A) {
         fz[0] = dz * (-1.5 * S[0][cz] - 0.5 * S[1][cz] + 0.5 * S[2][cz]);
         fz[1] = dz * (2.0 * S[0][cz] - 2.0 * S[2][cz]);
         fz[2] = dz * (-0.5 * S[0][cz] + 0.5 * S[1][cz] + 1.5 * S[2][cz]);
+        double t[3][2];                             // a direction's shuffles in flight
 #pragma unroll
-        for (int z = 0; z < 3; ++z) {
-          double v = fz[z] + (hx[0] * S[z][cx] + hy[0] * S[z][cy]);
-          v += hx[1] * __shfl(S[z][cx], nx[1]) + hx[2] * __shfl(S[z][cx], nx[2]);
-          v += hy[1] * __shfl(S[z][cy], ny[1]) + hy[2] * __shfl(S[z][cy], ny[2]);
-          if (elm) sR[f][c][27 * se + sq + 9 * z] = v;
-        }
+        for (int z = 0; z < 3; ++z)
+#pragma unroll
+          for (int d = 0; d < 2; ++d) t[z][d] = __shfl(S[z][cx], nx[d + 1]);
+#pragma unroll
+        for (int z = 0; z < 3; ++z) fz[z] += hx[0] * S[z][cx] + (hx[1] * t[z][0] + hx[2] * t[z][1]);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int z = 0; z < 3; ++z)
+#pragma unroll
+          for (int d = 0; d < 2; ++d) t[z][d] = __shfl(S[z][cy], ny[d + 1]);
+#pragma unroll
+        for (int z = 0; z < 3; ++z)
+          sR[f][c][elm ? 27 * se + sq + 9 * z : RNE * 27] =
+              fz[z] + (hy[0] * S[z][cy] + (hy[1] * t[z][0] + hy[2] * t[z][1]));
         __builtin_amdgcn_sched_barrier(0);
       }
     }
+    // loads of the finish and of the next layer, once the stresses have freed their
+    // registers
+    if (fin) {
+      minv = A.minvu[n];
+      if constexpr (UPDATE) {
+        ld3(A.x[0] + so, n * 24u, x2[0], x2[1], x2[2]);
+        ld3(A.x[1] + so, n * 24u, x3[0], x3[1], x3[2]);
+      }
+    }
+    if (ez + 1 < ez_end) {
+      load_plane(2 * ez + 3 + lp, r0, r1);
+      lm[0][0] = lm[2][0];
+      lm[0][1] = lm[2][1];
+#pragma unroll
+      for (int z = 1; z < 3; ++z) ld2(A.node, (sn + NXY * (unsigned)(2 * ez + 2 + z)) * 16u, lm[z][0], lm[z][1]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
     if constexpr (UPDATE) {
 #pragma unroll
       for (int c = 0; c < 3; ++c) {
