@@ -135,7 +135,7 @@ struct hr_ctx {
   // gradient post-processing: 1/Mg and restriction (geometry only, built once),
   // regularisation vectors, per-element costs, reduction partials, staging of
   // host material / gradient vectors
-  double *d_img = nullptr, *d_restr = nullptr, *d_reg = nullptr, *d_cost_el = nullptr, *d_red = nullptr;
+  double *d_img = nullptr, *d_restr = nullptr, *d_reg = nullptr, *d_red = nullptr;
   double *d_pm = nullptr, *d_pg = nullptr;
   double recompute = 1.0;
   hipStream_t stream = nullptr;
@@ -1050,7 +1050,7 @@ int hr_ctx_destroy(hr_ctx* ctx) {
   F(ctx->d_rec_tile_ptr); F(ctx->d_rec_node); F(ctx->d_rec_comp); F(ctx->d_rec_m); F(ctx->d_rec_perm);
   F(ctx->d_obs); F(ctx->d_gl); F(ctx->d_gm); F(ctx->d_part); F(ctx->d_scalar); F(ctx->d_tr_sorted);
   F(ctx->d_obs_sorted);
-  F(ctx->d_img); F(ctx->d_restr); F(ctx->d_reg); F(ctx->d_cost_el); F(ctx->d_red); F(ctx->d_pm); F(ctx->d_pg);
+  F(ctx->d_img); F(ctx->d_restr); F(ctx->d_reg); F(ctx->d_red); F(ctx->d_pm); F(ctx->d_pg);
   for (int c = 0; c < 3; ++c) F(ctx->d_tl[c]);
   F(ctx->d_D); F(ctx->d_E);
   for (hr_ctx::PullLists* pl : {&ctx->pl_src, &ctx->pl_rec}) {
@@ -2256,20 +2256,15 @@ int check_wreg(hr_ctx* ctx, const double* wreg) {
   return 0;
 }
 
-// Regularisation vectors of lam, mu (device) into ctx->d_reg (lambda, then mu)
-// and the two unscaled costs into ctx->d_red[RED_OUT + {0, 1}].
-constexpr int RED_OUT_COST = 4;
-int regularize(hr_ctx* ctx, int method, const double* wreg, const double* dl, const double* dm) {
+// Regularisation vectors of lam, mu (device) into ctx->d_reg (lambda, then mu), their
+// sums and those of gl, gm (device, or null) into ctx->d_red
+int regularize(hr_ctx* ctx, int method, const double* wreg, const double* dl, const double* dm, const double* gl,
+               const double* gm) {
   const size_t NN = (size_t)ctx->g.NN;
-  const long long nbe = reg_box_elements(ctx->g);
   if (!ctx->d_reg) if (int rc = dalloc(ctx, &ctx->d_reg, 2 * NN)) return rc;
-  if (!ctx->d_cost_el) if (int rc = dalloc(ctx, &ctx->d_cost_el, 2 * (size_t)nbe)) return rc;
-  if (!ctx->d_red) if (int rc = dalloc(ctx, &ctx->d_red, (size_t)dot_partials_size() + 8)) return rc;
-  HIPC(launch_regularization(ctx->g, ctx->d_zc, method == 0, wreg, dl, dm, ctx->d_reg, ctx->d_reg + NN,
-                             ctx->d_cost_el, ctx->stream));
-  const double* xs[2] = {ctx->d_cost_el, ctx->d_cost_el + 1};
-  const double* ys[2] = {nullptr, nullptr};
-  HIPC(launch_dots(2, nbe, 2, xs, ys, ctx->d_red, ctx->d_red + dot_partials_size() + RED_OUT_COST, ctx->stream));
+  if (!ctx->d_red) if (int rc = dalloc(ctx, &ctx->d_red, RED_SUMS + reg_partials_size(ctx->g))) return rc;
+  HIPC(launch_regularization(ctx->g, ctx->d_zc, method == 0, wreg, dl, dm, gl, gm, ctx->d_reg, ctx->d_reg + NN,
+                             ctx->d_red + RED_SUMS, ctx->d_red, ctx->stream));
   return 0;
 }
 
@@ -2316,9 +2311,9 @@ int hr_regularization(hr_ctx* ctx, int method, const double* wreg, const double*
   if (int rc = check_wreg(ctx, wreg)) return rc;
   const double *dl, *dm;
   if (int rc = stage_material(ctx, lam, mu, &dl, &dm)) return rc;
-  if (int rc = regularize(ctx, method, wreg, dl, dm)) return rc;
+  if (int rc = regularize(ctx, method, wreg, dl, dm, nullptr, nullptr)) return rc;
   const size_t NN = (size_t)ctx->g.NN;
-  if (cost) if (int rc = copy_scalars(ctx, cost, ctx->d_red + dot_partials_size() + RED_OUT_COST, 2)) return rc;
+  if (cost) if (int rc = copy_scalars(ctx, cost, ctx->d_red + RED_COST, 2)) return rc;
   if (int rc = from_dev(ctx, reg_lam, ctx->d_reg, NN)) return rc;
   if (int rc = from_dev(ctx, reg_mu, ctx->d_reg + NN, NN)) return rc;
   HIPC(hipStreamSynchronize(ctx->stream));
@@ -2343,35 +2338,18 @@ int hr_regularize_gradient(hr_ctx* ctx, int iter, int method, double factor, con
     if (int rc = to_dev(ctx, gl, g_lambda, NN)) return rc;
     if (int rc = to_dev(ctx, gm, g_mu, NN)) return rc;
   }
-  if (int rc = regularize(ctx, method, wreg, dl, dm)) return rc;
-  // ||g||^2 and ||reg||^2 of both fields (VecNorm, Program_Main.F90:433-441)
-  const double* rl = ctx->d_reg;
-  const double* rm = ctx->d_reg + NN;
-  const double* xs[4] = {gl, rl, gm, rm};
-  double* out = ctx->d_red + dot_partials_size();
-  HIPC(launch_dots(4, (long long)NN, 1, xs, xs, ctx->d_red, out, ctx->stream));
-  double h[6];
-  HIPC(hipMemcpyAsync(h, out, 6 * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-  HIPC(hipStreamSynchronize(ctx->stream));
-  // adaptive factor; a zero regularisation vector (homogeneous field) gets
-  // factor 0 where the reference divides by zero
-  const double fl = h[1] > 0.0 ? factor * std::sqrt(h[0]) / std::sqrt(h[1]) : 0.0;
-  const double fm = h[3] > 0.0 ? factor * std::sqrt(h[2]) / std::sqrt(h[3]) : 0.0;
-  const int add = iter != 1;
-  HIPC(launch_reg_update((long long)NN, add, fl, fm, rl, rm, ctx->d_img, gl, gm, ctx->stream));
+  // ||g||^2 and ||reg||^2 of both fields with them (VecNorm, Program_Main.F90:433-441)
+  if (int rc = regularize(ctx, method, wreg, dl, dm, gl, gm)) return rc;
+  HIPC(launch_reg_update((long long)NN, iter != 1, factor, ctx->d_reg, ctx->d_reg + NN, ctx->d_img, gl, gm, ctx->d_red,
+                         ctx->stream));
   if (!dev) {
     HIPC(hipMemcpyAsync(g_lambda, gl, NN * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
     HIPC(hipMemcpyAsync(g_mu, gm, NN * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
   }
-  const double c[2] = {add ? h[4] * fl : 0.0, add ? h[5] * fm : 0.0};
-  const double f2[2] = {fl, fm};
-  if (dev) {
-    if (cost_reg) HIPC(hipMemcpyAsync(cost_reg, c, 2 * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
-    if (reg_factor) HIPC(hipMemcpyAsync(reg_factor, f2, 2 * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
-  } else {
-    if (cost_reg) { cost_reg[0] = c[0]; cost_reg[1] = c[1]; }
-    if (reg_factor) { reg_factor[0] = f2[0]; reg_factor[1] = f2[1]; }
-  }
+  // one copy where the two outputs adjoin
+  const bool both = cost_reg && reg_factor == cost_reg + 2;
+  if (cost_reg) if (int rc = copy_scalars(ctx, cost_reg, ctx->d_red + RED_SCALED, both ? 4 : 2)) return rc;
+  if (reg_factor && !both) if (int rc = copy_scalars(ctx, reg_factor, ctx->d_red + RED_FACTOR, 2)) return rc;
   HIPC(hipStreamSynchronize(ctx->stream));
   return 0;
 }

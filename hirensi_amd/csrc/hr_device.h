@@ -75,19 +75,18 @@ hipError_t launch_sum(int n, const double* in, double* out, hipStream_t s);
 hipError_t launch_misfit(int nstep, int ngrp, const int* gptr, const int* gidx, int nrec, const double* tr,
                          const double* ob, double dt, double* part, double* out, hipStream_t s);
 // gradient post-processing (hr_reg.hip)
-long long reg_box_elements(const Geo& g);
+size_t reg_partials_size(const Geo& g);      // doubles of part below
 hipError_t launch_gradient_mass(const Geo& g, double* img, double* restr, hipStream_t s);
-// tv: 1 total variation, 0 TN; wreg: host (w_top, w_bot, w_Length) or nullptr;
-// cost_el: 2 x reg_box_elements(g)
+// tv: 1 total variation, 0 TN; wreg: host (w_top, w_bot, w_Length) or nullptr; gl, gm:
+// gradients whose norms are wanted too, or nullptr; red (RED_SUMS doubles): ||gl||^2,
+// ||gm||^2, ||rl||^2, ||rm||^2, the two unscaled costs, then launch_reg_update's scaled
+// costs and factors
+constexpr int RED_SUMS = 10, RED_COST = 4, RED_SCALED = 6, RED_FACTOR = 8;
 hipError_t launch_regularization(const Geo& g, const double* zc, int tv, const double* wreg, const double* lam,
-                                 const double* mu, double* rl, double* rm, double* cost_el, hipStream_t s);
-// out[v] = x[v] . y[v] (y[v] == nullptr: sum of x[v]), v < nd <= 4, over n
-// entries spaced by stride; part: dot_partials_size() doubles
-hipError_t launch_dots(int nd, long long n, long long stride, const double* const* x, const double* const* y,
-                       double* part, double* out, hipStream_t s);
-int dot_partials_size();
-hipError_t launch_reg_update(long long n, int add, double fl, double fm, const double* rl, const double* rm,
-                             const double* img, double* gl, double* gm, hipStream_t s);
+                                 const double* mu, const double* gl, const double* gm, double* rl, double* rm,
+                                 double* part, double* red, hipStream_t s);
+hipError_t launch_reg_update(long long n, int add, double factor, const double* rl, const double* rm,
+                             const double* img, double* gl, double* gm, double* red, hipStream_t s);
 }  // namespace hr
 
 namespace hr {

@@ -11,9 +11,8 @@
 // the gradient of a nodal field at q is three 3-term sums along the lattice
 // lines through q, and the element vector scatters back along the same lines.
 //
-// Assembly is by element colour: the elements of one colour (ex, ey, ez
-// parities) share no node, so one launch per colour adds its element vectors
-// into the nodal output without atomics, in a fixed order (deterministic).
+// Sums over nodes and elements are taken per block in a fixed order and added by
+// one block in block order, so that a repeated call gives the same bits.
 #include <hip/hip_runtime.h>
 
 #include "hr_device.h"
@@ -39,100 +38,252 @@ __device__ __forceinline__ double f90_int4(double x) {
 struct RegArgs {
   Geo g;
   const double* zc;          // lattice z coordinates
-  int px, py, pz;            // colour (element parities relative to the box origin)
-  int cx, cy, cz;            // elements of this colour per axis
+  int ntx, nty, ntz, tz;     // tiles, element layers per z-chunk
   int weighted;              // Weighted_Regularization
   double w_top, w_bot, w_len;
   const double* m[2];        // lambda, mu (nodal)
-  double* r[2];              // regularisation vectors (nodal, accumulated)
-  double* cost_el;           // per box element: [2 * e + field]
+  const double* gr[2];       // misfit gradients (null: their norms are not taken)
+  double* r[2];              // regularisation vectors (nodal)
+  double* part;              // per-block sums, columns as reg_tail_kernel reads them
 };
 
-// One thread per element of the colour.  TV: reg_I += sum_q W_q F_q
-// (grad N_I . grad m) / sqrt(|grad m|^2 + 0.01), cost += W_q F_q
-// int(|grad m|^2) / sqrt(...); TN: reg = ER m, cost = 1/2 m.ER m.
-template <bool TV>
-__global__ __launch_bounds__(128) void reg_color_kernel(RegArgs A) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= A.cx * A.cy * A.cz) return;
-  const Geo& g = A.g;
-  const int ia = t % A.cx, ib = (t / A.cx) % A.cy, ic = t / (A.cx * A.cy);
-  const int rx = A.px + 2 * ia, ry = A.py + 2 * ib, rz = A.pz + 2 * ic;  // element inside the box
-  const int ex = g.rlo[0] + rx, ey = g.rlo[1] + ry, ez = g.rlo[2] + rz;
-  const long long NX = g.NX, NXY = (long long)g.NX * g.NY;
-  const long long n0 = 2 * ex + NX * (2 * ey) + NXY * (2 * ez);
-  const long long re = rx + (long long)(g.rhi[0] - g.rlo[0]) * (ry + (long long)(g.rhi[1] - g.rlo[1]) * rz);
-  double fac[3];
+constexpr int REG_THREADS = 256;
+constexpr int REG_BLOCKS = 4;                    // blocks per CU (128 VGPRs without spills)
+constexpr int REG_STREAM = 1024;                 // blocks that clear the rest of the lattice
+constexpr int RT = 4, RO = 2 * RT + 1, RNE = (RT + 1) * (RT + 1);
+constexpr int REW = 7;                           // elements per wavefront (9 lanes each)
+static_assert(4 * REW >= RNE && 3 * RO * RO <= REG_THREADS, "one block of four wavefronts");
+
+// sum of v over the block (every thread calls it; the result is thread 0's)
+__device__ double block_sum(double v, double* sh) {
+  const int tid = threadIdx.x;
 #pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    if (A.weighted) {
-      const double z = A.zc[2 * ez + k];
-      const double f2 = fabs(z / A.w_len);
-      fac[k] = (1.0 - f2) * A.w_top + f2 * A.w_bot;
-    } else {
-      fac[k] = 1.0;
+  for (int w = 32; w > 0; w >>= 1) v += __shfl_down(v, w);
+  if ((tid & 63) == 0) sh[tid >> 6] = v;
+  __syncthreads();
+  const double s = (sh[0] + sh[1]) + (sh[2] + sh[3]);
+  __syncthreads();
+  return s;
+}
+
+// TV: reg_I = sum_q W_q F_q (grad N_I . grad m) / sqrt(|grad m|^2 + 0.01), cost =
+// sum_q W_q F_q int(|grad m|^2) / sqrt(...); TN: reg = ER m, cost = 1/2 m.ER m.
+//
+// Tile blocks: a block owns the nodes of 4 x 4 elements in x-y and of a chunk of element
+// layers and marches up the chunk; the elements on the low side of the tile and
+// the layer below the chunk are computed again.  Nine lanes take an element,
+// each a z-line of three GLL points: the line's nodal values come from memory
+// once, the neighbouring lines' values and fluxes by lane shuffles, and the
+// element vectors go through LDS to the nodes' owners (at most four elements of a layer).
+// So each node is written once, with its share of ||reg||^2 taken on the way.
+// Stream blocks: zeros outside the box and ||g||^2 over the lattice.
+//
+// The instructions bound it (700 per layer and wavefront, a fifth of them shuffles): 57
+// us at 64x64x32 elements with PML 6, for 75 MB of traffic.  One launch per element
+// colour, which read and wrote every vector entry 3.4 times, with separate passes for
+// the zeros and the sums, took 250 us there.  The point's |grad m|^2 keeps its separate
+// multiplies and adds, as the cost truncates it.
+template <bool TV>
+__global__ __launch_bounds__(REG_THREADS, REG_BLOCKS) void reg_kernel(const RegArgs A) {
+  __shared__ double sR[2][RNE * 27 + 1];         // element vectors, and a spare
+  __shared__ double sh[4];
+  const Geo& g = A.g;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int ntile = A.ntx * A.nty * A.ntz;
+  const unsigned NXY = (unsigned)(g.NX * g.NY);
+  if ((int)blockIdx.x >= ntile) {
+    const int b = blockIdx.x - ntile;
+    double s0 = 0.0, s1 = 0.0;
+    for (long long n = b * (long long)REG_THREADS + tid; n < g.NN; n += (long long)REG_STREAM * REG_THREADS) {
+      const unsigned u = (unsigned)n, k = u / NXY, jk = u / (unsigned)g.NX;
+      const int i = (int)(u - jk * (unsigned)g.NX), j = (int)(jk - k * (unsigned)g.NY);
+      const bool box = i >= 2 * g.rlo[0] && i <= 2 * g.rhi[0] && j >= 2 * g.rlo[1] && j <= 2 * g.rhi[1] &&
+                       (int)k >= 2 * g.rlo[2] && (int)k <= 2 * g.rhi[2];
+      if (!box || ntile == 0) A.r[0][n] = A.r[1][n] = 0.0;
+      if (A.gr[0]) {
+        const double a = A.gr[0][n], c = A.gr[1][n];
+        s0 += a * a;
+        s1 += c * c;
+      }
     }
+    if (A.gr[0]) {
+      s0 = block_sum(s0, sh);
+      s1 = block_sum(s1, sh);
+      if (tid == 0) {
+        A.part[b] = s0;
+        A.part[REG_STREAM + b] = s1;
+      }
+    }
+    return;
+  }
+  // XCD-aware order: XCD x = blockIdx % 8 takes a contiguous run of the tiles (the
+  // first ntile / 8 of each; the rest of the blocks follow in order)
+  const int C = ntile / 8;
+  const int t = (int)blockIdx.x < 8 * C ? (blockIdx.x & 7) * C + (blockIdx.x >> 3) : (int)blockIdx.x;
+  const int tx = t % A.ntx, tz = (t / A.ntx) % A.ntz, ty = t / (A.ntx * A.ntz);
+  const int ex0 = g.rlo[0] + RT * tx, ey0 = g.rlo[1] + RT * ty, ez0 = g.rlo[2] + A.tz * tz;
+  const int ez_end = min(ez0 + A.tz, g.rhi[2]);
+  const int ez_first = max(ez0 - 1, g.rlo[2]);
+  // element role: z-line (slx, sly) of window element se (lanes without an element
+  // compute on a node that is there and store nothing)
+  const int le = lane < 9 * REW ? lane / 9 : 0, sq = lane < 9 * REW ? lane - 9 * le : 0;
+  const int se = REW * (tid >> 6) + le;
+  const int slx = sq % 3, sly = sq / 3;
+  const int sex = ex0 - 1 + se % (RT + 1), sey = ey0 - 1 + se / (RT + 1);
+  const bool elm = lane < 9 * REW && se < RNE && sex >= g.rlo[0] && sex < g.rhi[0] && sey >= g.rlo[1] && sey < g.rhi[1];
+  const bool mine = elm && sex >= ex0 && sey >= ey0;      // the tile's own elements: their cost
+  const unsigned sn = elm ? (unsigned)((2 * sex + slx) + g.NX * (2 * sey + sly))
+                          : (unsigned)(2 * g.rlo[0] + g.NX * (2 * g.rlo[1]));
+  auto dm = [](int q, int a) { return a == 0 ? (q - 1) - 0.5 : (a == 1 ? -2.0 * (q - 1) : (q - 1) + 0.5); };
+  double fx[3], fy[3], hx[3], hy[3];     // L_a' at this line's point, L' of this line's point at point a (x, y)
+  int nx[3], ny[3];                      // and the lanes of those lines
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    fx[a] = dm(slx, a);
+    fy[a] = dm(sly, a);
+    hx[a] = g.dxi[0] * dm(a, slx);
+    hy[a] = g.dxi[1] * dm(a, sly);
+    nx[a] = 9 * le + a + 3 * sly;
+    ny[a] = 9 * le + slx + 3 * a;
   }
   const double d0 = g.dxi[0], d1 = g.dxi[1], d2 = g.dxi[2];
-  for (int f = 0; f < 2; ++f) {
-    const double* __restrict__ M = A.m[f];
-    double m[27], r[27];
+  // owner role: column oc of the plane group P (planes k % 3 == P)
+  const int P = tid / (RO * RO), oc = tid - P * (RO * RO);
+  const int ix = oc % RO, iy = oc / RO;
+  const int i = 2 * ex0 + ix, j = 2 * ey0 + iy;
+  const bool owned = P < 3 && (ix < 2 * RT || tx == A.ntx - 1) && (iy < 2 * RT || ty == A.nty - 1) && i <= 2 * g.rhi[0] &&
+                     j <= 2 * g.rhi[1];
+  int fq[4];                             // the node's places in its elements' vectors
 #pragma unroll
-    for (int c = 0; c < 3; ++c)
-#pragma unroll
-      for (int b = 0; b < 3; ++b)
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-          m[a + 3 * b + 9 * c] = M[n0 + a + NX * b + NXY * c];
-          r[a + 3 * b + 9 * c] = 0.0;
-        }
-    double cost = 0.0;
-#pragma unroll
-    for (int k = 0; k < 3; ++k)
-#pragma unroll
-      for (int j = 0; j < 3; ++j)
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {
-          const int q = i + 3 * j + 9 * k;
-          double gx = 0.0, gy = 0.0, gz = 0.0;
-#pragma unroll
-          for (int a = 0; a < 3; ++a) {
-            gx += dl(i, a) * m[a + 3 * j + 9 * k];
-            gy += dl(j, a) * m[i + 3 * a + 9 * k];
-            gz += dl(k, a) * m[i + 3 * j + 9 * a];
-          }
-          gx *= d0;
-          gy *= d1;
-          gz *= d2;
-          const double s = (gx * gx + gy * gy) + gz * gz;
-          double w = g.wq[q] * fac[k];
-          if (TV) {
-            const double den = sqrt(s + 0.01);
-            cost += (f90_int4(s) / den) * w;
-            w = w / den;
-          } else {
-            cost += s * w;
-          }
-          const double wx = w * gx * d0, wy = w * gy * d1, wz = w * gz * d2;
-#pragma unroll
-          for (int a = 0; a < 3; ++a) {
-            r[a + 3 * j + 9 * k] += dl(i, a) * wx;
-            r[i + 3 * a + 9 * k] += dl(j, a) * wy;
-            r[i + 3 * j + 9 * a] += dl(k, a) * wz;
-          }
-        }
-    double* __restrict__ R = A.r[f];
-#pragma unroll
-    for (int c = 0; c < 3; ++c)
-#pragma unroll
-      for (int b = 0; b < 3; ++b)
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-          const long long n = n0 + a + NX * b + NXY * c;
-          R[n] = R[n] + r[a + 3 * b + 9 * c];
-        }
-    A.cost_el[2 * re + f] = TV ? cost : 0.5 * cost;
+  for (int q = 0; q < 4; ++q) {
+    const int a = q & 1, b = q >> 1;
+    const int lx = (ix & 1) ? 1 : 2 - 2 * a, ly = (iy & 1) ? 1 : 2 - 2 * b;
+    const int exi = (ix >> 1) + ((ix & 1) ? 1 : a), eyi = (iy >> 1) + ((iy & 1) ? 1 : b);
+    const int ex = ex0 - 1 + exi, ey = ey0 - 1 + eyi;
+    const bool ok = owned && !((ix & 1) && a) && !((iy & 1) && b) && ex >= g.rlo[0] && ex < g.rhi[0] && ey >= g.rlo[1] &&
+                    ey < g.rhi[1];
+    fq[q] = ok ? 27 * (exi + (RT + 1) * eyi) + lx + 3 * ly : -1;
   }
+  double m[2][3], acc[2] = {0.0, 0.0}, cost[2] = {0.0, 0.0}, rr[2] = {0.0, 0.0};
+#pragma unroll
+  for (int f = 0; f < 2; ++f)
+#pragma unroll
+    for (int z = 0; z < 3; ++z) m[f][z] = A.m[f][sn + NXY * (unsigned)(2 * ez_first + z)];
+  for (int ez = ez_first; ez < ez_end; ++ez) {
+    const bool halo = ez < ez0;
+    const int p = ((P - 2 * ez) % 3 + 3) % 3;    // this group's plane within the layer
+    const int k = 2 * ez + p;
+    const bool next = ez + 1 < ez_end;
+    double w3[3], mn[2][2];
+#pragma unroll
+    for (int z = 0; z < 3; ++z) {
+      w3[z] = g.wq[sq + 9 * z];
+      if (A.weighted) {
+        const double f2 = fabs(A.zc[2 * ez + z] / A.w_len);
+        w3[z] *= (1.0 - f2) * A.w_top + f2 * A.w_bot;
+      }
+    }
+#pragma unroll
+    for (int f = 0; f < 2; ++f)
+#pragma unroll
+      for (int z = 0; z < 2; ++z) mn[f][z] = next ? A.m[f][sn + NXY * (unsigned)(2 * ez + 3 + z)] : 0.0;
+#pragma unroll
+    for (int f = 0; f < 2; ++f) {
+      double X[3], Y[3], Z[3];
+#pragma unroll
+      for (int z = 0; z < 3; ++z) {
+        double gx = 0.0, gy = 0.0, gz = 0.0;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+          gx += fx[a] * __shfl(m[f][z], nx[a]);
+          gy += fy[a] * __shfl(m[f][z], ny[a]);
+          gz += dl(z, a) * m[f][a];
+        }
+        gx *= d0;
+        gy *= d1;
+        gz *= d2;
+        const double s = (gx * gx + gy * gy) + gz * gz;
+        double w = w3[z], c;
+        if (TV) {
+          w = w * rsqrt(s + 0.01);
+          c = f90_int4(s) * w;
+        } else {
+          c = s * w;
+        }
+        if (mine && !halo) cost[f] += c;
+        X[z] = w * gx;
+        Y[z] = w * gy;
+        Z[z] = w * gz * d2;
+      }
+#pragma unroll
+      for (int z = 0; z < 3; ++z) {
+        double r = 0.0;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+          r = fma(hx[a], __shfl(X[z], nx[a]), r);
+          r = fma(hy[a], __shfl(Y[z], ny[a]), r);
+          r = fma(dl(a, z), Z[a], r);
+        }
+        sR[f][elm ? 27 * se + sq + 9 * z : RNE * 27] = r;
+      }
+      m[f][0] = m[f][2];
+      m[f][1] = mn[f][0];
+      m[f][2] = mn[f][1];
+    }
+    __syncthreads();
+    if (owned && (!halo || p == 2)) {
+      // a plane starts afresh unless the layer below started it
+      const bool fresh = p != 0 || ez == ez_first;
+#pragma unroll
+      for (int f = 0; f < 2; ++f) {
+        double s = fresh ? 0.0 : acc[f];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const double v = sR[f][(fq[q] >= 0 ? fq[q] : 0) + 9 * p];
+          s += fq[q] >= 0 ? v : 0.0;
+        }
+        acc[f] = s;
+      }
+      if (!halo && (p < 2 || ez == g.rhi[2] - 1)) {
+        const unsigned n = (unsigned)i + (unsigned)g.NX * (unsigned)j + NXY * (unsigned)k;
+#pragma unroll
+        for (int f = 0; f < 2; ++f) {
+          A.r[f][n] = acc[f];
+          rr[f] += acc[f] * acc[f];
+        }
+      }
+    }
+    __syncthreads();
+  }
+  double* const part = A.part + 2 * REG_STREAM;
+#pragma unroll
+  for (int f = 0; f < 2; ++f) {
+    const double a = block_sum(rr[f], sh), c = block_sum(cost[f], sh);
+    if (tid == 0) {
+      part[f * ntile + blockIdx.x] = a;
+      part[(2 + f) * ntile + blockIdx.x] = TV ? c : 0.5 * c;
+    }
+  }
+}
+
+// out = [||g_l||^2, ||g_m||^2 (when taken), ||r_l||^2, ||r_m||^2, cost_l, cost_m]: one
+// wavefront per sum
+__global__ __launch_bounds__(384) void reg_tail_kernel(int ntile, int norms, const double* __restrict__ part,
+                                                       double* __restrict__ out) {
+  const int v = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  if (v < 2 && !norms) return;
+  const double* const p = v < 2 ? part + v * REG_STREAM : part + 2 * REG_STREAM + (long long)(v - 2) * ntile;
+  const int n = v < 2 ? REG_STREAM : ntile;
+  double s[4] = {0.0, 0.0, 0.0, 0.0};
+  int q = lane;
+  for (; q + 192 < n; q += 256)
+#pragma unroll
+    for (int u = 0; u < 4; ++u) s[u] += p[q + 64 * u];
+  for (; q < n; q += 64) s[0] += p[q];
+  double a = (s[0] + s[1]) + (s[2] + s[3]);
+#pragma unroll
+  for (int w = 32; w > 0; w >>= 1) a += __shfl_down(a, w);
+  if (lane == 0) out[v] = a;
 }
 
 // Gradient mass at a lattice node: the GLL weights x det J of the box elements
@@ -167,57 +318,17 @@ __global__ __launch_bounds__(256) void gradient_mass_kernel(Geo g, double* __res
   }
 }
 
-__global__ __launch_bounds__(256) void fill2_kernel(long long n, double* __restrict__ a, double* __restrict__ b) {
-  for (long long q = blockIdx.x * (long long)blockDim.x + threadIdx.x; q < n; q += (long long)gridDim.x * blockDim.x) {
-    a[q] = 0.0;
-    b[q] = 0.0;
-  }
-}
-
-// Deterministic dot products: part[4 * blockIdx + v] = partial sums of
-// x_v . y_v over a fixed grid-stride split; the tail kernel adds the partials
-// in block order.
-constexpr int RED_BLOCKS = 256;
-constexpr int RED_THREADS = 256;
-
-struct DotArgs {
-  int nd;                    // number of dot products (<= 4)
-  long long n;
-  long long stride;          // element stride inside x and y
-  const double* x[4];
-  const double* y[4];        // nullptr: plain sum of x
-};
-
-__global__ __launch_bounds__(RED_THREADS) void dot_partial_kernel(DotArgs A, double* __restrict__ part) {
-  __shared__ double sh[RED_THREADS];
-  for (int v = 0; v < A.nd; ++v) {
-    double s = 0.0;
-    for (long long q = blockIdx.x * (long long)RED_THREADS + threadIdx.x; q < A.n; q += (long long)RED_BLOCKS * RED_THREADS)
-      s += A.y[v] ? A.x[v][q * A.stride] * A.y[v][q * A.stride] : A.x[v][q * A.stride];
-    sh[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = RED_THREADS / 2; w > 0; w >>= 1) {
-      if ((int)threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) part[blockIdx.x * 4 + v] = sh[0];
-    __syncthreads();
-  }
-}
-
-__global__ __launch_bounds__(64) void dot_tail_kernel(int nd, const double* __restrict__ part, double* __restrict__ out) {
-  if (threadIdx.x < nd) {
-    double s = 0.0;
-    for (int b = 0; b < RED_BLOCKS; ++b) s += part[b * 4 + threadIdx.x];
-    out[threadIdx.x] = s;
-  }
-}
-
-// g <- (g + f * reg) * img  (add = 1), g <- g * img (add = 0)
-__global__ __launch_bounds__(256) void reg_update_kernel(long long n, int add, double fl, double fm,
+// The adaptive factors f = factor ||g|| / ||reg|| (0 when ||reg|| = 0, a homogeneous
+// field, where the reference divides by zero) from the sums in red, then
+// g <- (g + f reg) img (add = 1), g <- g img (add = 0); red[6..9] = the scaled costs
+// and the factors.  One pass at copy speed; the factors are two divides a
+// thread, where reading the sums back first made the host wait between the passes.
+__global__ __launch_bounds__(256) void reg_update_kernel(long long n, int add, double factor,
                                                          const double* __restrict__ rl, const double* __restrict__ rm,
                                                          const double* __restrict__ img, double* __restrict__ gl,
-                                                         double* __restrict__ gm) {
+                                                         double* __restrict__ gm, double* red) {
+  const double fl = red[2] > 0.0 ? factor * sqrt(red[0]) / sqrt(red[2]) : 0.0;
+  const double fm = red[3] > 0.0 ? factor * sqrt(red[1]) / sqrt(red[3]) : 0.0;
   for (long long q = blockIdx.x * (long long)blockDim.x + threadIdx.x; q < n; q += (long long)gridDim.x * blockDim.x) {
     double a = gl[q], b = gm[q];
     if (add) {
@@ -226,6 +337,12 @@ __global__ __launch_bounds__(256) void reg_update_kernel(long long n, int add, d
     }
     gl[q] = a * img[q];
     gm[q] = b * img[q];
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    red[6] = add ? red[4] * fl : 0.0;
+    red[7] = add ? red[5] * fm : 0.0;
+    red[8] = fl;
+    red[9] = fm;
   }
 }
 
@@ -238,8 +355,32 @@ int grid_for(long long n, int threads) {
 
 }  // namespace
 
-long long reg_box_elements(const Geo& g) {
-  return (long long)(g.rhi[0] - g.rlo[0]) * (g.rhi[1] - g.rlo[1]) * (g.rhi[2] - g.rlo[2]);
+namespace {
+
+// Tiles and z-chunks of the regularisation kernel: the chunk with the fewest element
+// layers in sequence, rounds of blocks (REG_BLOCKS per CU run at once) times layers
+// per block, the halo layer with them; of equals the longest.  At 64x64x32 elements
+// (13 x 13 tiles) five layers, 1014 blocks: 57 us; four layers, 1183 blocks, 67 us.
+void reg_tiles(const Geo& g, int t[3], int& tz) {
+  const int R[3] = {g.rhi[0] - g.rlo[0], g.rhi[1] - g.rlo[1], g.rhi[2] - g.rlo[2]};
+  for (int d = 0; d < 2; ++d) t[d] = R[d] > 0 ? (R[d] + RT - 1) / RT : 0;
+  tz = R[2];
+  t[2] = R[2] > 0 ? 1 : 0;
+  const long long slots = 256 * REG_BLOCKS;
+  long long best = -1;
+  for (int c = R[2]; c >= 1; --c) {
+    const int n = (R[2] + c - 1) / c;
+    const long long cost = ((long long)t[0] * t[1] * n + slots - 1) / slots * (c + (n > 1));
+    if (best < 0 || cost < best) { best = cost; tz = c; t[2] = n; }
+  }
+}
+
+}  // namespace
+
+size_t reg_partials_size(const Geo& g) {
+  int t[3], tz;
+  reg_tiles(g, t, tz);
+  return 2 * REG_STREAM + 4 * (size_t)t[0] * t[1] * t[2];
 }
 
 hipError_t launch_gradient_mass(const Geo& g, double* img, double* restr, hipStream_t s) {
@@ -248,8 +389,8 @@ hipError_t launch_gradient_mass(const Geo& g, double* img, double* restr, hipStr
 }
 
 hipError_t launch_regularization(const Geo& g, const double* zc, int tv, const double* wreg, const double* lam,
-                                 const double* mu, double* rl, double* rm, double* cost_el, hipStream_t s) {
-  hipLaunchKernelGGL(fill2_kernel, dim3(grid_for(g.NN, 256)), dim3(256), 0, s, g.NN, rl, rm);
+                                 const double* mu, const double* gl, const double* gm, double* rl, double* rm,
+                                 double* part, double* red, hipStream_t s) {
   RegArgs A{};
   A.g = g;
   A.zc = zc;
@@ -261,48 +402,27 @@ hipError_t launch_regularization(const Geo& g, const double* zc, int tv, const d
   }
   A.m[0] = lam;
   A.m[1] = mu;
+  A.gr[0] = gl;
+  A.gr[1] = gm;
   A.r[0] = rl;
   A.r[1] = rm;
-  A.cost_el = cost_el;
-  const int R[3] = {g.rhi[0] - g.rlo[0], g.rhi[1] - g.rlo[1], g.rhi[2] - g.rlo[2]};
-  for (int col = 0; col < 8; ++col) {
-    A.px = col & 1;
-    A.py = (col >> 1) & 1;
-    A.pz = (col >> 2) & 1;
-    A.cx = (R[0] - A.px + 1) / 2;
-    A.cy = (R[1] - A.py + 1) / 2;
-    A.cz = (R[2] - A.pz + 1) / 2;
-    const long long ne = (long long)A.cx * A.cy * A.cz;
-    if (ne <= 0) continue;
-    const int blocks = (int)((ne + 127) / 128);
-    if (tv)
-      hipLaunchKernelGGL(reg_color_kernel<true>, dim3(blocks), dim3(128), 0, s, A);
-    else
-      hipLaunchKernelGGL(reg_color_kernel<false>, dim3(blocks), dim3(128), 0, s, A);
-  }
+  A.part = part;
+  int t[3];
+  reg_tiles(g, t, A.tz);
+  A.ntx = t[0];
+  A.nty = t[1];
+  A.ntz = t[2];
+  const int ntile = t[0] * t[1] * t[2];
+  if (tv) reg_kernel<true><<<ntile + REG_STREAM, REG_THREADS, 0, s>>>(A);
+  else reg_kernel<false><<<ntile + REG_STREAM, REG_THREADS, 0, s>>>(A);
+  reg_tail_kernel<<<1, 384, 0, s>>>(ntile, gl != nullptr, part, red);
   return hipGetLastError();
 }
 
-hipError_t launch_dots(int nd, long long n, long long stride, const double* const* x, const double* const* y,
-                       double* part, double* out, hipStream_t s) {
-  DotArgs A{};
-  A.nd = nd;
-  A.n = n;
-  A.stride = stride;
-  for (int v = 0; v < nd; ++v) {
-    A.x[v] = x[v];
-    A.y[v] = y[v];
-  }
-  hipLaunchKernelGGL(dot_partial_kernel, dim3(RED_BLOCKS), dim3(RED_THREADS), 0, s, A, part);
-  hipLaunchKernelGGL(dot_tail_kernel, dim3(1), dim3(64), 0, s, nd, part, out);
-  return hipGetLastError();
-}
-
-int dot_partials_size() { return RED_BLOCKS * 4; }
-
-hipError_t launch_reg_update(long long n, int add, double fl, double fm, const double* rl, const double* rm,
-                             const double* img, double* gl, double* gm, hipStream_t s) {
-  hipLaunchKernelGGL(reg_update_kernel, dim3(grid_for(n, 256)), dim3(256), 0, s, n, add, fl, fm, rl, rm, img, gl, gm);
+hipError_t launch_reg_update(long long n, int add, double factor, const double* rl, const double* rm,
+                             const double* img, double* gl, double* gm, double* red, hipStream_t s) {
+  hipLaunchKernelGGL(reg_update_kernel, dim3(grid_for(n, 256)), dim3(256), 0, s, n, add, factor, rl, rm, img, gl, gm,
+                     red);
   return hipGetLastError();
 }
 
