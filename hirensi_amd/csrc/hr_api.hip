@@ -774,9 +774,8 @@ int record_step(hr_ctx* ctx, int n) {
   if (ctx->f_nrec <= 0) return 0;
   const size_t nf = field_size(ctx), rows = (size_t)ctx->f_nstep + 1;
   const StepRef sr{ctx->dyn ? ctx->d_step : nullptr, ctx->f_nrec};
-  for (int q = 0; q < ctx->nshot; ++q)
-    HIPC(launch_record(ctx->f_nrec, ctx->d_rec_slot, ctx->x[1] + q * nf,
-                       ctx->d_traces + ((size_t)q * rows + n) * ctx->f_nrec, ctx->stream, sr));
+  HIPC(launch_record(ctx->f_nrec, ctx->d_rec_slot, ctx->nshot, ctx->x[1], (long long)nf,
+                     ctx->d_traces + (size_t)n * ctx->f_nrec, (long long)(rows * ctx->f_nrec), ctx->stream, sr));
   return 0;
 }
 
@@ -784,9 +783,8 @@ int record_step(hr_ctx* ctx, int n) {
 int store_slice(hr_ctx* ctx, double* base, size_t rows, size_t row) {
   const size_t nf = field_size(ctx), slice = 3 * (size_t)ctx->nbox;
   const StepRef sr{ctx->dyn ? ctx->d_step : nullptr, (long long)slice};
-  for (int q = 0; q < ctx->nshot; ++q)
-    HIPC(launch_store_box(ctx->g, ctx->box0, ctx->boxn, ctx->x[1] + q * nf, base + ((size_t)q * rows + row) * slice,
-                          ctx->stream, sr));
+  HIPC(launch_store_box(ctx->g, ctx->box0, ctx->boxn, ctx->nshot, ctx->x[1], (long long)nf, base + row * slice,
+                        (long long)(rows * slice), ctx->stream, sr));
   return 0;
 }
 
@@ -1846,11 +1844,12 @@ int hr_adjoint_gradient(hr_ctx* ctx, int nstep, double dt, int nrec, const long 
     HIPC(launch_permute_cols((long long)nshot * rows, nrec, ctx->d_rec_perm, ctx->d_obs, ctx->d_obs_sorted,
                              ctx->stream));
   }
-  // gradient accumulators on the RD box (sum over shots)
-  if (int rc = dalloc(ctx, &ctx->d_gl, ctx->nbox)) return rc;
-  if (int rc = dalloc(ctx, &ctx->d_gm, ctx->nbox)) return rc;
-  HIPC(hipMemsetAsync(ctx->d_gl, 0, ctx->nbox * sizeof(double), ctx->stream));
-  HIPC(hipMemsetAsync(ctx->d_gm, 0, ctx->nbox * sizeof(double), ctx->stream));
+  // gradient accumulators on the RD box, per shot
+  const size_t ngrad = (size_t)ctx->nbox * nshot;
+  if (int rc = dalloc(ctx, &ctx->d_gl, ngrad)) return rc;
+  if (int rc = dalloc(ctx, &ctx->d_gm, ngrad)) return rc;
+  HIPC(hipMemsetAsync(ctx->d_gl, 0, ngrad * sizeof(double), ctx->stream));
+  HIPC(hipMemsetAsync(ctx->d_gm, 0, ngrad * sizeof(double), ctx->stream));
   const size_t slice = 3 * (size_t)ctx->nbox;
   const double sgn[3] = {-1.0, 1.0, -1.0};
   const size_t nf = field_size(ctx);
@@ -1885,9 +1884,8 @@ int hr_adjoint_gradient(hr_ctx* ctx, int nstep, double dt, int nrec, const long 
       double* const a1 = P[1];
       const StepRef sr{ctx->dyn ? ctx->d_step : nullptr, (long long)slice};
       ctx->deferred.push_back([ctx, nshot, uh, uh_rows, uh_row, slice, a1, nf, dt, sr]() -> int {
-        for (int q = 0; q < nshot; ++q)
-          HIPC(launch_gradient(ctx->g, ctx->box0, ctx->boxn, uh + ((size_t)q * uh_rows + uh_row) * slice,
-                               a1 + q * nf, dt, ctx->d_gl, ctx->d_gm, ctx->stream, sr));
+        HIPC(launch_gradient(ctx->g, ctx->box0, ctx->boxn, nshot, uh + uh_row * slice, (long long)(uh_rows * slice),
+                             a1, (long long)nf, dt, ctx->d_gl, ctx->d_gm, ctx->stream, sr));
         return 0;
       });
     }
@@ -1966,7 +1964,7 @@ int hr_adjoint_gradient(hr_ctx* ctx, int nstep, double dt, int nrec, const long 
   }
   HIPC(hipMemsetAsync(dgl, 0, NN * sizeof(double), ctx->stream));
   HIPC(hipMemsetAsync(dgm, 0, NN * sizeof(double), ctx->stream));
-  HIPC(launch_gradient_finish(ctx->g, ctx->box0, ctx->boxn, ctx->d_gl, ctx->d_gm, dgl, dgm, ctx->stream));
+  HIPC(launch_gradient_finish(ctx->g, ctx->box0, ctx->boxn, nshot, ctx->d_gl, ctx->d_gm, dgl, dgm, ctx->stream));
   if (!dev) {
     HIPC(hipMemcpyAsync(g_lambda, dgl, NN * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
     HIPC(hipMemcpyAsync(g_mu, dgm, NN * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
@@ -2114,11 +2112,11 @@ int hr_gradient_accumulate(hr_ctx* ctx, const double* u, const double* p, double
   if (int rc = dalloc(ctx, &ctx->d_uslice, 3 * (size_t)ctx->nbox)) return rc;
   if (int rc = dalloc(ctx, &ctx->d_gl, ctx->nbox)) return rc;
   if (int rc = dalloc(ctx, &ctx->d_gm, ctx->nbox)) return rc;
-  HIPC(launch_store_box(ctx->g, ctx->box0, ctx->boxn, ctx->tmp, ctx->d_uslice, ctx->stream));
+  HIPC(launch_store_box(ctx->g, ctx->box0, ctx->boxn, 1, ctx->tmp, 0, ctx->d_uslice, 0, ctx->stream));
   HIPC(hipMemsetAsync(ctx->d_gl, 0, ctx->nbox * sizeof(double), ctx->stream));
   HIPC(hipMemsetAsync(ctx->d_gm, 0, ctx->nbox * sizeof(double), ctx->stream));
-  HIPC(launch_gradient(ctx->g, ctx->box0, ctx->boxn, ctx->d_uslice, ctx->tmp2, scale, ctx->d_gl, ctx->d_gm,
-                       ctx->stream));
+  HIPC(launch_gradient(ctx->g, ctx->box0, ctx->boxn, 1, ctx->d_uslice, 0, ctx->tmp2, 0, scale, ctx->d_gl,
+                       ctx->d_gm, ctx->stream));
   double *gl = g_lambda, *gm = g_mu;
   if (!dev) {
     if (int rc = dalloc(ctx, &ctx->d_pg, 2 * NN)) return rc;

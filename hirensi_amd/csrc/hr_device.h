@@ -51,16 +51,19 @@ struct StepRef {
   const int* step = nullptr;
   long long stride = 0;
 };
-hipError_t launch_record(int nrec, const long long* slot, const double* x2, double* row, hipStream_t s,
-                         StepRef sr = StepRef());
-hipError_t launch_store_box(const Geo& g, const int* box0, const int* boxn, const double* x2, double* hist,
-                            hipStream_t s, StepRef sr = StepRef());
-hipError_t launch_gradient(const Geo& g, const int* box0, const int* boxn, const double* uh, const double* p2,
-                           double dt, double* glam, double* gmu, hipStream_t s, StepRef sr = StepRef());
+// per-step kernels over all shots: strides between the shots' x2, rows, slices
+hipError_t launch_record(int nrec, const long long* slot, int nshot, const double* x2, long long xstride, double* row,
+                         long long rstride, hipStream_t s, StepRef sr = StepRef());
+hipError_t launch_store_box(const Geo& g, const int* box0, const int* boxn, int nshot, const double* x2,
+                            long long xstride, double* hist, long long hstride, hipStream_t s, StepRef sr = StepRef());
+// glam, gmu: one block of box sums per shot
+hipError_t launch_gradient(const Geo& g, const int* box0, const int* boxn, int nshot, const double* uh,
+                           long long ustride, const double* p2, long long pstride, double dt, double* glam, double* gmu,
+                           hipStream_t s, StepRef sr = StepRef());
 // *step = value; *step += delta (one lane, a vector store)
 hipError_t launch_step_set(int* step, int value, hipStream_t s);
 hipError_t launch_step_advance(int* step, int delta, hipStream_t s);
-hipError_t launch_gradient_finish(const Geo& g, const int* box0, const int* boxn, const double* glb,
+hipError_t launch_gradient_finish(const Geo& g, const int* box0, const int* boxn, int nshot, const double* glb,
                                   const double* gmb, double* gl, double* gm, hipStream_t s);
 hipError_t launch_permute_cols(long long nrows, int ncols, const long long* perm, const double* src, double* dst,
                                hipStream_t s);

@@ -10,16 +10,11 @@
 // Inactive entries are zero and never written.
 
 #include <hip/hip_runtime.h>
-#include "hr_device.h"
+#include "hr_lattice.h"
 
 #pragma clang fp contract(off)
 
 namespace hr {
-
-// 1D GLL derivative matrix: DM[a][b] = l_b'(xi_a), xi = -1, 0, 1
-__constant__ double c_dm[9] = {-1.5, 2.0, -0.5, -0.5, 0.0, 0.5, 0.5, -2.0, 1.5};
-
-__device__ __forceinline__ double DM(int a, int b) { return c_dm[3 * a + b]; }
 
 // ----------------------------------------------------- small kernels
 // lattice <- reference numbering (optionally scaled): out[slot[e]] = x[e] * r[e]
@@ -42,10 +37,13 @@ __global__ void scatter_eq_kernel(long long neq, const long long* __restrict__ s
   }
 }
 
-// receiver traces: row[r] = x2[slot[r]]
+// receiver traces of shot blockIdx.y: row[r] = x2[slot[r]]
 __global__ void record_kernel(int nrec, const long long* __restrict__ slot, const double* __restrict__ x2,
-                              double* __restrict__ row, const int* __restrict__ step, long long stride) {
+                              long long xstride, double* __restrict__ row, long long rstride,
+                              const int* __restrict__ step, long long stride) {
   const int r = blockIdx.x * blockDim.x + threadIdx.x;
+  x2 += blockIdx.y * xstride;
+  row += blockIdx.y * rstride;
   if (step) row += (long long)(*step) * stride;
   if (r < nrec) row[r] = x2[slot[r]];
 }
@@ -58,14 +56,16 @@ __global__ void step_advance_kernel(int* __restrict__ step, int delta) {
   if (threadIdx.x == 0) step[0] = step[0] + delta;
 }
 
-// displacement of the regular-domain node box -> history slice (3 x nbox,
-// component-major): a thread reads one node's three contiguous components and
+// displacement of the regular-domain node box of shot blockIdx.y -> history slice (3 x
+// nbox, component-major): a thread reads one node's three contiguous components and
 // writes them to the three component planes (each plane coalesced across lanes)
 __global__ void store_box_kernel(Geo g, int bi0, int bj0, int bk0, int bnx, int bny, int bnz,
-                                 const double* __restrict__ x2, double* __restrict__ hist,
-                                 const int* __restrict__ step, long long stride) {
+                                 const double* __restrict__ x2, long long xstride, double* __restrict__ hist,
+                                 long long hstride, const int* __restrict__ step, long long stride) {
   // 32-bit indices: 9 NN < 2^31 (checked by the host)
   const int nbox = bnx * bny * bnz;
+  x2 += blockIdx.y * xstride;
+  hist += blockIdx.y * hstride;
   if (step) hist += (long long)(*step) * stride;
   for (int r = blockIdx.x * blockDim.x + threadIdx.x; r < nbox; r += gridDim.x * blockDim.x) {
     const int bi = r % bnx, bj = (r / bnx) % bny, bk = r / (bnx * bny);
@@ -82,213 +82,190 @@ __global__ void store_box_kernel(Geo g, int bi0, int bj0, int bk0, int bnx, int 
 // sum over the regular-domain elements containing it of W * div u * div p and
 // W * [2 eps(u):eps(p) in the reference's component form], times dt.
 // u comes from the history slice (3 x nbox), p from the adjoint x2 (lattice).
-__global__ void gradient_kernel(Geo g, int bi0, int bj0, int bk0, int bnx, int bny, int bnz,
-                                const double* __restrict__ uh, const double* __restrict__ p2, double dt,
-                                double* __restrict__ glam, double* __restrict__ gmu) {
-  // 32-bit indices: 9 NN < 2^31 (checked by the host)
-  const int nbox = bnx * bny * bnz;
-  for (int r = blockIdx.x * blockDim.x + threadIdx.x; r < nbox; r += gridDim.x * blockDim.x) {
-    const int bi = r % bnx, bj = (r / bnx) % bny, bk = r / (bnx * bny);
-    const int pos[3] = {bi0 + bi, bj0 + bj, bk0 + bk};
-    const int n = pos[0] + g.NX * (pos[1] + g.NY * pos[2]);
-    const int stride[3] = {1, bnx, bnx * bny};
-    const int lstride[3] = {1, g.NX, g.NX * g.NY};
-    // per axis two element sides: s = 0 the element below (local 2; local 1 for an
-    // odd node), s = 1 the element above (local 0).  Only sides whose element is
-    // in the regular-domain range of the axis are used: their stencils stay in
-    // the regular-domain node box.
-    bool has[3][2];
-    int el[3][2], lo[3][2];
-    double du[3][2][3], dp[3][2][3];
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-      const int q = pos[a];
-      const bool odd = q & 1;
-      el[a][0] = odd ? (q - 1) >> 1 : (q >> 1) - 1;
-      lo[a][0] = odd ? 1 : 2;
-      el[a][1] = q >> 1;
-      lo[a][1] = 0;
-      has[a][0] = el[a][0] >= g.rlo[a] && el[a][0] < g.rhi[a];
-      has[a][1] = !odd && el[a][1] >= g.rlo[a] && el[a][1] < g.rhi[a];
-#pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        const int l = lo[a][s];
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-          double su = 0.0, sp = 0.0;
-          if (has[a][s]) {
-#pragma unroll
-            for (int m = 0; m < 3; ++m) {
-              const int off = m - l;
-              su += DM(l, m) * uh[c * nbox + r + off * stride[a]];
-              sp += DM(l, m) * p2[3 * (n + off * lstride[a]) + c];
-            }
-          }
-          du[a][s][c] = g.dxi[a] * su;
-          dp[a][s][c] = g.dxi[a] * sp;
-        }
-      }
-    }
-    double sl = 0.0, sm = 0.0;
-#pragma unroll
-    for (int sx = 0; sx < 2; ++sx)
-#pragma unroll
-      for (int sy = 0; sy < 2; ++sy)
-#pragma unroll
-        for (int sz = 0; sz < 2; ++sz) {
-          if (!(has[0][sx] && has[1][sy] && has[2][sz])) continue;
-          const double u1x = du[0][sx][0], u2x = du[0][sx][1], u3x = du[0][sx][2];
-          const double u1y = du[1][sy][0], u2y = du[1][sy][1], u3y = du[1][sy][2];
-          const double u1z = du[2][sz][0], u2z = du[2][sz][1], u3z = du[2][sz][2];
-          const double p1x = dp[0][sx][0], p2x = dp[0][sx][1], p3x = dp[0][sx][2];
-          const double p1y = dp[1][sy][0], p2y = dp[1][sy][1], p3y = dp[1][sy][2];
-          const double p1z = dp[2][sz][0], p2z = dp[2][sz][1], p3z = dp[2][sz][2];
-          const double sL = (u1x + u2y + u3z) * (p1x + p2y + p3z);
-          const double sM = 2.0 * (u1x * p1x + u2y * p2y + u3z * p3z) + (p1y + p2x) * (u1y + u2x) +
-                            (p1z + p3x) * (u1z + u3x) + (p3y + p2z) * (u3y + u2z);
-          const double W = g.wq[lo[0][sx] + 3 * lo[1][sy] + 9 * lo[2][sz]];
-          sl += sL * W;
-          sm += sM * W;
-        }
-    glam[r] += sl * dt;
-    gmu[r] += sm * dt;
-  }
-}
-
-// The same per-step gradient, tiled: a block owns GTX x GTY box nodes in x-y
-// and marches up a chunk of GZC planes.  Each value of u and p is read from
-// memory once per block (plus a halo of two nodes in x and y and two planes in z):
-// the thread of a column keeps the planes k-2..k+2 of its own u and p in
-// registers (z stencils), the plane k of the block's window sits in LDS (x and y
-// stencils).  Sums and their order are those of gradient_kernel, so the results
-// are identical.
-constexpr int GTX = 32, GTY = 8, GH = 2, GZC = 4;
-constexpr int GWX = GTX + 2 * GH, GWY = GTY + 2 * GH;
+//
+// Per axis a node has one element side (odd coordinate) or two (even: below and
+// above), each with its own derivatives; the weight W = w_x w_y w_z is the same for all
+// the elements of a node.  The sum over the up to eight elements of a product of
+// derivatives along axes a and b then splits into sums over sides: of products
+// for a = b, times the number of sides of the other two axes, and a product of sums
+// for a != b, times that of the third axis.  A side outside the box enters with
+// zero coefficients.
+//
+// A block owns GTX x GTY box columns and marches up a chunk of planes.  The thread of a
+// column keeps the planes k-2..k+2 of its own u and p in registers (z stencils); plane k
+// of the block's window, with a halo of two nodes, sits in LDS (x and y stencils).
+// What plane k + 1 needs is loaded before plane k is worked on, and the two LDS
+// planes alternate, so a plane costs one barrier and no load in its path.  All shots
+// go in one launch, each with accumulators of its own: one small box alone has too
+// few blocks for the GPU.
+// One call alone: 64x64x32 elements with PML 6, 41 -> 19 us (47 MB, about half
+// the copy rate); 32x32x16 with PML 4, 18 -> 6 us.
+constexpr int GTX = 32, GTY = 8, GH = 2;
+constexpr int GWX = GTX + 2 * GH, GWY = GTY + 2 * GH, GW = GWX * GWY;
 constexpr int GNT = GTX * GTY;
 // halo positions read by the stencils: rows 0, 1 and GWY-2, GWY-1 over the owned
 // columns (y stencils), columns 0, 1 and GWX-2, GWX-1 over the owned rows (x stencils)
 constexpr int GHALO = 2 * 2 * GTX + 2 * 2 * GTY;
+static_assert(GHALO <= GNT, "one halo position per thread");
+constexpr int GBLOCKS = 2;                     // blocks per CU: three spill 100 registers (79 us for 19)
 
-__global__ void __launch_bounds__(GNT) gradient_tile_kernel(Geo g, int bi0, int bj0, int bk0, int bnx, int bny,
-                                                            int bnz, const double* __restrict__ uh,
-                                                            const double* __restrict__ p2, double dt,
-                                                            double* __restrict__ glam, double* __restrict__ gmu,
-                                                            const int* __restrict__ step, long long stride) {
-  __shared__ double sU[3][GWY][GWX], sP[3][GWY][GWX];
-  if (step) uh += (long long)(*step) * stride;
+// one axis' sides of u and p: sums over the sides of each component, and of the
+// products of equal components
+struct Sides {
+  double u[3], p[3], d[3];
+};
+
+__global__ void __launch_bounds__(GNT, GBLOCKS) gradient_tile_kernel(
+    Geo g, int bi0, int bj0, int bk0, int bnx, int bny, int bnz, int ntx, int nty, int ntz, int tz, int nshot,
+    const double* __restrict__ uh, long long ustride, const double* __restrict__ p2, long long pstride, double dt,
+    double* __restrict__ glam, double* __restrict__ gmu, const int* __restrict__ step, long long stride) {
+#pragma clang fp contract(fast)
+  __shared__ double sU[2][3][GW], sP[2][3][GW];
   const int tid = threadIdx.x;
   const int tx = tid % GTX, ty = tid / GTX;
-  const int ti0 = blockIdx.x * GTX, tj0 = blockIdx.y * GTY;
-  const int kc0 = blockIdx.z * GZC, kc1 = min(kc0 + GZC, bnz);
+  const int ntile = ntx * nty * ntz, ntot = ntile * nshot;
+  // XCD-aware order: XCD x = blockIdx % 8 takes a contiguous run of the (shot, z, y, x) tiles
+  const int C = (ntot + 7) / 8;
+  const int li = (blockIdx.x & 7) * C + (blockIdx.x >> 3);
+  if (li >= ntot) return;
+  const int shot = li / ntile, t = li - shot * ntile;
+  const int nbox = bnx * bny * bnz;              // 32-bit: 9 NN < 2^31 (checked by the host)
+  if (step) uh += (long long)(*step) * stride;
+  uh += shot * ustride;
+  p2 += shot * pstride;
+  glam += (long long)shot * nbox;
+  gmu += (long long)shot * nbox;
+  const int ti0 = (t % ntx) * GTX, tj0 = ((t / ntx) % nty) * GTY;
+  const int kc0 = (t / (ntx * nty)) * tz, kc1 = min(kc0 + tz, bnz);
   const int bi = ti0 + tx, bj = tj0 + ty;
   const bool own = bi < bnx && bj < bny;
-  const int nbox = bnx * bny * bnz;              // 32-bit: 9 NN < 2^31 (checked by the host)
-  // u and p of box node (i, j, k) of this block's window (zero outside the box)
-  auto fetch = [&](int i, int j, int k, double* u, double* p) {
-    if (i >= 0 && j >= 0 && k >= 0 && i < bnx && j < bny && k < bnz) {
-      const int r = i + bnx * (j + bny * k);
-      const int n = (bi0 + i) + g.NX * ((bj0 + j) + g.NY * (bk0 + k));
+  // u and p of a box column at plane k, both clamped to the box: a position outside it
+  // meets zero coefficients only
+  const double *const u0p = uh, *const u1p = uh + nbox, *const u2p = uh + 2 * nbox;
+  auto fetch = [&](unsigned r0, unsigned n0, int k, double* u, double* p) {
+    const unsigned kk = (unsigned)min(max(k, 0), bnz - 1);
+    const unsigned r = (r0 + (unsigned)(bnx * bny) * kk) * 8u;
+    const unsigned n = (n0 + (unsigned)(g.NX * g.NY) * kk) * 24u;
+    u[0] = ldo(u0p, r);
+    u[1] = ldo(u1p, r);
+    u[2] = ldo(u2p, r);
+    ld3(p2, n, p[0], p[1], p[2]);
+  };
+  const int ci = min(bi, bnx - 1), cj = min(bj, bny - 1);
+  const unsigned r0 = (unsigned)(ci + bnx * cj), n0 = (unsigned)((bi0 + ci) + g.NX * ((bj0 + cj) + g.NY * bk0));
+  const int wo = (GH + tx) + GWX * (GH + ty);
+  // halo position of this thread
+  int hx = 0, hy = 0;
+  if (tid < 4 * GTX) { hy = tid / GTX; hx = GH + (tid - hy * GTX); if (hy >= 2) hy += GTY; }
+  else if (tid < GHALO) { const int q = tid - 4 * GTX; hy = GH + (q >> 2); hx = q & 3; if (hx >= 2) hx += GTX; }
+  const bool halo = tid < GHALO;
+  const int hi = min(max(ti0 + hx - GH, 0), bnx - 1), hj = min(max(tj0 + hy - GH, 0), bny - 1);
+  const unsigned hr0 = (unsigned)(hi + bnx * hj), hn0 = (unsigned)((bi0 + hi) + g.NX * ((bj0 + hj) + g.NY * bk0));
+  const int hw = hx + GWX * hy;
+  // x and y sides.  Side 0 is the element below (even node, its local point 2) or
+  // the one element of an odd node (local point 1), side 1 the element above (local
+  // point 0).  With a, b the side's other two values,
+  //   even, below  (3 (f - a) + b - a) / 2     odd  (a - b) / 2
+  //   above        (3 (a - f) + a - b) / 2
+  int ox[4], oy[4];
+  double cx[3], cy[3];
+  int cnt[3];
+  auto sides = [&](int q, int n, double dxi, int unit, int* o, double* c) {
+    const bool odd = q & 1, below = q >= 2, above = !odd && q + 2 <= n - 1;
+    o[0] = odd ? unit : -unit;
+    o[1] = odd ? -unit : -2 * unit;
+    o[2] = odd ? 0 : unit;
+    o[3] = odd ? 0 : 2 * unit;
+    c[0] = !odd && below ? 1.5 * dxi : 0.0;
+    c[1] = odd ? 0.5 * dxi : (below ? -0.5 * dxi : 0.0);
+    c[2] = above ? 0.5 * dxi : 0.0;
+    return (odd || below ? 1 : 0) + (above ? 1 : 0);
+  };
+  cnt[0] = sides(bi, bnx, g.dxi[0], 1, ox, cx);
+  cnt[1] = sides(bj, bny, g.dxi[1], GWX, oy, cy);
+  const double wxy = g.wq[1 + 3 * 1 + 9 * 1] * (bi & 1 ? 1.0 : 0.25) * (bj & 1 ? 1.0 : 0.25) * dt;
+  // own column: planes k-2 .. k+2 (index 0..4); halo of plane k
+  double qu[5][3], qp[5][3], hu[3], hp[3];
 #pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        u[c] = uh[c * nbox + r];
-        p[c] = p2[3 * n + c];
+  for (int d = 0; d < 5; ++d) fetch(r0, n0, kc0 - 2 + d, qu[d], qp[d]);
+  fetch(hr0, hn0, kc0, hu, hp);
+  for (int k = kc0; k < kc1; ++k) {
+    double(*const U)[GW] = sU[(k - kc0) & 1];
+    double(*const Q)[GW] = sP[(k - kc0) & 1];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) { U[c][wo] = qu[2][c]; Q[c][wo] = qp[2][c]; }
+    if (halo)
+#pragma unroll
+      for (int c = 0; c < 3; ++c) { U[c][hw] = hu[c]; Q[c][hw] = hp[c]; }
+    Sides Z;
+    if (k & 1) {
+      const double c = 0.5 * g.dxi[2];
+      cnt[2] = 1;
+#pragma unroll
+      for (int m = 0; m < 3; ++m) {
+        Z.u[m] = c * (qu[3][m] - qu[1][m]);
+        Z.p[m] = c * (qp[3][m] - qp[1][m]);
+        Z.d[m] = Z.u[m] * Z.p[m];
       }
     } else {
+      const double c0 = k >= 2 ? 0.5 * g.dxi[2] : 0.0, c1 = k + 2 <= bnz - 1 ? 0.5 * g.dxi[2] : 0.0;
+      cnt[2] = (k >= 2 ? 1 : 0) + (k + 2 <= bnz - 1 ? 1 : 0);
 #pragma unroll
-      for (int c = 0; c < 3; ++c) { u[c] = 0.0; p[c] = 0.0; }
-    }
-  };
-  // own column: planes k-2 .. k+2 (index 0..4)
-  double qu[5][3], qp[5][3];
-#pragma unroll
-  for (int d = 0; d < 4; ++d) fetch(bi, bj, kc0 - 2 + d, qu[d], qp[d]);
-  const int wx = GH + tx, wy = GH + ty;
-  for (int k = kc0; k < kc1; ++k) {
-    // this plane's accumulators, read with the plane's inputs
-    const int r = bi + bnx * (bj + bny * k);
-    double gl0 = 0.0, gm0 = 0.0;
-    if (own) { gl0 = glam[r]; gm0 = gmu[r]; }
-    fetch(bi, bj, k + 2, qu[4], qp[4]);
-#pragma unroll
-    for (int c = 0; c < 3; ++c) { sU[c][wy][wx] = qu[2][c]; sP[c][wy][wx] = qp[2][c]; }
-    for (int h = tid; h < GHALO; h += GNT) {
-      int hx, hy;
-      if (h < 4 * GTX) { hy = h / GTX; hx = GH + (h - hy * GTX); if (hy >= 2) hy += GTY; }
-      else { const int q = h - 4 * GTX; hy = GH + (q >> 2); hx = q & 3; if (hx >= 2) hx += GTX; }
-      double u[3], p[3];
-      fetch(ti0 + hx - GH, tj0 + hy - GH, k, u, p);
-#pragma unroll
-      for (int c = 0; c < 3; ++c) { sU[c][hy][hx] = u[c]; sP[c][hy][hx] = p[c]; }
-    }
-    __syncthreads();
-    if (own) {
-      const int pos[3] = {bi, bj, k};
-      const int bn[3] = {bnx, bny, bnz};
-      // per axis two element sides: s = 0 the element below (local 2; local 1 for an
-      // odd node), s = 1 the element above (local 0), within the box
-      bool has[3][2];
-      int lo[3][2];
-      double du[3][2][3], dp[3][2][3];
-#pragma unroll
-      for (int a = 0; a < 3; ++a) {
-        const int q = pos[a];
-        const bool odd = q & 1;
-        lo[a][0] = odd ? 1 : 2;
-        lo[a][1] = 0;
-        has[a][0] = odd ? true : q >= 2;
-        has[a][1] = !odd && q + 2 <= bn[a] - 1;
-#pragma unroll
-        for (int s = 0; s < 2; ++s) {
-          const int l = lo[a][s];
-#pragma unroll
-          for (int c = 0; c < 3; ++c) {
-            double su = 0.0, sp = 0.0;
-            if (has[a][s]) {
-#pragma unroll
-              for (int m = 0; m < 3; ++m) {
-                const int off = m - l;
-                double uv, pv;
-                if (a == 0) { uv = sU[c][wy][wx + off]; pv = sP[c][wy][wx + off]; }
-                else if (a == 1) { uv = sU[c][wy + off][wx]; pv = sP[c][wy + off][wx]; }
-                else { uv = qu[2 + off][c]; pv = qp[2 + off][c]; }
-                su += DM(l, m) * uv;
-                sp += DM(l, m) * pv;
-              }
-            }
-            du[a][s][c] = g.dxi[a] * su;
-            dp[a][s][c] = g.dxi[a] * sp;
-          }
-        }
+      for (int m = 0; m < 3; ++m) {
+        const double u0 = c0 * (3.0 * (qu[2][m] - qu[1][m]) + (qu[0][m] - qu[1][m]));
+        const double u1 = c1 * (3.0 * (qu[3][m] - qu[2][m]) + (qu[3][m] - qu[4][m]));
+        const double p0 = c0 * (3.0 * (qp[2][m] - qp[1][m]) + (qp[0][m] - qp[1][m]));
+        const double p1 = c1 * (3.0 * (qp[3][m] - qp[2][m]) + (qp[3][m] - qp[4][m]));
+        Z.u[m] = u0 + u1;
+        Z.p[m] = p0 + p1;
+        Z.d[m] = u0 * p0 + u1 * p1;
       }
-      double sl = 0.0, sm = 0.0;
-#pragma unroll
-      for (int sx = 0; sx < 2; ++sx)
-#pragma unroll
-        for (int sy = 0; sy < 2; ++sy)
-#pragma unroll
-          for (int sz = 0; sz < 2; ++sz) {
-            if (!(has[0][sx] && has[1][sy] && has[2][sz])) continue;
-            const double u1x = du[0][sx][0], u2x = du[0][sx][1], u3x = du[0][sx][2];
-            const double u1y = du[1][sy][0], u2y = du[1][sy][1], u3y = du[1][sy][2];
-            const double u1z = du[2][sz][0], u2z = du[2][sz][1], u3z = du[2][sz][2];
-            const double p1x = dp[0][sx][0], p2x = dp[0][sx][1], p3x = dp[0][sx][2];
-            const double p1y = dp[1][sy][0], p2y = dp[1][sy][1], p3y = dp[1][sy][2];
-            const double p1z = dp[2][sz][0], p2z = dp[2][sz][1], p3z = dp[2][sz][2];
-            const double sL = (u1x + u2y + u3z) * (p1x + p2y + p3z);
-            const double sM = 2.0 * (u1x * p1x + u2y * p2y + u3z * p3z) + (p1y + p2x) * (u1y + u2x) +
-                              (p1z + p3x) * (u1z + u3x) + (p3y + p2z) * (u3y + u2z);
-            const double W = g.wq[lo[0][sx] + 3 * lo[1][sy] + 9 * lo[2][sz]];
-            sl += sL * W;
-            sm += sM * W;
-          }
-      glam[r] = gl0 + sl * dt;
-      gmu[r] = gm0 + sm * dt;
     }
-    __syncthreads();
+    // the window moves up (index 1 is now plane k); the next plane's inputs
 #pragma unroll
     for (int d = 0; d < 4; ++d)
 #pragma unroll
       for (int c = 0; c < 3; ++c) { qu[d][c] = qu[d + 1][c]; qp[d][c] = qp[d + 1][c]; }
+    if (k + 1 < kc1) {
+      fetch(r0, n0, k + 3, qu[4], qp[4]);
+      if (halo) fetch(hr0, hn0, k + 1, hu, hp);
+    }
+    const unsigned r = (r0 + (unsigned)(bnx * bny * k)) * 8u;
+    const double gl0 = ldo(glam, r), gm0 = ldo(gmu, r);
+    __syncthreads();
+    Sides X, Y;
+    auto line = [&](const int* o, const double* c, Sides& S) {
+#pragma unroll
+      for (int m = 0; m < 3; ++m) {
+        const double* fu = U[m] + wo;
+        const double* fp = Q[m] + wo;
+        const double ua = fu[o[0]], pa = fp[o[0]], ub = fu[o[2]], pb = fp[o[2]];
+        const double u0 = c[0] * (qu[1][m] - ua) + c[1] * (ua - fu[o[1]]);
+        const double u1 = c[2] * (3.0 * (ub - qu[1][m]) + (ub - fu[o[3]]));
+        const double p0 = c[0] * (qp[1][m] - pa) + c[1] * (pa - fp[o[1]]);
+        const double p1 = c[2] * (3.0 * (pb - qp[1][m]) + (pb - fp[o[3]]));
+        S.u[m] = u0 + u1;
+        S.p[m] = p0 + p1;
+        S.d[m] = u0 * p0 + u1 * p1;
+        __builtin_amdgcn_sched_barrier(0);         // one component's reads at a time: no spills
+      }
+    };
+    const double nx = cnt[0], ny = cnt[1], nz = cnt[2];
+    const double nyz = ny * nz, nxz = nx * nz, nxy = nx * ny;
+    double sl = 0.0, dd = nxy * Z.d[2], sh = nxy * (Z.d[0] + Z.d[1]);
+    line(ox, cx, X);
+    dd += nyz * X.d[0];
+    sh += nyz * (X.d[1] + X.d[2]) + ny * (Z.p[0] * X.u[2] + X.p[2] * Z.u[0]);
+    sl += ny * (X.u[0] * Z.p[2] + Z.u[2] * X.p[0]);
+    line(oy, cy, Y);
+    dd += nxz * Y.d[1];
+    sh += nxz * (Y.d[0] + Y.d[2]) + nz * (Y.p[0] * X.u[1] + X.p[1] * Y.u[0]) + nx * (Y.p[2] * Z.u[1] + Z.p[1] * Y.u[2]);
+    sl += nz * (X.u[0] * Y.p[1] + Y.u[1] * X.p[0]) + nx * (Y.u[1] * Z.p[2] + Z.u[2] * Y.p[1]);
+    if (own) {
+      const double W = wxy * (k & 1 ? 1.0 : 0.25);
+      sto(glam, r, gl0 + (dd + sl) * W);
+      sto(gmu, r, gm0 + (2.0 * dd + sh) * W);
+    }
   }
 }
 
@@ -349,16 +326,21 @@ __global__ void sum_kernel(int n, const double* __restrict__ in, double* __restr
   }
 }
 
-// g <- -g for the regular-domain box, scattered to the nodal output
-__global__ void gradient_finish_kernel(Geo g, int bi0, int bj0, int bk0, int bnx, int bny, int bnz,
+// g <- -(sum over the shots of g) for the regular-domain box, scattered to the nodal output
+__global__ void gradient_finish_kernel(Geo g, int bi0, int bj0, int bk0, int bnx, int bny, int bnz, int nshot,
                                        const double* __restrict__ gl_box, const double* __restrict__ gm_box,
                                        double* __restrict__ gl, double* __restrict__ gm) {
   const long long nbox = (long long)bnx * bny * bnz;
   for (long long r = blockIdx.x * (long long)blockDim.x + threadIdx.x; r < nbox; r += (long long)gridDim.x * blockDim.x) {
     const int bi = (int)(r % bnx), bj = (int)((r / bnx) % bny), bk = (int)(r / ((long long)bnx * bny));
     const long long n = (long long)(bi0 + bi) + (long long)g.NX * ((long long)(bj0 + bj) + (long long)g.NY * (bk0 + bk));
-    gl[n] = gl_box[r] * -1.0;
-    gm[n] = gm_box[r] * -1.0;
+    double sl = 0.0, sm = 0.0;
+    for (int q = 0; q < nshot; ++q) {
+      sl += gl_box[q * nbox + r];
+      sm += gm_box[q * nbox + r];
+    }
+    gl[n] = sl * -1.0;
+    gm[n] = sm * -1.0;
   }
 }
 
@@ -429,8 +411,10 @@ hipError_t launch_scatter_eq(long long neq, const long long* slot, const double*
   hipLaunchKernelGGL(scatter_eq_kernel, dim3(grid_for(neq)), dim3(256), 0, s, neq, slot, raw, y, sc, l, z);
   return hipGetLastError();
 }
-hipError_t launch_record(int nrec, const long long* slot, const double* x2, double* row, hipStream_t s, StepRef sr) {
-  hipLaunchKernelGGL(record_kernel, dim3((nrec + 255) / 256), dim3(256), 0, s, nrec, slot, x2, row, sr.step, sr.stride);
+hipError_t launch_record(int nrec, const long long* slot, int nshot, const double* x2, long long xstride, double* row,
+                         long long rstride, hipStream_t s, StepRef sr) {
+  record_kernel<<<dim3((nrec + 255) / 256, nshot), 256, 0, s>>>(nrec, slot, x2, xstride, row, rstride, sr.step,
+                                                                sr.stride);
   return hipGetLastError();
 }
 hipError_t launch_step_set(int* step, int value, hipStream_t s) {
@@ -441,34 +425,40 @@ hipError_t launch_step_advance(int* step, int delta, hipStream_t s) {
   hipLaunchKernelGGL(step_advance_kernel, dim3(1), dim3(64), 0, s, step, delta);
   return hipGetLastError();
 }
-hipError_t launch_store_box(const Geo& g, const int* b0, const int* bn, const double* x2, double* hist, hipStream_t s,
-                            StepRef sr) {
+hipError_t launch_store_box(const Geo& g, const int* b0, const int* bn, int nshot, const double* x2, long long xstride,
+                            double* hist, long long hstride, hipStream_t s, StepRef sr) {
   const long long tot = (long long)bn[0] * bn[1] * bn[2];
-  hipLaunchKernelGGL(store_box_kernel, dim3(grid_for(tot)), dim3(256), 0, s, g, b0[0], b0[1], b0[2], bn[0], bn[1],
-                     bn[2], x2, hist, sr.step, sr.stride);
+  store_box_kernel<<<dim3(grid_for(tot), nshot), 256, 0, s>>>(g, b0[0], b0[1], b0[2], bn[0], bn[1], bn[2], x2, xstride,
+                                                              hist, hstride, sr.step, sr.stride);
   return hipGetLastError();
 }
-hipError_t launch_gradient(const Geo& g, const int* b0, const int* bn, const double* uh, const double* p2, double dt,
-                           double* glam, double* gmu, hipStream_t s, StepRef sr) {
-  const dim3 grid((bn[0] + GTX - 1) / GTX, (bn[1] + GTY - 1) / GTY, (bn[2] + GZC - 1) / GZC);
-  hipLaunchKernelGGL(gradient_tile_kernel, grid, dim3(GNT), 0, s, g, b0[0], b0[1], b0[2], bn[0], bn[1], bn[2], uh, p2,
-                     dt, glam, gmu, sr.step, sr.stride);
+hipError_t launch_gradient(const Geo& g, const int* b0, const int* bn, int nshot, const double* uh, long long ustride,
+                           const double* p2, long long pstride, double dt, double* glam, double* gmu, hipStream_t s,
+                           StepRef sr) {
+  // planes per chunk: the fewest planes in sequence, rounds of blocks times planes
+  // with the two that a chunk's start costs; of equals the longest
+  const int ntx = (bn[0] + GTX - 1) / GTX, nty = (bn[1] + GTY - 1) / GTY;
+  const long long slots = 256 * GBLOCKS;
+  long long best = -1;
+  int tz = bn[2];
+  for (int c = bn[2]; c >= 1; --c) {
+    const long long n = (long long)ntx * nty * ((bn[2] + c - 1) / c) * nshot;
+    const long long cost = (n + slots - 1) / slots * (c + 2);
+    if (best < 0 || cost < best) { best = cost; tz = c; }
+  }
+  const int ntz = (bn[2] + tz - 1) / tz;
+  const long long n = (long long)ntx * nty * ntz * nshot;
+  if (n <= 0) return hipSuccess;
+  gradient_tile_kernel<<<(unsigned)(8 * ((n + 7) / 8)), GNT, 0, s>>>(g, b0[0], b0[1], b0[2], bn[0], bn[1], bn[2], ntx,
+                                                                     nty, ntz, tz, nshot, uh, ustride, p2, pstride, dt,
+                                                                     glam, gmu, sr.step, sr.stride);
   return hipGetLastError();
 }
-
-// the node-per-thread form (kept as the reference for the tiled kernel's tests)
-hipError_t launch_gradient_pointwise(const Geo& g, const int* b0, const int* bn, const double* uh, const double* p2,
-                                     double dt, double* glam, double* gmu, hipStream_t s) {
-  const long long tot = (long long)bn[0] * bn[1] * bn[2];
-  hipLaunchKernelGGL(gradient_kernel, dim3(grid_for(tot)), dim3(256), 0, s, g, b0[0], b0[1], b0[2], bn[0], bn[1],
-                     bn[2], uh, p2, dt, glam, gmu);
-  return hipGetLastError();
-}
-hipError_t launch_gradient_finish(const Geo& g, const int* b0, const int* bn, const double* glb, const double* gmb,
+hipError_t launch_gradient_finish(const Geo& g, const int* b0, const int* bn, int nshot, const double* glb, const double* gmb,
                                   double* gl, double* gm, hipStream_t s) {
   const long long tot = (long long)bn[0] * bn[1] * bn[2];
   hipLaunchKernelGGL(gradient_finish_kernel, dim3(grid_for(tot)), dim3(256), 0, s, g, b0[0], b0[1], b0[2], bn[0],
-                     bn[1], bn[2], glb, gmb, gl, gm);
+                     bn[1], bn[2], nshot, glb, gmb, gl, gm);
   return hipGetLastError();
 }
 hipError_t launch_box_add(const Geo& g, const int* b0, const int* bn, const double* glb, const double* gmb, double* gl,

@@ -8,6 +8,10 @@
 namespace hr {
 namespace {
 
+// one double at a byte offset from a uniform base
+__device__ __forceinline__ double ldo(const double* p, unsigned off) {
+  return *reinterpret_cast<const double*>(reinterpret_cast<const char*>(p) + off);
+}
 __device__ __forceinline__ void sto(double* p, unsigned off, double v) {
   *reinterpret_cast<double*>(reinterpret_cast<char*>(p) + off) = v;
 }
