@@ -517,11 +517,11 @@ int launch_stage(hr_ctx* ctx, StageArgs& A, const Src3Spec* sp = nullptr) {
   if (counted) ctx->prof_all[A.stage] += 1;
   const bool prof = counted && (ctx->prof_tick++ % PROF_PERIOD) == 0;
   const bool split = ctx->version == 4 && A.stage >= 1 && A.stage <= 4;
-  // the split path runs its two kernels of stages 1 and 3 side by side where the
-  // nodal pass has more blocks than the GPU's CUs; below that the event waits cost
-  // more than the overlap gives (16x16x8: 17.9 ms against 22.5 ms per 200 steps,
-  // 70 blocks; 37x29x19: equal, 480 blocks)
-  const bool fork = ctx->concurrent && (A.stage & 1) && (long long)ctx->pnblk_nodal * ctx->nshot > 384;
+  // stages 1 and 3 of the split path: both passes in one launch, or on two streams where
+  // there is so much work that the events' cost no longer shows (4 shots of 48x48x24, 4380
+  // nodal blocks: 47.3 ms on two streams, 47.7 in one launch; 96x96x48, 5960: 25.9, 26.4;
+  // 64x64x32, 2100 blocks: equal; below that one launch is faster)
+  const bool fork = ctx->concurrent && (A.stage & 1) && (long long)ctx->pnblk_nodal * ctx->nshot > 3072;
   hr_ctx::StageEv ev{A.stage, !ctx->concurrent ? 1 : (!split ? 3 : (fork ? 2 : 1)), {nullptr, nullptr, nullptr}, {nullptr, nullptr, nullptr}};
   if (prof) {
     if (ctx->ev_open.size() >= 4096) if (int rc = drain_events(ctx)) return rc;
@@ -607,14 +607,14 @@ int launch_stage(hr_ctx* ctx, StageArgs& A, const Src3Spec* sp = nullptr) {
           HIPC(hipEventRecord(ctx->ev_join[1], ctx->cstream[1]));
         }
         if (prof) HIPC(hipEventRecord(ev.start[0], ctx->stream));
-        HIPC(launch_rd_pair(R, upd, ctx->stream));
+        HIPC(launch_elements(R, upd, ctx->stream));
         HIPC(hipStreamWaitEvent(ctx->stream, ctx->ev_join[0], 0));
         if (side_work) HIPC(hipStreamWaitEvent(ctx->stream, ctx->ev_join[1], 0));
       } else {
         if (int rc = run_deferred(ctx)) return rc;
         if (prof) HIPC(hipEventRecord(ev.start[0], ctx->stream));
-        if (elements) HIPC(launch_rd_pair(R, upd, ctx->stream));
-        HIPC(launch_split_nodal(B, last, A.transpose, ctx->stream));
+        if (elements) HIPC(launch_stage_pair(B, R, upd, A.transpose, ctx->stream));
+        else HIPC(launch_split_nodal(B, last, A.transpose, ctx->stream));
       }
       HIPC(launch_split_pull(B, A.transpose, ctx->stream));
       if (prof) HIPC(hipEventRecord(ev.end[0], ctx->stream));

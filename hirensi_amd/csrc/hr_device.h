@@ -210,5 +210,7 @@ constexpr int SPLIT_OWN = SPLIT_NT - 4;      // nodes (threads) per block of the
 hipError_t launch_split_nodal(const SplitArgs& A, int last, int transpose, hipStream_t s);
 hipError_t launch_split_pull(const SplitArgs& A, int transpose, hipStream_t s);
 void rd_tiles(const Geo& g, int tz, int t[3]);   // element pass tiles per axis (x, y, z-chunks)
-hipError_t launch_rd_pair(const RdArgs& A, int update, hipStream_t s);
+hipError_t launch_elements(const RdArgs& R, int update, hipStream_t s);
+// both passes of stages 1 and 3
+hipError_t launch_stage_pair(const SplitArgs& A, const RdArgs& R, int update, int transpose, hipStream_t s);
 }  // namespace hr

@@ -37,9 +37,9 @@ namespace {
 // logical blocks [x C, (x + 1) C) of the launch, so that each XCD's L2 holds a
 // contiguous run of the list (the neighbouring rows and planes of its nodes); a
 // launch has 8 C blocks and starts at logical block A.pb0.
-__device__ __forceinline__ int split_block(int nblk) {
+__device__ __forceinline__ int split_block(int blk, int nblk) {
   const int C = (nblk + 7) / 8;
-  return (blockIdx.x & 7) * C + (blockIdx.x >> 3);
+  return (blk & 7) * C + (blk >> 3);
 }
 // Flux records D of the split path, per shot 12 NN doubles: two arrays (ax =
 // y, z) of six doubles per lattice node, (G_{x,ax}, G_{y,ax}, G_{z,ax},
@@ -64,13 +64,19 @@ __device__ __forceinline__ void operator_inputs(const double* X, double& v1, dou
 // part of the update that does not need a4), and the new x1, x2 are written here.
 // The x-line sums read the x records of the block's entries from LDS:
 // consecutive list entries are x-neighbours.
+struct NodalLds {
+  double xr[6][SPLIT_NT];         // x flux records of the block's entries
+  unsigned xn[SPLIT_NT];          // their lattice nodes (~0: no entry)
+};
+
+// block `blk` of the pass over one shot
 template <bool LAST, bool TR>
-__global__ void __launch_bounds__(SPLIT_NT, LAST ? 2 : 3) pml_nodal_kernel(const SplitArgs A) {
+__device__ __forceinline__ void nodal_pass(const SplitArgs& A, int blk, int shot, NodalLds& sh) {
   constexpr int NIN = LAST ? 6 : 3;
-  __shared__ double sXr[6][SPLIT_NT];     // x flux records of the block's entries
-  __shared__ unsigned sXn[SPLIT_NT];      // their lattice nodes (~0: no entry)
+  double(&sXr)[6][SPLIT_NT] = sh.xr;
+  unsigned(&sXn)[SPLIT_NT] = sh.xn;
   const Geo3& g = A.g;
-  const int lb = split_block(A.pnbn);
+  const int lb = split_block(blk, A.pnbn);
   if (lb >= A.pnbn) return;
   const int tid = threadIdx.x;
   // list entry of this thread: the block owns [lb SPLIT_OWN, (lb + 1) SPLIT_OWN) and
@@ -81,7 +87,6 @@ __global__ void __launch_bounds__(SPLIT_NT, LAST ? 2 : 3) pml_nodal_kernel(const
   const bool valid = t >= 0 && sp_pml_node((unsigned)t, g.NX, g.NY, g.NZ, g.rlo, g.rhi, i, j, k);
   if (!valid) i = j = k = 0;
   const bool own = valid && tid >= 2 && tid < SPLIT_NT - 2;
-  const int shot = blockIdx.y;
   const unsigned n = (unsigned)i + (unsigned)g.NX * ((unsigned)j + (unsigned)g.NY * (unsigned)k);
   const long long so = (long long)shot * A.shot_stride;
   const unsigned NN = (unsigned)g.NN;
@@ -269,6 +274,13 @@ __global__ void __launch_bounds__(SPLIT_NT, LAST ? 2 : 3) pml_nodal_kernel(const
   }
 }
 
+// the pass alone (stages 2 and 4; it shares a launch with the element pass in 1 and 3)
+template <bool LAST, bool TR>
+__global__ void __launch_bounds__(SPLIT_NT, LAST ? 2 : 3) pml_nodal_kernel(const SplitArgs A) {
+  __shared__ NodalLds sh;
+  nodal_pass<LAST, TR>(A, blockIdx.x, blockIdx.y, sh);
+}
+
 // Sources at regular-domain-only nodes, which the element kernel finished: one
 // thread per node with entries (the list is in (shot, node) order).
 __device__ __forceinline__ void add_domain_sources(const SplitArgs& A, int q) {
@@ -315,7 +327,7 @@ __global__ void __launch_bounds__(SPLIT_NT, 2) pml_pull_kernel(const SplitArgs A
     if (blockIdx.y == 0) add_domain_sources(A, ((int)blockIdx.x - C8) * SPLIT_NT + tid);
     return;
   }
-  const int blk = split_block(A.pnb);
+  const int blk = split_block(blockIdx.x, A.pnb);
   if (blk >= A.pnb) return;
   const int shot = blockIdx.y;
   int e0 = 0, e1 = 0, jj = -1;          // this block's source entries (a uniform range)
@@ -497,17 +509,23 @@ constexpr int RT = 4, RW = 2 * RT + 3, RWP = RW * RW, RNE = (RT + 1) * (RT + 1),
 constexpr int REW = 7;                     // elements per wavefront (9 lanes each)
 static_assert(4 * REW >= RNE && 2 * RWP <= 256 && 3 * RO * RO <= 256, "one block of four wavefronts");
 
+struct RdLds {
+  double v[2][3][3][RWP];          // field, plane (k % 3), component, window position
+  double r[2][3][RNE * 27 + 1];    // nodal forces of the elements per field and component, a spare
+};
+
+// block `blk` of the pass
 template <bool UPDATE>
-__global__ void __launch_bounds__(256, 2) rd_pair_kernel(const RdArgs A) {
-  __shared__ double sV[2][3][3][RWP];      // field, plane (k % 3), component, window position
-  __shared__ double sR[2][3][RNE * 27 + 1];   // nodal forces of the elements per field and component, a spare
+__device__ __forceinline__ void element_pass(const RdArgs& A, int blk, RdLds& sh) {
+  double(&sV)[2][3][3][RWP] = sh.v;
+  double(&sR)[2][3][RNE * 27 + 1] = sh.r;
   const Geo3& g = A.g;
   const int tid = threadIdx.x, lane = tid & 63;
-  // XCD-aware order: XCD x = blockIdx % 8 takes a contiguous run of the (shot, y, z, x) tiles
+  // XCD-aware order: XCD x = blk % 8 takes a contiguous run of the (shot, y, z, x) tiles
   const int ntile = A.ntx * A.nty * A.ntz;
   const int ntot = ntile * A.nshot;
   const int C = (ntot + 7) / 8;
-  const int li = (blockIdx.x & 7) * C + (blockIdx.x >> 3);
+  const int li = (blk & 7) * C + (blk >> 3);
   if (li >= ntot) return;
   const int shot = li / ntile;
   const int t = li - shot * ntile;
@@ -750,6 +768,36 @@ __global__ void __launch_bounds__(256, 2) rd_pair_kernel(const RdArgs A) {
   }
 }
 
+// the element pass alone
+template <bool UPDATE>
+__global__ void __launch_bounds__(SPLIT_NT, 2) element_kernel(const RdArgs A) {
+  __shared__ RdLds sh;
+  element_pass<UPDATE>(A, blockIdx.x, sh);
+}
+
+// The element pass (the first nrd blocks) and the nodal pass of stages 1 and 3 in one
+// launch: the one is bound by LDS, the other by memory, and neither waits for the other,
+// so they share the CUs without the events of two streams, which cost 15-20 us a
+// stage.  The element blocks run longest and come first: mixed in with the nodal
+// blocks, one in two or in proportion, the pair took 5-20 % longer.
+// Against launches of their own (on two streams from 37x29x19 up), forward and adjoint
+// step on average: 16x16x8 elements 84 -> 74 us,
+// 37x29x19 150 -> 131, 4 shots of 32x32x16 341 -> 317, 64x64x32 equal.
+template <bool UPDATE, bool TR>
+__global__ void __launch_bounds__(SPLIT_NT, 2) stage_pair_kernel(const SplitArgs A, const RdArgs R, int nrd, int nn) {
+  __shared__ union {
+    NodalLds nodal;
+    RdLds element;
+  } sh;
+  const int b = blockIdx.x;
+  if (b < nrd) {
+    element_pass<UPDATE>(R, b, sh.element);
+    return;
+  }
+  const int shot = (b - nrd) / nn;
+  nodal_pass<false, TR>(A, (b - nrd) - shot * nn, shot, sh.nodal);
+}
+
 }  // namespace
 
 hipError_t launch_split_nodal(const SplitArgs& A, int last, int transpose, hipStream_t s) {
@@ -780,12 +828,28 @@ void rd_tiles(const Geo& g, int tz, int t[3]) {
   t[2] = (g.nez - g.rlo[2] + tz - 1) / tz;
 }
 
-hipError_t launch_rd_pair(const RdArgs& A, int update, hipStream_t s) {
-  const long long n = (long long)A.ntx * A.nty * A.ntz * A.nshot;
+hipError_t launch_elements(const RdArgs& R, int update, hipStream_t s) {
+  const long long n = (long long)R.ntx * R.nty * R.ntz * R.nshot;
   if (n <= 0) return hipSuccess;
   const unsigned nb = (unsigned)(8 * ((n + 7) / 8));
-  if (update) rd_pair_kernel<true><<<nb, 256, 0, s>>>(A);
-  else rd_pair_kernel<false><<<nb, 256, 0, s>>>(A);
+  if (update) element_kernel<true><<<nb, SPLIT_NT, 0, s>>>(R);
+  else element_kernel<false><<<nb, SPLIT_NT, 0, s>>>(R);
+  return hipGetLastError();
+}
+
+hipError_t launch_stage_pair(const SplitArgs& A, const RdArgs& R, int update, int transpose, hipStream_t s) {
+  if (A.nshot <= 0) return hipSuccess;
+  const long long n = (long long)R.ntx * R.nty * R.ntz * R.nshot;
+  const int nrd = (int)(8 * ((n + 7) / 8)), nn = 8 * ((A.pnbn + 7) / 8);
+  const unsigned nb = (unsigned)(nrd + nn * A.nshot);
+  if (nb == 0) return hipSuccess;
+  if (update) {
+    if (transpose) stage_pair_kernel<true, true><<<nb, SPLIT_NT, 0, s>>>(A, R, nrd, nn);
+    else stage_pair_kernel<true, false><<<nb, SPLIT_NT, 0, s>>>(A, R, nrd, nn);
+  } else {
+    if (transpose) stage_pair_kernel<false, true><<<nb, SPLIT_NT, 0, s>>>(A, R, nrd, nn);
+    else stage_pair_kernel<false, false><<<nb, SPLIT_NT, 0, s>>>(A, R, nrd, nn);
+  }
   return hipGetLastError();
 }
 

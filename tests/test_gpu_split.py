@@ -56,3 +56,30 @@ def test_split_path_at_tile_and_chunk_edges(shape, npml, tz):
     c3 = S.Context(mesh, model, version=3)
     tr3 = S.explicit_rk4_petsc_pml_3d(c3, nstep, dt, S.time_table(nstep, dt, 2, fr), src_eq, src_val, rec_eq)
     assert rel_l2(tr3, tr) < 1e-12
+
+
+def test_two_streams_match_one_launch():
+    """Stages 1 and 3 of a batch with more than 3072 nodal blocks run on two streams,
+    those of one shot in one launch; the same arithmetic, so 1e-13 relative."""
+    mesh = BoxMesh(24, 24, 12, npml=(5,) * 5)
+    model = random_model(mesh, seed=6)
+    lo, top, nshot, nstep, dt = mesh.rd_lo, mesh.NZ - 1, 18, 12, 1.0e-4
+    nodes = [mesh.node_index(2 * lo[0] + q, 2 * lo[1] + 7, top - q % 2) for q in range(nshot)]
+    rec_eq = receiver_dofs(mesh, nodes[::3])
+    src_eq = np.array([mesh.dof(n, q % 3) for q, n in enumerate(nodes)], dtype=np.int64)
+    ftab = np.stack([S.time_table(nstep, dt, 2, 400.0 + q) for q in range(nshot)])
+    one = np.ones(nshot)
+    print(f"two streams neq={mesh.neq} nshot={nshot}", flush=True)
+    ctx = S.Context(mesh, model)
+    tr = S.explicit_rk4_petsc_pml_3d_shots(ctx, nstep, dt, ftab, np.arange(nshot, dtype=np.int32), src_eq, one, rec_eq)
+    obs = 0.5 * tr
+    gl, gm, _ = S.explicit_rk4_petsc_pml_3d_adjoint_otd(ctx, nstep, dt, rec_eq, obs)
+    c1, sl, sm = S.Context(mesh, model), np.zeros(mesh.nnode), np.zeros(mesh.nnode)
+    for q in range(nshot):
+        t1 = S.explicit_rk4_petsc_pml_3d(c1, nstep, dt, ftab[q], src_eq[q:q + 1], one[:1], rec_eq)
+        assert rel_l2(tr[q], t1) < 1e-13, q
+        a, b, _ = S.explicit_rk4_petsc_pml_3d_adjoint_otd(c1, nstep, dt, rec_eq, obs[q])
+        sl += a
+        sm += b
+    assert np.abs(sl).max() > 0
+    assert rel_l2(gl, sl) < 1e-13 and rel_l2(gm, sm) < 1e-13
