@@ -153,9 +153,10 @@ struct hr_ctx {
   // split stage path (version 4): the flux records and interface sums of
   // split_shots shots, source entries by pull block and at regular-domain-only nodes
   bool split_ok = false;                      // the lattice fits the split path
-  int pnblk = 0;                              // SPLIT_NT-node blocks of the PML nodes (nodal pull)
-  int pnblk_nodal = 0;                        // SPLIT_OWN-node blocks of the PML nodes (nodal pass)
-  double* d_D = nullptr;
+  int pnblk = 0;                              // SPLIT_OWN-node blocks of the PML nodes
+  double* d_D = nullptr;                      // flux records: 12 NN doubles per shot, of odd stages, then of even ones
+  bool split_two = false;                     // there is room for both (else one, and a launch per pass)
+  SplitArgs split_prev{};                     // the stage whose pull is still to come
   double* d_E = nullptr;                      // two fields: 3 NN doubles per shot each
   int split_shots = 0;
   int rd_tz = 0;                              // layers per z-chunk of the element pass (0: rd_chunk's rule)
@@ -319,16 +320,24 @@ int build_pull_lists(hr_ctx* ctx, const std::vector<int>& ptr, const std::vector
   const int nblk = ctx->pnblk;
   const int gh[2] = {g.rhi[0], g.rhi[1]};
   struct Entry {
-    long long key;       // (shot, position in lattice order) of a PML node, (shot, node) of another
+    long long key;       // (shot, block, thread) of a PML node, (shot, node) of another
     int jj, shot;
   };
   std::vector<Entry> pml, rd;
   for (int q = 0; q < nshot; ++q)
     for (int jj = ptr[(size_t)q * nt]; jj < ptr[(size_t)(q + 1) * nt]; ++jj) {
       const int i = (int)(node[jj] % g.NX), j = (int)((node[jj] / g.NX) % g.NY), k = (int)(node[jj] / ((long long)g.NX * g.NY));
-      if (h_pml_node(g, i, j, k))
-        pml.push_back({(long long)q * nblk * SPLIT_NT + (long long)sp_pml_pos(i, j, k, g.NX, g.NY, g.rlo, gh), jj, q});
-      else
+      if (h_pml_node(g, i, j, k)) {
+        // the block that owns the node, and the neighbour block that forms its a as well
+        const long long pos = (long long)sp_pml_pos(i, j, k, g.NX, g.NY, g.rlo, gh);
+        const long long b = pos / SPLIT_OWN, r = pos - b * SPLIT_OWN;
+        auto add = [&](long long blk, long long slot) {
+          if (blk >= 0 && blk < nblk) pml.push_back({((long long)q * nblk + blk) * SPLIT_NT + slot, jj, q});
+        };
+        add(b, r + 2);
+        if (r < 2) add(b - 1, r + 2 + SPLIT_OWN);
+        if (r >= SPLIT_OWN - 2) add(b + 1, r + 2 - SPLIT_OWN);
+      } else
         rd.push_back({(long long)q * g.NN + node[jj], jj, q});
     }
   auto less = [](const Entry& a, const Entry& b) { return a.key != b.key ? a.key < b.key : a.jj < b.jj; };
@@ -521,7 +530,7 @@ int launch_stage(hr_ctx* ctx, StageArgs& A, const Src3Spec* sp = nullptr) {
   // there is so much work that the events' cost no longer shows (4 shots of 48x48x24, 4380
   // nodal blocks: 47.3 ms on two streams, 47.7 in one launch; 96x96x48, 5960: 25.9, 26.4;
   // 64x64x32, 2100 blocks: equal; below that one launch is faster)
-  const bool fork = ctx->concurrent && (A.stage & 1) && (long long)ctx->pnblk_nodal * ctx->nshot > 3072;
+  const bool fork = ctx->concurrent && (A.stage & 1) && (long long)ctx->pnblk * ctx->nshot > 3072;
   hr_ctx::StageEv ev{A.stage, !ctx->concurrent ? 1 : (!split ? 3 : (fork ? 2 : 1)), {nullptr, nullptr, nullptr}, {nullptr, nullptr, nullptr}};
   if (prof) {
     if (ctx->ev_open.size() >= 4096) if (int rc = drain_events(ctx)) return rc;
@@ -549,21 +558,24 @@ int launch_stage(hr_ctx* ctx, StageArgs& A, const Src3Spec* sp = nullptr) {
       B.shot_stride = (long long)field_size(ctx);
       if (ctx->split_shots < B.nshot || !ctx->d_D || !ctx->split_ok)
         return fail(ctx, 3, "split stage path without its buffers for %d shots", B.nshot);
-      const bool last = A.stage == 4;
+      const bool last = A.stage == 4, elements = A.stage == 1 || A.stage == 3;
       for (int a = 0; a < 3; ++a) { B.v[a] = A.in[a]; B.x[a] = A.in[3 + a]; }
       B.xn[0] = A.xnew[0]; B.xn[1] = A.xnew[1];
-      B.out = last ? A.xnew[2] : A.out;
+      // node-local terms: in place, but for stage 1, whose a1 other blocks still need them
+      // for when it is written; they go to the vector that the update writes last
+      B.a = A.stage == 3 && ctx->split_two ? nullptr : (last ? A.xnew[2] : A.out);
+      B.out = A.stage == 1 ? ctx->y[0] : (last ? A.xnew[2] : A.out);
       B.node = ctx->d_node; B.tab = ctx->d_tab; B.minvu = ctx->d_minvu; B.rwp = ctx->d_rwp;
       set_source(ctx, sp, B);
       B.h = A.h; B.h2 = A.hh; B.h3 = A.h6; B.h4 = A.h4;
       B.sc = last ? A.h4 : 1.0;
-      B.pnb = ctx->pnblk; B.pnbn = ctx->pnblk_nodal;
-      B.D = ctx->d_D;
+      B.pnbn = ctx->pnblk;
+      // the flux records of odd and even stages alternate
+      B.D = ctx->d_D + (elements || !ctx->split_two ? 0 : 12 * (size_t)ctx->g.NN * ctx->split_shots);
       // the element pass before stages 1 and 3 forms the interface sums of two stages
       const size_t ne = 3 * (size_t)ctx->g.NN * ctx->split_shots;
       double* const E[2] = {ctx->d_E, ctx->d_E + ne};
       B.E = E[(A.stage - 1) & 1];
-      const bool elements = A.stage == 1 || A.stage == 3;
       RdArgs R;
       if (elements) {
         std::memset(&R, 0, sizeof(R));
@@ -592,7 +604,7 @@ int launch_stage(hr_ctx* ctx, StageArgs& A, const Src3Spec* sp = nullptr) {
         HIPC(hipEventRecord(ctx->ev_fork, ctx->stream));
         HIPC(hipStreamWaitEvent(ctx->cstream[0], ctx->ev_fork, 0));
         if (prof) HIPC(hipEventRecord(ev.start[1], ctx->cstream[0]));
-        HIPC(launch_split_nodal(B, last, A.transpose, ctx->cstream[0]));
+        HIPC(launch_split_nodal(B, 0, A.transpose, ctx->cstream[0]));
         if (prof) HIPC(hipEventRecord(ev.end[1], ctx->cstream[0]));
         HIPC(hipEventRecord(ctx->ev_join[0], ctx->cstream[0]));
         const bool side_work = !ctx->deferred.empty();
@@ -614,9 +626,14 @@ int launch_stage(hr_ctx* ctx, StageArgs& A, const Src3Spec* sp = nullptr) {
         if (int rc = run_deferred(ctx)) return rc;
         if (prof) HIPC(hipEventRecord(ev.start[0], ctx->stream));
         if (elements) HIPC(launch_stage_pair(B, R, upd, A.transpose, ctx->stream));
-        else HIPC(launch_split_nodal(B, last, A.transpose, ctx->stream));
+        else if (ctx->split_two) HIPC(launch_pull_nodal(ctx->split_prev, B, last, A.transpose, ctx->stream));
+        else {
+          HIPC(launch_split_pull(ctx->split_prev, A.transpose, ctx->stream));
+          HIPC(launch_split_nodal(B, last, A.transpose, ctx->stream));
+        }
+        if (!elements) HIPC(launch_split_pull(B, A.transpose, ctx->stream));
       }
-      HIPC(launch_split_pull(B, A.transpose, ctx->stream));
+      if (elements) ctx->split_prev = B;      // its pull comes with the next stage's nodal pass
       if (prof) HIPC(hipEventRecord(ev.end[0], ctx->stream));
       if (prof) ctx->ev_open.push_back(ev);
       return 0;
@@ -714,9 +731,14 @@ int check_ready(hr_ctx* ctx) {
 int ensure_split(hr_ctx* ctx) {
   if (ctx->version != 4 || ctx->split_shots >= ctx->shot_cap) return 0;
   const size_t nd = 12 * (size_t)ctx->g.NN * ctx->shot_cap, ne = 6 * (size_t)ctx->g.NN * ctx->shot_cap;
-  if (int rc = dalloc(ctx, &ctx->d_D, nd)) return rc;
   if (int rc = dalloc(ctx, &ctx->d_E, ne)) return rc;
-  HIPC(hipMemsetAsync(ctx->d_D, 0, nd * sizeof(double), ctx->stream));
+  ctx->split_two = dalloc(ctx, &ctx->d_D, 2 * nd) == 0;
+  if (!ctx->split_two) {
+    (void)hipGetLastError();
+    ctx->err.clear();
+    if (int rc = dalloc(ctx, &ctx->d_D, nd)) return rc;
+  }
+  HIPC(hipMemsetAsync(ctx->d_D, 0, (ctx->split_two ? 2 : 1) * nd * sizeof(double), ctx->stream));
   ctx->split_shots = ctx->shot_cap;
   return 0;
 }
@@ -995,8 +1017,7 @@ int hr_ctx_create(const hr_mesh_desc* d, hr_ctx** out) {
     // 20 % faster per gradient than with the interface nodes last)
     const int gh[2] = {g.rhi[0], g.rhi[1]};
     const int pos = (int)sp_pml_count(g.NX, g.NY, g.NZ, g.rlo, gh);
-    ctx->pnblk = (pos + SPLIT_NT - 1) / SPLIT_NT;
-    ctx->pnblk_nodal = (pos + SPLIT_OWN - 1) / SPLIT_OWN;
+    ctx->pnblk = (pos + SPLIT_OWN - 1) / SPLIT_OWN;
     ctx->split_ok = true;
   } else {
     ctx->version = 3;

@@ -127,9 +127,10 @@ struct Src3 {                      // device-resident source entries of one solv
   int nrec;                        // adjoint: entries per shot (shared receivers)
   int nstep;
   int ntiles;
-  // the same entries at PML nodes, by block of the nodal PML pull: entries of
+  // the same entries at PML nodes, by block of the PML node list: entries of
   // (shot, block) are pblk_idx[pblk_ptr[s*pnblk+b] .. pblk_ptr[s*pnblk+b+1]), in node
-  // order, pblk_slot their node's place in the block
+  // order, pblk_slot their node's thread in the block (an entry at a block's edge is
+  // in two blocks, which both form that node's a)
   const int* pblk_ptr;
   const int* pblk_idx;
   const int* pblk_slot;
@@ -168,7 +169,8 @@ struct SplitArgs {
   const double* v[3];              // operator inputs
   const double* x[3];              // last stage: the state
   double* xn[2];                   // last stage: updated x1, x2
-  double* out;                     // a_s; last stage: updated x3
+  double* out;                     // node-local terms, from the nodal pass to the pull
+  double* a;                       // the pull's result: a_s (null: not kept); last stage: updated x3
   const double *node, *tab;        // node table (lambda, mu pairs), small table
   const double *minvu, *rwp;       // M^-1 of the displacement rows, sum of rho W over the PML elements per node (NN each)
   Src3 src;                        // as in Stage3Args
@@ -179,7 +181,7 @@ struct SplitArgs {
   long long shot_stride;
   double h, h2, h3, h4;            // h, h^2/2, h^3/6, h^4/24
   double sc;                       // scale of the stage's a in its output: 1, last stage h^4/24
-  int pnb, pnbn;                   // blocks of the pull (SPLIT_NT PML nodes) and of the nodal pass (SPLIT_OWN)
+  int pnbn;                        // blocks of the PML node list (SPLIT_OWN nodes each)
   double* D;                       // y- and z-line flux records, 12 NN doubles per shot
   const double* E;                 // regular-domain K sums of interface nodes, 3 NN doubles per shot
 };
@@ -204,10 +206,11 @@ hipError_t launch_stage3(const Stage3Args& A, int stage, int transpose, int tile
 // split stage path: the nodal pass over the PML nodes, the nodal pull, and the
 // regular-domain element pass
 constexpr int SPLIT_NT = 256;
-// list entries a nodal-pass block owns: it also computes two entries on each
+// list entries a block of the nodal kernels owns: it also computes two entries on each
 // side, for the x flux records of its own entries' x-lines
 constexpr int SPLIT_OWN = SPLIT_NT - 4;      // nodes (threads) per block of the nodal kernels
 hipError_t launch_split_nodal(const SplitArgs& A, int last, int transpose, hipStream_t s);
+hipError_t launch_pull_nodal(const SplitArgs& P, const SplitArgs& N, int last, int transpose, hipStream_t s);
 hipError_t launch_split_pull(const SplitArgs& A, int transpose, hipStream_t s);
 void rd_tiles(const Geo& g, int tz, int t[3]);   // element pass tiles per axis (x, y, z-chunks)
 hipError_t launch_elements(const RdArgs& R, int update, hipStream_t s);

@@ -58,36 +58,66 @@ __device__ __forceinline__ void operator_inputs(const double* X, double& v1, dou
   v3 = TR ? -X[2] : X[2];
 }
 
-// Node-local part of an RK4 stage at one PML node: the flux records of its y-
-// and z-lines, and into the stage output the node-local terms -M^-1 (diagonal
-// terms + x-line sums).  LAST: the output is the new x3 (scaled by h^4/24, on the
-// part of the update that does not need a4), and the new x1, x2 are written here.
-// The x-line sums read the x records of the block's entries from LDS:
-// consecutive list entries are x-neighbours.
+// A thread's list entry.  Block lb owns [lb SPLIT_OWN, (lb + 1) SPLIT_OWN) and computes
+// two entries more on each side, for their x records; a thread without an
+// entry runs node 0 (in bounds) and stores nothing.
+struct Entry {
+  int i, j, k;
+  bool valid, own;
+  unsigned n;
+};
+__device__ __forceinline__ Entry list_entry(const Geo3& g, int lb) {
+  Entry E;
+  const int tid = threadIdx.x;
+  const long long t = (long long)lb * SPLIT_OWN - 2 + tid;
+  E.i = E.j = E.k = 0;
+  E.valid = t >= 0 && sp_pml_node((unsigned)t, g.NX, g.NY, g.NZ, g.rlo, g.rhi, E.i, E.j, E.k);
+  if (!E.valid) E.i = E.j = E.k = 0;
+  E.own = E.valid && tid >= 2 && tid < SPLIT_NT - 2;
+  E.n = (unsigned)E.i + (unsigned)g.NX * ((unsigned)E.j + (unsigned)g.NY * (unsigned)E.k);
+  return E;
+}
+
 struct NodalLds {
   double xr[6][SPLIT_NT];         // x flux records of the block's entries
   unsigned xn[SPLIT_NT];          // their lattice nodes (~0: no entry)
 };
 
-// block `blk` of the pass over one shot
+// one vector's components at a node
+__device__ __forceinline__ void ld_node(const double* ip, unsigned offu, unsigned offs, double* v) {
+  ld3(ip, offu, v[0], v[1], v[2]);
+  ld2(ip, offs, v[3], v[4]);
+  ld2(ip, offs + 16u, v[5], v[6]);
+  ld2(ip, offs + 32u, v[7], v[8]);
+}
+// and its active components back
+__device__ __forceinline__ void st_node(double* dst, unsigned offu, unsigned offs, bool ua, int sm, const double* v) {
+  if (ua) st3(dst, offu, v[0], v[1], v[2]);
+  if (sm == 0x3f) st6(dst, offs, &v[3]);
+  else {
+    if (sm & 7) st3m(dst, offs, sm & 7, v[3], v[4], v[5]);
+    if (sm & 56) st3m(dst, offs + 24u, (sm >> 3) & 7, v[6], v[7], v[8]);
+  }
+}
+
+// Node-local part of an RK4 stage at one PML node: the flux records of its y-
+// and z-lines, and into the stage output the node-local terms -M^-1 (diagonal
+// terms + x-line sums).  LAST: the output is the new x3 (scaled by h^4/24, on the
+// part of the update that does not need a4), and the new x1, x2 are written here.
+// The x-line sums read the x records of the block's entries from LDS:
+// consecutive list entries are x-neighbours.  V[q]: the components of v1, v2, v3
+// and, LAST, x1, x2, x3.
 template <bool LAST, bool TR>
-__device__ __forceinline__ void nodal_pass(const SplitArgs& A, int blk, int shot, NodalLds& sh) {
+__device__ __forceinline__ void nodal_pass(const SplitArgs& A, const Entry& E, int shot,
+                                           const double (*V)[9], NodalLds& sh) {
   constexpr int NIN = LAST ? 6 : 3;
   double(&sXr)[6][SPLIT_NT] = sh.xr;
   unsigned(&sXn)[SPLIT_NT] = sh.xn;
   const Geo3& g = A.g;
-  const int lb = split_block(blk, A.pnbn);
-  if (lb >= A.pnbn) return;
   const int tid = threadIdx.x;
-  // list entry of this thread: the block owns [lb SPLIT_OWN, (lb + 1) SPLIT_OWN) and
-  // computes two more on each side for their x records; a thread without an
-  // entry runs node 0 (in bounds) and stores nothing
-  const long long t = (long long)lb * SPLIT_OWN - 2 + tid;
-  int i = 0, j = 0, k = 0;
-  const bool valid = t >= 0 && sp_pml_node((unsigned)t, g.NX, g.NY, g.NZ, g.rlo, g.rhi, i, j, k);
-  if (!valid) i = j = k = 0;
-  const bool own = valid && tid >= 2 && tid < SPLIT_NT - 2;
-  const unsigned n = (unsigned)i + (unsigned)g.NX * ((unsigned)j + (unsigned)g.NY * (unsigned)k);
+  const int i = E.i, j = E.j, k = E.k;
+  const bool valid = E.valid, own = E.own;
+  const unsigned n = E.n;
   const long long so = (long long)shot * A.shot_stride;
   const unsigned NN = (unsigned)g.NN;
   const unsigned SB = 8u * (3u * NN + (NN & 1u));
@@ -98,11 +128,10 @@ __device__ __forceinline__ void nodal_pass(const SplitArgs& A, int blk, int shot
   double XU[3][NIN], XS6[6][NIN];
 #pragma unroll
   for (int q = 0; q < NIN; ++q) {
-    const double* ip = (q < 3 ? A.v[q] : A.x[q - 3]) + so;
-    ld3(ip, offu, XU[0][q], XU[1][q], XU[2][q]);
-    ld2(ip, offs, XS6[0][q], XS6[1][q]);
-    ld2(ip, offs + 16u, XS6[2][q], XS6[3][q]);
-    ld2(ip, offs + 32u, XS6[4][q], XS6[5][q]);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) XU[c][q] = V[q][c];
+#pragma unroll
+    for (int m = 0; m < 6; ++m) XS6[m][q] = V[q][3 + m];
   }
   double lam, mu, ax, bx, ay, by, az, bz;
   ld2(nodet, n * 16u, lam, mu);
@@ -265,20 +294,29 @@ __device__ __forceinline__ void nodal_pass(const SplitArgs& A, int blk, int shot
     const double minv = m < 3 ? minv_u : (m < 6 ? minv_s : 0.5 * minv_s);
     pre[m] = pre[m] - sc * (minv * rx[m]);
   }
-  double* const dst = A.out + so;
-  if (ua) st3(dst, offu, pre[0], pre[1], pre[2]);
-  if (sm == 0x3f) st6(dst, offs, &pre[3]);
-  else {
-    if (sm & 7) st3m(dst, offs, sm & 7, pre[3], pre[4], pre[5]);
-    if (sm & 56) st3m(dst, offs + 24u, (sm >> 3) & 7, pre[6], pre[7], pre[8]);
-  }
+  st_node(A.out + so, offu, offs, ua, sm, pre);
 }
 
-// the pass alone (stages 2 and 4; it shares a launch with the element pass in 1 and 3)
+// block `blk` of the pass over one shot, on vectors in memory
+template <bool LAST, bool TR>
+__device__ __forceinline__ void nodal_block(const SplitArgs& A, int blk, int shot, NodalLds& sh) {
+  const int lb = split_block(blk, A.pnbn);
+  if (lb >= A.pnbn) return;
+  const Entry E = list_entry(A.g, lb);
+  const unsigned NN = (unsigned)A.g.NN;
+  const unsigned offu = E.n * 24u, offs = 8u * (3u * NN + (NN & 1u)) + E.n * 48u;
+  constexpr int NIN = LAST ? 6 : 3;
+  double V[NIN][9];
+#pragma unroll
+  for (int q = 0; q < NIN; ++q) ld_node((q < 3 ? A.v[q] : A.x[q - 3]) + (long long)shot * A.shot_stride, offu, offs, V[q]);
+  nodal_pass<LAST, TR>(A, E, shot, V, sh);
+}
+
+// the pass alone
 template <bool LAST, bool TR>
 __global__ void __launch_bounds__(SPLIT_NT, LAST ? 2 : 3) pml_nodal_kernel(const SplitArgs A) {
   __shared__ NodalLds sh;
-  nodal_pass<LAST, TR>(A, blockIdx.x, blockIdx.y, sh);
+  nodal_block<LAST, TR>(A, blockIdx.x, blockIdx.y, sh);
 }
 
 // Sources at regular-domain-only nodes, which the element kernel finished: one
@@ -300,7 +338,7 @@ __device__ __forceinline__ void add_domain_sources(const SplitArgs& A, int q) {
     s[1] += c == 1 ? v : 0.0;
     s[2] += c == 2 ? v : 0.0;
   }
-  double* const o = A.out + (long long)shot * A.shot_stride + 3 * n;
+  double* const o = A.a + (long long)shot * A.shot_stride + 3 * n;
 #pragma unroll
   for (int c = 0; c < 3; ++c) o[c] += A.sc * s[c];
 }
@@ -316,48 +354,42 @@ __device__ __forceinline__ void add_domain_sources(const SplitArgs& A, int q) {
 // each node finds its own through a table over the block's nodes; scanning the
 // entries node by node made the adjoint's pull of a 16 x 16 x 8 box, whose blocks
 // hold up to 64 receiver entries, 16-19 us long against 6.5 us without sources.
+struct PullLds {
+  double val[SPLIT_NT];                                // source entries: value,
+  int slot[SPLIT_NT], cmp[SPLIT_NT], first[SPLIT_NT];  // node in the block, component; a node's first
+};
+
+// the stage's a (or, in the last stage, its part of the new x3) of a node into out
 template <bool TR>
-__global__ void __launch_bounds__(SPLIT_NT, 2) pml_pull_kernel(const SplitArgs A) {
-  __shared__ double sVal[SPLIT_NT];                                 // source entries: value,
-  __shared__ int sSlot[SPLIT_NT], sCmp[SPLIT_NT], sFirst[SPLIT_NT]; // node in the block, component; a node's first
+__device__ __forceinline__ void pull_pass(const SplitArgs& A, const Entry& E, int lb, int shot, PullLds& sh,
+                                          double* out) {
+  double(&sVal)[SPLIT_NT] = sh.val;
+  int(&sSlot)[SPLIT_NT] = sh.slot;
+  int(&sCmp)[SPLIT_NT] = sh.cmp;
+  int(&sFirst)[SPLIT_NT] = sh.first;
   const Geo3& g = A.g;
   const int tid = threadIdx.x;
-  const int C8 = 8 * ((A.pnb + 7) / 8);
-  if ((int)blockIdx.x >= C8) {
-    if (blockIdx.y == 0) add_domain_sources(A, ((int)blockIdx.x - C8) * SPLIT_NT + tid);
-    return;
-  }
-  const int blk = split_block(blockIdx.x, A.pnb);
-  if (blk >= A.pnb) return;
-  const int shot = blockIdx.y;
   int e0 = 0, e1 = 0, jj = -1;          // this block's source entries (a uniform range)
   if (A.src_mode) {
-    const int pb = shot * A.src.pnblk + blk;
+    const int pb = shot * A.src.pnblk + lb;
     e0 = A.src.pblk_ptr[pb];
     e1 = A.src.pblk_ptr[pb + 1];
     if (tid < e1 - e0) jj = A.src.pblk_idx[e0 + tid];
   }
-  int i = 0, j = 0, k = 0;
-  // threads past the last node run node 0 (in bounds) and store nothing
-  const bool valid = sp_pml_node((unsigned)(blk * SPLIT_NT) + tid, g.NX, g.NY, g.NZ, g.rlo, g.rhi, i, j, k);
-  if (!valid) i = j = k = 0;
-  const unsigned n = (unsigned)i + (unsigned)g.NX * ((unsigned)j + (unsigned)g.NY * (unsigned)k);
+  const int i = E.i, j = E.j, k = E.k;
+  const unsigned n = E.n;
   const long long so = (long long)shot * A.shot_stride;
   const unsigned NN = (unsigned)g.NN;
   const unsigned SB = 8u * (3u * NN + (NN & 1u));
   const unsigned offu = n * 24u, offs = SB + n * 48u;
 
   // node-local terms the nodal pass wrote, and M^-1, issued with the records
-  double* const dst = A.out + so;
   const double minv_u = A.minvu[n];
   const double* __restrict__ tab = A.tab;
   const double sax = tab[TAB_STRETCH + 2 * i], say = tab[TAB_STRETCH + 2 * g.NX + 2 * j],
                saz = tab[TAB_STRETCH + 2 * g.NX + 2 * g.NY + 2 * k];
   double pre[9];
-  ld3(dst, offu, pre[0], pre[1], pre[2]);
-  ld2(dst, offs, pre[3], pre[4]);
-  ld2(dst, offs + 16u, pre[5], pre[6]);
-  ld2(dst, offs + 32u, pre[7], pre[8]);
+  ld_node(A.out + so, offu, offs, pre);
   double lam = 0.0, mu = 0.0;
   if constexpr (TR) ld2(A.node, n * 16u, lam, mu);
   // interface sums, read with the first batch where a regular-domain element
@@ -437,7 +469,6 @@ __global__ void __launch_bounds__(SPLIT_NT, 2) pml_pull_kernel(const SplitArgs A
   }
   // sources of this node: the block's entries are in node order, so a node's
   // entries follow its first one
-  const bool ua = u_act3(g, i, j, k);
   double src[3] = {0.0, 0.0, 0.0};
   for (int c0 = 0; c0 < e1 - e0; c0 += SPLIT_NT) {
     const int ne = min(e1 - e0 - c0, SPLIT_NT);
@@ -464,21 +495,78 @@ __global__ void __launch_bounds__(SPLIT_NT, 2) pml_pull_kernel(const SplitArgs A
       }
   }
   // finish on the node-local terms
-  if (!valid) return;
-  const int sm = smask3(g, i, j, k);
-  double out[9];
 #pragma unroll
   for (int m = 0; m < 9; ++m) {
     const double minv = m < 3 ? minv_u : (m < 6 ? minv_s : 0.5 * minv_s);
     const double sv = m < 3 ? src[m] : 0.0;
     out[m] = pre[m] + A.sc * (sv - minv * raw[m]);
   }
-  if (ua) st3(dst, offu, out[0], out[1], out[2]);
-  if (sm == 0x3f) st6(dst, offs, &out[3]);
-  else {
-    if (sm & 7) st3m(dst, offs, sm & 7, out[3], out[4], out[5]);
-    if (sm & 56) st3m(dst, offs + 24u, (sm >> 3) & 7, out[6], out[7], out[8]);
+}
+
+// the pull of stages 2 and 4
+template <bool TR>
+__global__ void __launch_bounds__(SPLIT_NT, 2) pml_pull_kernel(const SplitArgs A) {
+  __shared__ PullLds sh;
+  const int C8 = 8 * ((A.pnbn + 7) / 8);
+  if ((int)blockIdx.x >= C8) {
+    if (blockIdx.y == 0) add_domain_sources(A, ((int)blockIdx.x - C8) * SPLIT_NT + threadIdx.x);
+    return;
   }
+  const int lb = split_block(blockIdx.x, A.pnbn);
+  if (lb >= A.pnbn) return;
+  const Entry E = list_entry(A.g, lb);
+  double out[9];
+  pull_pass<TR>(A, E, lb, blockIdx.y, sh, out);
+  if (!E.own) return;
+  const unsigned NN = (unsigned)A.g.NN;
+  st_node(A.a + (long long)blockIdx.y * A.shot_stride, E.n * 24u, 8u * (3u * NN + (NN & 1u)) + E.n * 48u,
+          u_act3(A.g, E.i, E.j, E.k), smask3(A.g, E.i, E.j, E.k), out);
+}
+
+// The pull of stage 1 or 3 (P) and the nodal pass of the next stage (N) in one pass over
+// the PML nodes: the next stage's third input is the a that a node's pull has just
+// formed, so it is not read back, and a3, which nothing else reads at PML nodes, is not
+// written either (P.a null).  A block forms a for its two entries on each side as
+// well, hence a goes to another vector than the node-local terms it starts from, and
+// the flux records of odd and even stages alternate.
+// Bytes bound the two passes; in one they move 592 a node and stage against 666, and 880
+// against 1010 in the last.  64x64x32 elements: stages 1-2 82 us, as before, 3-4 113
+// against 126 us; 96x96x48 per step 1.62 -> 1.53 ms; 16x16x8, where launches
+// count, 74 -> 64 us.  Three blocks per CU (six registers spilled) are 1-3 % slower, the next
+// stage's other inputs loaded ahead of the pull no faster.
+template <bool LAST, bool TR>
+__global__ void __launch_bounds__(SPLIT_NT, 2) pull_nodal_kernel(const SplitArgs P, const SplitArgs N) {
+  __shared__ union {
+    PullLds pull;
+    NodalLds nodal;
+  } sh;
+  constexpr int NIN = LAST ? 6 : 3;
+  const int C8 = 8 * ((P.pnbn + 7) / 8);
+  if ((int)blockIdx.x >= C8) {
+    if (blockIdx.y == 0) add_domain_sources(P, ((int)blockIdx.x - C8) * SPLIT_NT + threadIdx.x);
+    return;
+  }
+  const int lb = split_block(blockIdx.x, P.pnbn);
+  if (lb >= P.pnbn) return;
+  const int shot = blockIdx.y;
+  const Entry E = list_entry(P.g, lb);
+  const long long so = (long long)shot * P.shot_stride;
+  const unsigned NN = (unsigned)P.g.NN;
+  const unsigned offu = E.n * 24u, offs = 8u * (3u * NN + (NN & 1u)) + E.n * 48u;
+  double V[NIN][9];
+  pull_pass<TR>(P, E, lb, shot, sh.pull, V[2]);
+  // inactive components are zero in every vector
+  const bool ua = u_act3(P.g, E.i, E.j, E.k);
+  const int sm = smask3(P.g, E.i, E.j, E.k);
+#pragma unroll
+  for (int m = 0; m < 9; ++m)
+    if (!(m < 3 ? ua : ((sm >> (m - 3)) & 1) != 0)) V[2][m] = 0.0;
+  if (P.a && E.own) st_node(P.a + so, offu, offs, ua, sm, V[2]);
+#pragma unroll
+  for (int q = 0; q < NIN; ++q)
+    if (q != 2) ld_node((q < 2 ? N.v[q] : N.x[q - 3]) + so, offu, offs, V[q]);
+  __syncthreads();      // the pull's LDS becomes the nodal pass's
+  nodal_pass<LAST, TR>(N, E, shot, V, sh.nodal);
 }
 
 // ------------------------------------------------- regular-domain element pass
@@ -795,7 +883,7 @@ __global__ void __launch_bounds__(SPLIT_NT, 2) stage_pair_kernel(const SplitArgs
     return;
   }
   const int shot = (b - nrd) / nn;
-  nodal_pass<false, TR>(A, (b - nrd) - shot * nn, shot, sh.nodal);
+  nodal_block<false, TR>(A, (b - nrd) - shot * nn, shot, sh.nodal);
 }
 
 }  // namespace
@@ -813,12 +901,31 @@ hipError_t launch_split_nodal(const SplitArgs& A, int last, int transpose, hipSt
   return hipGetLastError();
 }
 
-hipError_t launch_split_pull(const SplitArgs& A, int transpose, hipStream_t s) {
-  if (A.nshot <= 0 || A.pnb <= 0) return hipSuccess;
+namespace {
+// blocks of the pull: the list's, and those of the sources at regular-domain-only nodes
+dim3 pull_grid(const SplitArgs& A) {
   const int nsrc = A.src_mode ? (A.src.nrd + SPLIT_NT - 1) / SPLIT_NT : 0;
-  const dim3 grid(8 * ((A.pnb + 7) / 8) + nsrc, A.nshot);
-  if (transpose) pml_pull_kernel<true><<<grid, SPLIT_NT, 0, s>>>(A);
-  else pml_pull_kernel<false><<<grid, SPLIT_NT, 0, s>>>(A);
+  return dim3(8 * ((A.pnbn + 7) / 8) + nsrc, A.nshot);
+}
+}  // namespace
+
+hipError_t launch_split_pull(const SplitArgs& A, int transpose, hipStream_t s) {
+  if (A.nshot <= 0 || A.pnbn <= 0) return hipSuccess;
+  if (transpose) pml_pull_kernel<true><<<pull_grid(A), SPLIT_NT, 0, s>>>(A);
+  else pml_pull_kernel<false><<<pull_grid(A), SPLIT_NT, 0, s>>>(A);
+  return hipGetLastError();
+}
+
+hipError_t launch_pull_nodal(const SplitArgs& P, const SplitArgs& N, int last, int transpose, hipStream_t s) {
+  if (P.nshot <= 0 || P.pnbn <= 0) return hipSuccess;
+  const dim3 grid = pull_grid(P);
+  if (last) {
+    if (transpose) pull_nodal_kernel<true, true><<<grid, SPLIT_NT, 0, s>>>(P, N);
+    else pull_nodal_kernel<true, false><<<grid, SPLIT_NT, 0, s>>>(P, N);
+  } else {
+    if (transpose) pull_nodal_kernel<false, true><<<grid, SPLIT_NT, 0, s>>>(P, N);
+    else pull_nodal_kernel<false, false><<<grid, SPLIT_NT, 0, s>>>(P, N);
+  }
   return hipGetLastError();
 }
 
