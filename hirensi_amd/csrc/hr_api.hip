@@ -150,6 +150,7 @@ struct hr_ctx {
   // path: on the second side stream), so that it runs beside the stage kernels
   // instead of between stages.  The next launch_stage consumes it.
   std::vector<std::function<int()>> deferred;
+  OutArgs out{};                              // traces and history slice due with the next launch
   // split stage path (version 4): the flux records and interface sums of
   // split_shots shots, source entries by pull block and at regular-domain-only nodes
   bool split_ok = false;                      // the lattice fits the split path
@@ -511,13 +512,34 @@ int rd_chunk(const hr_ctx* ctx, int nshot) {
   return tz;
 }
 
-// queue the deferred per-step work on the main stream (in the order it was deferred)
+// the outputs due, of the state x
+OutArgs take_outputs(hr_ctx* ctx) {
+  OutArgs O = ctx->out;
+  ctx->out = OutArgs{};
+  O.nshot = ctx->nshot;
+  O.x2 = ctx->x[1];
+  O.xstride = (long long)field_size(ctx);
+  for (int d = 0; d < 3; ++d) { O.b0[d] = ctx->box0[d]; O.bn[d] = ctx->boxn[d]; }
+  O.NX = ctx->g.NX; O.NY = ctx->g.NY;
+  O.step = ctx->dyn ? ctx->d_step : nullptr;
+  return O;
+}
+
+// queue the outputs and the other deferred per-step work on the main stream (in the
+// order it was deferred)
 int run_deferred(hr_ctx* ctx) {
+  HIPC(launch_outputs(take_outputs(ctx), ctx->stream));
   std::vector<std::function<int()>> work;
   work.swap(ctx->deferred);
   for (auto& f : work)
     if (int rc = f()) return rc;
   return 0;
+}
+
+// forget what a solve that stopped on an error left
+void drop_deferred(hr_ctx* ctx) {
+  ctx->deferred.clear();
+  ctx->out = OutArgs{};
 }
 
 int launch_stage(hr_ctx* ctx, StageArgs& A, const Src3Spec* sp = nullptr) {
@@ -607,7 +629,7 @@ int launch_stage(hr_ctx* ctx, StageArgs& A, const Src3Spec* sp = nullptr) {
         HIPC(launch_split_nodal(B, 0, A.transpose, ctx->cstream[0]));
         if (prof) HIPC(hipEventRecord(ev.end[1], ctx->cstream[0]));
         HIPC(hipEventRecord(ctx->ev_join[0], ctx->cstream[0]));
-        const bool side_work = !ctx->deferred.empty();
+        const bool side_work = !ctx->deferred.empty() || output_blocks(ctx->out) > 0;
         if (side_work) {
           // the deferred kernels read the state the stage reads and write their
           // own outputs only; they queue on the context's stream, here the second side stream
@@ -623,9 +645,10 @@ int launch_stage(hr_ctx* ctx, StageArgs& A, const Src3Spec* sp = nullptr) {
         HIPC(hipStreamWaitEvent(ctx->stream, ctx->ev_join[0], 0));
         if (side_work) HIPC(hipStreamWaitEvent(ctx->stream, ctx->ev_join[1], 0));
       } else {
+        const OutArgs O = take_outputs(ctx);
         if (int rc = run_deferred(ctx)) return rc;
         if (prof) HIPC(hipEventRecord(ev.start[0], ctx->stream));
-        if (elements) HIPC(launch_stage_pair(B, R, upd, A.transpose, ctx->stream));
+        if (elements) HIPC(launch_stage_pair(B, R, O, upd, A.transpose, ctx->stream));
         else if (ctx->split_two) HIPC(launch_pull_nodal(ctx->split_prev, B, last, A.transpose, ctx->stream));
         else {
           HIPC(launch_split_pull(ctx->split_prev, A.transpose, ctx->stream));
@@ -791,22 +814,28 @@ int rk4_step(hr_ctx* ctx, double dt, int dir, int transpose, const double sgn[3]
   return 0;
 }
 
+// The outputs of the state x that go with the coming launch, or now (put_outputs):
 // receiver traces of every shot at the start of step n
-int record_step(hr_ctx* ctx, int n) {
-  if (ctx->f_nrec <= 0) return 0;
-  const size_t nf = field_size(ctx), rows = (size_t)ctx->f_nstep + 1;
-  const StepRef sr{ctx->dyn ? ctx->d_step : nullptr, ctx->f_nrec};
-  HIPC(launch_record(ctx->f_nrec, ctx->d_rec_slot, ctx->nshot, ctx->x[1], (long long)nf,
-                     ctx->d_traces + (size_t)n * ctx->f_nrec, (long long)(rows * ctx->f_nrec), ctx->stream, sr));
-  return 0;
+void record_step(hr_ctx* ctx, int n) {
+  if (ctx->f_nrec <= 0) return;
+  OutArgs& O = ctx->out;
+  O.nrec = ctx->f_nrec;
+  O.slot = ctx->d_rec_slot;
+  O.row = ctx->d_traces + (size_t)n * ctx->f_nrec;
+  O.rstride = ((long long)ctx->f_nstep + 1) * ctx->f_nrec;
 }
 
 // regular-domain displacement of every shot into history row `row` of blocks of `rows` rows per shot
-int store_slice(hr_ctx* ctx, double* base, size_t rows, size_t row) {
-  const size_t nf = field_size(ctx), slice = 3 * (size_t)ctx->nbox;
-  const StepRef sr{ctx->dyn ? ctx->d_step : nullptr, (long long)slice};
-  HIPC(launch_store_box(ctx->g, ctx->box0, ctx->boxn, ctx->nshot, ctx->x[1], (long long)nf, base + row * slice,
-                        (long long)(rows * slice), ctx->stream, sr));
+void store_slice(hr_ctx* ctx, double* base, size_t rows, size_t row) {
+  OutArgs& O = ctx->out;
+  const size_t slice = 3 * (size_t)ctx->nbox;
+  O.nbox = (int)ctx->nbox;
+  O.hist = base + row * slice;
+  O.hstride = (long long)(rows * slice);
+}
+
+int put_outputs(hr_ctx* ctx) {
+  HIPC(launch_outputs(take_outputs(ctx), ctx->stream));
   return 0;
 }
 
@@ -855,7 +884,7 @@ int run_steps(hr_ctx* ctx, int start, int count, int dir, const std::function<in
     const hipError_t ec = hipStreamEndCapture(ctx->stream, &g);
     if (rc || ec != hipSuccess) {
       if (g) (void)hipGraphDestroy(g);
-      ctx->deferred.clear();
+      drop_deferred(ctx);
       return rc ? rc : fail(ctx, 3, "hipStreamEndCapture failed: %s", hipGetErrorString(ec));
     }
     ctx->graph = g;
@@ -877,14 +906,15 @@ int run_forward_steps(hr_ctx* ctx, int n0, int n1, double* seg_hist, size_t seg_
   const double sgn[3] = {1.0, 1.0, 1.0};
   for (int n = n0; n < n1; ++n) {
     // the slice of the state at the start of step n, queued beside its stage 1
-    if (seg_hist) ctx->deferred.push_back([ctx, seg_hist, seg_rows, n, n0]() {
-      return store_slice(ctx, seg_hist, seg_rows, (size_t)(n - n0));
-    });
+    if (seg_hist) store_slice(ctx, seg_hist, seg_rows, (size_t)(n - n0));
     Src3Spec sp4[4];
     forward_sources(ctx, n, sp4);
     if (int rc = rk4_step(ctx, ctx->f_dt, +1, 0, sgn, sp4)) return rc;
   }
-  if (seg_hist) if (int rc = store_slice(ctx, seg_hist, seg_rows, (size_t)(n1 - n0))) return rc;
+  if (seg_hist) {
+    store_slice(ctx, seg_hist, seg_rows, (size_t)(n1 - n0));
+    if (int rc = put_outputs(ctx)) return rc;
+  }
   return 0;
 }
 
@@ -1491,7 +1521,7 @@ int forward_impl(hr_ctx* ctx, int nshot, int nstep, double dt, const double* fta
                  const long long* src_eq, const double* src_val, int nrec, const long long* rec_eq, double* traces,
                  int history, int segment, int scheme) {
   if (int rc = check_ready(ctx)) return rc;
-  ctx->deferred.clear();   // work left by a solve that stopped on an error
+  drop_deferred(ctx);   // work left by a solve that stopped on an error
   if (nshot < 1) return fail(ctx, 1, "nshot must be >= 1");
   if (nstep < 1 || !(dt > 0.0)) return fail(ctx, 1, "nstep must be >= 1 and dt > 0");
   if (!ftab) return fail(ctx, 1, "null time-function table");
@@ -1627,9 +1657,11 @@ int forward_impl(hr_ctx* ctx, int nshot, int nstep, double dt, const double* fta
   if (scheme == 1) {
     ctx->e_rows = 0;
     // traces row n = u at the start of step n (n >= 1; row 0 is u_0 = 0), as U_Store(:, ISTEP)
-    if (int rc = record_step(ctx, 0)) return rc;
+    record_step(ctx, 0);
+    if (int rc = put_outputs(ctx)) return rc;
     for (int n = 1; n <= nstep; ++n) {
-      if (int rc = record_step(ctx, n)) return rc;
+      record_step(ctx, n);
+      if (int rc = put_outputs(ctx)) return rc;
       if (int rc = cd_step(ctx, dt, n - 1)) return rc;
     }
     if (traces && nrec)
@@ -1666,17 +1698,14 @@ int forward_impl(hr_ctx* ctx, int nshot, int nstep, double dt, const double* fta
   };
   auto step_body = [&](int n) -> int {
     // traces and history slice of the state at the start of step n, queued beside its stage 1
-    ctx->deferred.push_back([ctx, n]() { return record_step(ctx, n); });
+    record_step(ctx, n);
     if (ctx->e_rows && n % ctx->e_every == 0) ctx->deferred.push_back([energy_at, n]() { return energy_at(n); });
-    if (ctx->h_store)
-      ctx->deferred.push_back([ctx, rows, n]() { return store_slice(ctx, ctx->d_hist, rows, (size_t)n); });
+    if (ctx->h_store) store_slice(ctx, ctx->d_hist, rows, (size_t)n);
     if (L > 0) {
       if (n % L == 0 && chain_slot[n / L] >= 0)
         if (int rc = snap_save(ctx, ctx->x, ctx->snap[chain_slot[n / L]], nshot)) return rc;
       if (n >= last0)
-        ctx->deferred.push_back([ctx, seg_rows, n, last0]() {
-          return store_slice(ctx, ctx->d_seg, seg_rows, (size_t)(n - last0));
-        });
+        store_slice(ctx, ctx->d_seg, seg_rows, (size_t)(n - last0));
     }
     Src3Spec sp4[4];
     forward_sources(ctx, n, sp4);
@@ -1689,10 +1718,11 @@ int forward_impl(hr_ctx* ctx, int nshot, int nstep, double dt, const double* fta
     for (int n = 0; n < nstep; ++n)
       if (int rc = step_body(n)) return rc;
   }
-  if (L > 0) if (int rc = store_slice(ctx, ctx->d_seg, seg_rows, (size_t)(nstep - last0))) return rc;
-  if (int rc = record_step(ctx, nstep)) return rc;
+  if (L > 0) store_slice(ctx, ctx->d_seg, seg_rows, (size_t)(nstep - last0));
+  record_step(ctx, nstep);
   if (ctx->e_rows && nstep % ctx->e_every == 0) if (int rc = energy_at(nstep)) return rc;
-  if (ctx->h_store) if (int rc = store_slice(ctx, ctx->d_hist, rows, (size_t)nstep)) return rc;
+  if (ctx->h_store) store_slice(ctx, ctx->d_hist, rows, (size_t)nstep);
+  if (int rc = put_outputs(ctx)) return rc;
   if (traces && nrec) {
     HIPC(hipMemcpyAsync(traces, ctx->d_traces, (size_t)nshot * rows * nrec * sizeof(double),
                         dev ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, ctx->stream));
@@ -1797,7 +1827,7 @@ int hr_misfit(hr_ctx* ctx, int nstep, double dt, int nrec, const double* dis_mea
 int hr_adjoint_gradient(hr_ctx* ctx, int nstep, double dt, int nrec, const long long* rec_eq, const double* dis_meas,
                         double* g_lambda, double* g_mu, double* misfit) {
   if (int rc = check_ready(ctx)) return rc;
-  ctx->deferred.clear();   // work left by a solve that stopped on an error
+  drop_deferred(ctx);   // work left by a solve that stopped on an error
   if (nstep != ctx->f_nstep || nrec != ctx->f_nrec || dt != ctx->f_dt)
     return fail(ctx, 1, "nstep/dt/nrec differ from the last hr_forward");
   if (ctx->f_history == HR_HISTORY_NONE) return fail(ctx, 2, "the last hr_forward kept no history");
@@ -1972,7 +2002,7 @@ int hr_adjoint_gradient(hr_ctx* ctx, int nstep, double dt, int nrec, const long 
   // the state buffers go back to the forward triple (the adjoint ones are context-owned)
   use(F, FY);
   if (status) {
-    ctx->deferred.clear();
+    drop_deferred(ctx);
     return status;
   }
   ctx->recompute = 1.0 + (double)recomputed / (double)nstep;
@@ -2053,7 +2083,7 @@ int hr_autotune(hr_ctx* ctx, int nshot, int steps, int* tz_best, double* ms_per_
   if (int rc = check_ready(ctx)) return rc;
   if (nshot < 1 || steps < 1) return fail(ctx, 1, "autotune needs nshot >= 1 and steps >= 1");
   if (int rc = ensure_shots(ctx, nshot)) return rc;
-  ctx->deferred.clear();
+  drop_deferred(ctx);
   hipEvent_t e0 = nullptr, e1 = nullptr;
   HIPC(hipEventCreate(&e0));
   HIPC(hipEventCreate(&e1));
@@ -2133,7 +2163,12 @@ int hr_gradient_accumulate(hr_ctx* ctx, const double* u, const double* p, double
   if (int rc = dalloc(ctx, &ctx->d_uslice, 3 * (size_t)ctx->nbox)) return rc;
   if (int rc = dalloc(ctx, &ctx->d_gl, ctx->nbox)) return rc;
   if (int rc = dalloc(ctx, &ctx->d_gm, ctx->nbox)) return rc;
-  HIPC(launch_store_box(ctx->g, ctx->box0, ctx->boxn, 1, ctx->tmp, 0, ctx->d_uslice, 0, ctx->stream));
+  OutArgs O = take_outputs(ctx);         // none is due here
+  O.nshot = 1;
+  O.x2 = ctx->tmp;
+  O.nbox = (int)ctx->nbox;
+  O.hist = ctx->d_uslice;
+  HIPC(launch_outputs(O, ctx->stream));
   HIPC(hipMemsetAsync(ctx->d_gl, 0, ctx->nbox * sizeof(double), ctx->stream));
   HIPC(hipMemsetAsync(ctx->d_gm, 0, ctx->nbox * sizeof(double), ctx->stream));
   HIPC(launch_gradient(ctx->g, ctx->box0, ctx->boxn, 1, ctx->d_uslice, 0, ctx->tmp2, 0, scale, ctx->d_gl,

@@ -51,12 +51,25 @@ struct StepRef {
   const int* step = nullptr;
   long long stride = 0;
 };
-// per-step kernels over all shots: strides between the shots' x2, rows, slices
-hipError_t launch_record(int nrec, const long long* slot, int nshot, const double* x2, long long xstride, double* row,
-                         long long rstride, hipStream_t s, StepRef sr = StepRef());
-hipError_t launch_store_box(const Geo& g, const int* box0, const int* boxn, int nshot, const double* x2,
-                            long long xstride, double* hist, long long hstride, hipStream_t s, StepRef sr = StepRef());
-// glam, gmu: one block of box sums per shot
+// A step's outputs of all shots: receiver traces (nrec 0: none) and the displacement of
+// the regular-domain node box as a history slice (nbox 0: none)
+struct OutArgs {
+  int nshot;
+  const double* x2;                // state vector, shots xstride apart
+  long long xstride;
+  int nrec;
+  const long long* slot;
+  double* row;                     // trace row, shots rstride apart
+  long long rstride;
+  int nbox, b0[3], bn[3], NX, NY;  // node box
+  double* hist;                    // slice, shots hstride apart
+  long long hstride;
+  const int* step;                 // captured loops: row and hist are those of step 0
+};
+constexpr int OUT_NT = 256;
+__host__ __device__ inline int output_blocks(const OutArgs& O) { return (O.nrec + OUT_NT - 1) / OUT_NT + (O.nbox + OUT_NT - 1) / OUT_NT; }
+hipError_t launch_outputs(const OutArgs& O, hipStream_t s);
+// uh, p2: shots ustride, pstride apart; glam, gmu: one block of box sums per shot
 hipError_t launch_gradient(const Geo& g, const int* box0, const int* boxn, int nshot, const double* uh,
                            long long ustride, const double* p2, long long pstride, double dt, double* glam, double* gmu,
                            hipStream_t s, StepRef sr = StepRef());
@@ -214,6 +227,7 @@ hipError_t launch_pull_nodal(const SplitArgs& P, const SplitArgs& N, int last, i
 hipError_t launch_split_pull(const SplitArgs& A, int transpose, hipStream_t s);
 void rd_tiles(const Geo& g, int tz, int t[3]);   // element pass tiles per axis (x, y, z-chunks)
 hipError_t launch_elements(const RdArgs& R, int update, hipStream_t s);
-// both passes of stages 1 and 3
-hipError_t launch_stage_pair(const SplitArgs& A, const RdArgs& R, int update, int transpose, hipStream_t s);
+// both passes of stages 1 and 3, and the step's outputs
+hipError_t launch_stage_pair(const SplitArgs& A, const RdArgs& R, const OutArgs& O, int update, int transpose,
+                             hipStream_t s);
 }  // namespace hr

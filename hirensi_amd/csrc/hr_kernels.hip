@@ -37,17 +37,6 @@ __global__ void scatter_eq_kernel(long long neq, const long long* __restrict__ s
   }
 }
 
-// receiver traces of shot blockIdx.y: row[r] = x2[slot[r]]
-__global__ void record_kernel(int nrec, const long long* __restrict__ slot, const double* __restrict__ x2,
-                              long long xstride, double* __restrict__ row, long long rstride,
-                              const int* __restrict__ step, long long stride) {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  x2 += blockIdx.y * xstride;
-  row += blockIdx.y * rstride;
-  if (step) row += (long long)(*step) * stride;
-  if (r < nrec) row[r] = x2[slot[r]];
-}
-
 // device-side step index of a captured time loop
 __global__ void step_set_kernel(int* __restrict__ step, int value) {
   if (threadIdx.x == 0) step[0] = value;
@@ -56,26 +45,8 @@ __global__ void step_advance_kernel(int* __restrict__ step, int delta) {
   if (threadIdx.x == 0) step[0] = step[0] + delta;
 }
 
-// displacement of the regular-domain node box of shot blockIdx.y -> history slice (3 x
-// nbox, component-major): a thread reads one node's three contiguous components and
-// writes them to the three component planes (each plane coalesced across lanes)
-__global__ void store_box_kernel(Geo g, int bi0, int bj0, int bk0, int bnx, int bny, int bnz,
-                                 const double* __restrict__ x2, long long xstride, double* __restrict__ hist,
-                                 long long hstride, const int* __restrict__ step, long long stride) {
-  // 32-bit indices: 9 NN < 2^31 (checked by the host)
-  const int nbox = bnx * bny * bnz;
-  x2 += blockIdx.y * xstride;
-  hist += blockIdx.y * hstride;
-  if (step) hist += (long long)(*step) * stride;
-  for (int r = blockIdx.x * blockDim.x + threadIdx.x; r < nbox; r += gridDim.x * blockDim.x) {
-    const int bi = r % bnx, bj = (r / bnx) % bny, bk = r / (bnx * bny);
-    const int n = (bi0 + bi) + g.NX * ((bj0 + bj) + g.NY * (bk0 + bk));
-    const double u0 = x2[3 * n], u1 = x2[3 * n + 1], u2 = x2[3 * n + 2];
-    hist[r] = u0;
-    hist[nbox + r] = u1;
-    hist[2 * nbox + r] = u2;
-  }
-}
+// traces and history slice of a state (hr_lattice.h)
+__global__ void __launch_bounds__(OUT_NT) output_kernel(const OutArgs O) { output_block(O, blockIdx.x, blockIdx.y); }
 
 // Per-step gradient accumulation (Update_g + ELEMENT_g_3D, Assemble_PETSc_3D.F90:556-661,
 // Element_Matrices_3D.F90:1725-1890): for every node of the regular-domain box,
@@ -411,10 +382,9 @@ hipError_t launch_scatter_eq(long long neq, const long long* slot, const double*
   hipLaunchKernelGGL(scatter_eq_kernel, dim3(grid_for(neq)), dim3(256), 0, s, neq, slot, raw, y, sc, l, z);
   return hipGetLastError();
 }
-hipError_t launch_record(int nrec, const long long* slot, int nshot, const double* x2, long long xstride, double* row,
-                         long long rstride, hipStream_t s, StepRef sr) {
-  record_kernel<<<dim3((nrec + 255) / 256, nshot), 256, 0, s>>>(nrec, slot, x2, xstride, row, rstride, sr.step,
-                                                                sr.stride);
+hipError_t launch_outputs(const OutArgs& O, hipStream_t s) {
+  if (output_blocks(O) <= 0) return hipSuccess;
+  output_kernel<<<dim3(output_blocks(O), O.nshot), OUT_NT, 0, s>>>(O);
   return hipGetLastError();
 }
 hipError_t launch_step_set(int* step, int value, hipStream_t s) {
@@ -423,13 +393,6 @@ hipError_t launch_step_set(int* step, int value, hipStream_t s) {
 }
 hipError_t launch_step_advance(int* step, int delta, hipStream_t s) {
   hipLaunchKernelGGL(step_advance_kernel, dim3(1), dim3(64), 0, s, step, delta);
-  return hipGetLastError();
-}
-hipError_t launch_store_box(const Geo& g, const int* b0, const int* bn, int nshot, const double* x2, long long xstride,
-                            double* hist, long long hstride, hipStream_t s, StepRef sr) {
-  const long long tot = (long long)bn[0] * bn[1] * bn[2];
-  store_box_kernel<<<dim3(grid_for(tot), nshot), 256, 0, s>>>(g, b0[0], b0[1], b0[2], bn[0], bn[1], bn[2], x2, xstride,
-                                                              hist, hstride, sr.step, sr.stride);
   return hipGetLastError();
 }
 hipError_t launch_gradient(const Geo& g, const int* b0, const int* bn, int nshot, const double* uh, long long ustride,

@@ -111,5 +111,32 @@ __device__ __forceinline__ double src_value(const Args& A, int jj, int shot, int
   return val;
 }
 
+// Block `blk` of a step's outputs of one shot: receiver traces row[r] = x2[slot[r]], then
+// the displacement of the regular-domain node box into the history slice (3 x
+// nbox, component-major): a thread reads one node's three contiguous components and
+// writes them to the three component planes (each plane coalesced across lanes).
+__device__ __forceinline__ void output_block(const OutArgs& O, int blk, int shot) {
+  const double* __restrict__ x2 = O.x2 + shot * O.xstride;
+  const int nrb = (O.nrec + OUT_NT - 1) / OUT_NT;
+  if (blk < nrb) {
+    const int r = blk * OUT_NT + (int)threadIdx.x;
+    double* row = O.row + shot * O.rstride;
+    if (O.step) row += (long long)(*O.step) * O.nrec;
+    if (r < O.nrec) row[r] = x2[O.slot[r]];
+    return;
+  }
+  const int r = (blk - nrb) * OUT_NT + (int)threadIdx.x;     // 32-bit: 9 NN < 2^31 (checked by the host)
+  if (r >= O.nbox) return;
+  double* hist = O.hist + shot * O.hstride;
+  if (O.step) hist += (long long)(*O.step) * 3 * O.nbox;
+  const int bi = r % O.bn[0], bj = (r / O.bn[0]) % O.bn[1], bk = r / (O.bn[0] * O.bn[1]);
+  const int n = (O.b0[0] + bi) + O.NX * ((O.b0[1] + bj) + O.NY * (O.b0[2] + bk));
+  double u0, u1, u2;
+  ld3(x2, (unsigned)n * 24u, u0, u1, u2);
+  hist[r] = u0;
+  hist[O.nbox + r] = u1;
+  hist[2 * (long long)O.nbox + r] = u2;
+}
+
 }  // namespace
 }  // namespace hr

@@ -868,11 +868,13 @@ __global__ void __launch_bounds__(SPLIT_NT, 2) element_kernel(const RdArgs A) {
 // so they share the CUs without the events of two streams, which cost 15-20 us a
 // stage.  The element blocks run longest and come first: mixed in with the nodal
 // blocks, one in two or in proportion, the pair took 5-20 % longer.
+// The traces and the history slice of the state that stage 1 reads are the last blocks.
 // Against launches of their own (on two streams from 37x29x19 up), forward and adjoint
 // step on average: 16x16x8 elements 84 -> 74 us,
 // 37x29x19 150 -> 131, 4 shots of 32x32x16 341 -> 317, 64x64x32 equal.
 template <bool UPDATE, bool TR>
-__global__ void __launch_bounds__(SPLIT_NT, 2) stage_pair_kernel(const SplitArgs A, const RdArgs R, int nrd, int nn) {
+__global__ void __launch_bounds__(SPLIT_NT, 2) stage_pair_kernel(const SplitArgs A, const RdArgs R, const OutArgs O,
+                                                                int nrd, int nn) {
   __shared__ union {
     NodalLds nodal;
     RdLds element;
@@ -880,6 +882,12 @@ __global__ void __launch_bounds__(SPLIT_NT, 2) stage_pair_kernel(const SplitArgs
   const int b = blockIdx.x;
   if (b < nrd) {
     element_pass<UPDATE>(R, b, sh.element);
+    return;
+  }
+  const int q = b - nrd - nn * A.nshot;
+  if (q >= 0) {
+    const int nb = output_blocks(O);
+    output_block(O, q % nb, q / nb);
     return;
   }
   const int shot = (b - nrd) / nn;
@@ -910,15 +918,15 @@ dim3 pull_grid(const SplitArgs& A) {
 }  // namespace
 
 hipError_t launch_split_pull(const SplitArgs& A, int transpose, hipStream_t s) {
-  if (A.nshot <= 0 || A.pnbn <= 0) return hipSuccess;
+  if (A.nshot <= 0 || pull_grid(A).x == 0) return hipSuccess;
   if (transpose) pml_pull_kernel<true><<<pull_grid(A), SPLIT_NT, 0, s>>>(A);
   else pml_pull_kernel<false><<<pull_grid(A), SPLIT_NT, 0, s>>>(A);
   return hipGetLastError();
 }
 
 hipError_t launch_pull_nodal(const SplitArgs& P, const SplitArgs& N, int last, int transpose, hipStream_t s) {
-  if (P.nshot <= 0 || P.pnbn <= 0) return hipSuccess;
   const dim3 grid = pull_grid(P);
+  if (P.nshot <= 0 || grid.x == 0) return hipSuccess;
   if (last) {
     if (transpose) pull_nodal_kernel<true, true><<<grid, SPLIT_NT, 0, s>>>(P, N);
     else pull_nodal_kernel<true, false><<<grid, SPLIT_NT, 0, s>>>(P, N);
@@ -944,18 +952,19 @@ hipError_t launch_elements(const RdArgs& R, int update, hipStream_t s) {
   return hipGetLastError();
 }
 
-hipError_t launch_stage_pair(const SplitArgs& A, const RdArgs& R, int update, int transpose, hipStream_t s) {
+hipError_t launch_stage_pair(const SplitArgs& A, const RdArgs& R, const OutArgs& O, int update, int transpose,
+                             hipStream_t s) {
   if (A.nshot <= 0) return hipSuccess;
   const long long n = (long long)R.ntx * R.nty * R.ntz * R.nshot;
   const int nrd = (int)(8 * ((n + 7) / 8)), nn = 8 * ((A.pnbn + 7) / 8);
-  const unsigned nb = (unsigned)(nrd + nn * A.nshot);
+  const unsigned nb = (unsigned)(nrd + nn * A.nshot + output_blocks(O) * O.nshot);
   if (nb == 0) return hipSuccess;
   if (update) {
-    if (transpose) stage_pair_kernel<true, true><<<nb, SPLIT_NT, 0, s>>>(A, R, nrd, nn);
-    else stage_pair_kernel<true, false><<<nb, SPLIT_NT, 0, s>>>(A, R, nrd, nn);
+    if (transpose) stage_pair_kernel<true, true><<<nb, SPLIT_NT, 0, s>>>(A, R, O, nrd, nn);
+    else stage_pair_kernel<true, false><<<nb, SPLIT_NT, 0, s>>>(A, R, O, nrd, nn);
   } else {
-    if (transpose) stage_pair_kernel<false, true><<<nb, SPLIT_NT, 0, s>>>(A, R, nrd, nn);
-    else stage_pair_kernel<false, false><<<nb, SPLIT_NT, 0, s>>>(A, R, nrd, nn);
+    if (transpose) stage_pair_kernel<false, true><<<nb, SPLIT_NT, 0, s>>>(A, R, O, nrd, nn);
+    else stage_pair_kernel<false, false><<<nb, SPLIT_NT, 0, s>>>(A, R, O, nrd, nn);
   }
   return hipGetLastError();
 }
