@@ -55,7 +55,7 @@ struct hr_ctx {
   double hel[3] = {1.0, 1.0, 1.0};          // element edges
   long long neq = 0;
   std::vector<long long> eq_slot;          // host copy of the numbering
-  long long* d_eq_slot = nullptr;
+  unsigned* d_eq_slot = nullptr;            // 32 bits: lattices past them are refused at creation or by the kernels
   // regular-domain node box
   int box0[3] = {0, 0, 0}, boxn[3] = {0, 0, 0};
   long long nbox = 0;
@@ -312,6 +312,12 @@ int upload(hr_ctx* ctx, T** d, const std::vector<T>& h) {
   return 0;
 }
 
+// the numbering's lattice slots on the device
+int upload_slots(hr_ctx* ctx) {
+  const std::vector<unsigned> s(ctx->eq_slot.begin(), ctx->eq_slot.end());
+  return upload(ctx, &ctx->d_eq_slot, s);
+}
+
 // Source entries of the split path: those at PML nodes by (shot, block) of the
 // nodal pull, in node order, the others in (shot, node) order (ptr: the (shot,
 // tile) lists of nshot shots over nt tiles)
@@ -493,19 +499,20 @@ Stage3Args args3(hr_ctx* ctx, const StageArgs& A, const Src3Spec* sp) {
 }
 
 // Element layers per z-chunk of the split path's element pass.  A block marches
-// up its chunk and computes one halo layer below it; 512 blocks (two per CU) run
-// at a time.  The chunk is the one with the fewest layers in sequence, rounds of
+// up its chunk and computes one halo layer below it; 512 blocks (two per CU; three
+// of the pass over one field) run at a time.  The chunk is the one with the fewest layers in sequence, rounds of
 // blocks times layers per block; of equals the longest, which repeats the
 // fewest halo layers.
-int rd_chunk(const hr_ctx* ctx, int nshot) {
+int rd_chunk(const hr_ctx* ctx, int nshot, int fields = 2) {
   if (ctx->rd_tz > 0) return ctx->rd_tz;
   const int layers = ctx->g.nez - ctx->g.rlo[2];
+  const int slots = fields == 2 ? 512 : 768;
   long long best = -1;
   int tz = layers;
   for (int c = layers; c >= 1; --c) {
     int t[3];
     rd_tiles(ctx->g, c, t);
-    const long long rounds = ((long long)t[0] * t[1] * t[2] * nshot + 511) / 512;
+    const long long rounds = ((long long)t[0] * t[1] * t[2] * nshot + slots - 1) / slots;
     const long long cost = rounds * (c + (t[2] > 1 ? 1 : 0));
     if (best < 0 || cost < best) { best = cost; tz = c; }
   }
@@ -547,12 +554,12 @@ int launch_stage(hr_ctx* ctx, StageArgs& A, const Src3Spec* sp = nullptr) {
   const bool counted = ctx->profiling && A.stage <= 4;
   if (counted) ctx->prof_all[A.stage] += 1;
   const bool prof = counted && (ctx->prof_tick++ % PROF_PERIOD) == 0;
-  const bool split = ctx->version == 4 && A.stage >= 1 && A.stage <= 4;
+  const bool split = ctx->version == 4 && A.stage <= 4;
   // stages 1 and 3 of the split path: both passes in one launch, or on two streams where
   // there is so much work that the events' cost no longer shows (4 shots of 48x48x24, 4380
   // nodal blocks: 47.3 ms on two streams, 47.7 in one launch; 96x96x48, 5960: 25.9, 26.4;
   // 64x64x32, 2100 blocks: equal; below that one launch is faster)
-  const bool fork = ctx->concurrent && (A.stage & 1) && (long long)ctx->pnblk * ctx->nshot > 3072;
+  const bool fork = ctx->concurrent && split && (A.stage & 1) && (long long)ctx->pnblk * ctx->nshot > 3072;
   hr_ctx::StageEv ev{A.stage, !ctx->concurrent ? 1 : (!split ? 3 : (fork ? 2 : 1)), {nullptr, nullptr, nullptr}, {nullptr, nullptr, nullptr}};
   if (prof) {
     if (ctx->ev_open.size() >= 4096) if (int rc = drain_events(ctx)) return rc;
@@ -580,6 +587,38 @@ int launch_stage(hr_ctx* ctx, StageArgs& A, const Src3Spec* sp = nullptr) {
       B.shot_stride = (long long)field_size(ctx);
       if (ctx->split_shots < B.nshot || !ctx->d_D || !ctx->split_ok)
         return fail(ctx, 3, "split stage path without its buffers for %d shots", B.nshot);
+      if (A.stage == 0) {
+        // an operator product: one shot, the sums of its single input
+        RdArgs R;
+        std::memset(&R, 0, sizeof(R));
+        B.nshot = 1;
+        B.v[0] = A.in[0];
+        B.out = B.a = A.out;
+        B.node = ctx->d_node; B.tab = ctx->d_tab; B.minvu = ctx->d_minvu; B.rwp = ctx->d_rwp;
+        B.sc = 1.0;
+        B.pnbn = ctx->pnblk;
+        B.D = ctx->d_D;
+        const int set = A.set_mask == 1 ? 0 : (A.set_mask == 2 ? 1 : 2);
+        if (set == 1) B.E = ctx->d_E;
+        R.g = B.g;
+        int t[3];
+        R.tz = rd_chunk(ctx, 1, 1);
+        rd_tiles(ctx->g, R.tz, t);
+        R.ntx = t[0]; R.nty = t[1]; R.ntz = t[2];
+        R.in[0] = A.in[0];
+        R.out[0] = A.out;
+        R.E[0] = ctx->d_E;
+        R.node = ctx->d_node;
+        R.nshot = 1;
+        if (int rc = run_deferred(ctx)) return rc;
+        if (prof) HIPC(hipEventRecord(ev.start[0], ctx->stream));
+        HIPC(launch_split_apply(B, R, set, A.transpose, ctx->stream));
+        if (prof) {
+          HIPC(hipEventRecord(ev.end[0], ctx->stream));
+          ctx->ev_open.push_back(ev);
+        }
+        return 0;
+      }
       const bool last = A.stage == 4, elements = A.stage == 1 || A.stage == 3;
       for (int a = 0; a < 3; ++a) { B.v[a] = A.in[a]; B.x[a] = A.in[3 + a]; }
       B.xn[0] = A.xnew[0]; B.xn[1] = A.xnew[1];
@@ -1053,7 +1092,7 @@ int hr_ctx_create(const hr_mesh_desc* d, hr_ctx** out) {
     ctx->version = 3;
   }
   if (int rc = setup_tiles(ctx)) return rc;
-  if (int rc = upload(ctx, &ctx->d_eq_slot, ctx->eq_slot)) return rc;
+  if (int rc = upload_slots(ctx)) return rc;
   // coordinates (origin: centred in x, y; top surface at z = 0)
   std::vector<double> xc(g.NX), yc(g.NY), zc(g.NZ);
   const double xmin = -0.5 * g.nex * d->h[0], ymin = -0.5 * g.ney * d->h[1], zmin = -(double)g.nez * d->h[2];
@@ -2213,7 +2252,7 @@ int hr_set_numbering(hr_ctx* ctx, const long long* id) {
         }
       }
   ctx->eq_slot.swap(slot);
-  if (int rc = upload(ctx, &ctx->d_eq_slot, ctx->eq_slot)) return rc;
+  if (int rc = upload_slots(ctx)) return rc;
   // MatShell scalings and the last forward were expressed in the old numbering
   for (int w = 0; w < 3; ++w) {
     ctx->shell[w].s = 1.0;

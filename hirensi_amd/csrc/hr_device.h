@@ -41,9 +41,9 @@ struct StageArgs {
 #include <hip/hip_runtime.h>
 namespace hr {
 // Host launchers (defined with the kernels).
-hipError_t launch_gather_eq(long long neq, const long long* slot, const double* x, const double* r, double* out,
+hipError_t launch_gather_eq(long long neq, const unsigned* slot, const double* x, const double* r, double* out,
                             hipStream_t s);
-hipError_t launch_scatter_eq(long long neq, const long long* slot, const double* raw, const double* y, double sc,
+hipError_t launch_scatter_eq(long long neq, const unsigned* slot, const double* raw, const double* y, double sc,
                              const double* l, double* z, hipStream_t s);
 // Device-side step index of a captured time loop: the kernel reads *step once and
 // offsets its per-step pointer by (*step) * stride elements (step null: no offset).
@@ -226,6 +226,8 @@ hipError_t launch_split_nodal(const SplitArgs& A, int last, int transpose, hipSt
 hipError_t launch_pull_nodal(const SplitArgs& P, const SplitArgs& N, int last, int transpose, hipStream_t s);
 hipError_t launch_split_pull(const SplitArgs& A, int transpose, hipStream_t s);
 void rd_tiles(const Geo& g, int tz, int t[3]);   // element pass tiles per axis (x, y, z-chunks)
+// operator product: A.v[0] = x, A.out = A.a = result, one shot; set 0 G, 1 K, 2 C
+hipError_t launch_split_apply(const SplitArgs& A, const RdArgs& R, int set, int transpose, hipStream_t s);
 hipError_t launch_elements(const RdArgs& R, int update, hipStream_t s);
 // both passes of stages 1 and 3, and the step's outputs
 hipError_t launch_stage_pair(const SplitArgs& A, const RdArgs& R, const OutArgs& O, int update, int transpose,

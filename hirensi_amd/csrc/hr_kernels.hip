@@ -18,7 +18,7 @@ namespace hr {
 
 // ----------------------------------------------------- small kernels
 // lattice <- reference numbering (optionally scaled): out[slot[e]] = x[e] * r[e]
-__global__ void gather_eq_kernel(long long neq, const long long* __restrict__ slot, const double* __restrict__ x,
+__global__ void gather_eq_kernel(long long neq, const unsigned* __restrict__ slot, const double* __restrict__ x,
                                  const double* __restrict__ r, double* __restrict__ out) {
   for (long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x; e < neq; e += (long long)gridDim.x * blockDim.x) {
     const double v = x[e];
@@ -27,7 +27,7 @@ __global__ void gather_eq_kernel(long long neq, const long long* __restrict__ sl
 }
 
 // reference numbering <- lattice: z[e] = y[e] + s * (l[e] * raw[slot[e]])
-__global__ void scatter_eq_kernel(long long neq, const long long* __restrict__ slot, const double* __restrict__ raw,
+__global__ void scatter_eq_kernel(long long neq, const unsigned* __restrict__ slot, const double* __restrict__ raw,
                                   const double* __restrict__ y, double s, const double* __restrict__ l,
                                   double* __restrict__ z) {
   for (long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x; e < neq; e += (long long)gridDim.x * blockDim.x) {
@@ -372,12 +372,12 @@ int grid_for(long long n) {
 }
 }  // namespace
 
-hipError_t launch_gather_eq(long long neq, const long long* slot, const double* x, const double* r, double* out,
+hipError_t launch_gather_eq(long long neq, const unsigned* slot, const double* x, const double* r, double* out,
                             hipStream_t s) {
   hipLaunchKernelGGL(gather_eq_kernel, dim3(grid_for(neq)), dim3(256), 0, s, neq, slot, x, r, out);
   return hipGetLastError();
 }
-hipError_t launch_scatter_eq(long long neq, const long long* slot, const double* raw, const double* y, double sc,
+hipError_t launch_scatter_eq(long long neq, const unsigned* slot, const double* raw, const double* y, double sc,
                              const double* l, double* z, hipStream_t s) {
   hipLaunchKernelGGL(scatter_eq_kernel, dim3(grid_for(neq)), dim3(256), 0, s, neq, slot, raw, y, sc, l, z);
   return hipGetLastError();

@@ -106,8 +106,8 @@ __device__ __forceinline__ void st_node(double* dst, unsigned offu, unsigned off
 // part of the update that does not need a4), and the new x1, x2 are written here.
 // The x-line sums read the x records of the block's entries from LDS:
 // consecutive list entries are x-neighbours.  V[q]: the components of v1, v2, v3
-// and, LAST, x1, x2, x3.
-template <bool LAST, bool TR>
+// and, LAST, x1, x2, x3.  RAW: an operator product, the plain sums with unit signs.
+template <bool LAST, bool TR, bool RAW = false>
 __device__ __forceinline__ void nodal_pass(const SplitArgs& A, const Entry& E, int shot,
                                            const double (*V)[9], NodalLds& sh) {
   constexpr int NIN = LAST ? 6 : 3;
@@ -149,7 +149,7 @@ __device__ __forceinline__ void nodal_pass(const SplitArgs& A, const Entry& E, i
 
   double v1u[3], vu2[3], v3u[3];
 #pragma unroll
-  for (int c = 0; c < 3; ++c) operator_inputs<TR>(XU[c], v1u[c], vu2[c], v3u[c]);
+  for (int c = 0; c < 3; ++c) operator_inputs<TR && !RAW>(XU[c], v1u[c], vu2[c], v3u[c]);
   // F[set][k], set 0 = w (G, v1), 1 = p (K, v2), 2 = e (C, v3)
   double F[3][3];
   F[2][0] = ay * az; F[2][1] = ax * az; F[2][2] = ax * ay;
@@ -185,7 +185,7 @@ __device__ __forceinline__ void nodal_pass(const SplitArgs& A, const Entry& E, i
     const double(*XS)[NIN] = &XS6[3 * hf];
     double s1[3], s2[3], s3[3];
 #pragma unroll
-    for (int tt = 0; tt < 3; ++tt) operator_inputs<TR>(XS[tt], s1[tt], s2[tt], s3[tt]);
+    for (int tt = 0; tt < 3; ++tt) operator_inputs<TR && !RAW>(XS[tt], s1[tt], s2[tt], s3[tt]);
 #pragma unroll
     for (int X = 0; X < 3; ++X) {
       const double* sv = X == 0 ? s1 : (X == 1 ? s2 : s3);
@@ -229,7 +229,7 @@ __device__ __forceinline__ void nodal_pass(const SplitArgs& A, const Entry& E, i
   double pre[9];
 #pragma unroll
   for (int m = 0; m < 9; ++m) {
-    const double minv = m < 3 ? minv_u : (m < 6 ? minv_s : 0.5 * minv_s);
+    const double minv = RAW ? -1.0 : (m < 3 ? minv_u : (m < 6 ? minv_s : 0.5 * minv_s));
     pre[m] = c3[m] - sc * (minv * dg[m]);
   }
   // x records to LDS; y and z records to memory
@@ -291,7 +291,7 @@ __device__ __forceinline__ void nodal_pass(const SplitArgs& A, const Entry& E, i
   }
 #pragma unroll
   for (int m = 0; m < 9; ++m) {
-    const double minv = m < 3 ? minv_u : (m < 6 ? minv_s : 0.5 * minv_s);
+    const double minv = RAW ? -1.0 : (m < 3 ? minv_u : (m < 6 ? minv_s : 0.5 * minv_s));
     pre[m] = pre[m] - sc * (minv * rx[m]);
   }
   st_node(A.out + so, offu, offs, ua, sm, pre);
@@ -359,8 +359,9 @@ struct PullLds {
   int slot[SPLIT_NT], cmp[SPLIT_NT], first[SPLIT_NT];  // node in the block, component; a node's first
 };
 
-// the stage's a (or, in the last stage, its part of the new x3) of a node into out
-template <bool TR>
+// the stage's a (or, in the last stage, its part of the new x3) of a node into out; RAW:
+// the operator product (E null: no element holds the operator)
+template <bool TR, bool RAW = false>
 __device__ __forceinline__ void pull_pass(const SplitArgs& A, const Entry& E, int lb, int shot, PullLds& sh,
                                           double* out) {
   double(&sVal)[SPLIT_NT] = sh.val;
@@ -398,8 +399,8 @@ __device__ __forceinline__ void pull_pass(const SplitArgs& A, const Entry& E, in
   const SpAxis ax3[3] = {sp_axis(i, g.nex, g.rlo[0], g.rhi[0]), sp_axis(j, g.ney, g.rlo[1], g.rhi[1]),
                          sp_axis(k, g.nez, g.rlo[2], g.nez)};
   const bool iface = sp_iface(ax3[0], ax3[1], ax3[2]);
-  double e3[3];
-  ld3(A.E + (long long)shot * 3 * g.NN, iface ? offu : 0u, e3[0], e3[1], e3[2]);
+  double e3[3] = {0.0, 0.0, 0.0};
+  if (!RAW || A.E) ld3(A.E + (long long)shot * 3 * g.NN, iface ? offu : 0u, e3[0], e3[1], e3[2]);
   const int sdyn = (e1 > e0 && A.step_dev) ? *A.step_dev : 0;
   if (e1 > e0) {
     if (jj >= 0) {
@@ -497,7 +498,7 @@ __device__ __forceinline__ void pull_pass(const SplitArgs& A, const Entry& E, in
   // finish on the node-local terms
 #pragma unroll
   for (int m = 0; m < 9; ++m) {
-    const double minv = m < 3 ? minv_u : (m < 6 ? minv_s : 0.5 * minv_s);
+    const double minv = RAW ? -1.0 : (m < 3 ? minv_u : (m < 6 ? minv_s : 0.5 * minv_s));
     const double sv = m < 3 ? src[m] : 0.0;
     out[m] = pre[m] + A.sc * (sv - minv * raw[m]);
   }
@@ -597,16 +598,17 @@ constexpr int RT = 4, RW = 2 * RT + 3, RWP = RW * RW, RNE = (RT + 1) * (RT + 1),
 constexpr int REW = 7;                     // elements per wavefront (9 lanes each)
 static_assert(4 * REW >= RNE && 2 * RWP <= 256 && 3 * RO * RO <= 256, "one block of four wavefronts");
 
+template <int NF>
 struct RdLds {
-  double v[2][3][3][RWP];          // field, plane (k % 3), component, window position
-  double r[2][3][RNE * 27 + 1];    // nodal forces of the elements per field and component, a spare
+  double v[NF][3][3][RWP];         // field, plane (k % 3), component, window position
+  double r[NF][3][RNE * 27 + 1];   // nodal forces of the elements per field and component, a spare
 };
 
-// block `blk` of the pass
-template <bool UPDATE>
-__device__ __forceinline__ void element_pass(const RdArgs& A, int blk, RdLds& sh) {
-  double(&sV)[2][3][3][RWP] = sh.v;
-  double(&sR)[2][3][RNE * 27 + 1] = sh.r;
+// block `blk` of the pass; NF = 1: K times one field, without the scaling by -M^-1
+template <int NF, bool UPDATE>
+__device__ __forceinline__ void element_pass(const RdArgs& A, int blk, RdLds<NF>& sh) {
+  double(&sV)[NF][3][3][RWP] = sh.v;
+  double(&sR)[NF][3][RNE * 27 + 1] = sh.r;
   const Geo3& g = A.g;
   const int tid = threadIdx.x, lane = tid & 63;
   // XCD-aware order: XCD x = blk % 8 takes a contiguous run of the (shot, y, z, x) tiles
@@ -623,7 +625,7 @@ __device__ __forceinline__ void element_pass(const RdArgs& A, int blk, RdLds& sh
   const int ez_first = max(ez0 - 1, g.rlo[2]);
   const long long so = (long long)shot * A.shot_stride;
   const double* const in0 = A.in[0] + so;
-  const double* const in1 = A.in[1] + so;
+  const double* const in1 = NF == 2 ? A.in[1] + so : nullptr;
   const unsigned NXY = (unsigned)(g.NX * g.NY);
 
   // load role: window position of one of the two new planes (regular-domain nodes only)
@@ -684,7 +686,7 @@ __device__ __forceinline__ void element_pass(const RdArgs& A, int blk, RdLds& sh
     if (ldr) {
       const unsigned o = (ln + NXY * (unsigned)k) * 24u;
       ld3(in0, o, r0[0], r0[1], r0[2]);
-      ld3(in1, o, r1[0], r1[1], r1[2]);
+      if constexpr (NF == 2) ld3(in1, o, r1[0], r1[1], r1[2]);
     }
   };
   auto put_plane = [&](int k, const double* r0, const double* r1) {
@@ -693,7 +695,7 @@ __device__ __forceinline__ void element_pass(const RdArgs& A, int blk, RdLds& sh
 #pragma unroll
       for (int c = 0; c < 3; ++c) {
         sV[0][s][c][lpos] = r0[c];
-        sV[1][s][c][lpos] = r1[c];
+        if constexpr (NF == 2) sV[NF - 1][s][c][lpos] = r1[c];
       }
     }
   };
@@ -708,9 +710,11 @@ __device__ __forceinline__ void element_pass(const RdArgs& A, int blk, RdLds& sh
 #pragma unroll
   for (int z = 0; z < 3; ++z) ld2(A.node, (sn + NXY * (unsigned)(2 * ez_first + z)) * 16u, lm[z][0], lm[z][1]);
 
-  double acc[2][3];
+  double acc[NF][3];
 #pragma unroll
-  for (int c = 0; c < 3; ++c) acc[0][c] = acc[1][c] = 0.0;
+  for (int f = 0; f < NF; ++f)
+#pragma unroll
+    for (int c = 0; c < 3; ++c) acc[f][c] = 0.0;
 
   for (int ez = ez_first; ez < ez_end; ++ez) {
     const bool halo = ez < ez0;
@@ -725,7 +729,7 @@ __device__ __forceinline__ void element_pass(const RdArgs& A, int blk, RdLds& sh
     __syncthreads();
     const int zs[3] = {(2 * ez) % 3, (2 * ez + 1) % 3, (2 * ez + 2) % 3};
 #pragma unroll
-    for (int f = 0; f < 2; ++f) {
+    for (int f = 0; f < NF; ++f) {
       double S[3][6];                               // W * stress at the line's points
       {
         double gz[3][3], u[3][3];                   // point, component
@@ -792,7 +796,7 @@ __device__ __forceinline__ void element_pass(const RdArgs& A, int blk, RdLds& sh
     // loads of the finish and of the next layer, once the stresses have freed their
     // registers
     if (fin) {
-      minv = A.minvu[n];
+      if constexpr (NF == 2) minv = A.minvu[n];
       if constexpr (UPDATE) {
         ld3(A.x[0] + so, n * 24u, x2[0], x2[1], x2[2]);
         ld3(A.x[1] + so, n * 24u, x3[0], x3[1], x3[2]);
@@ -818,7 +822,7 @@ __device__ __forceinline__ void element_pass(const RdArgs& A, int blk, RdLds& sh
       // a plane starts afresh unless the layer below started it
       const bool fresh = p != 0 || ez == ez_first;
 #pragma unroll
-      for (int f = 0; f < 2; ++f)
+      for (int f = 0; f < NF; ++f)
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
           double s = fresh ? 0.0 : acc[f][c];
@@ -833,13 +837,15 @@ __device__ __forceinline__ void element_pass(const RdArgs& A, int blk, RdLds& sh
     if (fin) {
       if (ifc) {
         const long long eo = (long long)shot * 3 * g.NN;
-        st3(A.E[0] + eo, n * 24u, acc[0][0], acc[0][1], acc[0][2]);
-        st3(A.E[1] + eo, n * 24u, acc[1][0], acc[1][1], acc[1][2]);
+#pragma unroll
+        for (int f = 0; f < NF; ++f) st3(A.E[f] + eo, n * 24u, acc[f][0], acc[f][1], acc[f][2]);
+      } else if constexpr (NF == 1) {
+        st3(A.out[0] + so, n * 24u, acc[0][0], acc[0][1], acc[0][2]);
       } else {
         double o0[3], o1[3];
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
-          const double s0 = -(minv * acc[0][c]), s1 = -(minv * acc[1][c]);
+          const double s0 = -(minv * acc[0][c]), s1 = -(minv * acc[NF - 1][c]);
           if constexpr (UPDATE) {
             const double a1 = own[0][c], a2 = own[1][c];
             o0[c] = x2[c] + (A.h * x3[c] + (A.h2 * a1 + (A.h3 * a2 + A.h4 * s0)));
@@ -859,8 +865,8 @@ __device__ __forceinline__ void element_pass(const RdArgs& A, int blk, RdLds& sh
 // the element pass alone
 template <bool UPDATE>
 __global__ void __launch_bounds__(SPLIT_NT, 2) element_kernel(const RdArgs A) {
-  __shared__ RdLds sh;
-  element_pass<UPDATE>(A, blockIdx.x, sh);
+  __shared__ RdLds<2> sh;
+  element_pass<2, UPDATE>(A, blockIdx.x, sh);
 }
 
 // The element pass (the first nrd blocks) and the nodal pass of stages 1 and 3 in one
@@ -877,11 +883,11 @@ __global__ void __launch_bounds__(SPLIT_NT, 2) stage_pair_kernel(const SplitArgs
                                                                 int nrd, int nn) {
   __shared__ union {
     NodalLds nodal;
-    RdLds element;
+    RdLds<2> element;
   } sh;
   const int b = blockIdx.x;
   if (b < nrd) {
-    element_pass<UPDATE>(R, b, sh.element);
+    element_pass<2, UPDATE>(R, b, sh.element);
     return;
   }
   const int q = b - nrd - nn * A.nshot;
@@ -892,6 +898,59 @@ __global__ void __launch_bounds__(SPLIT_NT, 2) stage_pair_kernel(const SplitArgs
   }
   const int shot = (b - nrd) / nn;
   nodal_block<false, TR>(A, (b - nrd) - shot * nn, shot, sh.nodal);
+}
+
+// Operator product with G (set 0), K (1) or C (2) on A.v[0], in place of a stage: the nodal
+// pass and, in the first nrd blocks, the element pass of K, or zeros at the
+// regular-domain-only nodes, which G and C do not reach; then the pull.
+// The tile classes of the fused stage kernel recompute each PML flux at up to five
+// nodes and put the elements' work on their own CUs only: K on 64x64x32 elements with
+// PML 6 took 130 us there against 64 + 35 us here, C^T on 45x37x22 45 against 14 + 12.
+template <bool TR>
+__global__ void __launch_bounds__(SPLIT_NT, 3) apply_pair_kernel(const SplitArgs A, const RdArgs R, int set, int nrd) {
+  __shared__ union {
+    NodalLds nodal;
+    RdLds<1> element;
+  } sh;
+  const int b = blockIdx.x;
+  if (b < nrd) {
+    if (set == 1) {
+      element_pass<1, false>(R, b, sh.element);
+      return;
+    }
+    const Geo3& g = A.g;
+    const int ni = 2 * (g.rhi[0] - g.rlo[0]) - 1, nj = 2 * (g.rhi[1] - g.rlo[1]) - 1, nk = g.NZ - 1 - 2 * g.rlo[2];
+    const int q = b * SPLIT_NT + (int)threadIdx.x;
+    if (q >= ni * nj * nk) return;
+    const int i = 2 * g.rlo[0] + 1 + q % ni, j = 2 * g.rlo[1] + 1 + (q / ni) % nj, k = 2 * g.rlo[2] + 1 + q / (ni * nj);
+    st3(A.out, 24u * (unsigned)(i + g.NX * (j + g.NY * k)), 0.0, 0.0, 0.0);
+    return;
+  }
+  const int lb = split_block(b - nrd, A.pnbn);
+  if (lb >= A.pnbn) return;
+  const Entry E = list_entry(A.g, lb);
+  const unsigned NN = (unsigned)A.g.NN;
+  double x[9], V[3][9];
+  ld_node(A.v[0], E.n * 24u, 8u * (3u * NN + (NN & 1u)) + E.n * 48u, x);
+#pragma unroll
+  for (int q = 0; q < 3; ++q)
+#pragma unroll
+    for (int m = 0; m < 9; ++m) V[q][m] = q == set ? x[m] : 0.0;
+  nodal_pass<false, TR, true>(A, E, 0, V, sh.nodal);
+}
+
+template <bool TR>
+__global__ void __launch_bounds__(SPLIT_NT, 2) apply_pull_kernel(const SplitArgs A) {
+  __shared__ PullLds sh;
+  const int lb = split_block(blockIdx.x, A.pnbn);
+  if (lb >= A.pnbn) return;
+  const Entry E = list_entry(A.g, lb);
+  double out[9];
+  pull_pass<TR, true>(A, E, lb, 0, sh, out);
+  if (!E.own) return;
+  const unsigned NN = (unsigned)A.g.NN;
+  st_node(A.a, E.n * 24u, 8u * (3u * NN + (NN & 1u)) + E.n * 48u, u_act3(A.g, E.i, E.j, E.k),
+          smask3(A.g, E.i, E.j, E.k), out);
 }
 
 }  // namespace
@@ -965,6 +1024,24 @@ hipError_t launch_stage_pair(const SplitArgs& A, const RdArgs& R, const OutArgs&
   } else {
     if (transpose) stage_pair_kernel<false, true><<<nb, SPLIT_NT, 0, s>>>(A, R, O, nrd, nn);
     else stage_pair_kernel<false, false><<<nb, SPLIT_NT, 0, s>>>(A, R, O, nrd, nn);
+  }
+  return hipGetLastError();
+}
+
+hipError_t launch_split_apply(const SplitArgs& A, const RdArgs& R, int set, int transpose, hipStream_t s) {
+  const Geo3& g = A.g;
+  long long n = (long long)R.ntx * R.nty * R.ntz;
+  if (set != 1) {
+    const long long only = (2ll * (g.rhi[0] - g.rlo[0]) - 1) * (2 * (g.rhi[1] - g.rlo[1]) - 1) * (g.NZ - 1 - 2 * g.rlo[2]);
+    n = g.rhi[0] > g.rlo[0] && g.rhi[1] > g.rlo[1] && only > 0 ? (only + SPLIT_NT - 1) / SPLIT_NT : 0;
+  }
+  const int nrd = (int)(8 * ((n + 7) / 8)), nn = 8 * ((A.pnbn + 7) / 8);
+  if (nrd + nn == 0) return hipSuccess;
+  if (transpose) apply_pair_kernel<true><<<nrd + nn, SPLIT_NT, 0, s>>>(A, R, set, nrd);
+  else apply_pair_kernel<false><<<nrd + nn, SPLIT_NT, 0, s>>>(A, R, set, nrd);
+  if (nn > 0) {
+    if (transpose) apply_pull_kernel<true><<<nn, SPLIT_NT, 0, s>>>(A);
+    else apply_pull_kernel<false><<<nn, SPLIT_NT, 0, s>>>(A);
   }
   return hipGetLastError();
 }

@@ -83,3 +83,22 @@ def test_two_streams_match_one_launch():
         sm += b
     assert np.abs(sl).max() > 0
     assert rel_l2(gl, sl) < 1e-13 and rel_l2(gm, sm) < 1e-13
+
+
+@pytest.mark.parametrize("shape,npml,tz", [((7, 11, 6), (1, 1, 1, 2, 1), 1), ((8, 6, 7), (2, 1, 1, 1, 2), 0),
+                                           ((6, 7, 5), (1, 4, 2, 2, 1), 3), ((11, 6, 9), (1, 2, 1, 1, 1), 8)])
+@pytest.mark.parametrize("which", [S.HR_K, S.HR_C, S.HR_G])
+def test_products_at_tile_and_chunk_edges(shape, npml, tz, which):
+    """Operator products on the split path, each after another operator's, whose result
+    the regular-domain nodes must not keep, against the oracle's assembled matrices."""
+    mesh = BoxMesh(*shape, npml=npml)
+    model = random_model(mesh, seed=9)
+    rng = np.random.default_rng(which)
+    x, y = rng.standard_normal(mesh.neq), rng.standard_normal(mesh.neq)
+    print(f"products {shape} npml={npml} tz={tz} which={which}", flush=True)
+    so, ctx = O.System(mesh, model), S.Context(mesh, model, tz=tz)
+    assert ctx.version() == 4
+    for tr in (False, True):
+        S.ShellMat(ctx, S.HR_K)._apply(tr, 3.0 * x, y, None)
+        z = S.ShellMat(ctx, which)._apply(tr, x, y, None)
+        assert rel_l2(z - y, so.matmult_add(which, x, np.zeros(mesh.neq), tr)) < 1e-12
