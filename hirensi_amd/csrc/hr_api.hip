@@ -60,11 +60,12 @@ struct hr_ctx {
   int box0[3] = {0, 0, 0}, boxn[3] = {0, 0, 0};
   long long nbox = 0;
   // node data (device)
-  double *d_xc = nullptr, *d_yc = nullptr, *d_zc = nullptr;
+  double* d_zc = nullptr;
   double* d_node = nullptr;                 // v3 node table (NT_COUNT x NN)
   double* d_tab = nullptr;                  // v3 small table (weights, per-axis stretch)
   Src3 src3_fwd{}, src3_adj{};              // source lists of the last forward / adjoint (device arrays)
-  std::vector<double> h_minv_u, h_wps, h_a;  // host copies for M^-1 of sources, diag M
+  std::vector<double> h_rho, h_s[3];        // element densities and stretch factors per axis (M^-1 of sources, diag M)
+  std::vector<double> h_c[3];               // lattice coordinates per axis
   bool have_material = false, have_pml = false;
   // state (device, 9*NN each)
   double* x[3] = {nullptr, nullptr, nullptr};
@@ -376,6 +377,30 @@ int build_pull_lists(hr_ctx* ctx, const std::vector<int>& ptr, const std::vector
   return 0;
 }
 
+// M^-1 of a node's displacement rows, as material_kernel forms it
+double node_minv_u(const hr_ctx* ctx, long long n) {
+  const Geo& g = ctx->g;
+  const int p[3] = {(int)(n % g.NX), (int)((n / g.NX) % g.NY), (int)(n / ((long long)g.NX * g.NY))};
+  const int ne[3] = {g.nex, g.ney, g.nez};
+  int lo[3], hi[3];
+  for (int d = 0; d < 3; ++d) {
+    lo[d] = p[d] >= 1 ? (p[d] - 1) / 2 : 0;
+    hi[d] = std::min(p[d] / 2, ne[d] - 1);
+  }
+  double mrd = 0.0, rwp = 0.0;
+  for (int ez = lo[2]; ez <= hi[2]; ++ez)
+    for (int ey = lo[1]; ey <= hi[1]; ++ey)
+      for (int ex = lo[0]; ex <= hi[0]; ++ex) {
+        const double rho = ctx->h_rho[(size_t)ex + (size_t)g.nex * ((size_t)ey + (size_t)g.ney * ez)];
+        const double W = g.wq[(p[0] - 2 * ex) + 3 * (p[1] - 2 * ey) + 9 * (p[2] - 2 * ez)];
+        const bool rd = ex >= g.rlo[0] && ex < g.rhi[0] && ey >= g.rlo[1] && ey < g.rhi[1] && ez >= g.rlo[2];
+        (rd ? mrd : rwp) += rho * W;
+      }
+  const double a = ctx->h_s[0][p[0]] * ctx->h_s[1][p[1]] * ctx->h_s[2][p[2]];
+  const double M = mrd + a * rwp;
+  return M > 0.0 ? 1.0 / M : 0.0;
+}
+
 // Sparse source grouped by owning tile.  entries: (lattice node, comp, M^-1)
 struct SrcBuild {
   std::vector<int> ptr;
@@ -409,7 +434,7 @@ SrcBuild build_src(hr_ctx* ctx, int n, const long long* eq) {
     slot_decode(g, slot, c, nd);
     s.node.push_back(nd);
     s.comp.push_back(c);
-    s.m.push_back(ctx->h_minv_u[nd]);
+    s.m.push_back(node_minv_u(ctx, nd));
     s.perm.push_back(kq.second);
   }
   return s;
@@ -1099,8 +1124,9 @@ int hr_ctx_create(const hr_mesh_desc* d, hr_ctx** out) {
   for (int i = 0; i < g.NX; ++i) xc[i] = xmin + (double)i * (0.5 * d->h[0]);
   for (int j = 0; j < g.NY; ++j) yc[j] = ymin + (double)j * (0.5 * d->h[1]);
   for (int k = 0; k < g.NZ; ++k) zc[k] = zmin + (double)k * (0.5 * d->h[2]);
-  if (int rc = upload(ctx, &ctx->d_xc, xc)) return rc;
-  if (int rc = upload(ctx, &ctx->d_yc, yc)) return rc;
+  ctx->h_c[0] = xc;
+  ctx->h_c[1] = yc;
+  ctx->h_c[2] = zc;
   if (int rc = upload(ctx, &ctx->d_zc, zc)) return rc;
   const size_t nf = field_size(ctx);
   for (int a = 0; a < 3; ++a) {
@@ -1126,7 +1152,7 @@ int hr_ctx_create(const hr_mesh_desc* d, hr_ctx** out) {
 int hr_ctx_destroy(hr_ctx* ctx) {
   if (!ctx) return 0;
   auto F = [](void* p) { if (p) (void)hipFree(p); };
-  F(ctx->d_eq_slot); F(ctx->d_xc); F(ctx->d_yc); F(ctx->d_zc);
+  F(ctx->d_eq_slot); F(ctx->d_zc);
   F(ctx->d_node); F(ctx->d_tab); F(ctx->d_ftab);
   for (int a = 0; a < 3; ++a) { F(ctx->x[a]); F(ctx->y[a]); F(ctx->gs[a]); F(ctx->shell[a].l); F(ctx->shell[a].r); }
   F(ctx->tmp); F(ctx->tmp2); F(ctx->d_traces); F(ctx->d_rec_slot); F(ctx->d_hist); F(ctx->d_seg);
@@ -1202,82 +1228,50 @@ int hr_set_material(hr_ctx* ctx, const double* lam, const double* mu, const doub
   if (!ctx->have_pml) return fail(ctx, 2, "call hr_set_pml before hr_set_material");
   const Geo& g = ctx->g;
   const size_t NN = (size_t)g.NN, nel = (size_t)g.nex * g.ney * g.nez;
-  std::vector<double> hl(NN), hm(NN), hr(nel);
-  if (ctx->flags & HR_DEVICE_PTRS) {
-    HIPC(hipMemcpy(hl.data(), lam, NN * sizeof(double), hipMemcpyDeviceToHost));
-    HIPC(hipMemcpy(hm.data(), mu, NN * sizeof(double), hipMemcpyDeviceToHost));
-    HIPC(hipMemcpy(hr.data(), rho_el, nel * sizeof(double), hipMemcpyDeviceToHost));
-  } else {
-    std::memcpy(hl.data(), lam, NN * sizeof(double));
-    std::memcpy(hm.data(), mu, NN * sizeof(double));
-    std::memcpy(hr.data(), rho_el, nel * sizeof(double));
-  }
+  const bool dev = ctx->flags & HR_DEVICE_PTRS;
+  // the densities stay on the host as well; a blocking copy, so that what the caller
+  // has queued on the default stream to fill lam and mu is done, too
+  std::vector<double> hr(nel);
+  if (dev) HIPC(hipMemcpy(hr.data(), rho_el, nel * sizeof(double), hipMemcpyDeviceToHost));
+  else std::memcpy(hr.data(), rho_el, nel * sizeof(double));
   for (size_t e = 0; e < nel; ++e)
     if (!(hr[e] > 0.0)) return fail(ctx, 1, "element %zu has non-positive density", e);
-  std::vector<double> mrd(NN, 0.0), rwp(NN, 0.0), wps(NN, 0.0);
-  for (int ez = 0; ez < g.nez; ++ez)
-    for (int ey = 0; ey < g.ney; ++ey)
-      for (int ex = 0; ex < g.nex; ++ex) {
-        const size_t e = (size_t)ex + (size_t)g.nex * ((size_t)ey + (size_t)g.ney * ez);
-        const bool rd = ex >= g.rlo[0] && ex < g.rhi[0] && ey >= g.rlo[1] && ey < g.rhi[1] && ez >= g.rlo[2];
-        for (int c = 0; c < 3; ++c)
-          for (int b = 0; b < 3; ++b)
-            for (int a = 0; a < 3; ++a) {
-              const long long n = lat(g, 2 * ex + a, 2 * ey + b, 2 * ez + c);
-              const double W = g.wq[a + 3 * b + 9 * c];
-              if (rd) mrd[n] += hr[e] * W;
-              else { rwp[n] += hr[e] * W; wps[n] += W; }
-            }
-      }
-  // coordinates
-  std::vector<double> xc(g.NX), yc(g.NY), zc(g.NZ);
-  HIPC(hipMemcpy(xc.data(), ctx->d_xc, g.NX * sizeof(double), hipMemcpyDeviceToHost));
-  HIPC(hipMemcpy(yc.data(), ctx->d_yc, g.NY * sizeof(double), hipMemcpyDeviceToHost));
-  HIPC(hipMemcpy(zc.data(), ctx->d_zc, g.NZ * sizeof(double), hipMemcpyDeviceToHost));
-  ctx->h_minv_u.assign(NN, 0.0);
-  ctx->h_a.assign(NN, 1.0);
-  for (int k = 0; k < g.NZ; ++k)
-    for (int j = 0; j < g.NY; ++j)
-      for (int i = 0; i < g.NX; ++i) {
-        const long long n = lat(g, i, j, k);
-        double s[6];
-        h_stretch(g.pml, xc[i], yc[j], zc[k], s);
-        const double a = s[0] * s[1] * s[2];
-        ctx->h_a[n] = a;
-        const double M = mrd[n] + a * rwp[n];
-        ctx->h_minv_u[n] = M > 0.0 ? 1.0 / M : 0.0;
-      }
-  ctx->h_wps = wps;
-  // v3 tables: node table [(lam, mu) pairs | (minv_u, minv_s, rwp, wps) quadruples]
-  // and [wq | per-axis stretch (a, b) pairs]
-  {
-    std::vector<double> nt((size_t)NT_COUNT * NN, 0.0);
-    double* quad = nt.data() + (size_t)NT_PAIR * NN;
-    for (size_t n = 0; n < NN; ++n) {
-      nt[2 * n] = hl[n];
-      nt[2 * n + 1] = hm[n];
-      quad[4 * n] = ctx->h_minv_u[n];
-      quad[4 * n + 1] = wps[n] > 0.0 ? 1.0 / (ctx->h_a[n] * wps[n]) : 0.0;
-      quad[4 * n + 2] = rwp[n];
-      quad[4 * n + 3] = wps[n];
-    }
-    if (int rc = upload(ctx, &ctx->d_node, nt)) return rc;
-    std::vector<double> tb(TAB_STRETCH + 2 * (size_t)(g.NX + g.NY + g.NZ), 0.0);
-    for (int q = 0; q < 27; ++q) tb[q] = g.wq[q];
-    double* ax = tb.data() + TAB_STRETCH;
-    double* ay = ax + 2 * g.NX;
-    double* az = ay + 2 * g.NY;
-    for (int i = 0; i < g.NX; ++i) { double s[6]; h_stretch(g.pml, xc[i], yc[0], zc[g.NZ - 1], s); ax[2 * i] = s[0]; ax[2 * i + 1] = s[3]; }
-    for (int j = 0; j < g.NY; ++j) { double s[6]; h_stretch(g.pml, xc[0], yc[j], zc[g.NZ - 1], s); ay[2 * j] = s[1]; ay[2 * j + 1] = s[4]; }
-    for (int k = 0; k < g.NZ; ++k) { double s[6]; h_stretch(g.pml, xc[0], yc[0], zc[k], s); az[2 * k] = s[2]; az[2 * k + 1] = s[5]; }
-    if (int rc = upload(ctx, &ctx->d_tab, tb)) return rc;
+  // stretch factors per axis: a = s_x s_y s_z, and the (a, b) pairs of the small table
+  const std::vector<double>&xc = ctx->h_c[0], &yc = ctx->h_c[1], &zc = ctx->h_c[2];
+  std::vector<double> tb(TAB_STRETCH + 2 * (size_t)(g.NX + g.NY + g.NZ), 0.0);
+  for (int q = 0; q < 27; ++q) tb[q] = g.wq[q];
+  double* ax = tb.data() + TAB_STRETCH;
+  double* ay = ax + 2 * g.NX;
+  double* az = ay + 2 * g.NY;
+  for (int i = 0; i < g.NX; ++i) { double s[6]; h_stretch(g.pml, xc[i], yc[0], zc[g.NZ - 1], s); ax[2 * i] = s[0]; ax[2 * i + 1] = s[3]; }
+  for (int j = 0; j < g.NY; ++j) { double s[6]; h_stretch(g.pml, xc[0], yc[j], zc[g.NZ - 1], s); ay[2 * j] = s[1]; ay[2 * j + 1] = s[4]; }
+  for (int k = 0; k < g.NZ; ++k) { double s[6]; h_stretch(g.pml, xc[0], yc[0], zc[k], s); az[2 * k] = s[2]; az[2 * k + 1] = s[5]; }
+  const double* const pairs[3] = {ax, ay, az};
+  const int nax[3] = {g.NX, g.NY, g.NZ};
+  for (int d = 0; d < 3; ++d) {
+    ctx->h_s[d].resize(nax[d]);
+    for (int q = 0; q < nax[d]; ++q) ctx->h_s[d][q] = pairs[d][2 * q];
   }
-  if (int rc = upload(ctx, &ctx->d_mrd, mrd)) return rc;
-  // the split path's nodal kernels read M^-1 of the u rows and the PML rho W sum
-  // from arrays of their own (8 bytes a node each); the stress rows' M^-1 and
-  // weight sum follow from the stretch factors and the element count
-  if (int rc = upload(ctx, &ctx->d_minvu, ctx->h_minv_u)) return rc;
-  if (int rc = upload(ctx, &ctx->d_rwp, rwp)) return rc;
+  if (int rc = dalloc(ctx, &ctx->d_node, (size_t)NT_COUNT * NN)) return rc;
+  if (int rc = dalloc(ctx, &ctx->d_tab, tb.size())) return rc;
+  if (int rc = dalloc(ctx, &ctx->d_mrd, NN)) return rc;
+  if (int rc = dalloc(ctx, &ctx->d_minvu, NN)) return rc;
+  if (int rc = dalloc(ctx, &ctx->d_rwp, NN)) return rc;
+  HIPC(hipMemcpyAsync(ctx->d_tab, tb.data(), tb.size() * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
+  // host arrays are staged where the quadruples go (nel < NN), which are formed last
+  const double *dl = lam, *dm = mu, *dr = rho_el;
+  if (!dev) {
+    double* const stage = ctx->d_node + NT_PAIR * NN;
+    HIPC(hipMemcpyAsync(stage, lam, NN * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
+    HIPC(hipMemcpyAsync(stage + NN, mu, NN * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
+    HIPC(hipMemcpyAsync(stage + 2 * NN, hr.data(), nel * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
+    dl = stage;
+    dm = stage + NN;
+    dr = stage + 2 * NN;
+  }
+  HIPC(launch_material(g, ctx->d_tab, dl, dm, dr, ctx->d_node, ctx->d_mrd, ctx->d_minvu, ctx->d_rwp, ctx->stream));
+  HIPC(hipStreamSynchronize(ctx->stream));
+  ctx->h_rho.swap(hr);
   ctx->have_material = true;
   // the history and traces of an earlier forward belong to the old operator
   ctx->f_nstep = 0;
@@ -1288,14 +1282,19 @@ int hr_set_material(hr_ctx* ctx, const double* lam, const double* mu, const doub
 int hr_get_diag_m(hr_ctx* ctx, double* m) {
   if (int rc = check_ready(ctx)) return rc;
   const Geo& g = ctx->g;
-  std::vector<double> hm(ctx->neq);
+  std::vector<double> hm(ctx->neq), quad((size_t)NT_QUAD * g.NN);
+  HIPC(hipMemcpy(quad.data(), ctx->d_node + NT_PAIR * (size_t)g.NN, quad.size() * sizeof(double), hipMemcpyDeviceToHost));
   for (long long e = 0; e < ctx->neq; ++e) {
     const long long slot = ctx->eq_slot[e];
     int c;
     long long n;
     slot_decode(g, slot, c, n);
-    if (c < 3) hm[e] = 1.0 / ctx->h_minv_u[n];
-    else hm[e] = (c < 6 ? 1.0 : 2.0) * ctx->h_a[n] * ctx->h_wps[n];
+    if (c < 3) hm[e] = 1.0 / quad[4 * n];
+    else {
+      const int i = (int)(n % g.NX), j = (int)((n / g.NX) % g.NY), k = (int)(n / ((long long)g.NX * g.NY));
+      const double a = ctx->h_s[0][i] * ctx->h_s[1][j] * ctx->h_s[2][k];
+      hm[e] = (c < 6 ? 1.0 : 2.0) * a * quad[4 * n + 3];
+    }
   }
   if (ctx->flags & HR_DEVICE_PTRS) HIPC(hipMemcpy(m, hm.data(), hm.size() * sizeof(double), hipMemcpyHostToDevice));
   else std::memcpy(m, hm.data(), hm.size() * sizeof(double));

@@ -51,6 +51,10 @@ struct StepRef {
   const int* step = nullptr;
   long long stride = 0;
 };
+// node table, regular-domain mass, M^-1 of the u rows and PML rho W sums of a material;
+// tab: the small table; lam, mu, rho (device) may lie where the quadruples go
+hipError_t launch_material(const Geo& g, const double* tab, const double* lam, const double* mu, const double* rho,
+                           double* node, double* mrd, double* minvu, double* rwp, hipStream_t s);
 // A step's outputs of all shots: receiver traces (nrec 0: none) and the displacement of
 // the regular-domain node box as a history slice (nbox 0: none)
 struct OutArgs {

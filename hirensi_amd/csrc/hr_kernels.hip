@@ -45,6 +45,65 @@ __global__ void step_advance_kernel(int* __restrict__ step, int delta) {
   if (threadIdx.x == 0) step[0] = step[0] + delta;
 }
 
+// The material's tables, a node per thread.  The sums over the elements that hold the
+// node are taken in element order.  First the pairs and the arrays, then
+// (material_quad_kernel) the quadruples, where host arrays may have been staged.
+// On the host, as loops over the elements with an upload of each table, they
+// took about 2 ms at 32x32x16 elements.
+__global__ void __launch_bounds__(256) material_kernel(Geo g, const double* __restrict__ tab,
+                                                       const double* __restrict__ lam, const double* __restrict__ mu,
+                                                       const double* __restrict__ rho, double* __restrict__ pairs,
+                                                       double* __restrict__ mrd, double* __restrict__ minvu,
+                                                       double* __restrict__ rwp) {
+  for (long long n = blockIdx.x * 256LL + threadIdx.x; n < g.NN; n += 256LL * gridDim.x) {
+    const int i = (int)(n % g.NX), j = (int)((n / g.NX) % g.NY), k = (int)(n / ((long long)g.NX * g.NY));
+    const int x0 = i >= 1 ? (i - 1) / 2 : 0, x1 = min(i / 2, g.nex - 1);
+    const int y0 = j >= 1 ? (j - 1) / 2 : 0, y1 = min(j / 2, g.ney - 1);
+    const int z0 = k >= 1 ? (k - 1) / 2 : 0, z1 = min(k / 2, g.nez - 1);
+    double sr = 0.0, sp = 0.0;
+    for (int ez = z0; ez <= z1; ++ez)
+      for (int ey = y0; ey <= y1; ++ey)
+        for (int ex = x0; ex <= x1; ++ex) {
+          const double m = rho[ex + (long long)g.nex * (ey + (long long)g.ney * ez)] *
+                           tab[(i - 2 * ex) + 3 * (j - 2 * ey) + 9 * (k - 2 * ez)];
+          if (ex >= g.rlo[0] && ex < g.rhi[0] && ey >= g.rlo[1] && ey < g.rhi[1] && ez >= g.rlo[2]) sr += m;
+          else sp += m;
+        }
+    const double a = tab[TAB_STRETCH + 2 * i] * tab[TAB_STRETCH + 2 * g.NX + 2 * j] *
+                     tab[TAB_STRETCH + 2 * (g.NX + g.NY) + 2 * k];
+    const double M = sr + a * sp;
+    mrd[n] = sr;
+    rwp[n] = sp;
+    minvu[n] = M > 0.0 ? 1.0 / M : 0.0;
+    pairs[2 * n] = lam[n];
+    pairs[2 * n + 1] = mu[n];
+  }
+}
+
+__global__ void __launch_bounds__(256) material_quad_kernel(Geo g, const double* __restrict__ tab,
+                                                            const double* __restrict__ minvu,
+                                                            const double* __restrict__ rwp,
+                                                            double* __restrict__ quad) {
+  for (long long n = blockIdx.x * 256LL + threadIdx.x; n < g.NN; n += 256LL * gridDim.x) {
+    const int i = (int)(n % g.NX), j = (int)((n / g.NX) % g.NY), k = (int)(n / ((long long)g.NX * g.NY));
+    const int x0 = i >= 1 ? (i - 1) / 2 : 0, x1 = min(i / 2, g.nex - 1);
+    const int y0 = j >= 1 ? (j - 1) / 2 : 0, y1 = min(j / 2, g.ney - 1);
+    const int z0 = k >= 1 ? (k - 1) / 2 : 0, z1 = min(k / 2, g.nez - 1);
+    double w = 0.0;
+    for (int ez = z0; ez <= z1; ++ez)
+      for (int ey = y0; ey <= y1; ++ey)
+        for (int ex = x0; ex <= x1; ++ex)
+          if (!(ex >= g.rlo[0] && ex < g.rhi[0] && ey >= g.rlo[1] && ey < g.rhi[1] && ez >= g.rlo[2]))
+            w += tab[(i - 2 * ex) + 3 * (j - 2 * ey) + 9 * (k - 2 * ez)];
+    const double a = tab[TAB_STRETCH + 2 * i] * tab[TAB_STRETCH + 2 * g.NX + 2 * j] *
+                     tab[TAB_STRETCH + 2 * (g.NX + g.NY) + 2 * k];
+    quad[4 * n] = minvu[n];
+    quad[4 * n + 1] = w > 0.0 ? 1.0 / (a * w) : 0.0;
+    quad[4 * n + 2] = rwp[n];
+    quad[4 * n + 3] = w;
+  }
+}
+
 // traces and history slice of a state (hr_lattice.h)
 __global__ void __launch_bounds__(OUT_NT) output_kernel(const OutArgs O) { output_block(O, blockIdx.x, blockIdx.y); }
 
@@ -382,6 +441,13 @@ hipError_t launch_scatter_eq(long long neq, const unsigned* slot, const double* 
   hipLaunchKernelGGL(scatter_eq_kernel, dim3(grid_for(neq)), dim3(256), 0, s, neq, slot, raw, y, sc, l, z);
   return hipGetLastError();
 }
+hipError_t launch_material(const Geo& g, const double* tab, const double* lam, const double* mu, const double* rho,
+                           double* node, double* mrd, double* minvu, double* rwp, hipStream_t s) {
+  material_kernel<<<grid_for(g.NN), 256, 0, s>>>(g, tab, lam, mu, rho, node, mrd, minvu, rwp);
+  material_quad_kernel<<<grid_for(g.NN), 256, 0, s>>>(g, tab, minvu, rwp, node + NT_PAIR * g.NN);
+  return hipGetLastError();
+}
+
 hipError_t launch_outputs(const OutArgs& O, hipStream_t s) {
   if (output_blocks(O) <= 0) return hipSuccess;
   output_kernel<<<dim3(output_blocks(O), O.nshot), OUT_NT, 0, s>>>(O);
