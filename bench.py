@@ -95,17 +95,17 @@ def stage_bytes(neq, nnode):
 
 
 def split_stage_bytes(mesh, transpose=False):
-    """Algorithmic bytes of one RK4 stage s of the split stage path (the default):
-    the nodal pass over the n_p PML nodes reads the 2+s raw inputs of all nine
-    components and four node-table doubles, writes the 12 flux-record doubles of
-    the y- and z-lines (the x-lines are summed in the pass, from LDS) and the
-    nine node-local outputs (stage 4: also x1, x2); the nodal pull reads the
-    flux records (each once), the node-local outputs, M^-1 of the u rows, the interface sums
-    of the n_i interface nodes (and lambda, mu when transposed) and writes nine outputs; the regular-domain
-    kernel reads, per regular-domain-only node, the displacement of the raw inputs
-    that enter its stage input (1, 2, 3, 3 vectors; stage 4: all six for the
-    update), lambda, mu and M^-1, and writes three outputs (stage 4: nine), and the
-    interface sums of the interface nodes."""
+    """Algorithmic bytes of the launches of RK4 stage s of the split stage path (the
+    default), each vector counted once per launch.  n_p PML nodes, n_r regular-domain-only
+    nodes, n_i interface nodes.  Stages 1 and 3: the nodal pass reads three vectors of
+    nine components and four node-table doubles and writes the 12 flux-record doubles of
+    the y- and z-lines and the nine node-local terms; the element pass reads two
+    displacement vectors (stage 3: x2, x3 as well), lambda, mu and M^-1 and writes two,
+    and two sums of each interface node.  Stages 2 and 4: the pull of the stage before
+    reads the node-local terms, the flux records and the interface sums and goes on as
+    this stage's nodal pass, which reads two more vectors (stage 4: x1, x2, x3 as well) and
+    the node table and writes a (stage 4: x1, x2 instead), flux records and
+    node-local terms; then this stage's own pull."""
     lo, hi = mesh.rd_lo, mesh.rd_hi
     nxy = mesh.NX * mesh.NY
     ax, ay = 2 * (hi[0] - lo[0]) - 1, 2 * (hi[1] - lo[1]) - 1
@@ -114,14 +114,12 @@ def split_stage_bytes(mesh, transpose=False):
     # interface nodes: the regular domain's node box less its interior
     bx, by, bz = ax + 2, ay + 2, mesh.NZ - 2 * lo[2]
     n_i = bx * by * bz - ax * ay * (bz - 1)
-    b = {}
-    for st in (1, 2, 3, 4):
-        k1 = n_p * (9 * (2 + st) + 4 + 12 + 9 + (18 if st == 4 else 0))
-        k3 = n_p * (12 + 9 + 1 + (2 if transpose else 0) + 9) + 3 * n_i
-        nv = 6 if st == 4 else {1: 1, 2: 2, 3: 3}[st]
-        k2 = n_r * (3 * nv + 2 + 2 + (9 if st == 4 else 3)) + 3 * n_i
-        b[st] = 8.0 * (k1 + k2 + k3)
-    return b
+    pull = n_p * (9 + 12 + 1 + (2 if transpose else 0) + 9) + 3 * n_i
+    nodal = n_p * (27 + 4 + 12 + 9)
+    element = {1: n_r * (6 + 3 + 6) + 6 * n_i, 3: n_r * (6 + 6 + 3 + 6) + 6 * n_i}
+    pn = {2: n_p * (9 + 12 + 18 + 4 + 9 + 12 + 9) + 3 * n_i, 4: n_p * (9 + 12 + 18 + 27 + 4 + 18 + 12 + 9) + 3 * n_i}
+    return {1: 8.0 * (nodal + element[1]), 2: 8.0 * (pn[2] + pull), 3: 8.0 * (nodal + element[3]),
+            4: 8.0 * (pn[4] + pull)}
 
 
 def traffic_file(split):
@@ -652,8 +650,8 @@ def main():
                      "frac": achieved / HBM_PEAK_GBS,
                      "traffic": tr["traffic_bytes_per_launch"] if tr else None,
                      "traffic_source": traffic_file(split) if tr else None,
-                     "kernel": ("RK4 stage, split path: nodal PML pass beside the regular-domain tile kernel, "
-                                "then the nodal PML pull" if split else
+                     "kernel": ("RK4 stage, split path (stages 1, 3: element and nodal pass; 2, 4: pull with the "
+                                "next nodal pass, pull)" if split else
                                 "stage kernel (all tile classes of one RK4 stage)"),
                      "launches": launches,
                      "avg_launch_us": avg_us,

@@ -134,22 +134,23 @@ struct hr_ctx {
   double *d_tr_sorted = nullptr, *d_obs_sorted = nullptr;
   size_t obs_cap = 0, sorted_cap = 0;
   // gradient post-processing: 1/Mg and restriction (geometry only, built once),
-  // regularisation vectors, per-element costs, reduction partials, staging of
-  // host material / gradient vectors
+  // regularisation vectors, sums and their partials, staging of host material /
+  // gradient vectors
   double *d_img = nullptr, *d_restr = nullptr, *d_reg = nullptr, *d_red = nullptr;
   double *d_pm = nullptr, *d_pg = nullptr;
   double recompute = 1.0;
   hipStream_t stream = nullptr;
-  // side streams (default priority) that run tile classes 1 and 2 of a stage
-  // concurrently with class 0 on the main stream; fork/join through events
+  // side streams (default priority): tile classes 1 and 2 of a fused stage beside class 0;
+  // the nodal pass and the deferred work of a large batch beside the element
+  // pass; fork/join through events
   hipStream_t cstream[2] = {nullptr, nullptr};
   hipEvent_t ev_fork = nullptr, ev_join[2] = {nullptr, nullptr};
   int concurrent = 1;
   // Per-step work (receiver traces, history slices, the per-step gradient) that
-  // only reads the state a stage-1 launch reads and does not write: queued beside
-  // the next stage launch (fused classes: on the main stream after the fork; split
-  // path: on the second side stream), so that it runs beside the stage kernels
-  // instead of between stages.  The next launch_stage consumes it.
+  // only reads the state a stage-1 launch reads and does not write: queued with the
+  // next stage launch (fused classes: on the main stream after the fork; split path:
+  // traces and slices as blocks of the launch and the rest before it, or all
+  // on the second side stream).  The next launch_stage consumes it.
   std::vector<std::function<int()>> deferred;
   OutArgs out{};                              // traces and history slice due with the next launch
   // split stage path (version 4): the flux records and interface sums of

@@ -17,9 +17,9 @@
 // besides.  K acts on v2 alone, and at regular-domain nodes nothing else does:
 // their a1 and a2 need x2 and x3 only and one pass forms both, a second one a3, a4
 // and the update, which leaves two element passes a step instead of four.
-// Measured against the stages on k1..k4 with four element passes (forward and
-// adjoint, one MI355X): 64x64x32 elements, PML 6: 0.68 -> 0.56 ms per step; 37x29x19:
-// 0.31 -> 0.16; 16x16x8: 0.23 -> 0.09.
+// Against the stages on k1..k4 with four element passes (forward and adjoint, one
+// MI355X): 64x64x32 elements, PML 6: 0.68 -> 0.56 ms per step; 37x29x19: 0.31 -> 0.16;
+// 16x16x8: 0.23 -> 0.09; with the passes as below 0.50, 0.119 and 0.062.
 
 #include <hip/hip_runtime.h>
 #include "hr_lattice.h"
@@ -589,11 +589,15 @@ __global__ void __launch_bounds__(SPLIT_NT, 2) pull_nodal_kernel(const SplitArgs
 // column once for the three points and keeps the column's lambda, mu in registers.
 // The loads of the finish and of the next layer are issued when the stresses have
 // freed their registers.  Both fields share the window pass and lambda, mu.
-// LDS bounds it: at 64x64x32 elements 52 of 78 us alone (counters), a quarter of that
-// bank conflicts that no padding of the window or the forces removed.  Beside the
-// nodal pass it takes 88 us there; the loads ahead of the stresses 100 us, three
-// blocks per CU (register spills) 92-112 us, and a form with one lattice column per
-// thread and half the LDS traffic 180 us (its widest parity class needs 300 registers).
+// LDS and the latency between its barriers bound it: at 64x64x32 elements 52 of 78 us
+// alone are LDS (counters), a quarter of that bank conflicts that no padding of the
+// window or the forces removed.  Beside the nodal pass it takes 92 us (first pass) and
+// 108 us there; the loads ahead of the stresses 100 us, three blocks per CU (register
+// spills) 92-112 us, a form with one lattice column per thread and half the LDS
+// traffic 180 us (its widest parity class needs 300 registers), a z-line's own value from
+// its register column (45 LDS reads for 63, but 182 registers and so two blocks per
+// CU for three) 102 us, 7 x 6 tiles of 512 threads (a quarter less halo work, one
+// block per CU) 15 % more at 96x96x48.
 constexpr int RT = 4, RW = 2 * RT + 3, RWP = RW * RW, RNE = (RT + 1) * (RT + 1), RO = 2 * RT + 1;
 constexpr int REW = 7;                     // elements per wavefront (9 lanes each)
 static_assert(4 * REW >= RNE && 2 * RWP <= 256 && 3 * RO * RO <= 256, "one block of four wavefronts");

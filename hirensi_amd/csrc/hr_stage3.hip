@@ -7,7 +7,7 @@
 // and the stage is one of the four of Solver_PETSc_Explicit.F90:1001-1046 (forward)
 // and :1319-1364 (adjoint, transposed with the signs -G, +K, -C), taken as
 // successive time derivatives (the scheme is in hr_split.hip, which runs the RK4
-// stages by default; this kernel runs single operators, the central-difference
+// stages and operator products by default; this kernel runs the central-difference
 // step, lattices too large for the split path and stage-kernel version 3).
 //
 // Work decomposition (same tiles as the v2 kernel): a workgroup owns TX x TY

@@ -257,14 +257,13 @@ int hr_get_history_plan(hr_ctx* ctx, int nstep, int nshot, int history, int segm
 int hr_revolve_schedule(int nseg, int nsnap, int max_actions, int* actions, int* nactions, long long* advances);
 
 /* Stage-kernel configuration: tile of 4 x ty elements in x-y (ty = 3), tz
- * elements per z-chunk (0: 10 for version 4, whose chunks start at the regular
- * domain's bottom layer; 7 for version 3), kernel version (0 keeps it): 4 (the default) splits
- * each RK4 stage into a nodal pass over the PML nodes, the tiled
- * regular-domain kernel and a nodal pull over the PML nodes; 3 runs the fused
- * tile classes (mixed, regular-domain, PML) for every stage.  Single-operator
- * applies and the central-difference step always use the fused kernel.  The
- * kernels of a stage run concurrently on side streams unless
- * HR_TILING_SERIAL_CLASSES is or-ed into version.  Invalidates the history of
+ * elements per z-chunk (0: by the box and the shots for version 4, whose chunks start at
+ * the regular domain's bottom layer; 7 for version 3), kernel version (0 keeps it): 4
+ * (the default) splits RK4 stages and operator products into nodal passes and
+ * pulls over the PML nodes and an element pass over the regular domain; 3 runs the fused
+ * tile classes (mixed, regular-domain, PML).  The central-difference step always
+ * uses the fused kernel.  Kernels run concurrently on side streams, where that
+ * is faster, unless HR_TILING_SERIAL_CLASSES is or-ed into version.  Invalidates the history of
  * the last hr_forward. */
 #define HR_TILING_SERIAL_CLASSES 0x100
 int hr_set_tiling(hr_ctx* ctx, int ty, int tz, int version);
