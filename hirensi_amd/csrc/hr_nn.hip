@@ -228,7 +228,10 @@ __device__ __forceinline__ bf16x4 read4(const unsigned short* p, const int o[4])
 // a channel chunk.  Bounded by the staging's latency and, per step, five LDS reads a
 // lane (four of two bytes); the matrix cores are 5-20 % busy.  16 -> 16 channels on 8 x
 // 16 x 32 x 32 voxels: 95 -> 23 us against the gather kernel, 128 -> 128 on 8 x 2 x 4 x
-// 4: 91 -> 23 us (216 dependent steps in 8 chunks).
+// 4: 91 -> 23 us (216 dependent steps in 8 chunks); with weights read 16 bytes a lane, the
+// 64 -> 64 layers of a 32 x 64 x 64 volume's third level 22 -> 18 us (without any weight
+// reads 16).  Operands of several steps read at once, or their places kept in
+// registers, cost the second block of a CU: 20-30 % slower over a network.
 template <int MT, int NT, int WM>
 __global__ void __launch_bounds__(256) conv3d_tile_kernel(const float* __restrict__ in,
                                                           const unsigned short* __restrict__ w,
@@ -304,12 +307,49 @@ __global__ void __launch_bounds__(256) conv3d_tile_kernel(const float* __restric
   float f0[CCH];
   // the weights of a whole chunk are loaded before they are needed: a chunk ahead
   // with one channel tile, else before the staging
-  bf16x4 a[CK / 16][MT];
+  constexpr int WU2 = (CK / 16 + 1) / 2;
+  bf16x4 a[2 * WU2][MT];
+  // rows that start at 16 bytes are read 16 bytes a lane, the four lanes of a row 64 in
+  // a row, for two steps at a time (half the requests, each a whole sector pair); `deal`
+  // then hands every lane the four weights of each step
+  const bool wide = MT == 1 && (cin & 7) == 0 && ((size_t)w & 15) == 0;
   auto weights = [&](int ci0) {
+    if (wide) {
+#pragma unroll
+      for (int u = 0; u < WU2; ++u) {
+        // the last pair is one step: its upper lanes read the lower ones' piece again
+        const int piece = 4 * u + (2 * u + 1 < CK / 16 ? kq : (kq & 1));
+        const uint4 q = *reinterpret_cast<const uint4*>(wrow[0] + ci0 * 27 + 8 * piece);
+        a[2 * u][0] = __builtin_bit_cast(bf16x4, make_uint2(q.x, q.y));
+        a[2 * u + 1][0] = __builtin_bit_cast(bf16x4, make_uint2(q.z, q.w));
+      }
+      return;
+    }
 #pragma unroll
     for (int s = 0; s < CK / 16; ++s)
 #pragma unroll
       for (int m = 0; m < MT; ++m) a[s][m] = *reinterpret_cast<const bf16x4*>(wrow[m] + ci0 * 27 + 16 * s + 4 * kq);
+  };
+  // lane group kq holds weights 32 u + 8 kq .. + 7 and needs 32 u + 4 kq .. + 3 (step 2 u)
+  // and 32 u + 16 + 4 kq .. + 3 (step 2 u + 1): exchange the piece's halves with
+  // lane bit 4, then with lane bit 5
+  auto deal = [&](bf16x4* an) {
+    if constexpr (MT == 1) {
+#pragma unroll
+      for (int u = 0; u < WU2; ++u) {
+        const uint2 lo = __builtin_bit_cast(uint2, an[2 * u]), hi = __builtin_bit_cast(uint2, an[2 * u + 1]);
+        unsigned x[2] = {lo.x, lo.y}, y[2] = {hi.x, hi.y};
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          auto t = __builtin_amdgcn_permlane16_swap(x[h], y[h], false, false);
+          t = __builtin_amdgcn_permlane32_swap(t[0], t[1], false, false);
+          x[h] = t[0];
+          y[h] = t[1];
+        }
+        an[2 * u] = __builtin_bit_cast(bf16x4, make_uint2(x[0], x[1]));
+        an[2 * u + 1] = __builtin_bit_cast(bf16x4, make_uint2(y[0], y[1]));
+      }
+    }
   };
   if (MT == 1 && aligned && cin >= CCH) weights(0);
   __syncthreads();
@@ -338,10 +378,11 @@ __global__ void __launch_bounds__(256) conv3d_tile_kernel(const float* __restric
     __syncthreads();
     if (ahead && ci0 + CCH < cin && tid < 3 * seg) fetch(tid, ci0 + CCH, f0);
     if (full) {
-      bf16x4 an[CK / 16];                    // this chunk's weights, the next one's on their way
+      bf16x4 an[2 * WU2];                    // this chunk's weights, the next one's on their way
       if constexpr (MT == 1) {
 #pragma unroll
-        for (int s = 0; s < CK / 16; ++s) an[s] = a[s][0];
+        for (int s = 0; s < 2 * WU2; ++s) an[s] = a[s][0];
+        if (wide) deal(an);
         if (ci0 + 2 * CCH <= cin) weights(ci0 + CCH);
       }
 #pragma unroll

@@ -79,3 +79,23 @@ def test_infinite_and_nan_inputs_stay_in_their_neighbourhood():
     y = torch.empty((nb, cout) + dims, device="cuda:0")
     assert L.hr_nn_conv3d(xd.data_ptr(), wd.data_ptr(), None, y.data_ptr(), cin, cout, nb, *dims, 0, s) == 0
     assert torch.equal(torch.isfinite(y.cpu()), torch.isfinite(ref))
+
+
+@pytest.mark.parametrize("cin,cout,dims", [(16, 16, (4, 8, 8)), (24, 40, (3, 5, 7)), (40, 70, (2, 4, 4)), (20, 33, (4, 4, 4)),
+                                           (128, 64, (2, 4, 8))])
+def test_weight_rows_at_every_alignment_give_the_same_bits(cin, cout, dims):
+    """Rows at 16 bytes are read 16 bytes a lane and dealt to the lanes, others in smaller
+    pieces: the same operands in the same order, so equal bits."""
+    from hirensi_amd import precond as PC
+    print(f"weight alignment cin={cin} cout={cout} dims={dims}", flush=True)
+    L, s = PC.lib(), torch.cuda.current_stream().cuda_stream
+    g = torch.Generator().manual_seed(cin + cout)
+    xd, w = torch.randn((2, cin) + dims, generator=g).to("cuda:0"), bits(torch.randn(cout * cin * 27, generator=g))
+    out = []
+    for shift in (0, 4, 1):                     # 16, 8 and 2 bytes
+        buf = torch.zeros(w.numel() + 8, dtype=torch.int16, device="cuda:0")
+        buf[shift:shift + w.numel()] = w
+        y = torch.empty((2, cout) + dims, device="cuda:0")
+        assert L.hr_nn_conv3d(xd.data_ptr(), buf.data_ptr() + 2 * shift, None, y.data_ptr(), cin, cout, 2, *dims, 0, s) == 0
+        out.append(y)
+    assert torch.equal(out[0], out[1]) and torch.equal(out[0], out[2])
