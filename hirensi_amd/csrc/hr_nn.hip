@@ -550,7 +550,42 @@ __global__ void __launch_bounds__(256) conv3d_wgrad_tile_kernel(const float* __r
         const int t = min(16 * h + r, 26);
         off[h] = (t / 9) * seg + ((t / 3) % 3 - 1) * pd.row + t % 3 - 1;
       }
-      for (int k0 = 0; k0 < n; k0 += 16) {
+      // four whole steps at a time: their places, then their operands in flight together
+      constexpr int G = 4;
+      int k0 = 0;
+      for (; k0 + 16 * G <= n; k0 += 16 * G) {
+        bf16x4 a[G][MT];
+        ushort4 q4[G];
+        short x[G][2][4];
+#pragma unroll
+        for (int s = 0; s < G; ++s) q4[s] = *reinterpret_cast<const ushort4*>(sQ + k0 + 16 * s + 4 * kq);
+#pragma unroll
+        for (int s = 0; s < G; ++s)
+#pragma unroll
+          for (int m = 0; m < MT; ++m)
+            a[s][m] = *reinterpret_cast<const bf16x4*>(sY + (16 * m + r) * WROW + k0 + 16 * s + 4 * kq);
+#pragma unroll
+        for (int s = 0; s < G; ++s)
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const unsigned short* const Xh = X + off[h];
+            x[s][h][0] = (short)Xh[q4[s].x];
+            x[s][h][1] = (short)Xh[q4[s].y];
+            x[s][h][2] = (short)Xh[q4[s].z];
+            x[s][h][3] = (short)Xh[q4[s].w];
+          }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s = 0; s < G; ++s)
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const bf16x4 b = {x[s][h][0], x[s][h][1], x[s][h][2], x[s][h][3]};
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+              acc[m][h] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[s][m], b, acc[m][h], 0, 0, 0);
+          }
+      }
+      for (; k0 < n; k0 += 16) {
         const int kk = k0 + 4 * kq;
         bf16x4 a[MT];
 #pragma unroll
