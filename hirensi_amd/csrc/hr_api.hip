@@ -153,6 +153,7 @@ struct hr_ctx {
   // on the second side stream).  The next launch_stage consumes it.
   std::vector<std::function<int()>> deferred;
   OutArgs out{};                              // traces and history slice due with the next launch
+  GradArgs grad{};                            // and the adjoint step's gradient
   // split stage path (version 4): the flux records and interface sums of
   // split_shots shots, source entries by pull block and at regular-domain-only nodes
   bool split_ok = false;                      // the lattice fits the split path
@@ -558,10 +559,17 @@ OutArgs take_outputs(hr_ctx* ctx) {
   return O;
 }
 
+GradArgs take_gradient(hr_ctx* ctx) {
+  const GradArgs G = ctx->grad;
+  ctx->grad = GradArgs{};
+  return G;
+}
+
 // queue the outputs and the other deferred per-step work on the main stream (in the
 // order it was deferred)
 int run_deferred(hr_ctx* ctx) {
   HIPC(launch_outputs(take_outputs(ctx), ctx->stream));
+  HIPC(launch_gradient(take_gradient(ctx), ctx->stream));
   std::vector<std::function<int()>> work;
   work.swap(ctx->deferred);
   for (auto& f : work)
@@ -573,6 +581,7 @@ int run_deferred(hr_ctx* ctx) {
 void drop_deferred(hr_ctx* ctx) {
   ctx->deferred.clear();
   ctx->out = OutArgs{};
+  ctx->grad = GradArgs{};
 }
 
 int launch_stage(hr_ctx* ctx, StageArgs& A, const Src3Spec* sp = nullptr) {
@@ -694,7 +703,7 @@ int launch_stage(hr_ctx* ctx, StageArgs& A, const Src3Spec* sp = nullptr) {
         HIPC(launch_split_nodal(B, 0, A.transpose, ctx->cstream[0]));
         if (prof) HIPC(hipEventRecord(ev.end[1], ctx->cstream[0]));
         HIPC(hipEventRecord(ctx->ev_join[0], ctx->cstream[0]));
-        const bool side_work = !ctx->deferred.empty() || output_blocks(ctx->out) > 0;
+        const bool side_work = !ctx->deferred.empty() || output_blocks(ctx->out) > 0 || gradient_blocks(ctx->grad) > 0;
         if (side_work) {
           // the deferred kernels read the state the stage reads and write their
           // own outputs only; they queue on the context's stream, here the second side stream
@@ -711,9 +720,14 @@ int launch_stage(hr_ctx* ctx, StageArgs& A, const Src3Spec* sp = nullptr) {
         if (side_work) HIPC(hipStreamWaitEvent(ctx->stream, ctx->ev_join[1], 0));
       } else {
         const OutArgs O = take_outputs(ctx);
+        // the gradient in the same launch where every block has its place at once, two
+        // on a CU; in more rounds its registers would cost the other blocks more than
+        // a launch (16x16x8 elements, 120 blocks: 126 -> 121 us forward and adjoint step)
+        GradArgs G{};
+        if (A.stage == 1 && stage_pair_blocks(B, R) + gradient_blocks(ctx->grad) <= 512) G = take_gradient(ctx);
         if (int rc = run_deferred(ctx)) return rc;
         if (prof) HIPC(hipEventRecord(ev.start[0], ctx->stream));
-        if (elements) HIPC(launch_stage_pair(B, R, O, upd, A.transpose, ctx->stream));
+        if (elements) HIPC(launch_stage_pair(B, R, O, G, upd, A.transpose, ctx->stream));
         else if (ctx->split_two) HIPC(launch_pull_nodal(ctx->split_prev, B, last, A.transpose, ctx->stream));
         else {
           HIPC(launch_split_pull(ctx->split_prev, A.transpose, ctx->stream));
@@ -1973,11 +1987,8 @@ int hr_adjoint_gradient(hr_ctx* ctx, int nstep, double dt, int nrec, const long 
       // queued beside stage 1 of the adjoint step, which reads but does not write p
       double* const a1 = P[1];
       const StepRef sr{ctx->dyn ? ctx->d_step : nullptr, (long long)slice};
-      ctx->deferred.push_back([ctx, nshot, uh, uh_rows, uh_row, slice, a1, nf, dt, sr]() -> int {
-        HIPC(launch_gradient(ctx->g, ctx->box0, ctx->boxn, nshot, uh + uh_row * slice, (long long)(uh_rows * slice),
-                             a1, (long long)nf, dt, ctx->d_gl, ctx->d_gm, ctx->stream, sr));
-        return 0;
-      });
+      ctx->grad = gradient_args(ctx->g, ctx->box0, ctx->boxn, nshot, uh + uh_row * slice, (long long)(uh_rows * slice), a1,
+                                (long long)nf, dt, ctx->d_gl, ctx->d_gm, sr);
     }
     // misfit sources r(t_n), their mean with r(t_{n-1}) and r(t_{n-1}) over the step of
     // -dt: s1 = r(t_n), s2 = (r(t_n) - r(t_{n-1})) / dt, s4 = 0 (the mean is exact)
@@ -2210,8 +2221,9 @@ int hr_gradient_accumulate(hr_ctx* ctx, const double* u, const double* p, double
   HIPC(launch_outputs(O, ctx->stream));
   HIPC(hipMemsetAsync(ctx->d_gl, 0, ctx->nbox * sizeof(double), ctx->stream));
   HIPC(hipMemsetAsync(ctx->d_gm, 0, ctx->nbox * sizeof(double), ctx->stream));
-  HIPC(launch_gradient(ctx->g, ctx->box0, ctx->boxn, 1, ctx->d_uslice, 0, ctx->tmp2, 0, scale, ctx->d_gl,
-                       ctx->d_gm, ctx->stream));
+  HIPC(launch_gradient(gradient_args(ctx->g, ctx->box0, ctx->boxn, 1, ctx->d_uslice, 0, ctx->tmp2, 0, scale, ctx->d_gl,
+                                     ctx->d_gm),
+                       ctx->stream));
   double *gl = g_lambda, *gm = g_mu;
   if (!dev) {
     if (int rc = dalloc(ctx, &ctx->d_pg, 2 * NN)) return rc;

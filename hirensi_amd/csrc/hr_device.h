@@ -73,10 +73,27 @@ struct OutArgs {
 constexpr int OUT_NT = 256;
 __host__ __device__ inline int output_blocks(const OutArgs& O) { return (O.nrec + OUT_NT - 1) / OUT_NT + (O.nbox + OUT_NT - 1) / OUT_NT; }
 hipError_t launch_outputs(const OutArgs& O, hipStream_t s);
-// uh, p2: shots ustride, pstride apart; glam, gmu: one block of box sums per shot
-hipError_t launch_gradient(const Geo& g, const int* box0, const int* boxn, int nshot, const double* uh,
-                           long long ustride, const double* p2, long long pstride, double dt, double* glam, double* gmu,
-                           hipStream_t s, StepRef sr = StepRef());
+// One adjoint step's gradient sums of all shots
+struct GradArgs {
+  int ntx, nty, ntz, tz, nshot;    // tiles, planes per z-chunk (gradient_args)
+  int NX, NY, b0[3], bn[3];        // node box
+  double dxi[3], wdt;              // centre point's weight x dt
+  const double* uh;                // history slice (3 x box), shots ustride apart
+  long long ustride;
+  const double* p2;                // adjoint x2, shots pstride apart
+  long long pstride;
+  double *glam, *gmu;              // a block of box sums per shot
+  const int* step;                 // captured loops: uh is the slice of step 0, stride elements a step
+  long long stride;
+};
+GradArgs gradient_args(const Geo& g, const int* box0, const int* boxn, int nshot, const double* uh, long long ustride,
+                       const double* p2, long long pstride, double dt, double* glam, double* gmu,
+                       StepRef sr = StepRef());
+// whole eights of blocks (0: none)
+__host__ __device__ inline int gradient_blocks(const GradArgs& G) {
+  return (int)(8 * (((long long)G.ntx * G.nty * G.ntz * G.nshot + 7) / 8));
+}
+hipError_t launch_gradient(const GradArgs& G, hipStream_t s);
 // *step = value; *step += delta (one lane, a vector store)
 hipError_t launch_step_set(int* step, int value, hipStream_t s);
 hipError_t launch_step_advance(int* step, int delta, hipStream_t s);
@@ -234,6 +251,7 @@ void rd_tiles(const Geo& g, int tz, int t[3]);   // element pass tiles per axis 
 hipError_t launch_split_apply(const SplitArgs& A, const RdArgs& R, int set, int transpose, hipStream_t s);
 hipError_t launch_elements(const RdArgs& R, int update, hipStream_t s);
 // both passes of stages 1 and 3, and the step's outputs
-hipError_t launch_stage_pair(const SplitArgs& A, const RdArgs& R, const OutArgs& O, int update, int transpose,
-                             hipStream_t s);
+int stage_pair_blocks(const SplitArgs& A, const RdArgs& R);   // of the two passes
+hipError_t launch_stage_pair(const SplitArgs& A, const RdArgs& R, const OutArgs& O, const GradArgs& G, int update,
+                             int transpose, hipStream_t s);
 }  // namespace hr

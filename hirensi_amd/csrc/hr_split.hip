@@ -22,6 +22,7 @@
 // 16x16x8: 0.23 -> 0.09; with the passes as below 0.50, 0.119 and 0.062.
 
 #include <hip/hip_runtime.h>
+#include "hr_gradient.h"
 #include "hr_lattice.h"
 #include "hr_split.h"
 
@@ -882,26 +883,40 @@ __global__ void __launch_bounds__(SPLIT_NT, 2) element_kernel(const RdArgs A) {
 // Against launches of their own (on two streams from 37x29x19 up), forward and adjoint
 // step on average: 16x16x8 elements 84 -> 74 us,
 // 37x29x19 150 -> 131, 4 shots of 32x32x16 341 -> 317, 64x64x32 equal.
-template <bool UPDATE, bool TR>
+// GRAD: the adjoint step's gradient sums as well, after the element blocks; their 236
+// registers leave two blocks on a CU, so only where all blocks fit at once (see
+// the launch's caller).
+template <bool UPDATE, bool TR, bool GRAD>
 __global__ void __launch_bounds__(SPLIT_NT, 2) stage_pair_kernel(const SplitArgs A, const RdArgs R, const OutArgs O,
-                                                                int nrd, int nn) {
+                                                                const GradArgs G, int nrd, int nn) {
+  static_assert(GNT == SPLIT_NT, "one block size");
   __shared__ union {
     NodalLds nodal;
     RdLds<2> element;
+    GradLds grad;
   } sh;
-  const int b = blockIdx.x;
+  int b = blockIdx.x;
   if (b < nrd) {
     element_pass<2, UPDATE>(R, b, sh.element);
     return;
   }
-  const int q = b - nrd - nn * A.nshot;
+  b -= nrd;
+  if constexpr (GRAD) {
+    const int ng = gradient_blocks(G);
+    if (b < ng) {
+      gradient_block(G, b, sh.grad);
+      return;
+    }
+    b -= ng;
+  }
+  const int q = b - nn * A.nshot;
   if (q >= 0) {
     const int nb = output_blocks(O);
     output_block(O, q % nb, q / nb);
     return;
   }
-  const int shot = (b - nrd) / nn;
-  nodal_block<false, TR>(A, (b - nrd) - shot * nn, shot, sh.nodal);
+  const int shot = b / nn;
+  nodal_block<false, TR>(A, b - shot * nn, shot, sh.nodal);
 }
 
 // Operator product with G (set 0), K (1) or C (2) on A.v[0], in place of a stage: the nodal
@@ -1015,19 +1030,25 @@ hipError_t launch_elements(const RdArgs& R, int update, hipStream_t s) {
   return hipGetLastError();
 }
 
-hipError_t launch_stage_pair(const SplitArgs& A, const RdArgs& R, const OutArgs& O, int update, int transpose,
-                             hipStream_t s) {
-  if (A.nshot <= 0) return hipSuccess;
+int stage_pair_blocks(const SplitArgs& A, const RdArgs& R) {
   const long long n = (long long)R.ntx * R.nty * R.ntz * R.nshot;
-  const int nrd = (int)(8 * ((n + 7) / 8)), nn = 8 * ((A.pnbn + 7) / 8);
-  const unsigned nb = (unsigned)(nrd + nn * A.nshot + output_blocks(O) * O.nshot);
+  return (int)(8 * ((n + 7) / 8)) + 8 * ((A.pnbn + 7) / 8) * A.nshot;
+}
+
+hipError_t launch_stage_pair(const SplitArgs& A, const RdArgs& R, const OutArgs& O, const GradArgs& G, int update,
+                             int transpose, hipStream_t s) {
+  if (A.nshot <= 0) return hipSuccess;
+  const int nn = 8 * ((A.pnbn + 7) / 8), nrd = stage_pair_blocks(A, R) - nn * A.nshot, ng = gradient_blocks(G);
+  if (ng > 0 && (update || !transpose)) return hipErrorInvalidValue;   // the gradient goes with the adjoint's stage 1
+  const unsigned nb = (unsigned)(nrd + nn * A.nshot + ng + output_blocks(O) * O.nshot);
   if (nb == 0) return hipSuccess;
-  if (update) {
-    if (transpose) stage_pair_kernel<true, true><<<nb, SPLIT_NT, 0, s>>>(A, R, O, nrd, nn);
-    else stage_pair_kernel<true, false><<<nb, SPLIT_NT, 0, s>>>(A, R, O, nrd, nn);
+  if (ng > 0) stage_pair_kernel<false, true, true><<<nb, SPLIT_NT, 0, s>>>(A, R, O, G, nrd, nn);
+  else if (update) {
+    if (transpose) stage_pair_kernel<true, true, false><<<nb, SPLIT_NT, 0, s>>>(A, R, O, G, nrd, nn);
+    else stage_pair_kernel<true, false, false><<<nb, SPLIT_NT, 0, s>>>(A, R, O, G, nrd, nn);
   } else {
-    if (transpose) stage_pair_kernel<false, true><<<nb, SPLIT_NT, 0, s>>>(A, R, O, nrd, nn);
-    else stage_pair_kernel<false, false><<<nb, SPLIT_NT, 0, s>>>(A, R, O, nrd, nn);
+    if (transpose) stage_pair_kernel<false, true, false><<<nb, SPLIT_NT, 0, s>>>(A, R, O, G, nrd, nn);
+    else stage_pair_kernel<false, false, false><<<nb, SPLIT_NT, 0, s>>>(A, R, O, G, nrd, nn);
   }
   return hipGetLastError();
 }
