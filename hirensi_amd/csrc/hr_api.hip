@@ -592,7 +592,7 @@ int launch_stage(hr_ctx* ctx, StageArgs& A, const Src3Spec* sp = nullptr) {
   const bool split = ctx->version == 4 && A.stage <= 4;
   // stages 1 and 3 of the split path: both passes in one launch, or on two streams where
   // there is so much work that the events' cost no longer shows (4 shots of 48x48x24, 4380
-  // nodal blocks: 47.3 ms on two streams, 47.7 in one launch; 96x96x48, 5960: 25.9, 26.4;
+  // nodal blocks: 44.7 ms on two streams, 45.0 in one launch; 96x96x48, 5960: 24.5, 25.0;
   // 64x64x32, 2100 blocks: equal; below that one launch is faster)
   const bool fork = ctx->concurrent && split && (A.stage & 1) && (long long)ctx->pnblk * ctx->nshot > 3072;
   hr_ctx::StageEv ev{A.stage, !ctx->concurrent ? 1 : (!split ? 3 : (fork ? 2 : 1)), {nullptr, nullptr, nullptr}, {nullptr, nullptr, nullptr}};
