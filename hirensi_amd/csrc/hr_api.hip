@@ -155,7 +155,8 @@ struct hr_ctx {
   OutArgs out{};                              // traces and history slice due with the next launch
   GradArgs grad{};                            // and the adjoint step's gradient
   // split stage path (version 4): the flux records and interface sums of
-  // split_shots shots, source entries by pull block and at regular-domain-only nodes
+  // split_shots shots (0: none, after an allocation that failed), source entries by pull
+  // block and at regular-domain-only nodes
   bool split_ok = false;                      // the lattice fits the split path
   int pnblk = 0;                              // SPLIT_OWN-node blocks of the PML nodes
   double* d_D = nullptr;                      // flux records: 12 NN doubles per shot, of odd stages, then of even ones
@@ -163,6 +164,7 @@ struct hr_ctx {
   SplitArgs split_prev{};                     // the stage whose pull is still to come
   double* d_E = nullptr;                      // two fields: 3 NN doubles per shot each
   int split_shots = 0;
+  double mem_limit = -1.0;                    // device bytes the context may hold (negative: no limit)
   int rd_tz = 0;                              // layers per z-chunk of the element pass (0: rd_chunk's rule)
   struct PullLists {
     int *ptr = nullptr, *idx = nullptr, *slot = nullptr, *rd_idx = nullptr, *rd_shot = nullptr;
@@ -228,6 +230,25 @@ int fail(hr_ctx* c, int code, const char* fmt, ...) {
     if (_e != hipSuccess) return fail(ctx, (int)_e, "%s failed: %s", #call, hipGetErrorString(_e)); \
   } while (0)
 
+// device bytes of the context's buffers (dalloc) and snapshots
+double held_bytes(const hr_ctx* ctx) {
+  double b = (double)ctx->snap.size() * (double)ctx->snap_elems * sizeof(double);
+  for (auto& kv : ctx->caps) b += (double)kv.second;
+  return b;
+}
+
+// hipMalloc within the context's limit (hr_limit_memory).  A failure leaves no
+// error behind for the next launch's check to find.
+hipError_t device_malloc(hr_ctx* ctx, void** p, size_t bytes) {
+  hipError_t e = hipErrorOutOfMemory;
+  if (ctx->mem_limit < 0.0 || held_bytes(ctx) + (double)bytes <= ctx->mem_limit) {
+    e = hipMalloc(p, bytes);
+    if (e != hipSuccess) (void)hipGetLastError();
+  }
+  if (e != hipSuccess) *p = nullptr;
+  return e;
+}
+
 // Grow-only device allocation: a pointer field keeps its buffer while the
 // request fits, so repeated solves allocate nothing (contents are not kept on
 // growth).
@@ -237,11 +258,10 @@ int dalloc(hr_ctx* ctx, T** p, size_t n) {
   auto it = ctx->caps.find((void*)p);
   if (*p && it != ctx->caps.end() && it->second >= n * sizeof(T)) return 0;
   if (*p) { (void)hipFree(*p); *p = nullptr; }
-  hipError_t e = hipMalloc((void**)p, n * sizeof(T));
-  if (e != hipSuccess) {
-    ctx->caps.erase((void*)p);
+  ctx->caps.erase((void*)p);
+  const hipError_t e = device_malloc(ctx, (void**)p, n * sizeof(T));
+  if (e != hipSuccess)
     return fail(ctx, (int)e, "hipMalloc of %zu bytes failed: %s", n * sizeof(T), hipGetErrorString(e));
-  }
   ctx->caps[(void*)p] = n * sizeof(T);
   return 0;
 }
@@ -589,7 +609,9 @@ int launch_stage(hr_ctx* ctx, StageArgs& A, const Src3Spec* sp = nullptr) {
   const bool counted = ctx->profiling && A.stage <= 4;
   if (counted) ctx->prof_all[A.stage] += 1;
   const bool prof = counted && (ctx->prof_tick++ % PROF_PERIOD) == 0;
-  const bool split = ctx->version == 4 && A.stage <= 4;
+  // an operator product needs the buffers of one shot, and takes the fused kernel where a
+  // batch that did not fit has left none
+  const bool split = ctx->version == 4 && A.stage <= 4 && (A.stage > 0 || ctx->split_shots > 0);
   // stages 1 and 3 of the split path: both passes in one launch, or on two streams where
   // there is so much work that the events' cost no longer shows (4 shots of 48x48x24, 4380
   // nodal blocks: 44.7 ms on two streams, 45.0 in one launch; 96x96x48, 5960: 24.5, 25.0;
@@ -620,7 +642,7 @@ int launch_stage(hr_ctx* ctx, StageArgs& A, const Src3Spec* sp = nullptr) {
       B.g = geo3(ctx);
       B.nshot = ctx->nshot;
       B.shot_stride = (long long)field_size(ctx);
-      if (ctx->split_shots < B.nshot || !ctx->d_D || !ctx->split_ok)
+      if (ctx->split_shots < (A.stage > 0 ? B.nshot : 1) || !ctx->split_ok)
         return fail(ctx, 3, "split stage path without its buffers for %d shots", B.nshot);
       if (A.stage == 0) {
         // an operator product: one shot, the sums of its single input
@@ -828,26 +850,27 @@ int check_ready(hr_ctx* ctx) {
 
 // state buffers for nshot shots (shot-major); contents are not kept on growth
 // flux records (y- and z-lines) and interface sums of the split path for
-// shot_cap shots; the records of regular-domain-only nodes are never written and
+// nshot shots; the records of regular-domain-only nodes are never written and
 // stay zero (the pull reads them)
 int ensure_split(hr_ctx* ctx) {
-  if (ctx->version != 4 || ctx->split_shots >= ctx->shot_cap) return 0;
-  const size_t nd = 12 * (size_t)ctx->g.NN * ctx->shot_cap, ne = 6 * (size_t)ctx->g.NN * ctx->shot_cap;
+  if (ctx->version != 4 || ctx->split_shots >= ctx->nshot) return 0;
+  const size_t nd = 12 * (size_t)ctx->g.NN * ctx->nshot, ne = 6 * (size_t)ctx->g.NN * ctx->nshot;
+  ctx->split_shots = 0;                  // a failure below leaves the buffers incomplete
   if (int rc = dalloc(ctx, &ctx->d_E, ne)) return rc;
   ctx->split_two = dalloc(ctx, &ctx->d_D, 2 * nd) == 0;
   if (!ctx->split_two) {
-    (void)hipGetLastError();
     ctx->err.clear();
     if (int rc = dalloc(ctx, &ctx->d_D, nd)) return rc;
   }
   HIPC(hipMemsetAsync(ctx->d_D, 0, (ctx->split_two ? 2 : 1) * nd * sizeof(double), ctx->stream));
-  ctx->split_shots = ctx->shot_cap;
+  ctx->split_shots = ctx->nshot;
   return 0;
 }
 
 int ensure_shots(hr_ctx* ctx, int nshot) {
   const size_t nf = field_size(ctx);
   if (nshot > ctx->shot_cap) {
+    ctx->shot_cap = 0;                   // a failure leaves vectors missing: the next solve takes them anew
     for (int a = 0; a < 3; ++a) {
       if (int rc = dalloc(ctx, &ctx->x[a], nf * nshot)) return rc;
       if (int rc = dalloc(ctx, &ctx->y[a], nf * nshot)) return rc;
@@ -1001,6 +1024,12 @@ int run_forward_steps(hr_ctx* ctx, int n0, int n1, double* seg_hist, size_t seg_
 
 // =================================================================== C ABI
 extern "C" {
+
+int hr_limit_memory(hr_ctx* ctx, double more) {
+  if (!ctx) return 1;
+  ctx->mem_limit = more < 0.0 ? -1.0 : held_bytes(ctx) + more;
+  return 0;
+}
 
 const char* hr_last_error(const hr_ctx* ctx) { return ctx ? ctx->err.c_str() : "null context"; }
 
@@ -1545,7 +1574,7 @@ int ensure_history_buffers(hr_ctx* ctx, int nshot) {
   const size_t need = (size_t)std::max(ctx->h_plan.s, ctx->h_nsnap);
   while (ctx->snap.size() < need) {
     double* p = nullptr;
-    hipError_t e = hipMalloc((void**)&p, elems * sizeof(double));
+    const hipError_t e = device_malloc(ctx, (void**)&p, elems * sizeof(double));
     if (e != hipSuccess) return fail(ctx, (int)e, "snapshot allocation failed: %s", hipGetErrorString(e));
     ctx->snap.push_back(p);
   }

@@ -17,3 +17,10 @@ bool ctx_device_ptrs(const hr_ctx* ctx);
 hipStream_t ctx_stream(const hr_ctx* ctx);
 int ctx_fail(hr_ctx* ctx, int code, const char* msg);
 }  // namespace hr
+
+extern "C" {
+// Device memory the context may take beyond what it holds (bytes; negative: no limit).
+// An allocation past it fails as one on a full GPU does: the paths that follow a
+// failed allocation are tested with it.
+int hr_limit_memory(hr_ctx* ctx, double more);
+}

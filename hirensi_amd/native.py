@@ -39,6 +39,9 @@ NN_FUSED_EXPORTS = (
     "hr_nn_conv3d_fused", "hr_nn_transpose_layers", "hr_nn_avgpool2_grad_act", "hr_nn_upsample2_grad_act",
 )
 
+# hirensi_amd/csrc/hr_internal.h: the tests' limit of a context's device memory
+INTERNAL_EXPORTS = ("hr_limit_memory",)
+
 
 class MeshDesc(C.Structure):
     _fields_ = [
@@ -125,7 +128,8 @@ def load():
     L.hr_set_graph.argtypes = [_vp, C.c_int]
     L.hr_synchronize.argtypes = [_vp]
     L.hr_get_graph_launches.argtypes = [_vp, C.POINTER(C.c_longlong)]
-    for name in EXPORTS:
+    L.hr_limit_memory.argtypes = [_vp, C.c_double]
+    for name in EXPORTS + INTERNAL_EXPORTS:
         getattr(L, name).restype = getattr(L, name).restype or C.c_int
     _lib = L
     return L
