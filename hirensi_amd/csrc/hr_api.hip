@@ -25,6 +25,16 @@ using namespace hr;
 namespace {
 // element layers per z-chunk of the fused tile classes (sweep of 3..8 at 64x64x32: 7 first)
 constexpr int DEFAULT_TZ = 7;
+// and where only the central-difference step runs them (version 4): as many chunks as
+// DEFAULT_TZ gives, of equal length, since the longest one bounds a small box (16x16x8
+// elements, 4 + 4 layers 68 us a step, 7 + 1 78; 24x24x12, 6 + 6 94, 7 + 5 83; 32x32x16,
+// 6 + 6 + 4 90, 7 + 7 + 2 98; 64x64x32 210 either way); a box of more chunks than the
+// kernel takes has longer ones.  tz > 0: the caller's length, within that limit.
+int fused_tz(int nez, int tz) {
+  const int least = (nez + HR_MAX_ZCHUNKS - 1) / HR_MAX_ZCHUNKS;
+  const int chunks = (nez + DEFAULT_TZ - 1) / DEFAULT_TZ;
+  return std::max(tz > 0 ? tz : (nez + chunks - 1) / chunks, least);
+}
 constexpr int DEFAULT_TY = 3;
 constexpr int DEFAULT_VERSION = 4;   // 4 = split stage path, 3 = fused tile classes
 
@@ -798,10 +808,18 @@ StageArgs base_args(hr_ctx* ctx) {
   return A;
 }
 
+// whether the fused kernel takes z-chunks of tz element layers
+int check_chunks(hr_ctx* ctx, int tz) {
+  const int n = (ctx->g.nez + tz - 1) / tz;
+  if (n > HR_MAX_ZCHUNKS) return fail(ctx, 1, "too many z-chunks (%d); raise tz", n);
+  return 0;
+}
+
 // Tile grid and the three tile-class lists of the stage kernel.  A tile's
 // window is its elements plus the low-side halo element in x, y and z.
 int setup_tiles(hr_ctx* ctx) {
   Geo& g = ctx->g;
+  if (int rc = check_chunks(ctx, g.tz)) return rc;
   g.tiles[0] = (g.nex + g.tx - 1) / g.tx;
   g.tiles[1] = (g.ney + g.ty - 1) / g.ty;
   // z-chunks of tz element layers (the kernel reads the boundaries, so chunks could differ;
@@ -810,7 +828,6 @@ int setup_tiles(hr_ctx* ctx) {
   zb.assign(1, 0);
   for (int z = g.tz; z < g.nez; z += g.tz) zb.push_back(z);
   zb.push_back(g.nez);
-  if ((int)zb.size() - 1 > HR_MAX_ZCHUNKS) return fail(ctx, 1, "too many z-chunks (%d); raise tz", (int)zb.size() - 1);
   g.tiles[2] = (int)zb.size() - 1;
   std::vector<int> lists[3];
   const int nt = ntiles(g);
@@ -1116,7 +1133,6 @@ int hr_ctx_create(const hr_mesh_desc* d, hr_ctx** out) {
   g.top_rule = d->top_stress_bc ? 1 : 0;
   g.tx = 4;
   g.ty = DEFAULT_TY;
-  g.tz = DEFAULT_TZ;
   // affine element: DJ = diag(h/2); DETJ and DJI as in ELEMENT_K_3D
   const double j11 = d->h[0] * 0.5, j22 = d->h[1] * 0.5, j33 = d->h[2] * 0.5;
   const double detj = j11 * j22 * j33 + 0.0 * 0.0 * 0.0 + 0.0 * 0.0 * 0.0 - 0.0 * j22 * 0.0 - 0.0 * 0.0 * j11 - j33 * 0.0 * 0.0;
@@ -1160,6 +1176,7 @@ int hr_ctx_create(const hr_mesh_desc* d, hr_ctx** out) {
   } else {
     ctx->version = 3;
   }
+  g.tz = ctx->version == 4 ? fused_tz(g.nez, 0) : DEFAULT_TZ;
   if (int rc = setup_tiles(ctx)) return rc;
   if (int rc = upload_slots(ctx)) return rc;
   // coordinates (origin: centred in x, y; top surface at z = 0)
@@ -1429,13 +1446,16 @@ int hr_set_tiling(hr_ctx* ctx, int ty, int tz, int version) {
     return fail(ctx, 1, "bad tiling (stage kernel version 3 or 4)");
   if (version == 4 && !ctx->split_ok) return fail(ctx, 1, "lattice too large for the split stage path (version 4)");
   Geo& g = ctx->g;
-  ctx->concurrent = serial ? 0 : 1;
   const int t = ty ? ty : DEFAULT_TY;
   if (t != 3) return fail(ctx, 1, "stage kernel tiles are 4 x 3 elements");
-  if (version) ctx->version = version;
+  if (!version) version = ctx->version;
+  const int ftz = version == 4 ? fused_tz(g.nez, tz) : (tz ? tz : DEFAULT_TZ);
+  if (int rc = check_chunks(ctx, ftz)) return rc;
+  ctx->concurrent = serial ? 0 : 1;
+  ctx->version = version;
   g.tx = 4;
   g.ty = t;
-  g.tz = tz ? tz : DEFAULT_TZ;
+  g.tz = ftz;
   ctx->rd_tz = tz;
   if (int rc = ensure_split(ctx)) return rc;
   return setup_tiles(ctx);

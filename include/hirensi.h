@@ -258,7 +258,7 @@ int hr_revolve_schedule(int nseg, int nsnap, int max_actions, int* actions, int*
 
 /* Stage-kernel configuration: tile of 4 x ty elements in x-y (ty = 3), tz
  * elements per z-chunk (0: by the box and the shots for version 4, whose chunks start at
- * the regular domain's bottom layer; 7 for version 3), kernel version (0 keeps it): 4
+ * the regular domain's bottom layer; 7 for version 3, which takes at most 64 chunks), kernel version (0 keeps it): 4
  * (the default) splits RK4 stages and operator products into nodal passes and
  * pulls over the PML nodes and an element pass over the regular domain; 3 runs the fused
  * tile classes (mixed, regular-domain, PML).  The central-difference step always

@@ -102,3 +102,32 @@ def test_products_at_tile_and_chunk_edges(shape, npml, tz, which):
         S.ShellMat(ctx, S.HR_K)._apply(tr, 3.0 * x, y, None)
         z = S.ShellMat(ctx, which)._apply(tr, x, y, None)
         assert rel_l2(z - y, so.matmult_add(which, x, np.zeros(mesh.neq), tr)) < 1e-12
+
+
+@pytest.mark.parametrize("nez,tz", [(449, 0), (500, 0), (470, 1)])
+def test_tall_boxes(nez, tz):
+    """More element layers than 64 chunks of the fused kernel's default length (or of the
+    caller's) hold: the RK4 stages and the central-difference step against the oracle.
+    Version 3, which runs those chunks for every stage, refuses and changes nothing."""
+    mesh = BoxMesh(3, 4, nez, npml=(1,) * 5)
+    model = random_model(mesh, seed=nez)
+    top, nstep, dt, fr = mesh.NZ - 1, 6, 1.0e-4, 400.0
+    src = np.array([mesh.dof(mesh.node_index(3, 4, top), 2), mesh.dof(mesh.node_index(3, 3, top - 440), 0)], dtype=np.int64)
+    rec = receiver_dofs(mesh, [mesh.node_index(3, 4, top - q) for q in (0, 1, 439, 440)])
+    print(f"tall box nez={nez} tz={tz} neq={mesh.neq}", flush=True)
+    B = np.zeros(mesh.neq)
+    B[src] = (1.0, 0.5)
+    row = {int(e): r for r, e in enumerate(mesh.store_eq)}
+    rows = np.array([row[int(e)] for e in rec])
+    so, ctx = O.System(mesh, model), S.Context(mesh, model, tz=tz)
+    assert ctx.version() == 4
+    tab = S.time_table(nstep, dt, 2, fr)
+    ref = so.forward(B, nstep, dt, lcase=2, fr=fr)[:, rows]
+    assert np.abs(ref).max() > 0
+    before = ctx.tiling()
+    with pytest.raises(S.HrError, match="z-chunks"):
+        ctx._check(ctx.L.hr_set_tiling(ctx.h, 0, 7, 3))
+    assert ctx.tiling() == before
+    assert rel_l2(S.explicit_rk4_petsc_pml_3d(ctx, nstep, dt, tab, src, B[src], rec), ref) < 1e-10
+    cd = so.cd_forward(B, nstep, dt, lcase=2, fr=fr)[:, rows]
+    assert rel_l2(S.explicit_central_difference_3(ctx, nstep, dt, src, B[src], rec, 2, fr), cd) < 1e-10
