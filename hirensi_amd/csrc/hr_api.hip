@@ -13,6 +13,7 @@
 #include <unordered_map>
 #include "hr_device.h"
 #include "hr_revolve.h"
+#include "hr_index.h"
 #include "hr_internal.h"
 #include "hr_split.h"
 #include "../../include/hirensi.h"
@@ -65,7 +66,7 @@ struct hr_ctx {
   double hel[3] = {1.0, 1.0, 1.0};          // element edges
   long long neq = 0;
   std::vector<long long> eq_slot;          // host copy of the numbering
-  unsigned* d_eq_slot = nullptr;            // 32 bits: lattices past them are refused at creation or by the kernels
+  unsigned* d_eq_slot = nullptr;            // 32 bits: LATTICE_NODES is checked at creation
   // regular-domain node box
   int box0[3] = {0, 0, 0}, boxn[3] = {0, 0, 0};
   long long nbox = 0;
@@ -1127,6 +1128,8 @@ int hr_ctx_create(const hr_mesh_desc* d, hr_ctx** out) {
   g.nex = d->nex; g.ney = d->ney; g.nez = d->nez;
   g.NX = 2 * g.nex + 1; g.NY = 2 * g.ney + 1; g.NZ = 2 * g.nez + 1;
   g.NN = (long long)g.NX * g.NY * g.NZ;
+  // more than the GPU holds: eleven vectors of 9 NN doubles alone are 378 GB there
+  if (g.NN > LATTICE_NODES) return fail(ctx, 1, "lattice of %lld nodes is too large (at most %lld)", g.NN, LATTICE_NODES);
   g.rlo[0] = d->npml[0]; g.rhi[0] = g.nex - d->npml[1];
   g.rlo[1] = d->npml[2]; g.rhi[1] = g.ney - d->npml[3];
   g.rlo[2] = d->npml[4]; g.rhi[2] = g.nez;

@@ -68,7 +68,7 @@ __device__ __forceinline__ void gradient_block(const GradArgs& A, int blk, GradL
   const int li = (blk & 7) * C + (blk >> 3);
   if (li >= ntot) return;
   const int shot = li / ntile, t = li - shot * ntile;
-  const int nbox = bnx * bny * bnz;              // 32-bit: 9 NN < 2^31 (checked by the host)
+  const int nbox = bnx * bny * bnz;              // and its byte offsets fit 32 bits (LATTICE_NODES)
   if (A.step) uh += (long long)(*A.step) * A.stride;
   uh += shot * A.ustride;
   p2 += shot * A.pstride;
@@ -82,16 +82,15 @@ __device__ __forceinline__ void gradient_block(const GradArgs& A, int blk, GradL
   // meets zero coefficients only
   const double *const u0p = uh, *const u1p = uh + nbox, *const u2p = uh + 2 * nbox;
   auto fetch = [&](unsigned r0, unsigned n0, int k, double* u, double* p) {
-    const unsigned kk = (unsigned)min(max(k, 0), bnz - 1);
-    const unsigned r = (r0 + (unsigned)(bnx * bny) * kk) * 8u;
-    const unsigned n = (n0 + (unsigned)(A.NX * A.NY) * kk) * 24u;
+    const int kk = min(max(k, 0), bnz - 1);
+    const unsigned r = (r0 + (unsigned)(bnx * bny) * (unsigned)kk) * 8u;
     u[0] = ldo(u0p, r);
     u[1] = ldo(u1p, r);
     u[2] = ldo(u2p, r);
-    ld3(p2, n, p[0], p[1], p[2]);
+    ld3(p2 + plane_doubles(A.NX, A.NY, bk0 + kk), n0, p[0], p[1], p[2]);
   };
   const int ci = min(bi, bnx - 1), cj = min(bj, bny - 1);
-  const unsigned r0 = (unsigned)(ci + bnx * cj), n0 = (unsigned)((bi0 + ci) + A.NX * ((bj0 + cj) + A.NY * bk0));
+  const unsigned r0 = (unsigned)(ci + bnx * cj), n0 = in_plane_bytes(A.NX, bi0 + ci, bj0 + cj);
   const int wo = (GH + tx) + GWX * (GH + ty);
   // halo position of this thread
   int hx = 0, hy = 0;
@@ -99,7 +98,7 @@ __device__ __forceinline__ void gradient_block(const GradArgs& A, int blk, GradL
   else if (tid < GHALO) { const int q = tid - 4 * GTX; hy = GH + (q >> 2); hx = q & 3; if (hx >= 2) hx += GTX; }
   const bool halo = tid < GHALO;
   const int hi = min(max(ti0 + hx - GH, 0), bnx - 1), hj = min(max(tj0 + hy - GH, 0), bny - 1);
-  const unsigned hr0 = (unsigned)(hi + bnx * hj), hn0 = (unsigned)((bi0 + hi) + A.NX * ((bj0 + hj) + A.NY * bk0));
+  const unsigned hr0 = (unsigned)(hi + bnx * hj), hn0 = in_plane_bytes(A.NX, bi0 + hi, bj0 + hj);
   const int hw = hx + GWX * hy;
   // x and y sides.  Side 0 is the element below (even node, its local point 2) or
   // the one element of an odd node (local point 1), side 1 the element above (local

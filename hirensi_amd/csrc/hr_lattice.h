@@ -4,6 +4,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include "hr_device.h"
+#include "hr_index.h"
 
 namespace hr {
 namespace {
@@ -125,14 +126,13 @@ __device__ __forceinline__ void output_block(const OutArgs& O, int blk, int shot
     if (r < O.nrec) row[r] = x2[O.slot[r]];
     return;
   }
-  const int r = (blk - nrb) * OUT_NT + (int)threadIdx.x;     // 32-bit: 9 NN < 2^31 (checked by the host)
+  const int r = (blk - nrb) * OUT_NT + (int)threadIdx.x;
   if (r >= O.nbox) return;
   double* hist = O.hist + shot * O.hstride;
   if (O.step) hist += (long long)(*O.step) * 3 * O.nbox;
   const int bi = r % O.bn[0], bj = (r / O.bn[0]) % O.bn[1], bk = r / (O.bn[0] * O.bn[1]);
-  const int n = (O.b0[0] + bi) + O.NX * ((O.b0[1] + bj) + O.NY * (O.b0[2] + bk));
   double u0, u1, u2;
-  ld3(x2, (unsigned)n * 24u, u0, u1, u2);
+  ld3(x2 + plane_doubles(O.NX, O.NY, O.b0[2] + bk), in_plane_bytes(O.NX, O.b0[0] + bi, O.b0[1] + bj), u0, u1, u2);
   hist[r] = u0;
   hist[O.nbox + r] = u1;
   hist[2 * (long long)O.nbox + r] = u2;
