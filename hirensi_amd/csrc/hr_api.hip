@@ -170,10 +170,10 @@ struct hr_ctx {
   // block and at regular-domain-only nodes
   bool split_ok = false;                      // the lattice fits the split path
   int pnblk = 0;                              // SPLIT_OWN-node blocks of the PML nodes
-  double* d_D = nullptr;                      // flux records: 12 NN doubles per shot, of odd stages, then of even ones
-  bool split_two = false;                     // there is room for both (else one, and a launch per pass)
+  double* d_D[2] = {nullptr, nullptr};        // flux records of odd and of even stages, 12 NN doubles per shot each;
+                                              // the second only where there is room (else a launch per pass)
   SplitArgs split_prev{};                     // the stage whose pull is still to come
-  double* d_E = nullptr;                      // two fields: 3 NN doubles per shot each
+  double* d_E = nullptr;                      // two fields: 3 sp_iface_count doubles per shot each
   int split_shots = 0;
   double mem_limit = -1.0;                    // device bytes the context may hold (negative: no limit)
   int rd_tz = 0;                              // layers per z-chunk of the element pass (0: rd_chunk's rule)
@@ -248,13 +248,29 @@ double held_bytes(const hr_ctx* ctx) {
   return b;
 }
 
+template <class T>
+void dfree(hr_ctx* ctx, T** p) {
+  if (*p) (void)hipFree(*p);
+  *p = nullptr;
+  ctx->caps.erase((void*)p);
+}
+
 // hipMalloc within the context's limit (hr_limit_memory).  A failure leaves no
-// error behind for the next launch's check to find.
+// error behind for the next launch's check to find.  Where there is no room the second
+// set of flux records is given back: it saves time only, so it must not keep a batch
+// or a stored history from fitting.  (No buffer is allocated between the stages of a
+// step or into a captured loop, which both hold the sets' addresses.)
 hipError_t device_malloc(hr_ctx* ctx, void** p, size_t bytes) {
-  hipError_t e = hipErrorOutOfMemory;
-  if (ctx->mem_limit < 0.0 || held_bytes(ctx) + (double)bytes <= ctx->mem_limit) {
-    e = hipMalloc(p, bytes);
+  auto take = [&]() {
+    if (ctx->mem_limit >= 0.0 && held_bytes(ctx) + (double)bytes > ctx->mem_limit) return hipErrorOutOfMemory;
+    const hipError_t e = hipMalloc(p, bytes);
     if (e != hipSuccess) (void)hipGetLastError();
+    return e;
+  };
+  hipError_t e = take();
+  if (e != hipSuccess && ctx->d_D[1]) {
+    dfree(ctx, &ctx->d_D[1]);
+    e = take();
   }
   if (e != hipSuccess) *p = nullptr;
   return e;
@@ -275,13 +291,6 @@ int dalloc(hr_ctx* ctx, T** p, size_t n) {
     return fail(ctx, (int)e, "hipMalloc of %zu bytes failed: %s", n * sizeof(T), hipGetErrorString(e));
   ctx->caps[(void*)p] = n * sizeof(T);
   return 0;
-}
-
-template <class T>
-void dfree(hr_ctx* ctx, T** p) {
-  if (*p) (void)hipFree(*p);
-  *p = nullptr;
-  ctx->caps.erase((void*)p);
 }
 
 // host <-> device copies honouring HR_DEVICE_PTRS
@@ -336,6 +345,8 @@ int tile_of(const hr_ctx* ctx, int i, int j, int k) {
   while (tz + 1 < g.tiles[2] && k >= 2 * ctx->zb[tz + 1]) ++tz;
   return tx + g.tiles[0] * (ty + g.tiles[1] * tz);
 }
+
+int iface_count(const hr_ctx* ctx) { return (int)sp_iface_count(ctx->boxn[0], ctx->boxn[1], ctx->boxn[2]); }
 
 int ntiles(const Geo& g) { return g.tiles[0] * g.tiles[1] * g.tiles[2]; }
 
@@ -655,6 +666,7 @@ int launch_stage(hr_ctx* ctx, StageArgs& A, const Src3Spec* sp = nullptr) {
       B.shot_stride = (long long)field_size(ctx);
       if (ctx->split_shots < (A.stage > 0 ? B.nshot : 1) || !ctx->split_ok)
         return fail(ctx, 3, "split stage path without its buffers for %d shots", B.nshot);
+      B.nif = iface_count(ctx);
       if (A.stage == 0) {
         // an operator product: one shot, the sums of its single input
         RdArgs R;
@@ -665,7 +677,7 @@ int launch_stage(hr_ctx* ctx, StageArgs& A, const Src3Spec* sp = nullptr) {
         B.node = ctx->d_node; B.tab = ctx->d_tab; B.minvu = ctx->d_minvu; B.rwp = ctx->d_rwp;
         B.sc = 1.0;
         B.pnbn = ctx->pnblk;
-        B.D = ctx->d_D;
+        B.D = ctx->d_D[0];
         const int set = A.set_mask == 1 ? 0 : (A.set_mask == 2 ? 1 : 2);
         if (set == 1) B.E = ctx->d_E;
         R.g = B.g;
@@ -676,6 +688,7 @@ int launch_stage(hr_ctx* ctx, StageArgs& A, const Src3Spec* sp = nullptr) {
         R.in[0] = A.in[0];
         R.out[0] = A.out;
         R.E[0] = ctx->d_E;
+        R.nif = B.nif;
         R.node = ctx->d_node;
         R.nshot = 1;
         if (int rc = run_deferred(ctx)) return rc;
@@ -692,7 +705,8 @@ int launch_stage(hr_ctx* ctx, StageArgs& A, const Src3Spec* sp = nullptr) {
       B.xn[0] = A.xnew[0]; B.xn[1] = A.xnew[1];
       // node-local terms: in place, but for stage 1, whose a1 other blocks still need them
       // for when it is written; they go to the vector that the update writes last
-      B.a = A.stage == 3 && ctx->split_two ? nullptr : (last ? A.xnew[2] : A.out);
+      const bool two = ctx->d_D[1] != nullptr;
+      B.a = A.stage == 3 && two ? nullptr : (last ? A.xnew[2] : A.out);
       B.out = A.stage == 1 ? ctx->y[0] : (last ? A.xnew[2] : A.out);
       B.node = ctx->d_node; B.tab = ctx->d_tab; B.minvu = ctx->d_minvu; B.rwp = ctx->d_rwp;
       set_source(ctx, sp, B);
@@ -700,9 +714,9 @@ int launch_stage(hr_ctx* ctx, StageArgs& A, const Src3Spec* sp = nullptr) {
       B.sc = last ? A.h4 : 1.0;
       B.pnbn = ctx->pnblk;
       // the flux records of odd and even stages alternate
-      B.D = ctx->d_D + (elements || !ctx->split_two ? 0 : 12 * (size_t)ctx->g.NN * ctx->split_shots);
+      B.D = ctx->d_D[elements || !two ? 0 : 1];
       // the element pass before stages 1 and 3 forms the interface sums of two stages
-      const size_t ne = 3 * (size_t)ctx->g.NN * ctx->split_shots;
+      const size_t ne = 3 * (size_t)B.nif * ctx->split_shots;
       double* const E[2] = {ctx->d_E, ctx->d_E + ne};
       B.E = E[(A.stage - 1) & 1];
       RdArgs R;
@@ -721,6 +735,7 @@ int launch_stage(hr_ctx* ctx, StageArgs& A, const Src3Spec* sp = nullptr) {
         R.out[0] = update ? ctx->y[1] : ctx->gs[0];
         R.out[1] = update ? ctx->y[2] : ctx->gs[1];
         R.E[0] = E[0]; R.E[1] = E[1];
+        R.nif = B.nif;
         R.node = ctx->d_node; R.minvu = ctx->d_minvu;
         R.nshot = B.nshot; R.shot_stride = B.shot_stride;
         R.h = A.h; R.h2 = A.hh; R.h3 = A.h6; R.h4 = A.h4;
@@ -761,7 +776,7 @@ int launch_stage(hr_ctx* ctx, StageArgs& A, const Src3Spec* sp = nullptr) {
         if (int rc = run_deferred(ctx)) return rc;
         if (prof) HIPC(hipEventRecord(ev.start[0], ctx->stream));
         if (elements) HIPC(launch_stage_pair(B, R, O, G, upd, A.transpose, ctx->stream));
-        else if (ctx->split_two) HIPC(launch_pull_nodal(ctx->split_prev, B, last, A.transpose, ctx->stream));
+        else if (two) HIPC(launch_pull_nodal(ctx->split_prev, B, last, A.transpose, ctx->stream));
         else {
           HIPC(launch_split_pull(ctx->split_prev, A.transpose, ctx->stream));
           HIPC(launch_split_nodal(B, last, A.transpose, ctx->stream));
@@ -872,15 +887,13 @@ int check_ready(hr_ctx* ctx) {
 // stay zero (the pull reads them)
 int ensure_split(hr_ctx* ctx) {
   if (ctx->version != 4 || ctx->split_shots >= ctx->nshot) return 0;
-  const size_t nd = 12 * (size_t)ctx->g.NN * ctx->nshot, ne = 6 * (size_t)ctx->g.NN * ctx->nshot;
+  const size_t nd = 12 * (size_t)ctx->g.NN * ctx->nshot, ne = 6 * (size_t)iface_count(ctx) * ctx->nshot;
   ctx->split_shots = 0;                  // a failure below leaves the buffers incomplete
   if (int rc = dalloc(ctx, &ctx->d_E, ne)) return rc;
-  ctx->split_two = dalloc(ctx, &ctx->d_D, 2 * nd) == 0;
-  if (!ctx->split_two) {
-    ctx->err.clear();
-    if (int rc = dalloc(ctx, &ctx->d_D, nd)) return rc;
-  }
-  HIPC(hipMemsetAsync(ctx->d_D, 0, (ctx->split_two ? 2 : 1) * nd * sizeof(double), ctx->stream));
+  if (int rc = dalloc(ctx, &ctx->d_D[0], nd)) return rc;
+  if (dalloc(ctx, &ctx->d_D[1], nd) != 0) ctx->err.clear();
+  for (double* D : ctx->d_D)
+    if (D) HIPC(hipMemsetAsync(D, 0, nd * sizeof(double), ctx->stream));
   ctx->split_shots = ctx->nshot;
   return 0;
 }
@@ -1230,7 +1243,7 @@ int hr_ctx_destroy(hr_ctx* ctx) {
   F(ctx->d_obs_sorted);
   F(ctx->d_img); F(ctx->d_restr); F(ctx->d_reg); F(ctx->d_red); F(ctx->d_pm); F(ctx->d_pg);
   for (int c = 0; c < 3; ++c) F(ctx->d_tl[c]);
-  F(ctx->d_D); F(ctx->d_E);
+  F(ctx->d_D[0]); F(ctx->d_D[1]); F(ctx->d_E);
   for (hr_ctx::PullLists* pl : {&ctx->pl_src, &ctx->pl_rec}) {
     F(pl->ptr); F(pl->idx); F(pl->slot); F(pl->rd_idx); F(pl->rd_shot);
   }
@@ -1552,7 +1565,8 @@ int plan_history(hr_ctx* ctx, int history, int segment, int nstep, int nshot) {
     HIPC(hipMemGetInfo(&fr, &tot));
     double held = 0.0;
     for (auto& kv : ctx->caps)
-      if (kv.first == (void*)&ctx->d_hist || kv.first == (void*)&ctx->d_seg) held += (double)kv.second;
+      if (kv.first == (void*)&ctx->d_hist || kv.first == (void*)&ctx->d_seg || kv.first == (void*)&ctx->d_D[1])
+        held += (double)kv.second;       // the second set of flux records is given back where there is no room
     held += (double)ctx->snap.size() * (double)ctx->snap_elems * sizeof(double);
     budget = 0.5 * ((double)fr + held);
   }

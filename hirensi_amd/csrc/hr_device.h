@@ -217,7 +217,8 @@ struct SplitArgs {
   double sc;                       // scale of the stage's a in its output: 1, last stage h^4/24
   int pnbn;                        // blocks of the PML node list (SPLIT_OWN nodes each)
   double* D;                       // y- and z-line flux records, 12 NN doubles per shot
-  const double* E;                 // regular-domain K sums of interface nodes, 3 NN doubles per shot
+  const double* E;                 // regular-domain K sums of the interface nodes (sp_iface_column), 3 nif doubles per shot
+  int nif;                         // interface nodes
 };
 
 // and its regular-domain element pass over two fields
@@ -227,7 +228,8 @@ struct RdArgs {
   const double* in[2];             // x2, x3 (update: a1, a2)
   const double* x[2];              // update: x2, x3
   double* out[2];                  // a1, a2 (update: new x2, x3)
-  double* E[2];                    // K sums of interface nodes per field
+  double* E[2];                    // K sums of the interface nodes per field (sp_iface_column)
+  int nif;                         // interface nodes
   const double *node, *minvu;
   int nshot;
   long long shot_stride;

@@ -137,6 +137,22 @@ constexpr unsigned sp_pml_pos(int i, int j, int k, int NX, int NY, const int lo[
   return base + R0 + ay * W + (unsigned)(j - 2 * hi[1]) * nx + (unsigned)i;
 }
 
+// Places of the interface nodes (nodes of the regular-domain box that PML elements hold
+// too), (bi, bj, bk) within the box of bnx x bny x bnz nodes: of each plane the rim,
+// its two rows in x before the rows' end nodes, then the bottom plane's inner
+// nodes.  The place is the column's plus bk rims, as an inner column has a node in plane
+// 0 only.
+constexpr unsigned sp_rim(int bnx, int bny) { return 2u * (unsigned)(bnx + bny - 2); }
+constexpr unsigned sp_iface_count(int bnx, int bny, int bnz) {
+  return (unsigned)bnz * sp_rim(bnx, bny) + (unsigned)((bnx - 2) * (bny - 2));
+}
+constexpr unsigned sp_iface_column(int bi, int bj, int bnx, int bny, int bnz) {
+  if (bj == 0) return (unsigned)bi;
+  if (bj == bny - 1) return (unsigned)(bnx + bi);
+  if (bi == 0 || bi == bnx - 1) return (unsigned)(2 * (bnx + bj - 1) + (bi == 0 ? 0 : 1));
+  return (unsigned)bnz * sp_rim(bnx, bny) + (unsigned)((bi - 1) + (bnx - 2) * (bj - 1));
+}
+
 // number of PML nodes
 constexpr unsigned sp_pml_count(int NX, int NY, int NZ, const int lo[3], const int hi[2]) {
   const unsigned nxy = (unsigned)NX * (unsigned)NY;

@@ -79,6 +79,15 @@ __device__ __forceinline__ Entry list_entry(const Geo3& g, int lb) {
   return E;
 }
 
+// place of a column's interface nodes in the regular-domain sums, and the step per plane
+__device__ __forceinline__ unsigned iface_column(const Geo3& g, int i, int j) {
+  return sp_iface_column(i - 2 * g.rlo[0], j - 2 * g.rlo[1], 2 * (g.rhi[0] - g.rlo[0]) + 1, 2 * (g.rhi[1] - g.rlo[1]) + 1,
+                         g.NZ - 2 * g.rlo[2]);
+}
+__device__ __forceinline__ unsigned iface_rim(const Geo3& g) {
+  return sp_rim(2 * (g.rhi[0] - g.rlo[0]) + 1, 2 * (g.rhi[1] - g.rlo[1]) + 1);
+}
+
 struct NodalLds {
   double xr[6][SPLIT_NT];         // x flux records of the block's entries
   unsigned xn[SPLIT_NT];          // their lattice nodes (~0: no entry)
@@ -396,12 +405,14 @@ __device__ __forceinline__ void pull_pass(const SplitArgs& A, const Entry& E, in
   if constexpr (TR) ld2(A.node, n * 16u, lam, mu);
   // interface sums, read with the first batch where a regular-domain element
   // holds the node; other lanes read the shot's first entry (one shared line)
-  // and drop it
+  // and drop it (a list of the interface nodes: as two lattice fields the sums took 6
+  // NN doubles a shot, and the pass is as fast)
   const SpAxis ax3[3] = {sp_axis(i, g.nex, g.rlo[0], g.rhi[0]), sp_axis(j, g.ney, g.rlo[1], g.rhi[1]),
                          sp_axis(k, g.nez, g.rlo[2], g.nez)};
   const bool iface = sp_iface(ax3[0], ax3[1], ax3[2]);
   double e3[3] = {0.0, 0.0, 0.0};
-  if (!RAW || A.E) ld3(A.E + (long long)shot * 3 * g.NN, iface ? offu : 0u, e3[0], e3[1], e3[2]);
+  const unsigned eo = (iface ? 24u : 0u) * (iface_column(g, i, j) + iface_rim(g) * (unsigned)(k - 2 * g.rlo[2]));   // (a select costs two registers, and a wave per SIMD)
+  if (!RAW || A.E) ld3(A.E + (long long)shot * 3 * A.nif, eo, e3[0], e3[1], e3[2]);
   const int sdyn = (e1 > e0 && A.step_dev) ? *A.step_dev : 0;
   if (e1 > e0) {
     if (jj >= 0) {
@@ -672,6 +683,7 @@ __device__ __forceinline__ void element_pass(const RdArgs& A, int blk, RdLds<NF>
   const bool owned = P < 3 && (ix < 2 * RT || tx == A.ntx - 1) && (iy < 2 * RT || ty == A.nty - 1) && i <= 2 * g.rhi[0] &&
                      j <= 2 * g.rhi[1];
   const int opos = (ix + 2) + RW * (iy + 2);
+  const unsigned ecol = 24u * iface_column(g, i, j), rim = iface_rim(g);
   // the node's places in the forces of the up to four elements of a layer that hold it:
   // an odd coordinate has one element (local point 1), an even one the element below
   // (local point 2) and the one above (local point 0)
@@ -841,9 +853,10 @@ __device__ __forceinline__ void element_pass(const RdArgs& A, int blk, RdLds<NF>
     }
     if (fin) {
       if (ifc) {
-        const long long eo = (long long)shot * 3 * g.NN;
+        const long long eo = (long long)shot * 3 * A.nif;
+        const unsigned o = ecol + 24u * rim * (unsigned)(k - 2 * g.rlo[2]);
 #pragma unroll
-        for (int f = 0; f < NF; ++f) st3(A.E[f] + eo, n * 24u, acc[f][0], acc[f][1], acc[f][2]);
+        for (int f = 0; f < NF; ++f) st3(A.E[f] + eo, o, acc[f][0], acc[f][1], acc[f][2]);
       } else if constexpr (NF == 1) {
         st3(A.out[0] + so, n * 24u, acc[0][0], acc[0][1], acc[0][2]);
       } else {

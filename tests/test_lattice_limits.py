@@ -1,6 +1,6 @@
-"""Lattices near and past the limits of 32-bit addresses: the displacement
-addresses of the kernels on state vectors, on the host, and the refusal at
-creation (before anything is allocated, so no GPU is needed)."""
+"""Addresses and sizes on the host: the displacement addresses of lattices past 32
+bits, the places of the interface nodes, and the refusal of a lattice that is too
+large at creation (before anything is allocated, so no GPU is needed)."""
 import ctypes as C
 import os
 import shutil
@@ -15,10 +15,11 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 
 
 @pytest.mark.skipif(shutil.which("g++") is None, reason="g++ absent")
-def test_displacement_addresses_of_large_lattices():
+@pytest.mark.parametrize("check", ["index_check", "iface_check"])
+def test_addresses(check):
     with tempfile.TemporaryDirectory() as tmp:
         exe = os.path.join(tmp, "ic")
-        subprocess.run(["g++", "-O1", "-std=c++17", os.path.join(HERE, "native", "index_check.cpp"), "-o", exe], check=True)
+        subprocess.run(["g++", "-O1", "-std=c++17", os.path.join(HERE, "native", check + ".cpp"), "-o", exe], check=True)
         r = subprocess.run([exe], capture_output=True, text=True)
     print(r.stdout)
     assert r.returncode == 0, r.stdout
