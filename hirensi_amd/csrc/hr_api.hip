@@ -176,7 +176,8 @@ struct hr_ctx {
   double* d_E = nullptr;                      // two fields: 3 sp_iface_count doubles per shot each
   int split_shots = 0;
   double mem_limit = -1.0;                    // device bytes the context may hold (negative: no limit)
-  int rd_tz = 0;                              // layers per z-chunk of the element pass (0: rd_chunk's rule)
+  int rd_tz = 0;                              // layers per z-chunk of the element pass (0: rd_chunk's rule),
+  int rd_tuned = 0, rd_tuned_shots = 0;       // and of the stages of a batch of the shots that hr_autotune timed
   struct PullLists {
     int *ptr = nullptr, *idx = nullptr, *slot = nullptr, *rd_idx = nullptr, *rd_shot = nullptr;
   } pl_src, pl_rec;
@@ -571,8 +572,10 @@ Stage3Args args3(hr_ctx* ctx, const StageArgs& A, const Src3Spec* sp) {
 // up its chunk and computes one halo layer below it; 512 blocks (two per CU; three
 // of the pass over one field) run at a time.  The chunk is the one with the fewest layers in sequence, rounds of
 // blocks times layers per block; of equals the longest, which repeats the
-// fewest halo layers.
+// fewest halo layers.  A length that hr_autotune found holds for what it timed: the
+// stages of a batch of as many shots.
 int rd_chunk(const hr_ctx* ctx, int nshot, int fields = 2) {
+  if (fields == 2 && ctx->rd_tuned > 0 && nshot == ctx->rd_tuned_shots) return ctx->rd_tuned;
   if (ctx->rd_tz > 0) return ctx->rd_tz;
   const int layers = ctx->g.nez - ctx->g.rlo[2];
   const int slots = fields == 2 ? 512 : 768;
@@ -1473,6 +1476,7 @@ int hr_set_tiling(hr_ctx* ctx, int ty, int tz, int version) {
   g.ty = t;
   g.tz = ftz;
   ctx->rd_tz = tz;
+  ctx->rd_tuned = 0;
   if (int rc = ensure_split(ctx)) return rc;
   return setup_tiles(ctx);
 }
@@ -2203,16 +2207,28 @@ int hr_autotune(hr_ctx* ctx, int nshot, int steps, int* tz_best, double* ms_per_
   hipEvent_t e0 = nullptr, e1 = nullptr;
   HIPC(hipEventCreate(&e0));
   HIPC(hipEventCreate(&e1));
-  const int tz0 = ctx->g.tz, rd0 = ctx->rd_tz;
+  const bool split = ctx->version == 4;
+  const int tz0 = ctx->g.tz, rd0 = ctx->rd_tz, rt0 = ctx->rd_tuned, rs0 = ctx->rd_tuned_shots;
   const double sgn[3] = {1.0, 1.0, 1.0};
   double best = -1.0;
-  int bt = tz0;
+  int bt = 0;
   int status = 0;
-  // z-chunk candidates: element layers per chunk of the stage-kernel tiles
-  for (int tz : {1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 16, 18, 20, 26, 32, 40}) {
-    if (tz > ctx->g.nez) continue;
-    ctx->g.tz = ctx->rd_tz = tz;
-    if (setup_tiles(ctx) != 0) continue;      // too many chunks for this mesh
+  // z-chunk candidates: element layers per chunk of the fused tiles (version 3), or of the
+  // element pass; there the length of rd_chunk's rule (0) comes last, when the clocks are
+  // up, and stays unless another one is faster by more than two timings of one differ
+  const int most = split ? ctx->g.nez - ctx->g.rlo[2] : ctx->g.nez;
+  if (split) {
+    ctx->rd_tz = ctx->rd_tuned = 0;
+    ctx->rd_tuned_shots = nshot;
+  }
+  const int rule = split ? rd_chunk(ctx, nshot) : 0;
+  for (int tz : {1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 16, 18, 20, 26, 32, 40, 0}) {
+    if (tz > most || (split ? tz == rule : tz == 0)) continue;
+    if (split) ctx->rd_tuned = tz;
+    else {
+      ctx->g.tz = tz;
+      if (setup_tiles(ctx) != 0) continue;    // too many chunks for this mesh
+    }
     // timed RK4 steps on the zero state without sources: the same launches and traffic
     if ((status = zero_state(ctx))) break;
     if ((status = rk4_step(ctx, 1.0e-4, +1, 0, sgn, nullptr))) break;
@@ -2226,12 +2242,18 @@ int hr_autotune(hr_ctx* ctx, int nshot, int steps, int* tz_best, double* ms_per_
       break;
     }
     const double per = (double)ms / steps;
-    if (best < 0.0 || per < best) { best = per; bt = tz; }
+    if (best < 0.0 || per < (tz ? 1.0 : 1.01) * best) { best = per; bt = tz; }
   }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
-  ctx->g.tz = status ? tz0 : bt;
-  ctx->rd_tz = status ? rd0 : bt;
+  if (status || best < 0.0) {
+    ctx->g.tz = tz0; ctx->rd_tz = rd0; ctx->rd_tuned = rt0; ctx->rd_tuned_shots = rs0;
+    if (!status) bt = tz0;
+  } else if (split) {
+    ctx->rd_tuned = bt;
+    bt = rd_chunk(ctx, nshot);
+  } else
+    ctx->g.tz = bt;
   if (int rc = setup_tiles(ctx)) return rc;
   if (int rc = zero_state(ctx)) return rc;
   if (status) return status;

@@ -57,3 +57,33 @@ def test_batched_shots_match_single_shots(history, segment):
     assert rel_l2(glb, gl1) < 1e-13 and rel_l2(gmb, gm1) < 1e-13
     assert abs(jb - j1) <= 1e-13 * abs(j1)
     assert abs(S.compute_misfit(cb, nstep, dt, dobs) - j1) <= 1e-13 * abs(j1)
+
+
+def test_a_tuned_chunk_holds_for_the_shots_it_was_timed_with():
+    """hr_autotune times the element pass for a batch of one size: solves of another
+    size and operator products keep the rule's chunk, and a length that the caller set
+    is replaced."""
+    mesh = BoxMesh(20, 12, 12, npml=(2,) * 5)
+    model = random_model(mesh, seed=3)
+    src = np.array([mesh.dof(mesh.surface_node(0.0, 0.0), 2)], dtype=np.int64)
+    dt = 1.0e-4
+
+    def chunk(ctx, nshot):
+        ftab = np.stack([S.time_table(2, dt, 2, 60.0)] * nshot)
+        S.explicit_rk4_petsc_pml_3d_shots(ctx, 2, dt, ftab, np.zeros(1, np.int32), src, np.ones(1), src,
+                                          history=S.HR_HISTORY_NONE, nshot=nshot)
+        return ctx.tiling()[1]
+
+    sizes = (1, 2, 12, 40)
+    plain = S.Context(mesh, model)
+    rule = {n: chunk(plain, n) for n in sizes}
+    print(f"rule's chunks {rule}", flush=True)
+    assert len(set(rule.values())) > 1
+    for set_tz in (0, 5):
+        ctx = S.Context(mesh, model, tz=set_tz)
+        if set_tz:
+            assert chunk(ctx, 2) == set_tz
+        tz, ms = ctx.autotune(nshot=12, steps=2)
+        assert ms > 0 and 1 <= tz <= 10
+        got = {n: chunk(ctx, n) for n in sizes}
+        assert got == {**rule, 12: tz}, (got, tz)
