@@ -13,6 +13,7 @@
 #include <unordered_map>
 #include "hr_device.h"
 #include "hr_revolve.h"
+#include "hr_due.h"
 #include "hr_index.h"
 #include "hr_internal.h"
 #include "hr_split.h"
@@ -58,6 +59,16 @@ struct Shell {
 };
 
 }  // namespace
+
+// a step's trace row and history slice (the base of the first shot's, elements per shot)
+struct TraceRow {
+  double* row = nullptr;
+  long long rstride = 0;
+};
+struct Slice {
+  double* hist = nullptr;
+  long long hstride = 0;
+};
 
 struct hr_ctx {
   std::string err;
@@ -163,8 +174,9 @@ struct hr_ctx {
   // traces and slices as blocks of the launch and the rest before it, or all
   // on the second side stream).  The next launch_stage consumes it.
   std::vector<std::function<int()>> deferred;
-  OutArgs out{};                              // traces and history slice due with the next launch
-  GradArgs grad{};                            // and the adjoint step's gradient
+  Due<TraceRow> due_row;                      // traces and history slice due with the next launch
+  Due<Slice> due_slice;
+  Due<GradArgs> due_grad;                     // and the adjoint step's gradient
   // split stage path (version 4): the flux records and interface sums of
   // split_shots shots (0: none, after an allocation that failed), source entries by pull
   // block and at regular-domain-only nodes
@@ -591,12 +603,11 @@ int rd_chunk(const hr_ctx* ctx, int nshot, int fields = 2) {
   return tz;
 }
 
-// the outputs due, of the state x
-OutArgs take_outputs(hr_ctx* ctx) {
-  OutArgs O = ctx->out;
-  ctx->out = OutArgs{};
-  O.nshot = ctx->nshot;
-  O.x2 = ctx->x[1];
+// outputs of x2 (shots field_size apart) with nothing due yet
+OutArgs output_args(const hr_ctx* ctx, const double* x2, int nshot) {
+  OutArgs O{};
+  O.nshot = nshot;
+  O.x2 = x2;
   O.xstride = (long long)field_size(ctx);
   for (int d = 0; d < 3; ++d) { O.b0[d] = ctx->box0[d]; O.bn[d] = ctx->boxn[d]; }
   O.NX = ctx->g.NX; O.NY = ctx->g.NY;
@@ -604,17 +615,27 @@ OutArgs take_outputs(hr_ctx* ctx) {
   return O;
 }
 
-GradArgs take_gradient(hr_ctx* ctx) {
-  const GradArgs G = ctx->grad;
-  ctx->grad = GradArgs{};
-  return G;
+// the outputs due, of the state x
+OutArgs take_outputs(hr_ctx* ctx) {
+  OutArgs O = output_args(ctx, ctx->x[1], ctx->nshot);
+  if (ctx->due_row.full()) {
+    const TraceRow t = ctx->due_row.take();
+    O.nrec = ctx->f_nrec; O.slot = ctx->d_rec_slot;
+    O.row = t.row; O.rstride = t.rstride;
+  }
+  if (ctx->due_slice.full()) {
+    const Slice t = ctx->due_slice.take();
+    O.nbox = (int)ctx->nbox;
+    O.hist = t.hist; O.hstride = t.hstride;
+  }
+  return O;
 }
 
 // queue the outputs and the other deferred per-step work on the main stream (in the
 // order it was deferred)
 int run_deferred(hr_ctx* ctx) {
   HIPC(launch_outputs(take_outputs(ctx), ctx->stream));
-  HIPC(launch_gradient(take_gradient(ctx), ctx->stream));
+  HIPC(launch_gradient(ctx->due_grad.take(), ctx->stream));
   std::vector<std::function<int()>> work;
   work.swap(ctx->deferred);
   for (auto& f : work)
@@ -625,8 +646,9 @@ int run_deferred(hr_ctx* ctx) {
 // forget what a solve that stopped on an error left
 void drop_deferred(hr_ctx* ctx) {
   ctx->deferred.clear();
-  ctx->out = OutArgs{};
-  ctx->grad = GradArgs{};
+  ctx->due_row.drop();
+  ctx->due_slice.drop();
+  ctx->due_grad.drop();
 }
 
 int launch_stage(hr_ctx* ctx, StageArgs& A, const Src3Spec* sp = nullptr) {
@@ -754,7 +776,7 @@ int launch_stage(hr_ctx* ctx, StageArgs& A, const Src3Spec* sp = nullptr) {
         HIPC(launch_split_nodal(B, 0, A.transpose, ctx->cstream[0]));
         if (prof) HIPC(hipEventRecord(ev.end[1], ctx->cstream[0]));
         HIPC(hipEventRecord(ctx->ev_join[0], ctx->cstream[0]));
-        const bool side_work = !ctx->deferred.empty() || output_blocks(ctx->out) > 0 || gradient_blocks(ctx->grad) > 0;
+        const bool side_work = !ctx->deferred.empty() || ctx->due_row.full() || ctx->due_slice.full() || ctx->due_grad.full();
         if (side_work) {
           // the deferred kernels read the state the stage reads and write their
           // own outputs only; they queue on the context's stream, here the second side stream
@@ -770,12 +792,13 @@ int launch_stage(hr_ctx* ctx, StageArgs& A, const Src3Spec* sp = nullptr) {
         HIPC(hipStreamWaitEvent(ctx->stream, ctx->ev_join[0], 0));
         if (side_work) HIPC(hipStreamWaitEvent(ctx->stream, ctx->ev_join[1], 0));
       } else {
-        const OutArgs O = take_outputs(ctx);
+        OutArgs O{};
+        if (outputs_ride(A.stage)) O = take_outputs(ctx);
         // the gradient in the same launch where every block has its place at once, two
         // on a CU; in more rounds its registers would cost the other blocks more than
         // a launch (16x16x8 elements, 120 blocks: 126 -> 121 us forward and adjoint step)
         GradArgs G{};
-        if (A.stage == 1 && stage_pair_blocks(B, R) + gradient_blocks(ctx->grad) <= 512) G = take_gradient(ctx);
+        if (A.stage == 1 && stage_pair_blocks(B, R) + gradient_blocks(ctx->due_grad.get()) <= 512) G = ctx->due_grad.take();
         if (int rc = run_deferred(ctx)) return rc;
         if (prof) HIPC(hipEventRecord(ev.start[0], ctx->stream));
         if (elements) HIPC(launch_stage_pair(B, R, O, G, upd, A.transpose, ctx->stream));
@@ -952,22 +975,17 @@ int rk4_step(hr_ctx* ctx, double dt, int dir, int transpose, const double sgn[3]
 
 // The outputs of the state x that go with the coming launch, or now (put_outputs):
 // receiver traces of every shot at the start of step n
-void record_step(hr_ctx* ctx, int n) {
-  if (ctx->f_nrec <= 0) return;
-  OutArgs& O = ctx->out;
-  O.nrec = ctx->f_nrec;
-  O.slot = ctx->d_rec_slot;
-  O.row = ctx->d_traces + (size_t)n * ctx->f_nrec;
-  O.rstride = ((long long)ctx->f_nstep + 1) * ctx->f_nrec;
+int record_step(hr_ctx* ctx, int n) {
+  if (ctx->f_nrec <= 0) return 0;
+  const TraceRow t{ctx->d_traces + (size_t)n * ctx->f_nrec, ((long long)ctx->f_nstep + 1) * ctx->f_nrec};
+  return ctx->due_row.put(t) ? 0 : fail(ctx, 3, "a trace row is still due");
 }
 
 // regular-domain displacement of every shot into history row `row` of blocks of `rows` rows per shot
-void store_slice(hr_ctx* ctx, double* base, size_t rows, size_t row) {
-  OutArgs& O = ctx->out;
+int store_slice(hr_ctx* ctx, double* base, size_t rows, size_t row) {
   const size_t slice = 3 * (size_t)ctx->nbox;
-  O.nbox = (int)ctx->nbox;
-  O.hist = base + row * slice;
-  O.hstride = (long long)(rows * slice);
+  const Slice t{base + row * slice, (long long)(rows * slice)};
+  return ctx->due_slice.put(t) ? 0 : fail(ctx, 3, "a history slice is still due");
 }
 
 int put_outputs(hr_ctx* ctx) {
@@ -1042,13 +1060,13 @@ int run_forward_steps(hr_ctx* ctx, int n0, int n1, double* seg_hist, size_t seg_
   const double sgn[3] = {1.0, 1.0, 1.0};
   for (int n = n0; n < n1; ++n) {
     // the slice of the state at the start of step n, queued beside its stage 1
-    if (seg_hist) store_slice(ctx, seg_hist, seg_rows, (size_t)(n - n0));
+    if (seg_hist) if (int rc = store_slice(ctx, seg_hist, seg_rows, (size_t)(n - n0))) return rc;
     Src3Spec sp4[4];
     forward_sources(ctx, n, sp4);
     if (int rc = rk4_step(ctx, ctx->f_dt, +1, 0, sgn, sp4)) return rc;
   }
   if (seg_hist) {
-    store_slice(ctx, seg_hist, seg_rows, (size_t)(n1 - n0));
+    if (int rc = store_slice(ctx, seg_hist, seg_rows, (size_t)(n1 - n0))) return rc;
     if (int rc = put_outputs(ctx)) return rc;
   }
   return 0;
@@ -1780,10 +1798,10 @@ int forward_impl(hr_ctx* ctx, int nshot, int nstep, double dt, const double* fta
   if (scheme == 1) {
     ctx->e_rows = 0;
     // traces row n = u at the start of step n (n >= 1; row 0 is u_0 = 0), as U_Store(:, ISTEP)
-    record_step(ctx, 0);
+    if (int rc = record_step(ctx, 0)) return rc;
     if (int rc = put_outputs(ctx)) return rc;
     for (int n = 1; n <= nstep; ++n) {
-      record_step(ctx, n);
+      if (int rc = record_step(ctx, n)) return rc;
       if (int rc = put_outputs(ctx)) return rc;
       if (int rc = cd_step(ctx, dt, n - 1)) return rc;
     }
@@ -1821,14 +1839,14 @@ int forward_impl(hr_ctx* ctx, int nshot, int nstep, double dt, const double* fta
   };
   auto step_body = [&](int n) -> int {
     // traces and history slice of the state at the start of step n, queued beside its stage 1
-    record_step(ctx, n);
+    if (int rc = record_step(ctx, n)) return rc;
     if (ctx->e_rows && n % ctx->e_every == 0) ctx->deferred.push_back([energy_at, n]() { return energy_at(n); });
-    if (ctx->h_store) store_slice(ctx, ctx->d_hist, rows, (size_t)n);
+    if (ctx->h_store) if (int rc = store_slice(ctx, ctx->d_hist, rows, (size_t)n)) return rc;
     if (L > 0) {
       if (n % L == 0 && chain_slot[n / L] >= 0)
         if (int rc = snap_save(ctx, ctx->x, ctx->snap[chain_slot[n / L]], nshot)) return rc;
       if (n >= last0)
-        store_slice(ctx, ctx->d_seg, seg_rows, (size_t)(n - last0));
+        if (int rc = store_slice(ctx, ctx->d_seg, seg_rows, (size_t)(n - last0))) return rc;
     }
     Src3Spec sp4[4];
     forward_sources(ctx, n, sp4);
@@ -1841,10 +1859,10 @@ int forward_impl(hr_ctx* ctx, int nshot, int nstep, double dt, const double* fta
     for (int n = 0; n < nstep; ++n)
       if (int rc = step_body(n)) return rc;
   }
-  if (L > 0) store_slice(ctx, ctx->d_seg, seg_rows, (size_t)(nstep - last0));
-  record_step(ctx, nstep);
+  if (L > 0) if (int rc = store_slice(ctx, ctx->d_seg, seg_rows, (size_t)(nstep - last0))) return rc;
+  if (int rc = record_step(ctx, nstep)) return rc;
   if (ctx->e_rows && nstep % ctx->e_every == 0) if (int rc = energy_at(nstep)) return rc;
-  if (ctx->h_store) store_slice(ctx, ctx->d_hist, rows, (size_t)nstep);
+  if (ctx->h_store) if (int rc = store_slice(ctx, ctx->d_hist, rows, (size_t)nstep)) return rc;
   if (int rc = put_outputs(ctx)) return rc;
   if (traces && nrec) {
     HIPC(hipMemcpyAsync(traces, ctx->d_traces, (size_t)nshot * rows * nrec * sizeof(double),
@@ -1861,8 +1879,10 @@ extern "C" {
 int hr_forward_shots(hr_ctx* ctx, int nshot, int nstep, double dt, const double* ftab, int nsrc, const int* src_shot,
                      const long long* src_eq, const double* src_val, int nrec, const long long* rec_eq, double* traces,
                      int history, int segment) {
-  return forward_impl(ctx, nshot, nstep, dt, ftab, nsrc, src_shot, src_eq, src_val, nrec, rec_eq, traces, history,
-                      segment, 0);
+  const int rc = forward_impl(ctx, nshot, nstep, dt, ftab, nsrc, src_shot, src_eq, src_val, nrec, rec_eq, traces,
+                              history, segment, 0);
+  if (rc && ctx) drop_deferred(ctx);
+  return rc;
 }
 
 int hr_forward_cd(hr_ctx* ctx, int nstep, double dt, const double* ftab, int nsrc, const long long* src_eq,
@@ -1875,8 +1895,10 @@ int hr_forward_cd(hr_ctx* ctx, int nstep, double dt, const double* ftab, int nsr
   if (ctx->flags & HR_DEVICE_PTRS) HIPC(hipMemcpy(f.data(), ftab, nstep * sizeof(double), hipMemcpyDeviceToHost));
   else std::memcpy(f.data(), ftab, nstep * sizeof(double));
   for (int n = 0; n < nstep; ++n) t3[3 * (size_t)n] = (dt * dt) * f[n];
-  return forward_impl(ctx, 1, nstep, dt, t3.data(), nsrc, nullptr, src_eq, src_val, nrec, rec_eq, traces,
-                      HR_HISTORY_NONE, 1, 1);
+  const int rc = forward_impl(ctx, 1, nstep, dt, t3.data(), nsrc, nullptr, src_eq, src_val, nrec, rec_eq, traces,
+                              HR_HISTORY_NONE, 1, 1);
+  if (rc) drop_deferred(ctx);
+  return rc;
 }
 
 int hr_forward(hr_ctx* ctx, int nstep, double dt, const double* ftab, int nsrc, const long long* src_eq,
@@ -2057,8 +2079,9 @@ int hr_adjoint_gradient(hr_ctx* ctx, int nstep, double dt, int nrec, const long 
       // queued beside stage 1 of the adjoint step, which reads but does not write p
       double* const a1 = P[1];
       const StepRef sr{ctx->dyn ? ctx->d_step : nullptr, (long long)slice};
-      ctx->grad = gradient_args(ctx->g, ctx->box0, ctx->boxn, nshot, uh + uh_row * slice, (long long)(uh_rows * slice), a1,
-                                (long long)nf, dt, ctx->d_gl, ctx->d_gm, sr);
+      if (!ctx->due_grad.put(gradient_args(ctx->g, ctx->box0, ctx->boxn, nshot, uh + uh_row * slice,
+                                           (long long)(uh_rows * slice), a1, (long long)nf, dt, ctx->d_gl, ctx->d_gm, sr)))
+        return fail(ctx, 3, "a step's gradient is still due");
     }
     // misfit sources r(t_n), their mean with r(t_{n-1}) and r(t_{n-1}) over the step of
     // -dt: s1 = r(t_n), s2 = (r(t_n) - r(t_{n-1})) / dt, s4 = 0 (the mean is exact)
@@ -2301,9 +2324,7 @@ int hr_gradient_accumulate(hr_ctx* ctx, const double* u, const double* p, double
   if (int rc = dalloc(ctx, &ctx->d_uslice, 3 * (size_t)ctx->nbox)) return rc;
   if (int rc = dalloc(ctx, &ctx->d_gl, ctx->nbox)) return rc;
   if (int rc = dalloc(ctx, &ctx->d_gm, ctx->nbox)) return rc;
-  OutArgs O = take_outputs(ctx);         // none is due here
-  O.nshot = 1;
-  O.x2 = ctx->tmp;
+  OutArgs O = output_args(ctx, ctx->tmp, 1);
   O.nbox = (int)ctx->nbox;
   O.hist = ctx->d_uslice;
   HIPC(launch_outputs(O, ctx->stream));

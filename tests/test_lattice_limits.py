@@ -15,8 +15,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 
 
 @pytest.mark.skipif(shutil.which("g++") is None, reason="g++ absent")
-@pytest.mark.parametrize("check", ["index_check", "iface_check"])
-def test_addresses(check):
+@pytest.mark.parametrize("check", ["index_check", "iface_check", "due_check"])
+def test_host_check(check):
     with tempfile.TemporaryDirectory() as tmp:
         exe = os.path.join(tmp, "ic")
         subprocess.run(["g++", "-O1", "-std=c++17", os.path.join(HERE, "native", check + ".cpp"), "-o", exe], check=True)
