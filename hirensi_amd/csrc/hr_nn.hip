@@ -817,6 +817,7 @@ bool launch_conv(const float* in, const unsigned short* w, const float* bias, co
   const size_t lds = CK * sizeof(int) + 3 * (size_t)seg * (sizeof(int) + CCH * sizeof(short));
   if (lds > LDS_LIMIT) return false;
   const long long nblk = whole ? (g.NB + spb - 1) / spb : (long long)g.NB * ((pd.V + NCB - 1) / NCB);
+  if (nblk >= 1 << 24) return false;         // 2^32 threads, where a launch wraps without an error
   const dim3 grid((unsigned)nblk, (unsigned)((cout + COB - 1) / COB));
   conv3d_tile_kernel<MT, NT, WM><<<grid, 256, lds, st>>>(in, w, bias, ep, out, cin, cout, pd, NCB, (int)seg);
   return true;
@@ -825,7 +826,8 @@ bool launch_conv(const float* in, const unsigned short* w, const float* bias, co
 // The tile by output channels, then by whether the larger column range still
 // gives every CU a block (256).  Wider tiles reuse a lane's LDS reads: more output
 // channels per wavefront first (each read feeds MT matrix operations), more
-// columns where there are few.  False: the rows are too long for the staging.
+// columns where there are few.  False: the rows are too long for the staging, or the
+// blocks too many for one launch (the gather kernel has 64 columns a block).
 bool conv_tiled(const float* in, const unsigned short* w, const float* bias, const Epilogue& ep, float* out, int cin,
                 int cout, const Vol& g, hipStream_t st) {
   const Pad pd(g);

@@ -99,3 +99,27 @@ def test_weight_rows_at_every_alignment_give_the_same_bits(cin, cout, dims):
         assert L.hr_nn_conv3d(xd.data_ptr(), buf.data_ptr() + 2 * shift, None, y.data_ptr(), cin, cout, 2, *dims, 0, s) == 0
         out.append(y)
     assert torch.equal(out[0], out[1]) and torch.equal(out[0], out[2])
+
+
+def test_a_batch_of_more_blocks_than_a_tile_can_launch():
+    """16 columns a block (rows of 280, more than 32 output channels) pass the launch limit of 2^32
+    threads at 2^28 columns, 52 GB here; the gather kernel has four times as
+    many columns a block.  Samples of the batch against the same samples alone, whose tiles
+    give the same bits."""
+    from hirensi_amd import precond as PC
+    L, s = PC.lib(), torch.cuda.current_stream().cuda_stream
+    cin, cout, nb, dims = 16, 33, 235, (64, 64, 280)
+    print(f"conv of {nb} x {dims} voxels, {cin} -> {cout} channels", flush=True)
+    if torch.cuda.mem_get_info()[0] < 60 << 30:
+        pytest.skip("needs 60 GB of device memory")
+    assert nb * dims[0] * dims[1] * dims[2] > 1 << 28
+    x = torch.empty((nb, cin) + dims, device="cuda:0").uniform_(-1, 1)
+    w = bits(torch.randn(cout * cin * 27, generator=torch.Generator().manual_seed(1)))
+    y = torch.empty((nb, cout) + dims, device="cuda:0")
+    one = torch.empty((1, cout) + dims, device="cuda:0")
+    assert L.hr_nn_conv3d(x.data_ptr(), w.data_ptr(), None, y.data_ptr(), cin, cout, nb, *dims, 0, s) == 0
+    for q in (0, 117, nb - 1):
+        assert L.hr_nn_conv3d(x[q].data_ptr(), w.data_ptr(), None, one.data_ptr(), cin, cout, 1, *dims, 0, s) == 0
+        assert torch.equal(y[q], one[0]) and float(one.abs().max()) > 0, q
+    del x, y
+    torch.cuda.empty_cache()
