@@ -15,10 +15,10 @@
 //
 // The tiled kernels stage the input of a block's columns in LDS, as BF16 and
 // zero-padded, and read all 27 taps from there; the gather kernels read every
-// tap from memory, for volumes whose rows are too long for the staging.  Both
-// accumulate the same products in the same order (K ascending in steps of 16 for a
-// convolution, the columns of a slice in steps of 16 for the weight gradient), so
-// their results agree bit for bit.
+// tap from memory, for volumes whose rows are too long for the staging and for convolutions of
+// too few channels to pay for it.  Both accumulate the same products in the same order (K
+// ascending in steps of 16 for a convolution, the columns of a slice in steps of 16
+// for the weight gradient), so their results agree bit for bit.
 
 #include <hip/hip_runtime.h>
 #include <cstdint>
@@ -805,9 +805,32 @@ bool odd(int D, int H, int W) { return (D | H | W) & 1; }
 // ------------------------------------------------------------ tiled launches
 constexpr size_t LDS_LIMIT = 64 * 1024;
 
+// What became of a tile: launched, its rows too long for the staging, or the gather
+// kernel is the faster one, or the only one whose blocks (64 columns each) one launch holds
+enum class Tile { DONE, TOO_LONG, GATHER };
+
+// Whether a tile beats the gather kernel.  With whole chunks of 16 channels and four
+// weights a load it always does (714 random shapes: 1.1-10 times).  A chunk of fewer
+// channels is staged at the cost of a whole one, and rows of weights that are no multiple
+// of 8 bytes are read weight by weight; what the tile saves is K's gathers.  So the K
+// steps that a chunk brings are held against a bound that grows with the places staged per
+// column, less where the blocks do not fill the GPU twice and the staging's loads are
+// hidden worse by others of their kind than the gathers' chain.  1318 random shapes of such
+// channels, rows of 2-280: the tile runs at 0.22-3.4 times the gather kernel's rate, where it
+// is taken at 0.80-3.4, nine in ten above 1; where it is not, at most 1.2.  One channel on
+// 2 x 32 x 64 x 64 voxels, the network's first layer: 20 us gathered, 29 tiled; 12 -> 24
+// channels there 227 and 89; 8 -> 16 on 2 x 8 x 33 x 100 26 and 28.
+bool tile_pays(int cin, int cout, const unsigned short* w, double places, long long blocks, double least, double slope) {
+  if (cin >= CCH && (cin & 3) == 0 && ((size_t)w & 7) == 0) return true;
+  const int steps = (27 * cin + 15) / 16, chunks = (cin + CCH - 1) / CCH;
+  if (blocks < 512) slope *= 0.3;
+  if (cout <= 4) slope *= 0.5;             // most lanes have no weights to read
+  return steps >= chunks * (least + slope * std::max(0.0, places - 10.0));
+}
+
 template <int MT, int NT, int WM>
-bool launch_conv(const float* in, const unsigned short* w, const float* bias, const Epilogue& ep, float* out, int cin,
-                 int cout, const Vol& g, hipStream_t st) {
+Tile launch_conv(const float* in, const unsigned short* w, const float* bias, const Epilogue& ep, float* out, int cin,
+                 int cout, const Vol& g, hipStream_t st, double least, double slope) {
   constexpr int NCB = 16 * NT * (4 / WM), COB = 16 * MT * WM;
   const Pad pd(g);
   const bool whole = pd.V < NCB;             // blocks of whole samples
@@ -815,37 +838,41 @@ bool launch_conv(const float* in, const unsigned short* w, const float* bias, co
   long long span = whole ? (long long)spb * pd.vol : pd.span(NCB, NCB, false);
   const long long seg = span + 2 * (pd.row + 1);
   const size_t lds = CK * sizeof(int) + 3 * (size_t)seg * (sizeof(int) + CCH * sizeof(short));
-  if (lds > LDS_LIMIT) return false;
+  if (lds > LDS_LIMIT) return Tile::TOO_LONG;
   const long long nblk = whole ? (g.NB + spb - 1) / spb : (long long)g.NB * ((pd.V + NCB - 1) / NCB);
-  if (nblk >= 1 << 24) return false;         // 2^32 threads, where a launch wraps without an error
-  const dim3 grid((unsigned)nblk, (unsigned)((cout + COB - 1) / COB));
+  const int ny = (cout + COB - 1) / COB;
+  // 2^24 blocks are 2^32 threads, where a launch wraps without an error
+  if (nblk >= 1 << 24 || !tile_pays(cin, cout, w, 3.0 * seg / (whole ? spb * pd.V : NCB), nblk * ny, least, slope))
+    return Tile::GATHER;
+  const dim3 grid((unsigned)nblk, (unsigned)ny);
   conv3d_tile_kernel<MT, NT, WM><<<grid, 256, lds, st>>>(in, w, bias, ep, out, cin, cout, pd, NCB, (int)seg);
-  return true;
+  return Tile::DONE;
 }
 
 // The tile by output channels, then by whether the larger column range still
 // gives every CU a block (256).  Wider tiles reuse a lane's LDS reads: more output
 // channels per wavefront first (each read feeds MT matrix operations), more
-// columns where there are few.  False: the rows are too long for the staging, or the
-// blocks too many for one launch (the gather kernel has 64 columns a block).
+// columns where there are few.  False: the gather kernel's.
 bool conv_tiled(const float* in, const unsigned short* w, const float* bias, const Epilogue& ep, float* out, int cin,
                 int cout, const Vol& g, hipStream_t st) {
+  if (cin < 2) return false;               // fewer K steps than any tile's bound below
   const Pad pd(g);
   const long long V = g.n(), ncol = V * g.NB;
   if (V * cin * 2 >= (1ll << 31) || pd.vol >= 1 << 23) return false;   // 32-bit voxel offsets, 24-bit places
   const int cot = (cout + 15) / 16;
-  if (cot == 1) {
-    if (ncol >= 256 * 256 && launch_conv<1, 4, 1>(in, w, bias, ep, out, cin, cout, g, st)) return true;
-    return launch_conv<1, 1, 1>(in, w, bias, ep, out, cin, cout, g, st);
-  }
-  if (cot == 2) {
-    if (ncol >= 256 * 128 && launch_conv<1, 4, 1>(in, w, bias, ep, out, cin, cout, g, st)) return true;
-    return launch_conv<1, 1, 2>(in, w, bias, ep, out, cin, cout, g, st);
-  }
   const long long y = (cot + 3) / 4;
-  if (ncol * y >= 64 * 256 && launch_conv<4, 1, 1>(in, w, bias, ep, out, cin, cout, g, st)) return true;
-  if (ncol * y >= 32 * 256 && launch_conv<2, 1, 2>(in, w, bias, ep, out, cin, cout, g, st)) return true;
-  return launch_conv<1, 1, 4>(in, w, bias, ep, out, cin, cout, g, st);
+  Tile t = Tile::TOO_LONG;
+  if (cot <= 2) {
+    const double least = cout <= 4 ? 4.0 : (cot == 1 ? 7.0 : 6.0);
+    if (ncol >= (cot == 1 ? 256 * 256 : 256 * 128)) t = launch_conv<1, 4, 1>(in, w, bias, ep, out, cin, cout, g, st, least, 1.0);
+    if (t != Tile::TOO_LONG) return t == Tile::DONE;
+    if (cot == 1) return launch_conv<1, 1, 1>(in, w, bias, ep, out, cin, cout, g, st, 8.0, 1.0) == Tile::DONE;
+    return launch_conv<1, 1, 2>(in, w, bias, ep, out, cin, cout, g, st, 7.0, 0.8) == Tile::DONE;
+  }
+  if (ncol * y >= 64 * 256) t = launch_conv<4, 1, 1>(in, w, bias, ep, out, cin, cout, g, st, 22.0, 0.5);
+  if (t == Tile::TOO_LONG && ncol * y >= 32 * 256) t = launch_conv<2, 1, 2>(in, w, bias, ep, out, cin, cout, g, st, 9.0, 1.2);
+  if (t == Tile::TOO_LONG) t = launch_conv<1, 1, 4>(in, w, bias, ep, out, cin, cout, g, st, 6.0, 0.1);
+  return t == Tile::DONE;
 }
 
 bool wgrad_tiled(const float* in, const float* dy, float* part, float* db, int cin, int cout, const Vol& g, int cslice,

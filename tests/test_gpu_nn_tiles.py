@@ -101,6 +101,25 @@ def test_weight_rows_at_every_alignment_give_the_same_bits(cin, cout, dims):
     assert torch.equal(out[0], out[1]) and torch.equal(out[0], out[2])
 
 
+# channels on both sides of the rule that leaves a convolution of few of them to the gather kernel
+# (K steps against the staged places, for every tile), on narrow and wide rows and small and
+# large grids, and rows of weights at 2 and 8 bytes
+@pytest.mark.parametrize("cout,nb,dims", [(16, 1, (3, 5, 17)), (16, 4, (8, 33, 100)), (3, 4, (16, 8, 192)), (32, 4, (16, 16, 33)),
+                                          (24, 2, (4, 4, 136)), (40, 2, (4, 6, 9)), (40, 2, (8, 33, 24)), (64, 2, (16, 32, 32))])
+def test_convolutions_of_few_channels(cout, nb, dims):
+    from hirensi_amd import precond as PC
+    print(f"few channels cout={cout} nb={nb} dims={dims}", flush=True)
+    L, s = PC.lib(), torch.cuda.current_stream().cuda_stream
+    for cin in (1, 2, 3, 4, 5, 9, 12, 15, 16, 17, 20):
+        g = torch.Generator().manual_seed(cin * 17 + cout)
+        x, w = torch.randn((nb, cin) + dims, generator=g), torch.randn(cout, cin * 27, generator=g) / np.sqrt(27.0 * cin)
+        b = torch.randn(cout, generator=g)
+        xd, wd, bd = x.to("cuda:0"), bits(w), b.to("cuda:0")
+        y = torch.empty((nb, cout) + dims, device="cuda:0")
+        assert L.hr_nn_conv3d(xd.data_ptr(), wd.data_ptr(), bd.data_ptr(), y.data_ptr(), cin, cout, nb, *dims, 0, s) == 0
+        assert rel(y, F.conv3d(bf(x), bf(w).view(cout, cin, 3, 3, 3), b, padding=1)) < 1e-5, cin
+
+
 def test_a_batch_of_more_blocks_than_a_tile_can_launch():
     """16 columns a block (rows of 280, more than 32 output channels) pass the launch limit of 2^32
     threads at 2^28 columns, 52 GB here; the gather kernel has four times as
