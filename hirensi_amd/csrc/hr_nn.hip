@@ -887,6 +887,16 @@ bool wgrad_tiled(const float* in, const float* dy, float* part, float* db, int c
   const size_t lds = sizeof(short) * ((size_t)16 * MT * WROW + WU + (size_t)WCH * 3 * seg);
   if (lds > LDS_LIMIT || seg >= 65536) return false;
   const unsigned nx = (unsigned)((cin + WCH - 1) / WCH), ny = (unsigned)((cout + 16 * MT - 1) / (16 * MT));
+  // While few blocks are at work a slice's chunks come one after another, each as long as
+  // five steps of the gather kernel (three with half the rows of the output gradient, where
+  // a single chunk is as fast), so those that short slices or samples of few voxels
+  // cut shorter are left to it: 24 -> 64 channels on 8 x 48 voxels 37 us gathered, 49 tiled;
+  // 5 -> 64 on 32 voxels 7.0 and 10.8; 40 -> 32 on 8 x 16 15 and 30; but with 30 x 42
+  // blocks, 120 -> 64 on 8 x 336, 116 and 40.
+  const long long most = (V & 15) == 0 ? std::min<long long>(V, WU) : WU;
+  const long long chunks = (cslice + most - 1) / most + ((V & 15) == 0 && g.NB > 1 && cslice % V && V % cslice ? 1 : 0);
+  const long long steps = cslice / 16;
+  if ((long long)nx * ny * ns < 32 && (MT == 4 ? steps < 5 * chunks : MT == 2 && chunks > 1 && steps < 3 * chunks)) return false;
   const unsigned rows = ny * (unsigned)ns;
   const dim3 grid(nx + (db ? ((unsigned)cout + rows - 1) / rows : 0), ny, (unsigned)ns);
   if (ns > 65535) return false;

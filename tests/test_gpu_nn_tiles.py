@@ -120,6 +120,26 @@ def test_convolutions_of_few_channels(cout, nb, dims):
         assert rel(y, F.conv3d(bf(x), bf(w).view(cout, cin, 3, 3, 3), b, padding=1)) < 1e-5, cin
 
 
+@pytest.mark.parametrize("cin,cout,nb,dims,ns", [(24, 64, 8, (1, 3, 16), 1), (1, 64, 8, (3, 2, 16), 12), (3, 40, 5, (1, 1, 16), 2),
+                                                 (5, 33, 3, (4, 4, 4), 3), (5, 33, 3, (4, 4, 4), 1)])
+def test_weight_gradients_of_small_samples(cin, cout, nb, dims, ns):
+    """Samples that cut the staged chunks short, on both sides of the rule that leaves them to the
+    gather kernel."""
+    from hirensi_amd import precond as PC
+    print(f"weight gradient cin={cin} cout={cout} nb={nb} dims={dims} slices={ns}", flush=True)
+    L, s = PC.lib(), torch.cuda.current_stream().cuda_stream
+    g = torch.Generator().manual_seed(cin + 7 * cout)
+    x, dy = torch.randn((nb, cin) + dims, generator=g), torch.randn((nb, cout) + dims, generator=g)
+    xd, dyd = x.to("cuda:0"), dy.to("cuda:0")
+    dw, db = torch.empty(cout * cin * 27, device="cuda:0"), torch.empty(cout, device="cuda:0")
+    part = torch.empty(ns * dw.numel(), device="cuda:0")
+    assert L.hr_nn_conv3d_wgrad(xd.data_ptr(), dyd.data_ptr(), part.data_ptr(), ns, dw.data_ptr(), db.data_ptr(), cin,
+                                cout, nb, *dims, s) == 0
+    ref = torch.nn.grad.conv3d_weight(bf(x), (cout, cin, 3, 3, 3), bf(dy), padding=1).reshape(-1)
+    assert rel(dw, ref) < 1e-5
+    assert rel(db, dy.sum(dim=(0, 2, 3, 4))) < 1e-5
+
+
 def test_a_batch_of_more_blocks_than_a_tile_can_launch():
     """16 columns a block (rows of 280, more than 32 output channels) pass the launch limit of 2^32
     threads at 2^28 columns, 52 GB here; the gather kernel has four times as
