@@ -262,8 +262,9 @@ __device__ __forceinline__ void nodal_pass(const SplitArgs& A, const Entry& E, i
   // the x-line of the pull: side-scaled stencil over the x-neighbours' records.
   // The neighbour at lattice offset di (|di| <= 2) is at most |di| entries away
   // in the list (no PML node between, or one); one that is not a PML node (a
-  // regular-domain node) has no record, and offsets outside the lattice have zero
-  // coefficients.
+  // regular-domain node) has no record; offsets outside the lattice, and of an element that
+  // does not hold the node, have zero coefficients and are not read, so that a
+  // non-finite value reaches the nodes that share a PML element with it only.
   double cs0, cs1, cu[5];
   sp_side_scales(AX, AY, AZ, cs0, cs1);
   sp_stencil(AX.odd, cs0, cs1, cu);
@@ -274,7 +275,7 @@ __device__ __forceinline__ void nodal_pass(const SplitArgs& A, const Entry& E, i
     int slot = -1;
     if (di == 0) {
       slot = tid;
-    } else if (i + di >= 0 && i + di < g.NX) {
+    } else if (cu[d] != 0.0) {
       const unsigned ne = (unsigned)((int)n + di);
       const int near = tid + (di > 0 ? 1 : -1);
       if (di == 2 || di == -2) slot = sXn[tid + di] == ne ? tid + di : (sXn[near] == ne ? near : -1);
@@ -425,8 +426,6 @@ __device__ __forceinline__ void pull_pass(const SplitArgs& A, const Entry& E, in
   // M^-1 of the stress rows: 1 / (a W), a the stretch-factor product, W the PML weight sum
   const double minv_s = 1.0 / (((sax * say) * saz) * (g.detj * sp_pml_weight(ax3[0], ax3[1], ax3[2])));
   const double* const Dp = A.D + (long long)shot * 12 * g.NN;
-  const int cc[3] = {i, j, k};
-  const int nax[3] = {g.NX, g.NY, g.NZ};
   const int str[3] = {1, g.NX, g.NX * g.NY};
   // y- and z-lines (the x-line terms are in the node-local terms): per axis
   // su = sum_d cu[d] G_{.,ax}(n + (d - 2) str), sd the same with the s-row
@@ -444,9 +443,8 @@ __device__ __forceinline__ void pull_pass(const SplitArgs& A, const Entry& E, in
       // odd coordinates have no +-2 terms: skipped (a row of consecutive list
       // entries shares the y and z coordinates)
       if ((d == 0 || d == 4) && ax3[ax].odd) continue;
-      // offsets outside the lattice have zero coefficients: read the node itself
-      const int p = cc[ax] + d - 2;
-      const unsigned m = (p >= 0 && p < nax[ax]) ? (unsigned)((int)n + (d - 2) * str[ax]) : n;
+      // where the coefficient is zero (outside the lattice, among others) the node itself is read
+      const unsigned m = cu[d] != 0.0 ? (unsigned)((int)n + (d - 2) * str[ax]) : n;
       const unsigned o = d_rec(ax, NN, m);
       double G0, G1, G2, W0, W1, W2;
       ld2(Dp, o, G0, G1);

@@ -131,3 +131,27 @@ def test_tall_boxes(nez, tz):
     assert rel_l2(S.explicit_rk4_petsc_pml_3d(ctx, nstep, dt, tab, src, B[src], rec), ref) < 1e-10
     cd = so.cd_forward(B, nstep, dt, lcase=2, fr=fr)[:, rows]
     assert rel_l2(S.explicit_central_difference_3(ctx, nstep, dt, src, B[src], rec, 2, fr), cd) < 1e-10
+
+
+@pytest.mark.parametrize("shape,npml", [((7, 6, 5), (2, 1, 1, 2, 1)), ((6, 7, 5), (1, 4, 2, 2, 1))])
+def test_a_non_finite_entry_reaches_no_more_than_on_the_fused_kernel(shape, npml):
+    """Zero coefficients multiply nothing: entries of a product that a NaN or an infinity in
+    x makes non-finite on the split path are so on the fused kernel too (also around a
+    regular domain of one element)."""
+    mesh = BoxMesh(*shape, npml=npml)
+    model = random_model(mesh, seed=2)
+    rng = np.random.default_rng(3)
+    x, zero = rng.standard_normal(mesh.neq), np.zeros(mesh.neq)
+    print(f"non-finite entries {shape} npml={npml}", flush=True)
+    c4, c3 = S.Context(mesh, model), S.Context(mesh, model, version=3)
+    dofs = rng.choice(mesh.neq, 40, replace=False)
+    for which in (S.HR_K, S.HR_C, S.HR_G):
+        for tr in (False, True):
+            reached = 0                                # C and G do not reach regular-domain-only nodes
+            for q, d in enumerate(dofs):
+                xx = x.copy()
+                xx[d] = np.inf if q % 4 == 0 else np.nan
+                a, b = (~np.isfinite(S.ShellMat(c, which)._apply(tr, xx, zero, None)) for c in (c4, c3))
+                assert not (a & ~b).any(), (which, tr, d)
+                reached += b.any()
+            assert reached > len(dofs) // 2, (which, tr)
