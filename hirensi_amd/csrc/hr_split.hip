@@ -19,7 +19,7 @@
 // and the update, which leaves two element passes a step instead of four.
 // Against the stages on k1..k4 with four element passes (forward and adjoint, one
 // MI355X): 64x64x32 elements, PML 6: 0.68 -> 0.56 ms per step; 37x29x19: 0.31 -> 0.16;
-// 16x16x8: 0.23 -> 0.09; with the passes as below 0.50, 0.119 and 0.062.
+// 16x16x8: 0.23 -> 0.09; with the passes as below 0.49, 0.118 and 0.061.
 
 #include <hip/hip_runtime.h>
 #include "hr_gradient.h"
@@ -32,12 +32,10 @@
 namespace hr {
 namespace {
 
-// Blocks of consecutive PML nodes in lattice order (sp_pml_node), one node per
-// thread (nodal pull: SPLIT_NT nodes; nodal pass: SPLIT_OWN nodes and two on each
-// side).  XCD x = blockIdx % 8 takes the
-// logical blocks [x C, (x + 1) C) of the launch, so that each XCD's L2 holds a
-// contiguous run of the list (the neighbouring rows and planes of its nodes); a
-// launch has 8 C blocks and starts at logical block A.pb0.
+// Blocks of consecutive PML nodes in lattice order (sp_pml_node), one node per thread:
+// SPLIT_OWN nodes and two on each side.  XCD x = blockIdx % 8 takes the logical
+// blocks [x C, (x + 1) C) of the launch, so that each XCD's L2 holds a contiguous run of
+// the list (the neighbouring rows and planes of its nodes); a launch has 8 C blocks.
 __device__ __forceinline__ int split_block(int blk, int nblk) {
   const int C = (nblk + 7) / 8;
   return (blk & 7) * C + (blk >> 3);
@@ -426,6 +424,8 @@ __device__ __forceinline__ void pull_pass(const SplitArgs& A, const Entry& E, in
   // M^-1 of the stress rows: 1 / (a W), a the stretch-factor product, W the PML weight sum
   const double minv_s = 1.0 / (((sax * say) * saz) * (g.detj * sp_pml_weight(ax3[0], ax3[1], ax3[2])));
   const double* const Dp = A.D + (long long)shot * 12 * g.NN;
+  const int cc[3] = {i, j, k};
+  const int nax[3] = {g.NX, g.NY, g.NZ};
   const int str[3] = {1, g.NX, g.NX * g.NY};
   // y- and z-lines (the x-line terms are in the node-local terms): per axis
   // su = sum_d cu[d] G_{.,ax}(n + (d - 2) str), sd the same with the s-row
@@ -443,8 +443,13 @@ __device__ __forceinline__ void pull_pass(const SplitArgs& A, const Entry& E, in
       // odd coordinates have no +-2 terms: skipped (a row of consecutive list
       // entries shares the y and z coordinates)
       if ((d == 0 || d == 4) && ax3[ax].odd) continue;
-      // where the coefficient is zero (outside the lattice, among others) the node itself is read
-      const unsigned m = cu[d] != 0.0 ? (unsigned)((int)n + (d - 2) * str[ax]) : n;
+      // where the coefficient is zero the node itself is read: outside the lattice, and two
+      // nodes away across a regular-domain element (one away there is no record).  The
+      // product's pull is 2 % faster with addresses that do not wait for the
+      // coefficients, the stages' pulls 1 % slower
+      const int p = cc[ax] + d - 2;
+      const bool use = RAW ? p >= 0 && p < nax[ax] && ((d != 0 && d != 4) || cu[d] != 0.0) : cu[d] != 0.0;
+      const unsigned m = use ? (unsigned)((int)n + (d - 2) * str[ax]) : n;
       const unsigned o = d_rec(ax, NN, m);
       double G0, G1, G2, W0, W1, W2;
       ld2(Dp, o, G0, G1);
@@ -542,8 +547,8 @@ __global__ void __launch_bounds__(SPLIT_NT, 2) pml_pull_kernel(const SplitArgs A
 // the flux records of odd and even stages alternate.
 // Bytes bound the two passes; in one they move 592 a node and stage against 666, and 880
 // against 1010 in the last.  64x64x32 elements: stages 1-2 82 us, as before, 3-4 113
-// against 126 us; 96x96x48 per step 1.62 -> 1.53 ms; 16x16x8, where launches
-// count, 74 -> 64 us.  Three blocks per CU (six registers spilled) are 1-3 % slower, the next
+// against 126 us (80 and 105 since neighbours of zero coefficient are not read); 96x96x48 per
+// step 1.62 -> 1.53 ms; 16x16x8, where launches count, 74 -> 64 us.  Three blocks per CU (six registers spilled) are 1-3 % slower, the next
 // stage's other inputs loaded ahead of the pull no faster.
 template <bool LAST, bool TR>
 __global__ void __launch_bounds__(SPLIT_NT, 2) pull_nodal_kernel(const SplitArgs P, const SplitArgs N) {
