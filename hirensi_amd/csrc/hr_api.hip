@@ -700,7 +700,7 @@ int launch_stage(hr_ctx* ctx, StageArgs& A, const Src3Spec* sp = nullptr) {
         B.v[0] = A.in[0];
         B.out = B.a = A.out;
         B.node = ctx->d_node; B.tab = ctx->d_tab; B.minvu = ctx->d_minvu; B.rwp = ctx->d_rwp;
-        B.sc = 1.0;
+        B.sc = B.ss = 1.0;
         B.pnbn = ctx->pnblk;
         B.D = ctx->d_D[0];
         const int set = A.set_mask == 1 ? 0 : (A.set_mask == 2 ? 1 : 2);
@@ -737,6 +737,7 @@ int launch_stage(hr_ctx* ctx, StageArgs& A, const Src3Spec* sp = nullptr) {
       set_source(ctx, sp, B);
       B.h = A.h; B.h2 = A.hh; B.h3 = A.h6; B.h4 = A.h4;
       B.sc = last ? A.h4 : 1.0;
+      B.ss = last ? A.h : 1.0;
       B.pnbn = ctx->pnblk;
       // the flux records of odd and even stages alternate
       B.D = ctx->d_D[elements || !two ? 0 : 1];
@@ -993,7 +994,7 @@ int put_outputs(hr_ctx* ctx) {
   return 0;
 }
 
-// forward sources of step n: B values times s1, s2, s4 of the stages (stage 3 has none)
+// forward sources of step n: B values times s1, s2 and the last stage's (stage 3 has none)
 void forward_sources(hr_ctx* ctx, int n, Src3Spec sp4[4]) {
   for (int s = 0; s < 4; ++s) {
     sp4[s] = Src3Spec();
@@ -1705,13 +1706,12 @@ int forward_impl(hr_ctx* ctx, int nshot, int nstep, double dt, const double* fta
   if (dev && scheme == 0) HIPC(hipMemcpy(ctx->ftab.data(), ftab, nft * sizeof(double), hipMemcpyDeviceToHost));
   else std::memcpy(ctx->ftab.data(), ftab, nft * sizeof(double));
   if (scheme == 0) {
-    // f0, fm, f1 of a step -> the sources of stages 1, 2 and 4 (hr_split.hip).  The
-    // differences come first: where they vanish, a small dt cannot make 0 x inf of them
+    // f0, fm, f1 of a step -> the sources of stages 1, 2 and 4 (hr_split.hip)
     for (size_t q = 0; q < (size_t)nstep * nshot; ++q) {
       double* f = ctx->ftab.data() + 3 * q;
       const double f0 = f[0], fm = f[1], f1 = f[2];
       f[1] = 2.0 * (fm - f0) / dt;
-      f[2] = 4.0 * ((f0 - fm) + (f1 - fm)) / dt / dt / dt;
+      f[2] = ((f0 - fm) + (f1 - fm)) / 6.0;
     }
   }
   if (ctx->ftab_cap < nft) {

@@ -155,7 +155,7 @@ struct Src3 {                      // device-resident source entries of one solv
   const int* comp;                 // component 0..2
   const double* m;                 // M^-1 of that DOF
   const double* val;               // forward: B entries
-  const double* ftab;              // forward: time function f(T), f(T+dt/2), f(T+dt): nshot x nstep x 3
+  const double* ftab;              // forward: source factors of stages 1, 2 and 4 (f0, 2 (fm - f0) / dt, (f0 - 2 fm + f1) / 6): nshot x nstep x 3
   const double* tr;                // adjoint: traces per shot, (nstep+1) rows of nrec, columns in entry order
   const double* obs;               // adjoint: observations, same layout
   int nrec;                        // adjoint: entries per shot (shared receivers)
@@ -214,7 +214,7 @@ struct SplitArgs {
   int nshot;
   long long shot_stride;
   double h, h2, h3, h4;            // h, h^2/2, h^3/6, h^4/24
-  double sc;                       // scale of the stage's a in its output: 1, last stage h^4/24
+  double sc, ss;                   // scales of the stage's a in its output and of its source: 1, last stage h^4/24, h
   int pnbn;                        // blocks of the PML node list (SPLIT_OWN nodes each)
   double* D;                       // y- and z-line flux records, 12 NN doubles per shot
   const double* E;                 // regular-domain K sums of the interface nodes (sp_iface_column), 3 nif doubles per shot

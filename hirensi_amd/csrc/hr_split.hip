@@ -10,7 +10,8 @@
 //   a3 = L(x3, a1, a2),       a4 = L(a1, a2, a3) + s4,
 //   x1 += h x2 + h^2/2 x3 + h^3/6 a1 + h^4/24 a2        (x2, x3 likewise, from one
 //   component later), s1 = f0, s2 = 2 (fm - f0) / h, s4 = 4 (f0 - 2 fm + f1) / h^3
-// for the source at the start, middle and end of the step.  Expanding the
+// for the source at the start, middle and end of the step (s4 goes into x3 alone, as
+// h times (f0 - 2 fm + f1) / 6: neither 1 / h^3 nor h^4 is formed for it).  Expanding the
 // classical k1..k4 in powers of the operator gives the same polynomial in h, source
 // terms included, so the step is the reference's RK4 up to rounding; but a stage
 // reads three vectors instead of 3, 4, 5 and 6, and the last one the state
@@ -349,14 +350,14 @@ __device__ __forceinline__ void add_domain_sources(const SplitArgs& A, int q) {
   }
   double* const o = A.a + (long long)shot * A.shot_stride + 3 * n;
 #pragma unroll
-  for (int c = 0; c < 3; ++c) o[c] += A.sc * s[c];
+  for (int c = 0; c < 3; ++c) o[c] += A.ss * s[c];
 }
 
 // Pull of an RK4 stage at one PML node: the PML elements' terms from the flux
 // records along the y- and z-lines through the node (side-scaled 5-point
 // stencils; the x-line terms are in the node-local terms), the regular-domain K
 // sums of an interface node from E, the sources, then out = (node-local terms)
-// + sc (src - M^-1 sums), sc = 1, or h^4/24 in the last stage.  The blocks past
+// - sc (M^-1 sums) + ss src, sc = ss = 1, in the last stage h^4/24 and h.  The blocks past
 // the node blocks add the sources at regular-domain-only nodes.
 //
 // A block's source entries are evaluated by as many threads at once into LDS and
@@ -410,7 +411,7 @@ __device__ __forceinline__ void pull_pass(const SplitArgs& A, const Entry& E, in
                          sp_axis(k, g.nez, g.rlo[2], g.nez)};
   const bool iface = sp_iface(ax3[0], ax3[1], ax3[2]);
   double e3[3] = {0.0, 0.0, 0.0};
-  const unsigned eo = (iface ? 24u : 0u) * (iface_column(g, i, j) + iface_rim(g) * (unsigned)(k - 2 * g.rlo[2]));   // (a select costs two registers, and a wave per SIMD)
+  const unsigned eo = (iface ? 24u : 0u) * (iface_column(g, i, j) + iface_rim(g) * (unsigned)(k - 2 * g.rlo[2]));
   if (!RAW || A.E) ld3(A.E + (long long)shot * 3 * A.nif, eo, e3[0], e3[1], e3[2]);
   const int sdyn = (e1 > e0 && A.step_dev) ? *A.step_dev : 0;
   if (e1 > e0) {
@@ -515,7 +516,7 @@ __device__ __forceinline__ void pull_pass(const SplitArgs& A, const Entry& E, in
   for (int m = 0; m < 9; ++m) {
     const double minv = RAW ? -1.0 : (m < 3 ? minv_u : (m < 6 ? minv_s : 0.5 * minv_s));
     const double sv = m < 3 ? src[m] : 0.0;
-    out[m] = pre[m] + A.sc * (sv - minv * raw[m]);
+    out[m] = (pre[m] + A.sc * -(minv * raw[m])) + A.ss * sv;
   }
 }
 
@@ -899,7 +900,7 @@ __global__ void __launch_bounds__(SPLIT_NT, 2) element_kernel(const RdArgs A) {
 // Against launches of their own (on two streams from 37x29x19 up), forward and adjoint
 // step on average: 16x16x8 elements 84 -> 74 us,
 // 37x29x19 150 -> 131, 4 shots of 32x32x16 341 -> 317, 64x64x32 equal.
-// GRAD: the adjoint step's gradient sums as well, after the element blocks; their 236
+// GRAD: the adjoint step's gradient sums as well, after the element blocks; their 240
 // registers leave two blocks on a CU, so only where all blocks fit at once (see
 // the launch's caller).
 template <bool UPDATE, bool TR, bool GRAD>

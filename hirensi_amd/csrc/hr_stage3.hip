@@ -751,7 +751,7 @@ __global__ void __launch_bounds__(NT3, HAS_RD ? (HAS_PML ? 3 : 5) : (S == 1 ? 3 
               out[m] = gout;
             } else if constexpr (S == 4) {
               const int cm = (NS == 9) ? m : (m < 3 ? m : 0);
-              out[m] = c3o[cm] + A.h4 * gout;
+              out[m] = (c3o[cm] + A.h4 * -(minv * raw[m])) + A.h * src;   // the source's scale: hr_split.hip
             } else {
               const int cm = (NS == 9) ? m : (m < 3 ? m : 0);
               out[m] = c3o[cm] + gout;                        // u_{n+1}

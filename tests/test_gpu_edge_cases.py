@@ -68,3 +68,22 @@ def test_argument_errors_are_reported():
     # the context still works after the errors
     tr = S.explicit_rk4_petsc_pml_3d(ctx, nstep, dt, ftab, src_eq, src_val, rec_eq)
     assert np.isfinite(tr).all()
+
+
+@pytest.mark.parametrize("version", [4, 3])
+@pytest.mark.parametrize("dt", [1.0e-80, 1.0e-100])
+def test_time_steps_whose_fourth_power_underflows(version, dt):
+    """The stages' sources hold neither 1 / dt^3 nor dt^4."""
+    mesh, model, rec_eq, src_eq, src_val = small_case(seed=5)
+    nstep, fr = 5, 0.02 / dt
+    print(f"dt={dt} version={version}", flush=True)
+    B = np.zeros(mesh.neq)
+    np.add.at(B, src_eq, src_val)
+    pos = {int(e): r for r, e in enumerate(mesh.store_eq)}
+    ref = O.System(mesh, model).forward(B, nstep, dt, lcase=2, fr=fr)[:, [pos[int(e)] for e in rec_eq]]
+    ctx = S.Context(mesh, model, version=version)
+    tr = S.explicit_rk4_petsc_pml_3d(ctx, nstep, dt, S.time_table(nstep, dt, 2, fr), src_eq, src_val, rec_eq,
+                                     history=S.HR_HISTORY_NONE)
+    big = np.abs(ref).max()
+    assert big > 0
+    assert rel_l2(tr / big, ref / big) < 1e-10
