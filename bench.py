@@ -83,12 +83,12 @@ def step_bytes(neq, nnode):
 
 
 def stage_bytes(neq, nnode):
-    """Algorithmic bytes of one launch of the stage kernel for RK4 stage s:
-    stage s reads its 2+s input vectors (x1, x2, x3, g1..g_{s-1}), M^-1 and
-    lambda, mu; stages 1-3 write g_s; stage 4 writes the updated x1, x2, x3."""
+    """Algorithmic bytes of one launch of the fused stage kernel (version 3) for RK4
+    stage s: three vectors (of x1, x2, x3, a1, a2, a3, those from the s-th on), M^-1 and
+    lambda, mu read, a_s written; stage 4 reads x1, x2, x3 as well and writes them updated."""
     b = {}
     for s in (1, 2, 3, 4):
-        reads = (2 + s) * neq + neq + 2 * nnode
+        reads = (3 if s < 4 else 6) * neq + neq + 2 * nnode
         writes = neq if s < 4 else 3 * neq
         b[s] = 8.0 * (reads + writes)
     return b

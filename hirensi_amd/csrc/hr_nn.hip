@@ -226,7 +226,7 @@ __device__ __forceinline__ bf16x4 read4(const unsigned short* p, const int o[4])
 // tiles each.  K runs in steps of 16 over (channel, tap) as in the weights'
 // rows; the places of a step's operands come from a table over the CK entries of
 // a channel chunk.  Bounded by the staging's latency and, per step, five LDS reads a
-// lane (four of two bytes); the matrix cores are 5-20 % busy.  16 -> 16 channels on 8 x
+// lane (four of two bytes); the matrix cores are 3-8 % busy (counters).  16 -> 16 channels on 8 x
 // 16 x 32 x 32 voxels: 95 -> 23 us against the gather kernel, 128 -> 128 on 8 x 2 x 4 x
 // 4: 91 -> 23 us (216 dependent steps in 8 chunks); with weights read 16 bytes a lane, the
 // 64 -> 64 layers of a 32 x 64 x 64 volume's third level 22 -> 18 us (without any weight
